@@ -29,6 +29,31 @@ int hip_fail(hipError_t e, const char *what);
 constexpr int kBlock = 256;        // threads per workgroup for streaming kernels
 constexpr int kMaxRedBlocks = 2048; // partial sums per reduction
 
+// All a product needs to know about a 64-row slice of an operator with a
+// dictionary, in one cache line (one scalar load): the slot offsets; which
+// tuples its rows hold (b >= 0: tuple b in the lanes of `mask`, tuple a in
+// the others; b < 0: row r holds tuple a + dict_id[r]); up to two tail
+// entries, their columns, the position of the first value in the value
+// storage (0 where there is none: a valid one) and, in `flags`, their
+// number and lanes (two of one lane in their order); or, for more than two rows of one tail entry each
+// (number 3), `col` as the mask of their lanes.
+struct DictRec {
+    int32_t off[kStencilMaxW];
+    int32_t a, b;
+    uint64_t mask;
+    int32_t col[2];
+    int32_t pos;
+    uint32_t flags;  // bits 0-1: tail entries; 8-13 and 16-21: their lanes
+};
+// kDictFast: a full slice (64 rows of the operator) whose slots need no
+// clamp and whose tail the record describes.  kDictLine: slots 2, 3 and 4
+// of it are the offsets -1, 0 and 1.  kDictFree: slot 7 is unused (offset
+// 0, values 0).
+constexpr uint32_t kDictFast = 1u << 24, kDictFree = 1u << 25, kDictLine = 1u << 26;
+constexpr uint32_t kDictMany = 3u;
+constexpr int kDictLineW = 7;  // slots from which a slice can be one of these
+static_assert(sizeof(DictRec) == 64, "slice dictionary record layout");
+
 }  // namespace gip
 
 struct gip_ctx {
@@ -90,6 +115,17 @@ struct gip_mat {
     int32_t *d_sym_flag;
     uint64_t sym_version;  // val_version + 1 the symmetric values were made from (0: never)
     int32_t sym_ok;        // 1: in use, -1: the values are not symmetric
+    // dictionary of the slot values (gip_dict.hip): the distinct tuples of a
+    // row's slot values and diagonal, dict_n of them (0: none), current while
+    // dict_version == val_version + 1
+    int32_t dict_n;
+    uint64_t dict_version;
+    gip::DictRec *d_dict_rec;  // per slice: which tuples its rows hold
+    uint16_t *d_dict_id;       // per row, read for slices of more than two tuples
+    int32_t dict_ids;          // there are such slices
+    double *d_dict_tab, *d_dict_soa, *d_dict_diag;  // tuples, 8 per row of the table; slot by slot; a_ii
+    float *d_dict_tab32, *d_dict_soa32;
+    int32_t st_empty;  // stencil layout: some row has no entries
     // a_ii per row (the stored values of a DIAG operator), for Jacobi; for
     // the other layouts refreshed from d_diag_src (each row's last diagonal
     // entry's position in the value storage, -1 for none) when values change
@@ -108,6 +144,11 @@ int reduce_grid(int n);
 // a stencil operator's slot values; *ok is true when the PCG's product may
 // read them.  Allocates on first use.
 int mat_sym_prepare(gip_ctx *c, gip_mat *A, bool *ok);
+// Makes the dictionary of a stencil operator's slot values from its current
+// values where it pays (dict_n stays 0 otherwise), and frees it.
+int mat_dict_build(gip_ctx *c, gip_mat *A);
+void mat_dict_free(gip_mat *A);
+inline bool mat_dict_ok(const gip_mat *A) { return A->dict_n > 0 && A->dict_version == A->val_version + 1; }
 // Looks up the no-alloc PCG scratch array's address on `device` (current);
 // called once per device by gip_init.
 int pcg_scratch_setup(int device);

@@ -386,6 +386,22 @@ __global__ __launch_bounds__(kBlock) void k_iter_spmv_sym(EllView A, PcgDev d, c
     iter_spmv<W, false, true>(A, d, p);
 }
 
+// K1 with the slot values from the dictionary: a wavefront's partial goes to
+// its slice's place, as above, so the sums and their order are the same.
+template <int SW, int R>
+__global__ __launch_bounds__(kBlock) void k_iter_spmv_dict(EllView A, PcgDev d, const double *__restrict__ p) {
+    const int st = state_load(d.state);
+    dict_rows<R, SW, double, double>(
+        A, A.val, d.n, p, [](int) { return 0; },
+        [&](int row, bool ok, bool any, double sum, double own, int) {
+            if (st != ST_RUN) return;
+            if (ok && any) d.Ap[row] = sum;
+            if (ok && !any) sum = d.Ap[row];  // empty row: Ap keeps its value
+            const double acc = wave_sum_dpp(ok ? own * sum : 0.0);
+            if ((threadIdx.x & 63) == 0) d.chunk[row >> 6] = acc;
+        });
+}
+
 // The direction p_k = 1.0 s + beta p_{k-1} read at any column j of the
 // product, computed exactly as the direction update computes it on the
 // solved rows (:113, no contraction: the same bits); past the solved rows
@@ -966,6 +982,22 @@ __global__ __launch_bounds__(kBlock) void k_m_spmv_small(EllView A, PcgDev d, co
     m_spmv<W, true>(A, d, p);
 }
 
+// (as k_iter_spmv_dict)
+template <int SW, int R>
+__global__ __launch_bounds__(kBlock) void k_m_spmv_dict(EllView A, PcgDev d, const float *__restrict__ p) {
+    dict_rows<R, SW, float, float>(
+        A, A.val32, d.n, p, [](int) { return 0; },
+        [&](int row, bool ok, bool, float sum, float own, int) {
+            if (ok) d.Ap32[row] = sum;
+            const double acc = wave_sum_dpp(ok ? (double)own * (double)sum : 0.0);
+            const double sa = d.deflate ? wave_sum_dpp(ok ? (double)sum : 0.0) : 0.0;
+            if ((threadIdx.x & 63) == 0) {
+                d.chunk[row >> 6] = acc;
+                if (d.deflate) d.chunk_s[row >> 6] = sa;
+            }
+        });
+}
+
 template <bool SMALL>
 __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
     float *__restrict__ r = d.r32, *__restrict__ s = d.s32;
@@ -1505,6 +1537,13 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
         int rc = mat_sym_prepare(c, const_cast<gip_mat *>(A), &sym);
         if (rc) return rc;
     }
+    // the dictionary of its slot values, where the operator has one, before
+    // either form of the stored values; in FP32 from 2^21 rows on, below
+    // which the values stay in the caches (us per iteration without and with
+    // it: FP64 81^3 30.9 / 27.9, 97^3 37.9 / 31.5, 128^3 58.5 / 46.6, 256^3
+    // 423.7 / 324.1; mixed 97^3 31.5 / 32.3, 128^3 45.0 / 42.3, 256^3
+    // 250.8 / 211.1)
+    const bool dict = S->fold && A->st_w >= 7 && mat_dict_ok(A) && (!mixed || S->n >= 1 << 21);
     PcgDev d = make_dev(S, b, x, o->precond ? 1 : 0);
     EllView v = view(A);
     const int pollk = o->poll > 0 ? o->poll : 16;
@@ -1562,7 +1601,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                 if (S->fold && !S->rows) {
                     if (k > 0) k_iter_dir<<<S->grid, kBlock, 0, st>>>(d, S->p, k);
                     const bool smp = sample_begin(k);
-                    if (sym)
+                    if (dict)
+                        DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p);
+                    else if (sym)
                         SYM_LAUNCH(A, k_iter_spmv_sym, v, d, S->p);
                     else
                         DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, S->p);
@@ -1573,7 +1614,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                     // (partials: p.Ap in chunk, then r.s in chunk and r.r in chunk_s)
                     if (k > 0) k_iter_dir_rows<<<S->nchunk, kBlock, 0, st>>>(d, S->p, k);
                     const bool smp = sample_begin(k);
-                    if (sym)
+                    if (dict)
+                        DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p);
+                    else if (sym)
                         SYM_LAUNCH(A, k_iter_spmv_sym, v, d, S->p);
                     else
                         DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, S->p);
@@ -1627,7 +1670,10 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                 if (S->fold) {
                     if (k > 0) k_m_dir<<<S->grid, kBlock, 0, st>>>(d, S->p32, k, pending);
                     const bool smp = sample_begin(k);
-                    DISPATCH_WG(A, S->nchunk, k_m_spmv, v, d, S->p32);
+                    if (dict)
+                        DICT_LAUNCH(k_m_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p32);
+                    else
+                        DISPATCH_WG(A, S->nchunk, k_m_spmv, v, d, S->p32);
                     sample_end(smp);
                     k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
                     k_m_update<false><<<S->grid, kBlock, 0, st>>>(d, k);

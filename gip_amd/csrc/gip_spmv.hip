@@ -89,6 +89,34 @@ __global__ __launch_bounds__(kBlock) void k_stencil(EllView A, int nrows, const 
         y[out] = a * sum + b * y[out];
 }
 
+// The same products with the slot values from the dictionary.
+struct NoLoads {
+    __device__ int operator()(int) const { return 0; }
+};
+
+template <int MODE, int SW, int R>
+__global__ __launch_bounds__(kBlock) void k_stencil_dict(EllView A, int nrows, const double *__restrict__ x,
+                                                        double *__restrict__ y, double a, double b,
+                                                        const int32_t *__restrict__ scatter) {
+    dict_rows<R, SW, double, double>(A, A.val, nrows, x, NoLoads{}, [&](int row, bool ok, bool any, double sum, double, int) {
+        if (!ok || !any) return;
+        const int out = scatter ? scatter[row] : row;
+        if (MODE == 0)
+            y[out] = sum;
+        else
+            y[out] = a * sum + b * y[out];
+    });
+}
+
+template <int SW, int R>
+__global__ __launch_bounds__(kBlock) void k_stencil32_dict(EllView A, int nrows, const float *__restrict__ x,
+                                                          float *__restrict__ y) {
+    dict_rows<R, SW, float, float>(A, A.val32, nrows, x, NoLoads{},
+                                        [&](int row, bool ok, bool any, float sum, float, int) {
+                                            if (ok) y[row] = any ? sum : 0.0f;
+                                        });
+}
+
 template <int W>
 __global__ __launch_bounds__(kBlock) void k_stencil32(EllView A, int nrows, const float *__restrict__ x,
                                                      float *__restrict__ y) {
@@ -330,9 +358,16 @@ int spmv_launch(gip_ctx *c, const gip_mat *A, const double *x, double *y, double
 #undef GIP_ELL_CASE
     } else if (A->format == GIP_FMT_STENCIL) {
         const EllView v = view(A);
+        const bool dict = mat_dict_ok(A), two = dict_two(A->nrows);
 #define GIP_ST_CASE(Wc)                                                                   \
     case Wc:                                                                              \
-        if (mode == 0)                                                                    \
+        if (dict && mode == 0 && two)                                                     \
+            k_stencil_dict<0, -Wc, 2><<<(g + 1) / 2, kBlock, 0, st>>>(v, A->nrows, x, y, a, b, scatter); \
+        else if (dict && mode == 0)                                                       \
+            k_stencil_dict<0, -Wc, 1><<<g, kBlock, 0, st>>>(v, A->nrows, x, y, a, b, scatter); \
+        else if (dict)                                                                    \
+            k_stencil_dict<1, -Wc, 1><<<g, kBlock, 0, st>>>(v, A->nrows, x, y, a, b, scatter); \
+        else if (mode == 0)                                                               \
             k_stencil<0, Wc><<<g, kBlock, 0, st>>>(v, A->nrows, x, y, a, b, scatter);     \
         else                                                                              \
             k_stencil<1, Wc><<<g, kBlock, 0, st>>>(v, A->nrows, x, y, a, b, scatter);     \
@@ -393,6 +428,11 @@ int spmv32_launch(gip_ctx *c, const gip_mat *A, const float *x, float *y) {
         if (!A->d_ell_val32) return set_error(GIP_EINVAL, "operator has no FP32 values");
         const EllView v = view(A);
         const int g = nblocks(A->nrows);
+        if (mat_dict_ok(A) && A->st_w >= 7) {
+            DICT_LAUNCH(k_stencil32_dict, A->st_w, g, c->stream, v, A->nrows, x, y);
+            GIP_LAUNCH_CHECK("spmv32 kernel");
+            return GIP_OK;
+        }
         switch (-A->st_w) {
             case -7: k_stencil32<-7><<<g, kBlock, 0, c->stream>>>(v, A->nrows, x, y); break;
             case -8: k_stencil32<-8><<<g, kBlock, 0, c->stream>>>(v, A->nrows, x, y); break;
@@ -599,6 +639,8 @@ int gip_mat_create(gip_ctx *c, int32_t nrows, int32_t ncols, int32_t nnz, const 
         A->st_w = plan.w;
         A->st_tail_base = plan.tail_base;
         A->st_tail_nnz = (int32_t)plan.tcol.size();
+        for (const StencilHdr &h : plan.hdr)
+            if (h.empty) A->st_empty = 1;
         std::vector<double> sval((size_t)plan.stored, 0.0);
         for (int32_t j = 0; j < nnz; ++j) sval[(size_t)plan.pos[(size_t)j]] = val[j];
         rc = upload(c, &A->d_ell_val, sval.data(), sval.size());
@@ -640,7 +682,9 @@ int gip_mat_create(gip_ctx *c, int32_t nrows, int32_t ncols, int32_t nnz, const 
         hipError_t e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) rc = hip_fail(e, "gip_mat_create upload");
     }
+    if (!rc) rc = mat_dict_build(c, A);
     if (rc) {
+        mat_dict_free(A);
         free_mat_arrays(A);
         delete A;
         return rc;
@@ -654,6 +698,7 @@ int gip_mat_destroy(gip_mat *A) {
     hipSetDevice(A->ctx->device);
     hipStreamSynchronize(A->ctx->stream);
     if (A->transpose) gip_mat_destroy(A->transpose);
+    mat_dict_free(A);
     free_mat_arrays(A);
     delete A;
     return GIP_OK;
@@ -851,7 +896,9 @@ int gip_mat_set_values(gip_mat *A, const double *host) {
         if (A->d_val32) k_to_f32<<<nblocks(A->nnz), kBlock, 0, c->stream>>>(A->nnz, A->d_val, A->d_val32);
     }
     GIP_LAUNCH_CHECK("gip_mat_set_values");
-    return diag_refresh(c, A);
+    int rc = diag_refresh(c, A);
+    if (!rc && A->format == GIP_FMT_STENCIL) rc = mat_dict_build(c, A);
+    return rc;
 }
 
 int gip_mat_diag_inv(const gip_mat *A, double *dinv) {
@@ -998,6 +1045,7 @@ int gip_dcsrmv_t(gip_ctx *c, const gip_mat *Ac, const double *x, double *y, int3
     if (A->nnz) {
         k_refresh<<<nblocks(A->nnz), kBlock, 0, c->stream>>>(A->nnz, value_store(A), A->d_tsrc, value_store(T), A->d_tdst);
         GIP_LAUNCH_CHECK("gip_dcsrmv_t refresh");
+        ++T->val_version;  // what was made from earlier values is stale
     }
     if (ncols_out) {
         k_fill0<<<nblocks(ncols_out), kBlock, 0, c->stream>>>(ncols_out, y);

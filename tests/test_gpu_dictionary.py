@@ -1,0 +1,108 @@
+"""The dictionary of a stencil operator's slot values (gip_dict.hip): from
+2^18 rows on, an operator whose rows repeat a few value tuples is multiplied
+from the distinct tuples.  The values are the stored ones bit for bit, so
+every product must equal the CSR layout's bitwise: at the smallest size, on
+meshes whose lines fill slices (scalar tuples), straddle them (per-row ids)
+and end in a partial slice, for the operators of every shape, after changes
+of the values (made again, one value off, no repetition left, rebuilt on the
+device), and in FP32.
+"""
+import numpy as np
+import pytest
+
+from gip_amd import cavity, hip
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = hip.Device(0)
+    yield d
+    d.close()
+
+
+def _products(dev, A, C, seed, fp32=False):
+    """y = A x and y = a A x + b y over random x, both layouts, bitwise."""
+    rng = np.random.default_rng(seed)
+    m, n = A.cols_needed, A.nrows
+    dx = dev.to_device(rng.standard_normal(m))
+    y0 = rng.standard_normal(n)
+    for op in (lambda M, y: M.spmv(dx, y), lambda M, y: M.spmv_ab(dx, y, -1.25, 0.5)):
+        got, want = dev.to_device(y0), dev.to_device(y0)
+        op(A, got)
+        op(C, want)
+        assert np.array_equal(got.download(), want.download())
+    if fp32:
+        sx = dev.to_device(rng.standard_normal(m).astype(np.float32))
+        got, want = dev.array(n, np.float32), dev.array(n, np.float32)
+        A.spmv32(sx, got)
+        C.spmv32(sx, want)
+        assert np.array_equal(got.download(), want.download())
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 64), (64, 64, 63), (128, 64, 33), (63, 65, 67), (97, 97, 97),
+                                   (256, 32, 40), (129, 130, 16), (192, 48, 48)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("beta", [0.0, 1.5])
+def test_laplacian_products_bitwise(dev, shape, beta):
+    c = cavity.generate(*shape, beta=beta, gamma=1e-3, ops=cavity.OP_BITS["L"])
+    L = c.op("L")
+    print(f"[dictionary {shape} beta {beta}] rows {L.nrows}", flush=True)
+    A = hip.Matrix.from_csr(dev, L, fp32=True)
+    C = hip.Matrix.from_csr(dev, L, fmt=hip.FMT_CSR, fp32=True)
+    assert A.info()["format"] == hip.FMT_STENCIL
+    assert np.array_equal(A.values(), L.val)
+    _products(dev, A, C, 1, fp32=True)
+
+
+@pytest.mark.parametrize("n", [64, 72])
+def test_every_operator_bitwise(dev, n):
+    c = cavity.generate(n, gamma=1e-3)
+    for name in cavity.OPS:
+        op = c.op(name)
+        print(f"[dictionary {name} {n}^3] rows {op.nrows}", flush=True)
+        A, C = hip.Matrix.from_csr(dev, op), hip.Matrix.from_csr(dev, op, fmt=hip.FMT_CSR)
+        _products(dev, A, C, 2)
+        # the transposed product refreshes its operator's values on each call
+        if name in ("D", "Gx", "SO"):
+            x = dev.to_device(np.random.default_rng(3).standard_normal(A.nrows))
+            cols = max(A.cols_needed, C.cols_needed)
+            got, want = dev.array(cols), dev.array(cols)
+            for M, y in ((A, got), (C, want)):
+                M.spmv_t(x, y, cols)
+            assert np.array_equal(got.download(), want.download())
+            v = op.val * 1.5
+            A.set_values(v)
+            C.set_values(v)
+            for M, y in ((A, got), (C, want)):
+                M.spmv_t(x, y, cols)
+            assert np.array_equal(got.download(), want.download())
+        A.destroy()
+        C.destroy()
+
+
+@pytest.mark.parametrize("n", [64, 66])
+def test_changed_values(dev, n):
+    c = cavity.generate(n, gamma=1e-3)
+    L = c.op("L")
+    A = hip.Matrix.from_csr(dev, L, fp32=True)
+    C = hip.Matrix.from_csr(dev, L, fmt=hip.FMT_CSR, fp32=True)
+    rng = np.random.default_rng(4)
+    one = L.val.copy()
+    one[L.nnz // 2] = np.nextafter(one[L.nnz // 2], 0.0)
+    signs = np.where(rng.random(L.nnz) < 0.5, -0.0, L.val)  # zeros of both signs, many tuples
+    for v in (2.0 * L.val, one, rng.standard_normal(L.nnz), signs, L.val):
+        A.set_values(v)
+        C.set_values(v)
+        assert np.array_equal(A.values(), v)
+        _products(dev, A, C, 5, fp32=True)
+    # values rebuilt on the device by a product: the dictionary made before is stale
+    D = c.op("D")
+    A, C = hip.Matrix.from_csr(dev, D), hip.Matrix.from_csr(dev, D, fmt=hip.FMT_CSR)
+    E = hip.Matrix.from_csr(dev, c.op("Ec"))
+    mf = dev.to_device(rng.standard_normal(c.n_faces))
+    for M in (A, C):
+        E.spmv_vals(mf, M)
+    _products(dev, A, C, 6)
+    assert np.array_equal(A.values(), C.values())
