@@ -168,7 +168,8 @@ __global__ __launch_bounds__(kBlock) void k_dict_assign(DictTable T, int n, int 
                                                         const StencilTail *__restrict__ tail,
                                                         const StencilHdr *__restrict__ hdr,
                                                         const int32_t *__restrict__ tcol, int tail_base, int cmax,
-                                                        DictRec *__restrict__ rec, uint16_t *__restrict__ ids) {
+                                                        DictRec *__restrict__ rec, DictSel *__restrict__ sel,
+                                                        uint16_t *__restrict__ ids) {
     const int r = blockIdx.x * kBlock + threadIdx.x, sl = r >> 6, lane = r & 63;
     if (sl >= ns) return;  // whole wavefronts
     int id = -1;
@@ -256,6 +257,7 @@ __global__ __launch_bounds__(kBlock) void k_dict_assign(DictTable T, int n, int 
         if (w > 7 && q.off[7] == 0) q.flags |= kDictFree;
         if (b < 0) T.count[2] = -1;  // some slice needs its rows' ids
         rec[sl] = q;
+        sel[sl] = DictSel{a, b, mask};
     }
     if (bad) atomicOr(T.count + 1, 1);
 }
@@ -270,11 +272,12 @@ inline int blocks(int64_t n) { return (int)((n + kBlock - 1) / kBlock); }
 }  // namespace
 
 void mat_dict_free(gip_mat *A) {
-    void *ptrs[] = {A->d_dict_rec, A->d_dict_id, A->d_dict_tab, A->d_dict_soa, A->d_dict_diag, A->d_dict_tab32,
+    void *ptrs[] = {A->d_dict_rec, A->d_dict_sel, A->d_dict_id, A->d_dict_tab, A->d_dict_soa, A->d_dict_diag, A->d_dict_tab32,
                     A->d_dict_soa32};
     for (void *p : ptrs)
         if (p) hipFree(p);
     A->d_dict_rec = nullptr;
+    A->d_dict_sel = nullptr;
     A->d_dict_id = nullptr;
     A->d_dict_tab = A->d_dict_soa = A->d_dict_diag = nullptr;
     A->d_dict_tab32 = A->d_dict_soa32 = nullptr;
@@ -326,6 +329,7 @@ int mat_dict_build(gip_ctx *c, gip_mat *A) {
     };
     get(&d_rows, (size_t)nd);
     get(&A->d_dict_rec, (size_t)A->nslices);
+    get(&A->d_dict_sel, (size_t)A->nslices);
     get(&A->d_dict_id, (size_t)n);
     get(&A->d_dict_tab, (size_t)nd * 8);
     get(&A->d_dict_soa, (size_t)nd * w);
@@ -348,7 +352,7 @@ int mat_dict_build(gip_ctx *c, gip_mat *A) {
             k_dict_assign<<<blocks((int64_t)A->nslices * 64), kBlock, 0, st>>>(
                 T, n, A->nslices, nd, w, A->d_ell_val, A->d_diag, A->d_dict_tab, A->d_dict_diag, A->d_st_off,
                 A->d_st_tail, A->d_st_hdr, A->d_st_tcol, (int)A->st_tail_base, std::max(0, A->cols_needed - 1), A->d_dict_rec,
-                A->d_dict_id);
+                A->d_dict_sel, A->d_dict_id);
             if (A->d_dict_tab32) {
                 k_dict_f32<<<blocks((int64_t)nd * 8), kBlock, 0, st>>>((int64_t)nd * 8, A->d_dict_tab, A->d_dict_tab32);
                 k_dict_f32<<<blocks((int64_t)nd * w), kBlock, 0, st>>>((int64_t)nd * w, A->d_dict_soa, A->d_dict_soa32);

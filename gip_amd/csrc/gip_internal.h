@@ -45,6 +45,12 @@ struct DictRec {
     int32_t pos;
     uint32_t flags;  // bits 0-1: tail entries; 8-13 and 16-21: their lanes
 };
+// The tuples of a slice alone, for the sweeps that need only the diagonal's
+// (the four slices of a workgroup's chunk share a cache line).
+struct DictSel {
+    int32_t a, b;
+    uint64_t mask;
+};
 // kDictFast: a full slice (64 rows of the operator) whose slots need no
 // clamp and whose tail the record describes.  kDictLine: slots 2, 3 and 4
 // of it are the offsets -1, 0 and 1.  kDictFree: slot 7 is unused (offset
@@ -121,6 +127,7 @@ struct gip_mat {
     int32_t dict_n;
     uint64_t dict_version;
     gip::DictRec *d_dict_rec;  // per slice: which tuples its rows hold
+    gip::DictSel *d_dict_sel;
     uint16_t *d_dict_id;       // per row, read for slices of more than two tuples
     int32_t dict_ids;          // there are such slices
     double *d_dict_tab, *d_dict_soa, *d_dict_diag;  // tuples, 8 per row of the table; slot by slot; a_ii

@@ -118,6 +118,11 @@ struct PcgDev {
     double *part;  // P_COUNT x kMaxRedBlocks partials; each array has one
                    // producer grid size and stays zero past it
     int precond;
+    // the Jacobi inverse per tuple of the operator's dictionary (LEAN sweeps)
+    const DictSel *dc_sel;
+    const uint16_t *dc_id;
+    const double *ddinv;
+    const float *ddinv32;
     __device__ double *P(int k) const { return part + k * kMaxRedBlocks; }
 };
 
@@ -190,6 +195,21 @@ __device__ inline double *sa_part(const PcgDev &d, int k) { return d.P((k & 1) ?
 __device__ inline bool deflating(const PcgDev &d, double zaz) { return d.deflate && zaz > 0.0 && isfinite(zaz); }
 __device__ inline double m_denom(double dn, double sap, double zaz, bool dfl) {
     return dfl ? dn - sap * sap / zaz : dn;
+}
+
+// LEAN sweeps (long iterations on an operator with a dictionary): the
+// preconditioned residual s = Dinv r is not stored.  The direction sweep
+// reads r instead of s and forms it again, with the inverse diagonal from
+// the dictionary, so the update writes r alone: two vector streams of its
+// five less.  The same expression on the same values: the same bits.
+__device__ inline double s_of(const PcgDev &d, int row, double r) {
+    if (!d.precond) return r;
+    double si = 0.0;
+    si = si + r * dict_one(d.dc_sel, d.dc_id, d.ddinv, row);  // :99-105
+    return si;
+}
+__device__ inline float s_of(const PcgDev &d, int row, float r) {
+    return d.precond ? r * dict_one(d.dc_sel, d.dc_id, d.ddinv32, row) : r;
 }
 
 // ---- setup ---------------------------------------------------------------
@@ -599,9 +619,10 @@ constexpr int kRowsMin = 1 << 23;
 
 // K0 (k >= 1): rho_k, the convergence test, x += alpha_{k-1} p,
 // beta, p = 1.0 s + beta p
+template <bool LEAN>
 __global__ __launch_bounds__(kBlock) void k_iter_dir(PcgDev d, double *__restrict__ p, int k) {
     double *__restrict__ x = d.x;
-    const double *__restrict__ s = d.s;
+    const double *__restrict__ s = LEAN ? d.r : d.s;
     const int st = state_load(d.state);
     if (st != ST_RUN && st != conv_stamp(k)) return;
     const double rho = sum_partials<RED_SUM>(d.P(P_RS), d.G);  // :107
@@ -618,7 +639,8 @@ __global__ __launch_bounds__(kBlock) void k_iter_dir(PcgDev d, double *__restric
     const double beta = rho / rho_slot(d, k - 1);  // :109
     if (leader()) d.sc[S_RHO0 + (k & 1)] = rho;
     FOR_ROWS(d.n, row) {
-        const double xo = x[row], si = s[row], po = p[row];
+        const double xo = x[row], sr = s[row], po = p[row];
+        const double si = LEAN ? s_of(d, row, sr) : sr;
         x[row] = xo + alpha * po;       // :95 of iteration k-1
         p[row] = 1.0 * si + beta * po;  // :113
     }
@@ -627,6 +649,7 @@ __global__ __launch_bounds__(kBlock) void k_iter_dir(PcgDev d, double *__restric
 // K2: alpha_k from the folded p.Ap partials, r += (-alpha) Ap, s = Dinv r,
 // partials of r.s and r.r (one per workgroup); each row's operands are
 // loaded together (one round trip per row)
+template <bool LEAN>
 __global__ __launch_bounds__(kBlock) void k_iter_update_grid(PcgDev d, int k) {
     if (!running(d)) return;
     double *__restrict__ r = d.r, *__restrict__ s = d.s;
@@ -648,17 +671,19 @@ __global__ __launch_bounds__(kBlock) void k_iter_update_grid(PcgDev d, int k) {
     double rs = 0.0, rr = 0.0;
     FOR_ROWS(d.n, row) {
         const double ro = r[row], apr = Ap[row];
-        const double di = precond ? dinv[row] : 0.0;
+        const double di = precond && !LEAN ? dinv[row] : 0.0;
         const double ri = ro + malpha * apr;  // :97
         r[row] = ri;
         double si;
-        if (precond) {  // :99-105
+        if (LEAN) {
+            si = s_of(d, row, ri);
+        } else if (precond) {  // :99-105
             si = 0.0;
             si = si + ri * di;
         } else {
             si = ri;
         }
-        s[row] = si;
+        if (!LEAN) s[row] = si;
         rs = rs + ri * si;
         rr = rr + ri * ri;
     }
@@ -691,6 +716,7 @@ __device__ inline double ntload(const double *p) { return __builtin_nontemporal_
 __device__ inline void ntstore(double *p, double v) { __builtin_nontemporal_store(v, p); }
 
 // K0 of iteration k >= 1
+template <bool LEAN>
 __global__ __launch_bounds__(kBlock) void k_iter_dir_rows(PcgDev d, double *__restrict__ p, int k) {
     const int st = state_load(d.state);
     const int row = blockIdx.x * kBlock + threadIdx.x;
@@ -705,7 +731,8 @@ __global__ __launch_bounds__(kBlock) void k_iter_dir_rows(PcgDev d, double *__re
     const double beta = d.sc[S_BETA];
     // nontemporal accesses: each array is streamed once per sweep (a plain
     // stream of this mix runs 8% faster with them on this device)
-    const double xo = ntload(x + row), si = ntload(d.s + row), po = ntload(p + row);
+    const double xo = ntload(x + row), sr = ntload((LEAN ? d.r : d.s) + row), po = ntload(p + row);
+    const double si = LEAN ? s_of(d, row, sr) : sr;
     ntstore(x + row, xo + alpha * po);       // :95 of iteration k-1
     ntstore(p + row, 1.0 * si + beta * po);  // :113
 }
@@ -748,6 +775,7 @@ __global__ __launch_bounds__(kBlock) void k_alpha_fin(PcgDev d, int k) {
 }
 
 // K2 of iteration k
+template <bool LEAN>
 __global__ __launch_bounds__(kBlock) void k_iter_update_rows(PcgDev d, int k) {
     if (!running(d)) return;
     const int row = blockIdx.x * kBlock + threadIdx.x;
@@ -755,17 +783,19 @@ __global__ __launch_bounds__(kBlock) void k_iter_update_rows(PcgDev d, int k) {
     double rs = 0.0, rr = 0.0;
     if (row < d.n) {
         const double ro = ntload(d.r + row), apr = ntload(d.Ap + row);
-        const double di = d.precond ? ntload(d.dinv + row) : 0.0;
+        const double di = d.precond && !LEAN ? ntload(d.dinv + row) : 0.0;
         const double ri = ro + malpha * apr;  // :97
         ntstore(d.r + row, ri);
         double si;
-        if (d.precond) {  // :99-105
+        if (LEAN) {
+            si = s_of(d, row, ri);
+        } else if (d.precond) {  // :99-105
             si = 0.0;
             si = si + ri * di;
         } else {
             si = ri;
         }
-        ntstore(d.s + row, si);
+        if (!LEAN) ntstore(d.s + row, si);
         rs = ri * si;
         rr = ri * ri;
     }
@@ -833,9 +863,10 @@ __global__ __launch_bounds__(kBlock) void k_fin(PcgDev d) {
 // K0 (k >= 1): rho_k, the correction update xc += alpha_{k-1} p of the
 // previous iteration (`pending`: not yet folded by a defect correction),
 // beta (0 after a restart: the previous rho slot is +inf), p32 = s32 + beta p32
+template <bool LEAN>
 __global__ __launch_bounds__(kBlock) void k_m_dir(PcgDev d, float *__restrict__ p, int k, int pending) {
     float *__restrict__ xc = d.xc32;
-    const float *__restrict__ s = d.s32;
+    const float *__restrict__ s = LEAN ? d.r32 : d.s32;
     if (!running(d)) return;
     const double rho = sum_partials<RED_SUM>(d.P(P_RS), d.G);
     const float a32 = pending ? (float)alpha_slot(d, k - 1) : 0.0f;  // alpha_{k-1}, as K2 of k-1 formed it
@@ -845,8 +876,9 @@ __global__ __launch_bounds__(kBlock) void k_m_dir(PcgDev d, float *__restrict__ 
     // solve at 256^3 over four runs: 392-394 ms with them, 403-405 without;
     // the sweeps' own times are unchanged within noise)
     FOR_ROWS(d.n, row) {
-        const float xo = __builtin_nontemporal_load(xc + row), si = __builtin_nontemporal_load(s + row),
+        const float xo = __builtin_nontemporal_load(xc + row), sr = __builtin_nontemporal_load(s + row),
                     po = __builtin_nontemporal_load(p + row);
+        const float si = LEAN ? s_of(d, row, sr) : sr;
         if (pending) __builtin_nontemporal_store(xo + a32 * po, xc + row);
         __builtin_nontemporal_store(si + beta * po, p + row);
     }
@@ -998,7 +1030,7 @@ __global__ __launch_bounds__(kBlock) void k_m_spmv_dict(EllView A, PcgDev d, con
         });
 }
 
-template <bool SMALL>
+template <bool SMALL, bool LEAN = false>
 __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
     float *__restrict__ r = d.r32, *__restrict__ s = d.s32;
     const float *__restrict__ Ap = d.Ap32, *__restrict__ dinv = d.dinv32;
@@ -1044,7 +1076,7 @@ __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
         FOR_ROWS(d.n, row) {
             // every operand first, so the row costs one memory round trip
             const float ro = __builtin_nontemporal_load(r + row), apr = __builtin_nontemporal_load(Ap + row);
-            const float di = precond ? __builtin_nontemporal_load(dinv + row) : 0.0f;
+            const float di = precond && !LEAN ? __builtin_nontemporal_load(dinv + row) : 0.0f;
             float azr = 0.0f;
             if (dfl && !listed) {
                 azr = az[row];
@@ -1062,8 +1094,8 @@ __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
             const float wr = dfl ? apr - c32 * azr : apr;  // (P A p)_row
             const float ri = ro - a32 * wr;
             __builtin_nontemporal_store(ri, r + row);
-            const float si = precond ? ri * di : ri;
-            __builtin_nontemporal_store(si, s + row);
+            const float si = LEAN ? s_of(d, row, ri) : precond ? ri * di : ri;
+            if (!LEAN) __builtin_nontemporal_store(si, s + row);
             rs = rs + (double)ri * (double)si;
             rr = rr + (double)ri * (double)ri;
         }
@@ -1221,6 +1253,15 @@ __global__ __launch_bounds__(kBlock) void k_to32(int n, const double *__restrict
     if (i < n) b[i] = (float)a[i];
 }
 
+__global__ __launch_bounds__(kBlock) void k_tuple_inv(int n, const double *__restrict__ diag, double *__restrict__ inv,
+                                                      float *__restrict__ inv32) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const double v = 1.0 / diag[i];
+    inv[i] = v;
+    inv32[i] = (float)v;
+}
+
 // z = 1 on rows [0, n), 0 on [n, n_all); az = 0 on [0, n)
 __global__ __launch_bounds__(kBlock) void k_ones(int n, int n_all, double *__restrict__ z, double *__restrict__ az,
                                                  AzList *azl) {
@@ -1298,6 +1339,9 @@ struct gip_pcg {
     float *r32, *p32, *s32, *Ap32, *xc32, *dinv32;
     double *p2;   // second direction buffer of the fused iteration (small operators)
     float *p32b;  // its FP32 counterpart
+    double *ddinv;   // the Jacobi inverse per tuple of the operator's dictionary
+    float *ddinv32;  // (FP64, FP32), made from dictionary `dict_version`
+    uint64_t dict_version;
     double *az;   // A 1 (MIXED coarse step)
     float *az32;  // its FP32 copy (MIXED deflation)
     AzList *azl;  // the FP32 copy's nonzeros, when few
@@ -1345,6 +1389,14 @@ static int pcg_grid(int n) {
             KERNEL<-8><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__);                    \
     } while (0)
 
+#define LEAN_LAUNCH(KERNEL, GRID, ...)                                                \
+    do {                                                                              \
+        if (lean)                                                                     \
+            KERNEL<true><<<GRID, kBlock, 0, st>>>(__VA_ARGS__);                       \
+        else                                                                          \
+            KERNEL<false><<<GRID, kBlock, 0, st>>>(__VA_ARGS__);                      \
+    } while (0)
+
 static PcgDev make_dev(gip_pcg *S, const double *b, double *x, int precond) {
     PcgDev d;
     d.n = S->n;
@@ -1373,6 +1425,10 @@ static PcgDev make_dev(gip_pcg *S, const double *b, double *x, int precond) {
     d.iters = S->state + 1;
     d.part = S->part;
     d.precond = precond;
+    d.dc_sel = S->A->d_dict_sel;
+    d.dc_id = S->A->d_dict_id;
+    d.ddinv = S->ddinv;
+    d.ddinv32 = S->ddinv32;
     return d;
 }
 
@@ -1431,6 +1487,18 @@ int gip_pcg_create(gip_ctx *c, const gip_mat *A, int32_t n_all, gip_pcg **out) {
         return rc;
     }
     int rc = A->diag_missing ? GIP_OK : gip_mat_diag_inv(A, S->dinv);
+    if (!rc && S->fold && mat_dict_ok(A)) {
+        // the same inverse, once per tuple (the diagonal is part of the tuple)
+        const int nd = A->dict_n;
+        e = hipMalloc((void **)&S->ddinv, (size_t)nd * 8);
+        if (e == hipSuccess) e = hipMalloc((void **)&S->ddinv32, (size_t)nd * 4);
+        if (e == hipSuccess) {
+            k_tuple_inv<<<(nd + kBlock - 1) / kBlock, kBlock, 0, c->stream>>>(nd, A->d_dict_diag, S->ddinv, S->ddinv32);
+            e = hipGetLastError();
+            S->dict_version = A->dict_version;
+        }
+        if (e != hipSuccess) rc = hip_fail(e, "gip_pcg_create dictionary");
+    }
     if (!rc) {
         e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) rc = hip_fail(e, "gip_pcg_create sync");
@@ -1448,7 +1516,8 @@ int gip_pcg_destroy(gip_pcg *S) {
     hipSetDevice(S->ctx->device);
     hipStreamSynchronize(S->ctx->stream);
     void *ptrs[] = {S->r,    S->p,      S->s,  S->Ap, S->dinv, S->r32,   S->p32,  S->s32,  S->Ap32,
-                    S->xc32, S->dinv32, S->az, S->sc, S->part, S->chunk, S->state, S->p2, S->p32b, S->az32, S->azl};
+                    S->xc32, S->dinv32, S->az, S->sc, S->part, S->chunk, S->state, S->p2, S->p32b, S->az32, S->azl,
+                    S->ddinv, S->ddinv32};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (S->h_state) hipHostFree(S->h_state);
@@ -1544,6 +1613,14 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     // 423.7 / 324.1; mixed 97^3 31.5 / 32.3, 128^3 45.0 / 42.3, 256^3
     // 250.8 / 211.1)
     const bool dict = S->fold && A->st_w >= 7 && mat_dict_ok(A) && (!mixed || S->n >= 1 << 21);
+    // ... and its inverse diagonal, while the solver's (taken when it was
+    // created) is the one of the operator's present values.  us per
+    // iteration with s stored and not: FP64 128^3 46.6 / 43.5, 200^3 195 /
+    // 165, 256^3 324 / 300; mixed 256^3 211 / 197, but 200^3 117 / 122: where
+    // slices need their rows' ids, those and the record cost the FP32 sweeps
+    // what s and Dinv did.
+    const bool lean = dict && (!mixed || !A->dict_ids) &&
+                      (!o->precond || (S->ddinv && S->dict_version == A->dict_version));
     PcgDev d = make_dev(S, b, x, o->precond ? 1 : 0);
     EllView v = view(A);
     const int pollk = o->poll > 0 ? o->poll : 16;
@@ -1599,7 +1676,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             int chunk = std::min(fixed ? 4096 : pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold && !S->rows) {
-                    if (k > 0) k_iter_dir<<<S->grid, kBlock, 0, st>>>(d, S->p, k);
+                    if (k > 0) LEAN_LAUNCH(k_iter_dir, S->grid, d, S->p, k);
                     const bool smp = sample_begin(k);
                     if (dict)
                         DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p);
@@ -1609,10 +1686,10 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                         DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, S->p);
                     sample_end(smp);
                     k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
-                    k_iter_update_grid<<<S->grid, kBlock, 0, st>>>(d, k);
+                    LEAN_LAUNCH(k_iter_update_grid, S->grid, d, k);
                 } else if (S->fold) {
                     // (partials: p.Ap in chunk, then r.s in chunk and r.r in chunk_s)
-                    if (k > 0) k_iter_dir_rows<<<S->nchunk, kBlock, 0, st>>>(d, S->p, k);
+                    if (k > 0) LEAN_LAUNCH(k_iter_dir_rows, S->nchunk, d, S->p, k);
                     const bool smp = sample_begin(k);
                     if (dict)
                         DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p);
@@ -1623,7 +1700,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                     sample_end(smp);
                     k_fold_two<<<S->gdn, kBlock, 0, st>>>(d, d.chunk, nullptr, P_DN, P_DN);
                     k_alpha_fin<<<1, kBlock, 0, st>>>(d, k);
-                    k_iter_update_rows<<<S->nchunk, kBlock, 0, st>>>(d, k);
+                    LEAN_LAUNCH(k_iter_update_rows, S->nchunk, d, k);
                     k_fold_two<<<S->gdn, kBlock, 0, st>>>(d, d.chunk, d.chunk_s, P_RS, P_RR);
                     k_beta_fin<<<1, kBlock, 0, st>>>(d, k + 1);
                 } else {
@@ -1668,7 +1745,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             int chunk = std::min(pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold) {
-                    if (k > 0) k_m_dir<<<S->grid, kBlock, 0, st>>>(d, S->p32, k, pending);
+                    if (k > 0) LEAN_LAUNCH(k_m_dir, S->grid, d, S->p32, k, pending);
                     const bool smp = sample_begin(k);
                     if (dict)
                         DICT_LAUNCH(k_m_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p32);
@@ -1676,7 +1753,10 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                         DISPATCH_WG(A, S->nchunk, k_m_spmv, v, d, S->p32);
                     sample_end(smp);
                     k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
-                    k_m_update<false><<<S->grid, kBlock, 0, st>>>(d, k);
+                    if (lean)
+                        k_m_update<false, true><<<S->grid, kBlock, 0, st>>>(d, k);
+                    else
+                        k_m_update<false><<<S->grid, kBlock, 0, st>>>(d, k);
                 } else {
                     const bool smp = sample_begin(k);
                     if (k > 0)

@@ -251,10 +251,10 @@ __device__ inline T at_byte(const T *a, uint32_t byte) {
 
 // One value per tuple (the inverse diagonal, say) for a row.
 template <class V>
-__device__ inline V dict_one(const EllView &A, const V *tuple_val, int row) {
-    const_as<DictRec> *r = as_const(A.dc_rec) + __builtin_amdgcn_readfirstlane(row >> 6);
+__device__ inline V dict_one(const DictSel *sel, const uint16_t *ids, const V *tuple_val, int row) {
+    const_as<DictSel> *r = as_const(sel) + __builtin_amdgcn_readfirstlane(row >> 6);
     const int a = r->a, b = r->b;
-    if (b < 0) return tuple_val[a + A.dc_id[row]];
+    if (b < 0) return tuple_val[a + ids[row]];
     const V va = as_const(tuple_val)[a], vb = as_const(tuple_val)[b];
     return ((r->mask >> (row & 63)) & 1ull) ? vb : va;
 }
