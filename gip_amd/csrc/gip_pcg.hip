@@ -100,6 +100,7 @@ struct AzList {
 struct PcgDev {
     int n, G;      // solved rows, workgroups of the sweeping kernels (<= kMaxRedBlocks)
     int nchunk;    // 256-row chunks: workgroups of the product kernels
+    int wpc;       // product partials per chunk the fold reads (one per wavefront, or one)
     int Gdn;       // p.Ap partials the next kernels read (<= kMaxRedBlocks)
     double *chunk; // partials of the product: with the fold, kWaves per
                    // 256-row chunk (one per wavefront); without it, one per
@@ -160,24 +161,38 @@ __device__ inline double dpp_row_shr(double v) {
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-__device__ inline double read_lane(double v, int lane) {
+// Wavefront sums by DPP: an inclusive scan of each row of 16 lanes, then row
+// 0's total onto row 1's and row 2's onto row 3's (row broadcast), then lane
+// 31's onto the last row: a fixed order, no LDS, no lane reads.  The total
+// is in lane 63 (18 vector instructions).
+template <int CTRL, int ROWS>
+__device__ inline double dpp_row_bcast(double v) {
     const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
-
-// Sum over the wavefront with DPP row shifts (an inclusive scan of each row
-// of 16 lanes) and four lane reads, the same value in every lane; a fixed
-// order, but not wave_sum's.  The wavefront partials of the long
-// iterations' products and of the FP64 update use it (FP64 solve at 256^3
-// 1163 -> 1155 ms against the shuffle sum).
-__device__ inline double wave_sum_dpp(double v) {
+__device__ inline double half_sum_dpp(double v) {  // lanes 31 and 63: the totals of their halves
     v = v + dpp_row_shr<0x111>(v);
     v = v + dpp_row_shr<0x112>(v);
     v = v + dpp_row_shr<0x114>(v);
     v = v + dpp_row_shr<0x118>(v);
-    return ((read_lane(v, 15) + read_lane(v, 31)) + read_lane(v, 47)) + read_lane(v, 63);
+    return v + dpp_row_bcast<0x142, 0xa>(v);
+}
+__device__ inline double wave_sum_63(double v) {
+    v = half_sum_dpp(v);
+    return v + dpp_row_bcast<0x143, 0xc>(v);
+}
+// Two sums for little more than one: the lower half of the wavefront takes
+// a, the upper half b (each lane's value and the one 32 lanes on), and the
+// halves are summed together.  a's total is in lane 31, b's in lane 63.
+__device__ inline double wave_sum_two(double a, double b) {
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    const double p = __longlong_as_double(((long long)hi[0] << 32) | (long long)lo[0]);
+    const double q = __longlong_as_double(((long long)hi[1] << 32) | (long long)lo[1]);
+    return half_sum_dpp(p + q);
 }
 __device__ inline double rho_slot(const PcgDev &d, int k) { return d.sc[S_RHO0 + (k & 1)]; }
 // p.Ap partials of iteration k in the fused (small-operator) iteration
@@ -197,6 +212,12 @@ __device__ inline double m_denom(double dn, double sap, double zaz, bool dfl) {
     return dfl ? dn - sap * sap / zaz : dn;
 }
 
+// Rows a thread of a grid-stride update sweep has in flight: a LEAN row's
+// two streams alone leave the memory idle (us per iteration with 1, 2, 4
+// rows: mixed 256^3 205 / 197 / 211, FP64 200^3 171 / 167 / 167); a row of
+// five streams does not gain (mixed 160^3 clustered 79.4 / 79.4 / 82.3).
+template <bool LEAN>
+constexpr int kSweepU = LEAN ? 2 : 1;
 // LEAN sweeps (long iterations on an operator with a dictionary): the
 // preconditioned residual s = Dinv r is not stored.  The direction sweep
 // reads r instead of s and forms it again, with the inverse diagonal from
@@ -369,8 +390,8 @@ __device__ inline void iter_spmv(const EllView &A, const PcgDev &d, const double
             acc = pr * sum;
         }
         // one partial per wavefront: no barrier, each wavefront retires alone
-        acc = wave_sum_dpp(acc);
-        if ((threadIdx.x & 63) == 0) d.chunk[c * kWaves + (threadIdx.x >> 6)] = acc;
+        acc = wave_sum_63(acc);
+        if ((threadIdx.x & 63) == 63) d.chunk[c * kWaves + (threadIdx.x >> 6)] = acc;
         return;
     }
     const int st = state_load(d.state);
@@ -406,10 +427,25 @@ __global__ __launch_bounds__(kBlock) void k_iter_spmv_sym(EllView A, PcgDev d, c
     iter_spmv<W, false, true>(A, d, p);
 }
 
-// K1 with the slot values from the dictionary: a wavefront's partial goes to
-// its slice's place, as above, so the sums and their order are the same.
+// K1 with the slot values from the dictionary.  The wavefront sums of a
+// chunk's four slices are added here, in the order the fold adds them, and
+// stored as one value per chunk (an 8-byte store per slice and sum took 12
+// of 73 us in the FP32 product at 256^3): the same sums in the same order.
+template <int R, int M>
+__device__ inline void chunk_store(const PcgDev &d, const double (&sh)[4 * R][M]) {
+    __syncthreads();
+    const int t = threadIdx.x, c = dict_block(blockIdx.x, gridDim.x) * R + t / M;
+    if (t < R * M && c < d.nchunk) {
+        double v = 0.0;
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j) v = v + sh[t / M * 4 + j][t % M];
+        (t % M ? d.chunk_s : d.chunk)[c] = v;
+    }
+}
+
 template <int SW, int R>
 __global__ __launch_bounds__(kBlock) void k_iter_spmv_dict(EllView A, PcgDev d, const double *__restrict__ p) {
+    __shared__ double sh[4 * R][1];
     const int st = state_load(d.state);
     dict_rows<R, SW, double, double>(
         A, A.val, d.n, p, [](int) { return 0; },
@@ -417,9 +453,11 @@ __global__ __launch_bounds__(kBlock) void k_iter_spmv_dict(EllView A, PcgDev d, 
             if (st != ST_RUN) return;
             if (ok && any) d.Ap[row] = sum;
             if (ok && !any) sum = d.Ap[row];  // empty row: Ap keeps its value
-            const double acc = wave_sum_dpp(ok ? own * sum : 0.0);
-            if ((threadIdx.x & 63) == 0) d.chunk[row >> 6] = acc;
+            const double acc = wave_sum_63(ok ? own * sum : 0.0);
+            if ((threadIdx.x & 63) == 63) sh[(row >> 6) & (4 * R - 1)][0] = acc;
         });
+    if (st != ST_RUN) return;
+    chunk_store<R, 1>(d, sh);
 }
 
 // The direction p_k = 1.0 s + beta p_{k-1} read at any column j of the
@@ -523,13 +561,11 @@ __global__ __launch_bounds__(kBlock) void k_fold_dn(PcgDev d) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     double v = 0.0, sa = 0.0;
     if (i < d.nchunk) {
-        const double *w = d.chunk + (size_t)i * kWaves;
-#pragma unroll
-        for (int j = 0; j < kWaves; ++j) v = v + w[j];
+        const double *w = d.chunk + (size_t)i * d.wpc;
+        for (int j = 0; j < d.wpc; ++j) v = v + w[j];
         if (d.deflate) {
-            const double *ws = d.chunk_s + (size_t)i * kWaves;
-#pragma unroll
-            for (int j = 0; j < kWaves; ++j) sa = sa + ws[j];
+            const double *ws = d.chunk_s + (size_t)i * d.wpc;
+            for (int j = 0; j < d.wpc; ++j) sa = sa + ws[j];
         }
     }
     if (d.deflate) {
@@ -669,24 +705,28 @@ __global__ __launch_bounds__(kBlock) void k_iter_update_grid(PcgDev d, int k) {
     store_alpha(d, k, alpha);
     const double malpha = -1.0 * alpha;
     double rs = 0.0, rr = 0.0;
-    FOR_ROWS(d.n, row) {
-        const double ro = r[row], apr = Ap[row];
-        const double di = precond && !LEAN ? dinv[row] : 0.0;
-        const double ri = ro + malpha * apr;  // :97
-        r[row] = ri;
-        double si;
-        if (LEAN) {
-            si = s_of(d, row, ri);
-        } else if (precond) {  // :99-105
-            si = 0.0;
-            si = si + ri * di;
-        } else {
-            si = ri;
-        }
-        if (!LEAN) s[row] = si;
-        rs = rs + ri * si;
-        rr = rr + ri * ri;
-    }
+    struct In {
+        double r, ap, di;
+    };
+    sweep_rows<kSweepU<LEAN>>(
+        d.n,
+        [&](int row) {
+            return In{r[row], Ap[row], !precond ? 0.0 : LEAN ? dict_one(d.dc_sel, d.dc_id, d.ddinv, row) : dinv[row]};
+        },
+        [&](int row, const In &v) {
+            const double ri = v.r + malpha * v.ap;  // :97
+            r[row] = ri;
+            double si;
+            if (precond) {  // :99-105
+                si = 0.0;
+                si = si + ri * v.di;
+            } else {
+                si = ri;
+            }
+            if (!LEAN) s[row] = si;
+            rs = rs + ri * si;
+            rr = rr + ri * ri;
+        });
     double red[2] = {rs, rr};
     block_reduce_n<2>(red);
     if (threadIdx.x == 0) {
@@ -737,19 +777,18 @@ __global__ __launch_bounds__(kBlock) void k_iter_dir_rows(PcgDev d, double *__re
     ntstore(p + row, 1.0 * si + beta * po);  // :113
 }
 
-// the per-wavefront partials of a and b, folded in index order into the
-// Gdn partials of arrays ia and ib (b may be null)
-__global__ __launch_bounds__(kBlock) void k_fold_two(PcgDev d, const double *__restrict__ a,
+// the `per` partials of each of the nwg workgroups of a sweep (a, and b
+// where not null), folded in index order into one partial per workgroup of
+// this kernel, arrays ia and ib
+__global__ __launch_bounds__(kBlock) void k_fold_two(PcgDev d, int nwg, int per, const double *__restrict__ a,
                                                     const double *__restrict__ b, int ia, int ib) {
     if (!running(d)) return;
     const int i = blockIdx.x * kBlock + threadIdx.x;
     double va = 0.0, vb = 0.0;
-    if (i < d.nchunk) {
-#pragma unroll
-        for (int j = 0; j < kWaves; ++j) va = va + a[(size_t)i * kWaves + j];
+    if (i < nwg) {
+        for (int j = 0; j < per; ++j) va = va + a[(size_t)i * per + j];
         if (b)
-#pragma unroll
-            for (int j = 0; j < kWaves; ++j) vb = vb + b[(size_t)i * kWaves + j];
+            for (int j = 0; j < per; ++j) vb = vb + b[(size_t)i * per + j];
     }
     double red[2] = {va, vb};
     block_reduce_n<2>(red);
@@ -774,39 +813,47 @@ __global__ __launch_bounds__(kBlock) void k_alpha_fin(PcgDev d, int k) {
     if (threadIdx.x == 0) alpha_finish(d, k, dn);
 }
 
-// K2 of iteration k
+// K2 of iteration k: kUpdateRows slices per wavefront, their loads in flight
+// together and their rows summed before the wavefront's two sums, which
+// with one slice and two separate sums held the kernel to 4.7 TB/s (256^3
+// with a dictionary: 86 -> 61 us, 6.6 TB/s; FP64 iteration at 256^3
+// clustered 428 -> 421 us).
+constexpr int kUpdateRows = 2;
 template <bool LEAN>
 __global__ __launch_bounds__(kBlock) void k_iter_update_rows(PcgDev d, int k) {
     if (!running(d)) return;
-    const int row = blockIdx.x * kBlock + threadIdx.x;
+    const int wv = blockIdx.x * kWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     const double malpha = -1.0 * alpha_slot(d, k);
-    double rs = 0.0, rr = 0.0;
-    if (row < d.n) {
-        const double ro = ntload(d.r + row), apr = ntload(d.Ap + row);
-        const double di = d.precond && !LEAN ? ntload(d.dinv + row) : 0.0;
-        const double ri = ro + malpha * apr;  // :97
-        ntstore(d.r + row, ri);
+    double rs = 0.0, rr = 0.0, ro[kUpdateRows], apr[kUpdateRows], di[kUpdateRows];
+#pragma unroll
+    for (int u = 0; u < kUpdateRows; ++u) {
+        const int at = (wv * kUpdateRows + u) * 64 + lane, row = at < d.n ? at : d.n - 1;
+        ro[u] = ntload(d.r + row);
+        apr[u] = ntload(d.Ap + row);
+        di[u] = !d.precond ? 0.0 : LEAN ? dict_one(d.dc_sel, d.dc_id, d.ddinv, row) : ntload(d.dinv + row);
+    }
+#pragma unroll
+    for (int u = 0; u < kUpdateRows; ++u) {
+        const int row = (wv * kUpdateRows + u) * 64 + lane;
+        const double ri = ro[u] + malpha * apr[u];  // :97
         double si;
-        if (LEAN) {
-            si = s_of(d, row, ri);
-        } else if (d.precond) {  // :99-105
+        if (d.precond) {  // :99-105
             si = 0.0;
-            si = si + ri * di;
+            si = si + ri * di[u];
         } else {
             si = ri;
         }
-        if (!LEAN) ntstore(d.s + row, si);
-        rs = ri * si;
-        rr = ri * ri;
+        if (row < d.n) {
+            ntstore(d.r + row, ri);
+            if (!LEAN) ntstore(d.s + row, si);
+            rs = rs + ri * si;
+            rr = rr + ri * ri;
+        }
     }
     // one partial per wavefront: no barrier
-    rs = wave_sum_dpp(rs);
-    rr = wave_sum_dpp(rr);
-    const int wv = blockIdx.x * kWaves + (threadIdx.x >> 6);
-    if ((threadIdx.x & 63) == 0) {
-        d.chunk[wv] = rs;
-        d.chunk_s[wv] = rr;
-    }
+    const double t = wave_sum_two(rs, rr);
+    if (lane == 31) d.chunk[wv] = t;
+    if (lane == 63) d.chunk_s[wv] = t;
     if (leader()) *d.iters = k + 1;
 }
 
@@ -823,10 +870,10 @@ __device__ inline void beta_finish(const PcgDev &d, int k, double rho, double rr
     d.sc[S_RHO0 + (k & 1)] = rho;
 }
 
-__global__ __launch_bounds__(kBlock) void k_beta_fin(PcgDev d, int k) {
+__global__ __launch_bounds__(kBlock) void k_beta_fin(PcgDev d, int k, int np) {
     if (!running(d)) return;
     double sums[2];
-    sum_partials_n<2>({d.P(P_RS), d.P(P_RR)}, d.Gdn, sums);
+    sum_partials_n<2>({d.P(P_RS), d.P(P_RR)}, np, sums);
     if (threadIdx.x == 0) beta_finish(d, k, sums[0], sums[1]);
 }
 
@@ -971,13 +1018,10 @@ __device__ inline void m_spmv(const EllView &A, const PcgDev &d, const float *__
             acc = (double)pr * (double)sum;
             sa = (double)sum;
         }
-        acc = wave_sum_dpp(acc);
-        const int wv = c * kWaves + (threadIdx.x >> 6);
-        if ((threadIdx.x & 63) == 0) d.chunk[wv] = acc;
-        if (d.deflate) {
-            sa = wave_sum_dpp(sa);
-            if ((threadIdx.x & 63) == 0) d.chunk_s[wv] = sa;
-        }
+        const int wv = c * kWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+        acc = wave_sum_two(acc, sa);
+        if (lane == 31) d.chunk[wv] = acc;
+        if (lane == 63) d.chunk_s[wv] = acc;
         return;
     }
     const int st = state_load(d.state);
@@ -1017,17 +1061,16 @@ __global__ __launch_bounds__(kBlock) void k_m_spmv_small(EllView A, PcgDev d, co
 // (as k_iter_spmv_dict)
 template <int SW, int R>
 __global__ __launch_bounds__(kBlock) void k_m_spmv_dict(EllView A, PcgDev d, const float *__restrict__ p) {
+    __shared__ double sh[4 * R][2];
     dict_rows<R, SW, float, float>(
         A, A.val32, d.n, p, [](int) { return 0; },
         [&](int row, bool ok, bool, float sum, float own, int) {
             if (ok) d.Ap32[row] = sum;
-            const double acc = wave_sum_dpp(ok ? (double)own * (double)sum : 0.0);
-            const double sa = d.deflate ? wave_sum_dpp(ok ? (double)sum : 0.0) : 0.0;
-            if ((threadIdx.x & 63) == 0) {
-                d.chunk[row >> 6] = acc;
-                if (d.deflate) d.chunk_s[row >> 6] = sa;
-            }
+            const int lane = threadIdx.x & 63;
+            const double acc = wave_sum_two(ok ? (double)own * (double)sum : 0.0, ok ? (double)sum : 0.0);
+            if ((lane & 31) == 31) sh[(row >> 6) & (4 * R - 1)][lane >> 5] = acc;
         });
+    chunk_store<R, 2>(d, sh);
 }
 
 template <bool SMALL, bool LEAN = false>
@@ -1073,32 +1116,40 @@ __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
         const bool listed = naz <= kAzList;
 #pragma unroll
         for (int j = 0; j < kAzList; ++j) li[j] = j < naz ? li[j] : -1;
-        FOR_ROWS(d.n, row) {
-            // every operand first, so the row costs one memory round trip
-            const float ro = __builtin_nontemporal_load(r + row), apr = __builtin_nontemporal_load(Ap + row);
-            const float di = precond && !LEAN ? __builtin_nontemporal_load(dinv + row) : 0.0f;
-            float azr = 0.0f;
-            if (dfl && !listed) {
-                azr = az[row];
-            } else {
-                // rows compared with the list only in a chunk that holds a
-                // listed row (a workgroup-uniform test per chunk)
-                const int base = __builtin_amdgcn_readfirstlane(row - (int)threadIdx.x);
-                bool hit = false;
+        struct In {
+            float r, ap, di;
+        };
+        sweep_rows<kSweepU<LEAN>>(
+            d.n,
+            [&](int row) {
+                return In{__builtin_nontemporal_load(r + row), __builtin_nontemporal_load(Ap + row),
+                          !precond ? 0.0f
+                          : LEAN   ? dict_one(d.dc_sel, d.dc_id, d.ddinv32, row)
+                                   : __builtin_nontemporal_load(dinv + row)};
+            },
+            [&](int row, const In &v) {
+                float azr = 0.0f;
+                if (dfl && !listed) {
+                    azr = az[row];
+                } else {
+                    // rows compared with the list only in a chunk that holds a
+                    // listed row (a workgroup-uniform test per chunk)
+                    const int base = __builtin_amdgcn_readfirstlane(row - (int)threadIdx.x);
+                    bool hit = false;
 #pragma unroll
-                for (int j = 0; j < kAzList; ++j) hit = hit || (unsigned)(li[j] - base) < (unsigned)kBlock;
-                if (hit)
+                    for (int j = 0; j < kAzList; ++j) hit = hit || (unsigned)(li[j] - base) < (unsigned)kBlock;
+                    if (hit)
 #pragma unroll
-                    for (int j = 0; j < kAzList; ++j) azr = row == li[j] ? lv[j] : azr;
-            }
-            const float wr = dfl ? apr - c32 * azr : apr;  // (P A p)_row
-            const float ri = ro - a32 * wr;
-            __builtin_nontemporal_store(ri, r + row);
-            const float si = LEAN ? s_of(d, row, ri) : precond ? ri * di : ri;
-            if (!LEAN) __builtin_nontemporal_store(si, s + row);
-            rs = rs + (double)ri * (double)si;
-            rr = rr + (double)ri * (double)ri;
-        }
+                        for (int j = 0; j < kAzList; ++j) azr = row == li[j] ? lv[j] : azr;
+                }
+                const float wr = dfl ? v.ap - c32 * azr : v.ap;  // (P A p)_row
+                const float ri = v.r - a32 * wr;
+                __builtin_nontemporal_store(ri, r + row);
+                const float si = precond ? ri * v.di : ri;
+                if (!LEAN) __builtin_nontemporal_store(si, s + row);
+                rs = rs + (double)ri * (double)si;
+                rr = rr + (double)ri * (double)ri;
+            });
     } else {
         ThreadRows t(d.n);
         float ro = 0.0f, apr = 0.0f, di = 0.0f, azr = 0.0f;
@@ -1402,6 +1453,7 @@ static PcgDev make_dev(gip_pcg *S, const double *b, double *x, int precond) {
     d.n = S->n;
     d.G = S->grid;
     d.nchunk = S->nchunk;
+    d.wpc = kWaves;
     d.Gdn = S->gdn;
     d.chunk = S->fold ? S->chunk : S->part + P_DN * kMaxRedBlocks;
     d.chunk_s = S->fold ? S->chunk + (size_t)S->nchunk * kWaves : nullptr;
@@ -1622,6 +1674,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     const bool lean = dict && (!mixed || !A->dict_ids) &&
                       (!o->precond || (S->ddinv && S->dict_version == A->dict_version));
     PcgDev d = make_dev(S, b, x, o->precond ? 1 : 0);
+    if (dict) d.wpc = 1;
     EllView v = view(A);
     const int pollk = o->poll > 0 ? o->poll : 16;
     const int use_coarse = o->coarse >= 0 ? 1 : 0;
@@ -1698,11 +1751,12 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                     else
                         DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, S->p);
                     sample_end(smp);
-                    k_fold_two<<<S->gdn, kBlock, 0, st>>>(d, d.chunk, nullptr, P_DN, P_DN);
+                    k_fold_two<<<S->gdn, kBlock, 0, st>>>(d, S->nchunk, d.wpc, d.chunk, nullptr, P_DN, P_DN);
                     k_alpha_fin<<<1, kBlock, 0, st>>>(d, k);
-                    LEAN_LAUNCH(k_iter_update_rows, S->nchunk, d, k);
-                    k_fold_two<<<S->gdn, kBlock, 0, st>>>(d, d.chunk, d.chunk_s, P_RS, P_RR);
-                    k_beta_fin<<<1, kBlock, 0, st>>>(d, k + 1);
+                    const int uwg = (S->nchunk + kUpdateRows - 1) / kUpdateRows, ufold = (uwg + kBlock - 1) / kBlock;
+                    LEAN_LAUNCH(k_iter_update_rows, uwg, d, k);
+                    k_fold_two<<<ufold, kBlock, 0, st>>>(d, uwg, kWaves, d.chunk, d.chunk_s, P_RS, P_RR);
+                    k_beta_fin<<<1, kBlock, 0, st>>>(d, k + 1, ufold);
                 } else {
                     const bool smp = sample_begin(k);
                     if (k > 0 && o->tol > 0.0)

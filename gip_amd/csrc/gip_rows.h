@@ -675,6 +675,31 @@ struct RowSweep {
     for (RowSweep rs__(n); rs__.c < rs__.c1; rs__.c += rs__.step) \
         for (int row = rs__.c * kBlock + (int)threadIdx.x; row < (rs__.c + 1) * kBlock && row < (n); row = (n))
 
+// FOR_ROWS with U rows' loads in flight: load(row) requests a row's operands
+// (called for every lane: a row past the sweep is read as the last row),
+// use(row, operands) takes them; a thread's rows in the same order.
+template <int U, class LOAD, class USE>
+__device__ inline void sweep_rows(int n, const LOAD &load, const USE &use) {
+    if constexpr (U == 1) {
+        FOR_ROWS(n, row) use(row, load(row));
+        return;
+    }
+    RowSweep rs(n);
+    for (; rs.c < rs.c1; rs.c += U * rs.step) {
+        decltype(load(0)) v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int c = rs.c + u * rs.step, row = c * kBlock + (int)threadIdx.x;
+            v[u] = load(c < rs.c1 && row < n ? row : n - 1);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int c = rs.c + u * rs.step, row = c * kBlock + (int)threadIdx.x;
+            if (c < rs.c1 && row < n) use(row, v[u]);
+        }
+    }
+}
+
 // The rows FOR_ROWS gives this thread, as a cursor, so that a kernel can
 // request its first row's operands before its prologue and each next row's
 // right after storing the current one.  Only the last chunk of the matrix
