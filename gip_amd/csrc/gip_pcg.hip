@@ -653,21 +653,32 @@ __global__ __launch_bounds__(kBlock) void k_iter_update(PcgDev d, int k) {
 // past the switch 224^3 834.0 / 776.4, 256^3 1418 / 1286).
 constexpr int kRowsMin = 1 << 23;
 
-// K0 (k >= 1): rho_k, the convergence test, x += alpha_{k-1} p,
-// beta, p = 1.0 s + beta p
-template <bool LEAN>
-__global__ __launch_bounds__(kBlock) void k_iter_dir(PcgDev d, double *__restrict__ p, int k) {
+// The x updates of the long iterations (x += alpha_k p_k, :95) are made two
+// at a time by the direction sweep of every second iteration, which reads
+// p_{k-1} anyway: x is read and written half as often for one more read of
+// the direction before (two direction buffers by parity; the older one is
+// the one being overwritten).  In order, so the same bits.  Nine streams
+// instead of ten per two sweeps.
+__device__ inline double x_two(double x, double a2, double p2, double a1, double p1) {
+    const double t = x + a2 * p2;  // iteration k-2
+    return t + a1 * p1;            // iteration k-1
+}
+
+// K0 (k >= 1): rho_k, the convergence test, beta, p_k = 1.0 s + beta p_{k-1}
+// into pnew (which holds p_{k-2}); PAIR: the x updates of k-2 and k-1
+template <bool LEAN, bool PAIR>
+__global__ __launch_bounds__(kBlock) void k_iter_dir(PcgDev d, const double *__restrict__ pold,
+                                                    double *__restrict__ pnew, int k) {
     double *__restrict__ x = d.x;
     const double *__restrict__ s = LEAN ? d.r : d.s;
     const int st = state_load(d.state);
     if (st != ST_RUN && st != conv_stamp(k)) return;
     const double rho = sum_partials<RED_SUM>(d.P(P_RS), d.G);  // :107
-    const double alpha = alpha_slot(d, k - 1);
+    const double a1 = PAIR ? alpha_slot(d, k - 1) : 0.0, a2 = PAIR ? alpha_slot(d, k - 2) : 0.0;
     const double tol2 = d.sc[S_TOL2];
     if (tol2 >= 0.0) {
         const double rr = sum_partials<RED_SUM>(d.P(P_RR), d.G);
         if (rr <= tol2) {  // every workgroup reaches the same decision
-            x_update(d, p, alpha);
             if (leader()) state_store(d.state, conv_stamp(k));
             return;
         }
@@ -675,10 +686,11 @@ __global__ __launch_bounds__(kBlock) void k_iter_dir(PcgDev d, double *__restric
     const double beta = rho / rho_slot(d, k - 1);  // :109
     if (leader()) d.sc[S_RHO0 + (k & 1)] = rho;
     FOR_ROWS(d.n, row) {
-        const double xo = x[row], sr = s[row], po = p[row];
+        const double sr = s[row], po = pold[row];
+        const double xo = PAIR ? x[row] : 0.0, pp = PAIR ? pnew[row] : 0.0;
         const double si = LEAN ? s_of(d, row, sr) : sr;
-        x[row] = xo + alpha * po;       // :95 of iteration k-1
-        p[row] = 1.0 * si + beta * po;  // :113
+        if (PAIR) x[row] = x_two(xo, a2, pp, a1, po);
+        pnew[row] = 1.0 * si + beta * po;  // :113
     }
 }
 
@@ -755,26 +767,22 @@ __global__ __launch_bounds__(kBlock) void k_iter_update_grid(PcgDev d, int k) {
 __device__ inline double ntload(const double *p) { return __builtin_nontemporal_load(p); }
 __device__ inline void ntstore(double *p, double v) { __builtin_nontemporal_store(v, p); }
 
-// K0 of iteration k >= 1
-template <bool LEAN>
-__global__ __launch_bounds__(kBlock) void k_iter_dir_rows(PcgDev d, double *__restrict__ p, int k) {
-    const int st = state_load(d.state);
+// K0 of iteration k >= 1 (as k_iter_dir)
+template <bool LEAN, bool PAIR>
+__global__ __launch_bounds__(kBlock) void k_iter_dir_rows(PcgDev d, const double *__restrict__ pold,
+                                                         double *__restrict__ pnew, int k) {
+    if (!running(d)) return;
     const int row = blockIdx.x * kBlock + threadIdx.x;
     if (row >= d.n) return;
-    const double alpha = alpha_slot(d, k - 1);
-    double *__restrict__ x = d.x;
-    if (st == conv_stamp(k)) {  // converged after iteration k-1: its x update only
-        x[row] = x[row] + alpha * p[row];  // :95
-        return;
-    }
-    if (st != ST_RUN) return;
+    const double a1 = PAIR ? alpha_slot(d, k - 1) : 0.0, a2 = PAIR ? alpha_slot(d, k - 2) : 0.0;
     const double beta = d.sc[S_BETA];
     // nontemporal accesses: each array is streamed once per sweep (a plain
     // stream of this mix runs 8% faster with them on this device)
-    const double xo = ntload(x + row), sr = ntload((LEAN ? d.r : d.s) + row), po = ntload(p + row);
+    const double sr = ntload((LEAN ? d.r : d.s) + row), po = ntload(pold + row);
+    const double xo = PAIR ? ntload(d.x + row) : 0.0, pp = PAIR ? ntload(pnew + row) : 0.0;
     const double si = LEAN ? s_of(d, row, sr) : sr;
-    ntstore(x + row, xo + alpha * po);       // :95 of iteration k-1
-    ntstore(p + row, 1.0 * si + beta * po);  // :113
+    if (PAIR) ntstore(d.x + row, x_two(xo, a2, pp, a1, po));
+    ntstore(pnew + row, 1.0 * si + beta * po);  // :113
 }
 
 // the `per` partials of each of the nwg workgroups of a sweep (a, and b
@@ -878,12 +886,24 @@ __global__ __launch_bounds__(kBlock) void k_beta_fin(PcgDev d, int k, int np) {
 }
 
 
-// x += alpha_k p of the last iteration k, unless a breakdown stopped the solve
-__global__ __launch_bounds__(kBlock) void k_x_flush_rows(PcgDev d, const double *__restrict__ p, int k) {
-    const int st = state_load(d.state);
-    if (st != ST_RUN && st != conv_stamp(k + 1)) return;
-    const int row = blockIdx.x * kBlock + threadIdx.x;
-    if (row < d.n) d.x[row] = d.x[row] + alpha_slot(d, k) * p[row];
+// The x updates still due when a long solve has stopped: of its `iters`
+// iterations K0 of every even iteration k >= 2 has applied those before k
+// (after a breakdown in iteration `iters`, whose K0 ran, that one's too).
+// Directions by parity in pa (even) and pb.
+__global__ __launch_bounds__(kBlock) void k_x_flush_pair(PcgDev d, const double *__restrict__ pa,
+                                                        const double *__restrict__ pb) {
+    const int it = *d.iters;
+    if (it < 1) return;
+    const bool broke = (state_load(d.state) & ST_MASK) == ST_BREAK;
+    if (broke && !(it & 1)) return;
+    const bool two = !(it & 1);
+    const double a1 = alpha_slot(d, it - 1), a2 = two ? alpha_slot(d, it - 2) : 0.0;
+    const double *__restrict__ p1 = ((it - 1) & 1) ? pb : pa;
+    FOR_ROWS(d.n, row) {
+        double x = d.x[row];
+        if (two) x = x + a2 * pa[row];
+        d.x[row] = x + a1 * p1[row];
+    }
 }
 
 // one workgroup after the last iteration: the final convergence test on the
@@ -907,27 +927,34 @@ __global__ __launch_bounds__(kBlock) void k_fin(PcgDev d) {
 
 // ---- MIXED iteration (FP32 vectors and operator, FP64 dot accumulation) --------
 
-// K0 (k >= 1): rho_k, the correction update xc += alpha_{k-1} p of the
-// previous iteration (`pending`: not yet folded by a defect correction),
-// beta (0 after a restart: the previous rho slot is +inf), p32 = s32 + beta p32
-template <bool LEAN>
-__global__ __launch_bounds__(kBlock) void k_m_dir(PcgDev d, float *__restrict__ p, int k, int pending) {
+// K0 (k >= 1): rho_k, beta (0 after a restart: the previous rho slot is
+// +inf), p32 = s32 + beta p32 into pnew; PAIR: the correction updates
+// xc += alpha p of iterations k-2 and k-1 (not yet folded by a defect
+// correction), two at a time as in k_iter_dir
+template <bool LEAN, bool PAIR>
+__global__ __launch_bounds__(kBlock) void k_m_dir(PcgDev d, const float *__restrict__ pold, float *__restrict__ pnew,
+                                                 int k) {
     float *__restrict__ xc = d.xc32;
     const float *__restrict__ s = LEAN ? d.r32 : d.s32;
     if (!running(d)) return;
     const double rho = sum_partials<RED_SUM>(d.P(P_RS), d.G);
-    const float a32 = pending ? (float)alpha_slot(d, k - 1) : 0.0f;  // alpha_{k-1}, as K2 of k-1 formed it
+    const float a1 = PAIR ? (float)alpha_slot(d, k - 1) : 0.0f;  // as K2 formed them
+    const float a2 = PAIR ? (float)alpha_slot(d, k - 2) : 0.0f;
     const float beta = (float)(rho / rho_slot(d, k - 1));
     if (leader()) d.sc[S_RHO0 + (k & 1)] = rho;
     // nontemporal accesses: each array is streamed once per sweep (mixed
     // solve at 256^3 over four runs: 392-394 ms with them, 403-405 without;
     // the sweeps' own times are unchanged within noise)
     FOR_ROWS(d.n, row) {
-        const float xo = __builtin_nontemporal_load(xc + row), sr = __builtin_nontemporal_load(s + row),
-                    po = __builtin_nontemporal_load(p + row);
+        const float sr = __builtin_nontemporal_load(s + row), po = __builtin_nontemporal_load(pold + row);
+        const float xo = PAIR ? __builtin_nontemporal_load(xc + row) : 0.0f,
+                    pp = PAIR ? __builtin_nontemporal_load(pnew + row) : 0.0f;
         const float si = LEAN ? s_of(d, row, sr) : sr;
-        if (pending) __builtin_nontemporal_store(xo + a32 * po, xc + row);
-        __builtin_nontemporal_store(si + beta * po, p + row);
+        if (PAIR) {
+            const float t = xo + a2 * pp;
+            __builtin_nontemporal_store(t + a1 * po, xc + row);
+        }
+        __builtin_nontemporal_store(si + beta * po, pnew + row);
     }
 }
 
@@ -1209,11 +1236,15 @@ __global__ __launch_bounds__(kBlock) void k_m_status(PcgDev d) {
     if (threadIdx.x == 0) d.sc[S_RR] = rr;
 }
 
-// x += (xc + alpha_k p) (the last iteration's pending update first), xc = 0
-__global__ __launch_bounds__(kBlock) void k_m_fold(PcgDev d, const float *__restrict__ p, int k) {
-    const float a32 = (float)alpha_slot(d, k);
+// x += xc, with the last iterations' pending updates xc += alpha p first
+// (two: those of k-1 in p2 and k in p; one: that of k), xc = 0
+__global__ __launch_bounds__(kBlock) void k_m_fold(PcgDev d, const float *__restrict__ p, const float *__restrict__ p2,
+                                                  int k, int pending) {
+    const float a1 = (float)alpha_slot(d, k), a2 = pending > 1 ? (float)alpha_slot(d, k - 1) : 0.0f;
     FOR_ROWS(d.n, row) {
-        const float xcv = d.xc32[row] + a32 * p[row];
+        float xcv = d.xc32[row];
+        if (pending > 1) xcv = xcv + a2 * p2[row];
+        if (pending) xcv = xcv + a1 * p[row];
         d.x[row] = d.x[row] + (double)xcv;
         d.xc32[row] = 0.0f;
     }
@@ -1388,7 +1419,7 @@ struct gip_pcg {
     int n, n_all, grid;
     double *r, *p, *s, *Ap, *dinv;
     float *r32, *p32, *s32, *Ap32, *xc32, *dinv32;
-    double *p2;   // second direction buffer of the fused iteration (small operators)
+    double *p2;   // second direction buffer (directions alternate by parity)
     float *p32b;  // its FP32 counterpart
     double *ddinv;   // the Jacobi inverse per tuple of the operator's dictionary
     float *ddinv32;  // (FP64, FP32), made from dictionary `dict_version`
@@ -1519,7 +1550,7 @@ int gip_pcg_create(gip_ctx *c, const gip_mat *A, int32_t n_all, gip_pcg **out) {
     };
     dalloc((void **)&S->r, n * 8);
     dalloc((void **)&S->p, na * 8);
-    if (!S->fold) dalloc((void **)&S->p2, na * 8);
+    dalloc((void **)&S->p2, na * 8);
     dalloc((void **)&S->s, n * 8);
     dalloc((void **)&S->Ap, n * 8);
     dalloc((void **)&S->dinv, n * 8);
@@ -1597,10 +1628,8 @@ static int ensure_mixed(gip_pcg *S) {
     // there (the correction leaves the ghost values of x unchanged)
     GIP_HIP_TRY(hipMalloc(&S->p32, na * 4));
     GIP_HIP_TRY(hipMemsetAsync(S->p32, 0, na * 4, S->ctx->stream));
-    if (!S->fold) {
-        GIP_HIP_TRY(hipMalloc(&S->p32b, na * 4));
-        GIP_HIP_TRY(hipMemsetAsync(S->p32b, 0, na * 4, S->ctx->stream));
-    }
+    GIP_HIP_TRY(hipMalloc(&S->p32b, na * 4));
+    GIP_HIP_TRY(hipMemsetAsync(S->p32b, 0, na * 4, S->ctx->stream));
     if (S->n) {
         k_to32<<<(S->n + kBlock - 1) / kBlock, kBlock, 0, S->ctx->stream>>>(S->n, S->dinv, S->dinv32);
         GIP_LAUNCH_CHECK("dinv32");
@@ -1679,10 +1708,22 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     const int pollk = o->poll > 0 ? o->poll : 16;
     const int use_coarse = o->coarse >= 0 ? 1 : 0;
     d.deflate = mixed && use_coarse;
-    // direction of iteration k: one buffer with the fold, alternating by
-    // parity in the fused iteration
-    auto pdir = [&](int k) { return (!S->fold && (k & 1)) ? S->p2 : S->p; };
-    auto pdir32 = [&](int k) { return (!S->fold && (k & 1)) ? S->p32b : S->p32; };
+    // direction of iteration k: two buffers by parity
+    auto pdir = [&](int k) { return (k & 1) ? S->p2 : S->p; };
+    auto pdir32 = [&](int k) { return (k & 1) ? S->p32b : S->p32; };
+    // the instance of a long direction sweep: LEAN, and whether it makes the
+    // pending x updates
+#define DIR_LAUNCH(KERNEL, GRID, PAIR, ...)                        \
+    do {                                                           \
+        if (lean && (PAIR))                                        \
+            KERNEL<true, true><<<GRID, kBlock, 0, st>>>(__VA_ARGS__);   \
+        else if (lean)                                             \
+            KERNEL<true, false><<<GRID, kBlock, 0, st>>>(__VA_ARGS__);  \
+        else if (PAIR)                                             \
+            KERNEL<false, true><<<GRID, kBlock, 0, st>>>(__VA_ARGS__);  \
+        else                                                       \
+            KERNEL<false, false><<<GRID, kBlock, 0, st>>>(__VA_ARGS__); \
+    } while (0)
     // time_products: events around one product launch (k >= 1) per host
     // poll, read after the poll's synchronisation
     const bool timing = o->time_products != 0;
@@ -1729,27 +1770,27 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             int chunk = std::min(fixed ? 4096 : pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold && !S->rows) {
-                    if (k > 0) LEAN_LAUNCH(k_iter_dir, S->grid, d, S->p, k);
+                    if (k > 0) DIR_LAUNCH(k_iter_dir, S->grid, k >= 2 && !(k & 1), d, pdir(k - 1), pdir(k), k);
                     const bool smp = sample_begin(k);
                     if (dict)
-                        DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p);
+                        DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, pdir(k));
                     else if (sym)
-                        SYM_LAUNCH(A, k_iter_spmv_sym, v, d, S->p);
+                        SYM_LAUNCH(A, k_iter_spmv_sym, v, d, pdir(k));
                     else
-                        DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, S->p);
+                        DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, pdir(k));
                     sample_end(smp);
                     k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
                     LEAN_LAUNCH(k_iter_update_grid, S->grid, d, k);
                 } else if (S->fold) {
                     // (partials: p.Ap in chunk, then r.s in chunk and r.r in chunk_s)
-                    if (k > 0) LEAN_LAUNCH(k_iter_dir_rows, S->nchunk, d, S->p, k);
+                    if (k > 0) DIR_LAUNCH(k_iter_dir_rows, S->nchunk, k >= 2 && !(k & 1), d, pdir(k - 1), pdir(k), k);
                     const bool smp = sample_begin(k);
                     if (dict)
-                        DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p);
+                        DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, pdir(k));
                     else if (sym)
-                        SYM_LAUNCH(A, k_iter_spmv_sym, v, d, S->p);
+                        SYM_LAUNCH(A, k_iter_spmv_sym, v, d, pdir(k));
                     else
-                        DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, S->p);
+                        DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, pdir(k));
                     sample_end(smp);
                     k_fold_two<<<S->gdn, kBlock, 0, st>>>(d, S->nchunk, d.wpc, d.chunk, nullptr, P_DN, P_DN);
                     k_alpha_fin<<<1, kBlock, 0, st>>>(d, k);
@@ -1775,13 +1816,15 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                 sample_read();
             }
         }
-        if (S->rows) {
-            if (k > 0) k_x_flush_rows<<<S->nchunk, kBlock, 0, st>>>(d, S->p, k - 1);
-            k_fin_rows<<<1, kBlock, 0, st>>>(d);
-        } else {
-            if (k > 0) k_x_flush<<<S->grid, kBlock, 0, st>>>(d, pdir(k - 1), k - 1);
-            k_fin<<<1, kBlock, 0, st>>>(d);
+        if (S->fold) {
+            if (k > 0) k_x_flush_pair<<<S->grid, kBlock, 0, st>>>(d, S->p, S->p2);
+        } else if (k > 0) {
+            k_x_flush<<<S->grid, kBlock, 0, st>>>(d, pdir(k - 1), k - 1);
         }
+        if (S->rows)
+            k_fin_rows<<<1, kBlock, 0, st>>>(d);
+        else
+            k_fin<<<1, kBlock, 0, st>>>(d);
         GIP_LAUNCH_CHECK("pcg final test");
     } else {
         // FP64 residual of x0 (with the coarse step), FP32 copies, first direction
@@ -1794,17 +1837,18 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
         double last_rr = S->h_sc[S_TRUE_RR];
         const double it = o->inner_tol > 0.0 ? o->inner_tol : 0.1;
         const double inner2 = it * it;
-        int k = 0, pending = 0;  // pending: the last iteration's correction update is not yet applied
+        int k = 0, pending = 0;  // pending: the correction updates not yet applied (at most two)
         while (k < o->maxit && S->h_state[0] == ST_RUN) {
             int chunk = std::min(pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold) {
-                    if (k > 0) LEAN_LAUNCH(k_m_dir, S->grid, d, S->p32, k, pending);
+                    if (k > 0) DIR_LAUNCH(k_m_dir, S->grid, pending == 2, d, pdir32(k - 1), pdir32(k), k);
+                    pending = pending == 2 ? 1 : pending + 1;
                     const bool smp = sample_begin(k);
                     if (dict)
-                        DICT_LAUNCH(k_m_spmv_dict, A->st_w, S->nchunk, st, v, d, S->p32);
+                        DICT_LAUNCH(k_m_spmv_dict, A->st_w, S->nchunk, st, v, d, pdir32(k));
                     else
-                        DISPATCH_WG(A, S->nchunk, k_m_spmv, v, d, S->p32);
+                        DISPATCH_WG(A, S->nchunk, k_m_spmv, v, d, pdir32(k));
                     sample_end(smp);
                     k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
                     if (lean)
@@ -1819,8 +1863,8 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                         DISPATCH_WG(A, S->nchunk, k_m_spmv_small, v, d, S->p32);
                     sample_end(smp);
                     k_m_update<true><<<S->grid, kBlock, 0, st>>>(d, k);
+                    pending = 1;
                 }
-                pending = 1;
             }
             k_m_status<<<1, kBlock, 0, st>>>(d);
             GIP_LAUNCH_CHECK("mixed iteration");
@@ -1830,7 +1874,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             const double rr32 = S->h_sc[S_RR], tol2 = S->h_sc[S_TOL2];
             const bool near_target = tol2 >= 0.0 && rr32 <= tol2;
             if (rr32 <= inner2 * last_rr || near_target || k >= o->maxit) {
-                k_m_fold<<<S->grid, kBlock, 0, st>>>(d, pdir32(k - 1), k - 1);
+                k_m_fold<<<S->grid, kBlock, 0, st>>>(d, pdir32(k - 1), pdir32(k), k - 1, pending);
                 pending = 0;
                 DISPATCH_W(A, k_m_resid, v, d);
                 k_m_coarse<<<S->grid, kBlock, 0, st>>>(d, use_coarse);

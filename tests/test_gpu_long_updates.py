@@ -1,0 +1,104 @@
+"""The long iterations make their x updates two at a time (gip_pcg.hip,
+k_iter_dir): whatever iteration a solve stops at, x must hold every update.
+One to six fixed iterations and a stop at each of a few tolerances, on both
+long forms (more than 2^19 and more than 2^23 rows), with and without a
+dictionary, against the oracle; the mixed solve with corrections after one,
+two and three iterations; a breakdown in the second iteration.
+"""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from gip_amd import cavity, hip
+from oracle import pyoracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = hip.Device(0)
+    yield d
+    d.close()
+
+
+def _line(n, scale=None):
+    """A shifted 1-D Laplacian (a few distinct rows: a dictionary), or one scaled row by row (none)."""
+    T = sp.diags([-1.0, 2.05, -1.0], [-1, 0, 1], shape=(n, n)).tocsr()
+    if scale is not None:
+        S = sp.diags(scale)
+        T = (S @ T @ S).tocsr()
+    T.sort_indices()
+    return T
+
+
+@pytest.mark.parametrize("n,plain", [(2 ** 19 + 1, False), (2 ** 19 + 300, True), (2 ** 23 + 65, False)])
+def test_x_holds_every_update(dev, n, plain):
+    rng = np.random.default_rng(n)
+    T = _line(n, 1.0 + 0.1 * rng.random(n) if plain else None)
+    b, x0 = rng.standard_normal(n), 0.1 * rng.standard_normal(n)
+    orc = pyoracle.Csr(T.indptr, T.indices, T.data, n)
+    M = hip.Matrix(dev, T.indptr, T.indices, T.data, ncols=n, fp32=True)
+    solver = hip.PCG(M, n)
+    db, dx0, dx = dev.to_device(b), dev.to_device(x0), dev.array(n)
+    for maxit in range(0, 7):
+        r = solver.solve(db, dx, dx0, maxit=maxit)
+        want, st, it, rel = pyoracle.pcg(orc, b, x0, n, maxit)
+        assert r.iters == it == maxit and r.status == 0
+        assert np.linalg.norm(dx.download() - want) <= 1e-12 * np.linalg.norm(want), maxit
+    for tol in (0.5, 0.2, 0.1, 0.05, 0.02):
+        r = solver.solve(db, dx, dx0, maxit=100, tol=tol, poll=3)
+        want, st, it, rel = pyoracle.pcg(orc, b, x0, n, 100, tol=tol)
+        assert r.iters == it and r.status == 0
+        assert np.linalg.norm(dx.download() - want) <= 1e-12 * np.linalg.norm(want), tol
+    for poll in (1, 2, 3):
+        r = solver.solve(db, dx, dx0, maxit=200, tol=1e-10, precision=hip.PCG_MIXED, poll=poll)
+        x = dx.download()
+        print(f"[n={n} mixed poll {poll}] iters {r.iters} corrections {r.corrections}", flush=True)
+        assert r.status == 0 and np.linalg.norm(b - T @ x) <= 1.01e-10 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("shape", [(96, 96, 64), (128, 256, 257)], ids=lambda s: "x".join(map(str, s)))
+def test_cavity_iterates(dev, shape):
+    c = cavity.generate(*shape, gamma=1e-3, ops=cavity.OP_BITS["L"])
+    L, n, nall = c.op("L"), c.n_inner, c.n_all
+    b = np.zeros(nall)
+    b[:n] = cavity.rhs_normal(n, 4)
+    x0 = np.zeros(nall)
+    A = hip.Matrix.from_csr(dev, L)
+    solver = hip.PCG(A, nall)
+    dx, orc = dev.array(nall), pyoracle.Csr.of(L)
+    for maxit in (1, 2, 3, 6):
+        for precond in (True, False):
+            r = solver.solve(dev.to_device(b), dx, dev.to_device(x0), maxit=maxit, precond=precond)
+            assert r.iters == maxit
+            if precond:
+                want, st, it, rel = pyoracle.pcg(orc, b, x0, n, maxit)
+                assert np.linalg.norm(dx.download() - want) <= 1e-12 * np.linalg.norm(want), maxit
+    # a solver made before its operator's values changed keeps their diagonal
+    A.set_values(2.0 * L.val)
+    r = solver.solve(dev.to_device(b), dx, dev.to_device(x0), maxit=5)
+    got = dx.download()
+    F = hip.Matrix(dev, L.rowptr, L.col, 2.0 * L.val, nrows=n)
+    fresh = hip.PCG(F, nall)
+    fresh.solve(dev.to_device(b), dx, dev.to_device(x0), maxit=5)
+    want = dx.download()
+    assert np.linalg.norm(got - want) <= 1e-12 * np.linalg.norm(want)
+
+
+def test_breakdown_keeps_the_updates_made(dev):
+    """A right-hand side the solve meets exactly after two iterations: the third
+    breaks down (p.Ap = 0) with x complete, whatever parity it stops at."""
+    n = 2 ** 19 + 64
+    T = sp.identity(n, format="csr") * 2.0
+    T = (T + sp.csr_matrix(([1.0, 1.0], ([0, 1], [1, 0])), shape=(n, n))).tocsr()
+    T.sort_indices()
+    M = hip.Matrix(dev, T.indptr, T.indices, T.data, ncols=n)
+    solver = hip.PCG(M, n)
+    b = np.ones(n)
+    dx = dev.array(n)
+    r = solver.solve(dev.to_device(b), dx, dev.to_device(np.zeros(n)), maxit=50, raise_on_breakdown=False)
+    x = dx.download()
+    print(f"[breakdown] iters {r.iters} status {r.status}", flush=True)
+    assert np.all(np.isfinite(x))
+    assert np.linalg.norm(b - T @ x) <= 1e-9 * np.linalg.norm(b)
