@@ -108,6 +108,8 @@ struct PcgDev {
     double *chunk_s;  // long operators: a second array of per-wavefront partials (FP64: r.r; MIXED: 1.Ap)
     double *x, *r, *s, *Ap;
     const double *b, *dinv;
+    SP<double> *sp[2];   // small operators: the pairs (s, p) by iteration parity
+    SP<float> *sp32[2];  // (iteration k's p, then its s, go into those of parity k)
     float *r32, *s32, *Ap32, *xc32;
     const float *dinv32;
     const float *az32;  // A 1 in FP32 (MIXED deflation)
@@ -236,16 +238,19 @@ __device__ inline float s_of(const PcgDev &d, int row, float r) {
 // ---- setup ---------------------------------------------------------------
 
 // x = x0 (all), direction buffers = x0 outside the solved rows,
-// Ap = (A x0)_i or x0_i on empty rows, r = b + (-1.0) Ap   (:55-70)
+// Ap = (A x0)_i or x0_i on empty rows, r = b + (-1.0) Ap   (:55-70); p null:
+// the directions are the pairs' (small operators)
 template <int W>
 __global__ __launch_bounds__(kBlock) void k_setup_resid(EllView A, PcgDev d, const double *__restrict__ x0, int n_all,
                                                         double *__restrict__ p, double *__restrict__ p2) {
     const int stride = gridDim.x * kBlock;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < n_all; i += stride) {
         d.x[i] = x0[i];
-        if (i >= d.n) {
+        if (i >= d.n && p) {
             p[i] = x0[i];
-            if (p2) p2[i] = x0[i];
+            p2[i] = x0[i];
+        } else if (i >= d.n) {
+            d.sp[0][i] = d.sp[1][i] = SP<double>{0.0, x0[i]};
         }
     }
     Operand<double> xo{x0};
@@ -270,7 +275,10 @@ __global__ __launch_bounds__(kBlock) void k_setup_dir(PcgDev d, double *__restri
         } else {
             pi = ri;
         }
-        p[row] = pi;
+        if (p)
+            p[row] = pi;
+        else
+            d.sp[0][row].p = pi;
         rs = rs + ri * pi;
         bb = bb + d.b[row] * d.b[row];
         rr = rr + ri * ri;
@@ -310,15 +318,6 @@ __device__ inline void store_alpha(const PcgDev &d, int k, double alpha) {
     if (leader()) d.sc[S_ALPHA0 + (k & 1)] = alpha;
 }
 
-// x += alpha_k p over the solved rows
-__device__ inline void x_update(const PcgDev &d, const double *__restrict__ p, double alpha) {
-    double *__restrict__ x = d.x;
-    FOR_ROWS(d.n, row) {
-        const double xo = x[row], po = p[row];
-        x[row] = xo + alpha * po;  // :95
-    }
-}
-
 // A product operand that also keeps the value it reads at the row's own
 // column (the p_i of p.Ap, which the row's diagonal entry reads anyway), so
 // that the product does not load it a second time (FP64 product: 1.8%
@@ -350,58 +349,67 @@ struct SelfOperand {
 // partial arrays are summed one at a time, which keeps the register count,
 // and with it the occupancy of the sweep, low.
 
-// x += alpha_k p of the last iteration k
-__global__ __launch_bounds__(kBlock) void k_x_flush(PcgDev d, const double *__restrict__ p, int k) {
+// x += alpha_k p of the last iteration k (small operators)
+__global__ __launch_bounds__(kBlock) void k_x_flush(PcgDev d, int k) {
     if (!running(d)) return;
-    x_update(d, p, alpha_slot(d, k));
+    const double alpha = alpha_slot(d, k);
+    const SP<double> *__restrict__ sp = d.sp[k & 1];
+    FOR_ROWS(d.n, row) d.x[row] = d.x[row] + alpha * sp[row].p;  // :95
 }
 
 // K1: Ap = A p (empty rows keep Ap), p.Ap partials; one row per thread.
 // Long operators: workgroups in dispatch order, one partial per wavefront
 // (with the direction and update sweeps in dispatch order too, 2% faster
 // per FP64 iteration at 256^3 than the XCD-contiguous order, which keeps
-// the neighbour gathers in one XCD's L2).  SMALL: XCD-contiguous order,
-// one partial per chunk.  Both test the state word after the row's loads
-// instead of before them, taking its latency off the kernel's critical
-// path (FP64 solve at 256^3: 1256 -> 1238 ms); a finished solve then still
+// the neighbour gathers in one XCD's L2).  The state word is tested after
+// the row's loads instead of before them, taking its latency off the kernel's
+// critical path (FP64 solve at 256^3: 1256 -> 1238 ms); a finished solve then still
 // reads the operator, but stores nothing.  (The same reordering in the
 // long direction and update sweeps made the solve slower: 1303 ms.)
 // SYM: the slot values from the operator's symmetric form (stencil layout).
-template <int W, bool SMALL, bool SYM = false>
+template <int W, bool SYM = false>
 __device__ inline void iter_spmv(const EllView &A, const PcgDev &d, const double *__restrict__ p) {
-    if constexpr (!SMALL) {
-        const int st = state_load(d.state);  // tested after the row's loads, before any store
-        const int c = blockIdx.x;
-        const int row = c * kBlock + threadIdx.x;
-        double acc = 0.0, sum = 0.0, pr = 0.0;
-        bool any = false;
-        if (row < d.n) {
-            const SelfOperand<double> po{p, row, 0.0, false};
-            if constexpr (SYM)
-                any = row_dot_sym<W, double, double>(A, A.val, A.sym, po, row, sum);
-            else
-                any = row_dot<W, double, double>(A, A.val, po, row, sum);
-            if (!any) sum = d.Ap[row];  // empty row: Ap keeps its value
-            pr = po.found ? po.self : p[row];
-        }
-        if (st != ST_RUN) return;
-        if (row < d.n) {
-            if (any) d.Ap[row] = sum;
-            acc = pr * sum;
-        }
-        // one partial per wavefront: no barrier, each wavefront retires alone
-        acc = wave_sum_63(acc);
-        if ((threadIdx.x & 63) == 63) d.chunk[c * kWaves + (threadIdx.x >> 6)] = acc;
-        return;
+    const int st = state_load(d.state);  // tested after the row's loads, before any store
+    const int c = blockIdx.x;
+    const int row = c * kBlock + threadIdx.x;
+    double acc = 0.0, sum = 0.0, pr = 0.0;
+    bool any = false;
+    if (row < d.n) {
+        const SelfOperand<double> po{p, row, 0.0, false};
+        if constexpr (SYM)
+            any = row_dot_sym<W, double, double>(A, A.val, A.sym, po, row, sum);
+        else
+            any = row_dot<W, double, double>(A, A.val, po, row, sum);
+        if (!any) sum = d.Ap[row];  // empty row: Ap keeps its value
+        pr = po.found ? po.self : p[row];
     }
+    if (st != ST_RUN) return;
+    if (row < d.n) {
+        if (any) d.Ap[row] = sum;
+        acc = pr * sum;
+    }
+    // one partial per wavefront: no barrier, each wavefront retires alone
+    acc = wave_sum_63(acc);
+    if ((threadIdx.x & 63) == 63) d.chunk[c * kWaves + (threadIdx.x >> 6)] = acc;
+}
+
+template <int W>
+__global__ __launch_bounds__(kBlock) void k_iter_spmv(EllView A, PcgDev d, const double *__restrict__ p) {
+    iter_spmv<W>(A, d, p);
+}
+
+// the first product of a small operator: p_0 from the pairs, XCD-contiguous
+// order, one partial per chunk
+template <int W>
+__global__ __launch_bounds__(kBlock) void k_iter_spmv_small(EllView A, PcgDev d) {
     const int st = state_load(d.state);
     const int c = xcd_block(blockIdx.x, gridDim.x);
     const int row = c * kBlock + threadIdx.x;
     double pr = 0.0, sum = 0.0;
     bool any = false;
     if (row < d.n) {
-        Operand<double> po{p};
-        pr = p[row];
+        const PairOperand<double> po{d.sp[0]};
+        pr = po.at(row);
         any = row_dot<W, double, double>(A, A.val, po, row, sum);
         if (!any) sum = d.Ap[row];  // empty row: Ap keeps its value
     }
@@ -413,18 +421,8 @@ __device__ inline void iter_spmv(const EllView &A, const PcgDev &d, const double
 }
 
 template <int W>
-__global__ __launch_bounds__(kBlock) void k_iter_spmv(EllView A, PcgDev d, const double *__restrict__ p) {
-    iter_spmv<W, false>(A, d, p);
-}
-
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_iter_spmv_small(EllView A, PcgDev d, const double *__restrict__ p) {
-    iter_spmv<W, true>(A, d, p);
-}
-
-template <int W>
 __global__ __launch_bounds__(kBlock) void k_iter_spmv_sym(EllView A, PcgDev d, const double *__restrict__ p) {
-    iter_spmv<W, false, true>(A, d, p);
+    iter_spmv<W, true>(A, d, p);
 }
 
 // K1 with the slot values from the dictionary.  The wavefront sums of a
@@ -460,61 +458,146 @@ __global__ __launch_bounds__(kBlock) void k_iter_spmv_dict(EllView A, PcgDev d, 
     chunk_store<R, 1>(d, sh);
 }
 
-// The direction p_k = 1.0 s + beta p_{k-1} read at any column j of the
-// product, computed exactly as the direction update computes it on the
-// solved rows (:113, no contraction: the same bits); past the solved rows
-// (ghost columns) the direction keeps its value.
-struct DirOperand {
-    const double *__restrict__ s, *__restrict__ p;
-    double beta;
-    int n;
-    __device__ inline double at(int j) const {
-        const double po = p[j], si = s[j < n ? j : 0];
-        return j < n ? 1.0 * si + beta * po : po;
+// ---- small operators: prologue and epilogue sums ----------------------------
+//
+// M sums of at most 64 K (WAVE: every wavefront sums all of them by itself,
+// no LDS and no barrier) or 256 K partials (each wavefront its share, one
+// exchange), the same in every lane of every workgroup.  The loads are
+// issued unconditionally at load(), early in a kernel: a slot past n is the
+// array's last entry, a zero whenever n < kMaxRedBlocks.
+constexpr int kSmallK = 8;  // partials per lane
+constexpr int kWaveParts = 64 * kSmallK;
+
+__device__ inline double lane_value(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+template <int M, bool WAVE>
+struct SmallSums {
+    double v[M][kSmallK];
+    __device__ inline void load(const double *const (&part)[M], int n) {
+        const int step = WAVE ? 64 : kBlock, t = WAVE ? threadIdx.x & 63 : threadIdx.x;
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int k = 0; k < kSmallK; ++k) {
+                const int i = t + k * step;
+                v[m][k] = part[m][i < n ? i : kMaxRedBlocks - 1];
+            }
+    }
+    __device__ inline void reduce(double (&out)[M]) {
+        static_assert(M <= 2, "at most two sums");
+        __shared__ double sh[kWaves][2];
+        double acc[2] = {0.0, 0.0};
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int k = 0; k < kSmallK; ++k) acc[m] = acc[m] + v[m][k];
+        const double t = M == 1 ? wave_sum_63(acc[0]) : wave_sum_two(acc[0], acc[1]);
+        if (WAVE) {
+            out[0] = lane_value(t, M == 1 ? 63 : 31);
+            if (M > 1) out[M - 1] = lane_value(t, 63);
+            return;
+        }
+        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+        if (M == 1 ? lane == 63 : (lane & 31) == 31) sh[w][M == 1 ? 0 : lane >> 5] = t;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            double a = sh[0][m];
+#pragma unroll
+            for (int k = 1; k < kWaves; ++k) a = a + sh[k][m];
+            out[m] = a;
+        }
+    }
+};
+
+// M sums over the workgroup, in thread 0 (sh: used nowhere else in the kernel)
+template <int M>
+__device__ inline void small_block_sum(double (&v)[M]) {
+    static_assert(M <= 2, "at most two sums");
+    __shared__ double sh[kWaves][2];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double t = M == 1 ? wave_sum_63(v[0]) : wave_sum_two(v[0], v[M - 1]);
+    if (M == 1 ? lane == 63 : (lane & 31) == 31) sh[w][M == 1 ? 0 : lane >> 5] = t;
+    __syncthreads();
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            v[m] = sh[0][m];
+#pragma unroll
+            for (int k = 1; k < kWaves; ++k) v[m] = v[m] + sh[k][m];
+        }
+}
+
+// The operand row of the fused kernels, requested ahead where the layout
+// lets the kernel know its width (W: as kernel_width).
+template <int W, class T>
+struct RowPre {
+    StencilPre<(W < 0 ? -W : 1), T> st;
+    EllPre<(W > 0 ? W : 1), T> el;
+    __device__ inline void load(const EllView &A, const T *val, const SP<T> *sp, int row) {
+        if constexpr (W < 0)
+            stencil_row_pre<(W < 0 ? -W : 1), T>(A, val, sp, row, st);
+        else if constexpr (W > 0)
+            ell_row_pre<(W > 0 ? W : 1), T>(A, val, sp, row, el);
+    }
+    __device__ inline bool sum(const EllView &A, const T *val, const DirOperand<T> &x, int row, T &out) const {
+        if constexpr (W < 0) {
+            return stencil_row_fin<(W < 0 ? -W : 1), T>(A, val, x, row, st, out);
+        } else if constexpr (W > 0) {
+            out = T(0);
+#pragma unroll
+            for (int k = 0; k < (W > 0 ? W : 1); ++k)
+                out = out + dir_at(el.g[k], el.c[k], x.beta, x.n) * el.v[k];
+            return true;
+        } else {
+            return row_dot<0, T, T>(A, val, x, row, out);
+        }
     }
 };
 
 // Small operators, k >= 1: K0 and K1 in one kernel over the product's grid
 // (one row per thread).  rho_k, the convergence test, x += alpha_{k-1} p_{k-1}
-// on the thread's row, p_k = 1.0 s + beta p_{k-1} into the other direction
-// buffer, Ap = A p_k with p_k formed at every column read, and the p_k.Ap
+// on the thread's row, p_k = 1.0 s + beta p_{k-1} into the other pairs,
+// Ap = A p_k with p_k formed at every column read, and the p_k.Ap
 // partials of iteration k (read by K2 of k while this kernel's own
 // partials of k-1 stay intact: two partial arrays by parity).
 // TOL: a solve with a tolerance (the r.r partials and the convergence
 // test); without one (the reference's fixed iteration count) the prologue
 // sums the rho partials only.
-template <int W, bool TOL>
-__device__ inline void iter_dirprod(const EllView &A, const PcgDev &d, const double *__restrict__ pold,
-                                    double *__restrict__ pnew, int k) {
+template <int W, bool TOL, bool WAVE>
+__device__ inline void iter_dirprod(const EllView &A, const PcgDev &d, int k) {
+    const SP<double> *__restrict__ old = d.sp[(k - 1) & 1];
     const int st = state_load(d.state);
     const int c = xcd_block(blockIdx.x, gridDim.x);
     const int row = c * kBlock + threadIdx.x;
     const bool own = row < d.n;
-    double xo = 0.0, si = 0.0, po = 0.0;
+    double xo = 0.0;
+    SP<double> me{0.0, 0.0};
     if (own) {
         xo = d.x[row];
-        si = d.s[row];
-        po = pold[row];
+        me = old[row];
     }
     const double tol2 = TOL ? early_load(d.sc + S_TOL2) : -1.0;
     const double rho_prev = early_load(d.sc + S_RHO0 + ((k - 1) & 1));
     const double alpha = early_load(d.sc + S_ALPHA0 + ((k - 1) & 1));  // alpha_{k-1}, as K2 of k-1 formed it (:93)
     constexpr int NS = TOL ? 2 : 1;
-    PaddedSums<NS> ps;
+    SmallSums<NS, WAVE> ps;
     if constexpr (TOL)
-        ps.load({d.P(P_RS), d.P(P_RR)}, {d.G, d.G});
+        ps.load({d.P(P_RS), d.P(P_RR)}, d.G);
     else
-        ps.load({d.P(P_RS)}, {d.G});
-    // stencil layout: the operator's loads (none depends on beta) go out
-    // while the prologue's are in flight
-    constexpr int SW = W < 0 ? -W : 1;
-    StencilPre<SW, double> q;
-    if (W < 0 && own) stencil_row_pre<SW, double>(A, A.val, row, q);
+        ps.load({d.P(P_RS)}, d.G);
+    RowPre<W, double> q;
+    if (own) q.load(A, A.val, old, row);
     double sums[NS];
     ps.reduce(sums);
     if (st != ST_RUN && st != conv_stamp(k)) return;
     if (TOL && tol2 >= 0.0 && sums[NS - 1] <= tol2) {  // every workgroup reaches the same decision
-        if (own) d.x[row] = xo + alpha * po;
+        if (own) d.x[row] = xo + alpha * me.p;
         if (leader()) state_store(d.state, conv_stamp(k));
         return;
     }
@@ -522,35 +605,22 @@ __device__ inline void iter_dirprod(const EllView &A, const PcgDev &d, const dou
     if (leader()) d.sc[S_RHO0 + (k & 1)] = sums[0];
     double pr = 0.0, sum = 0.0;
     if (own) {
-        d.x[row] = xo + alpha * po;  // :95 of iteration k-1
-        pr = 1.0 * si + beta * po;   // :113
-        pnew[row] = pr;
-        const DirOperand op{d.s, pold, beta, d.n};
-        bool any;
-        if constexpr (W < 0)
-            any = stencil_row_fin<SW, double, double>(A, A.val, op, row, q, sum);  // :87
-        else
-            any = row_dot<W, double, double>(A, A.val, op, row, sum);
-        if (any)
+        d.x[row] = xo + alpha * me.p;    // :95 of iteration k-1
+        pr = 1.0 * me.s + beta * me.p;   // :113
+        d.sp[k & 1][row].p = pr;
+        if (q.sum(A, A.val, DirOperand<double>{old, beta, d.n}, row, sum))  // :87
             d.Ap[row] = sum;
         else
             sum = d.Ap[row];  // empty row: Ap keeps its value
     }
-    double acc = own ? pr * sum : 0.0;
-    acc = block_reduce<RED_SUM>(acc);
-    if (threadIdx.x == 0) dn_part(d, k)[c] = acc;
+    double acc[1] = {own ? pr * sum : 0.0};
+    small_block_sum<1>(acc);
+    if (threadIdx.x == 0) dn_part(d, k)[c] = acc[0];
 }
 
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_iter_dirprod(EllView A, PcgDev d, const double *__restrict__ pold,
-                                                         double *__restrict__ pnew, int k) {
-    iter_dirprod<W, true>(A, d, pold, pnew, k);
-}
-
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_iter_dirprod_fixed(EllView A, PcgDev d, const double *__restrict__ pold,
-                                                               double *__restrict__ pnew, int k) {
-    iter_dirprod<W, false>(A, d, pold, pnew, k);
+template <int W, bool TOL, bool WAVE>
+__global__ __launch_bounds__(kBlock) void k_iter_dirprod(EllView A, PcgDev d, int k) {
+    iter_dirprod<W, TOL, WAVE>(A, d, k);
 }
 
 // the per-wavefront partials of the long products, folded in index order:
@@ -582,58 +652,50 @@ __global__ __launch_bounds__(kBlock) void k_fold_dn(PcgDev d) {
 }
 
 // K2 (operators of at most 2^19 rows): alpha_k, r += (-alpha) Ap, s = Dinv r,
-// partials of r.s and r.r; each row's operands are loaded together (one
-// round trip per row), requested before the prologue's sums
+// partials of r.s and r.r; one row per thread, its operands requested before
+// the prologue's sums
+template <bool WAVE>
 __global__ __launch_bounds__(kBlock) void k_iter_update(PcgDev d, int k) {
-    double *__restrict__ r = d.r, *__restrict__ s = d.s;
-    const double *__restrict__ Ap = d.Ap, *__restrict__ dinv = d.dinv;
     const bool precond = d.precond != 0;
-    double rs = 0.0, rr = 0.0;
-    {
-        ThreadRows t(d.n);
-        double ro = 0.0, apr = 0.0, di = 0.0;
-        const int st = state_load(d.state);
-        if (t.valid()) {
-            ro = r[t.row];
-            apr = Ap[t.row];
-            if (precond) di = dinv[t.row];
-        }
-        const double rho = early_load(d.sc + S_RHO0 + (k & 1));
-        double sums[1];
-        sum_padded<1>({dn_part(d, k)}, {d.Gdn}, sums);
-        const double dn = sums[0];
-        if (st != ST_RUN) return;
-        const double alpha = rho / dn;
-        if (dn == 0.0 || !isfinite(dn) || !isfinite(alpha)) {
-            if (leader()) state_store(d.state, ST_BREAK);
-            return;
-        }
-        store_alpha(d, k, alpha);
-        const double malpha = -1.0 * alpha;
-        while (t.valid()) {
-            const int row = t.row;
-            const double ri = ro + malpha * apr;  // :97
-            r[row] = ri;
-            double si;
-            if (precond) {  // :99-105
-                si = 0.0;
-                si = si + ri * di;
-            } else {
-                si = ri;
-            }
-            s[row] = si;
-            rs = rs + ri * si;
-            rr = rr + ri * ri;
-            t.next();
-            if (t.valid()) {
-                ro = r[t.row];
-                apr = Ap[t.row];
-                if (precond) di = dinv[t.row];
-            }
-        }
+    const ThreadRows t(d.n);
+    const bool own = t.valid();
+    double ro = 0.0, apr = 0.0, di = 0.0;
+    const int st = state_load(d.state);
+    if (own) {
+        ro = d.r[t.row];
+        apr = d.Ap[t.row];
+        if (precond) di = d.dinv[t.row];
     }
-    double red[2] = {rs, rr};
-    block_reduce_n<2>(red);
+    const double rho = early_load(d.sc + S_RHO0 + (k & 1));
+    SmallSums<1, WAVE> ps;
+    ps.load({dn_part(d, k)}, d.Gdn);
+    double sums[1];
+    ps.reduce(sums);
+    const double dn = sums[0];
+    if (st != ST_RUN) return;
+    const double alpha = rho / dn;
+    if (dn == 0.0 || !isfinite(dn) || !isfinite(alpha)) {
+        if (leader()) state_store(d.state, ST_BREAK);
+        return;
+    }
+    store_alpha(d, k, alpha);
+    const double malpha = -1.0 * alpha;
+    double red[2] = {0.0, 0.0};
+    if (own) {
+        const double ri = ro + malpha * apr;  // :97
+        d.r[t.row] = ri;
+        double si;
+        if (precond) {  // :99-105
+            si = 0.0;
+            si = si + ri * di;
+        } else {
+            si = ri;
+        }
+        d.sp[k & 1][t.row].s = si;
+        red[0] = ri * si;
+        red[1] = ri * ri;
+    }
+    small_block_sum<2>(red);
     if (threadIdx.x == 0) {
         d.P(P_RS)[blockIdx.x] = red[0];
         d.P(P_RR)[blockIdx.x] = red[1];
@@ -958,106 +1020,88 @@ __global__ __launch_bounds__(kBlock) void k_m_dir(PcgDev d, const float *__restr
     }
 }
 
-// (as DirOperand, in FP32: the direction update's float expression)
-struct DirOperand32 {
-    const float *__restrict__ s, *__restrict__ p;
-    float beta;
-    int n;
-    __device__ inline float at(int j) const {
-        const float po = p[j], si = s[j < n ? j : 0];
-        return j < n ? si + beta * po : po;
-    }
-};
-
 // Small operators, k >= 1: k_m_dir and the FP32 product in one kernel (as
-// k_iter_dirprod)
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_m_dirprod(EllView A, PcgDev d, const float *__restrict__ pold,
-                                                      float *__restrict__ pnew, int k, int pending) {
+// iter_dirprod)
+template <int W, bool WAVE>
+__global__ __launch_bounds__(kBlock) void k_m_dirprod(EllView A, PcgDev d, int k, int pending) {
+    const SP<float> *__restrict__ old = d.sp32[(k - 1) & 1];
     const int st = state_load(d.state);
     const int c = xcd_block(blockIdx.x, gridDim.x);
     const int row = c * kBlock + threadIdx.x;
     const bool own = row < d.n;
-    float xo = 0.0f, si = 0.0f, po = 0.0f;
+    float xo = 0.0f;
+    SP<float> me{0.0f, 0.0f};
     if (own) {
         xo = d.xc32[row];
-        si = d.s32[row];
-        po = pold[row];
+        me = old[row];
     }
     const double rho_prev = early_load(d.sc + S_RHO0 + ((k - 1) & 1));
     const double alpha = early_load(d.sc + S_ALPHA0 + ((k - 1) & 1));  // alpha_{k-1}, as K2 of k-1 formed it
-    const double zaz = early_load(d.sc + S_ZAZ);
-    PaddedSums<1> ps;
-    ps.load({d.P(P_RS)}, {d.G});
-    constexpr int SW = W < 0 ? -W : 1;
-    StencilPre<SW, float> q;
-    if (W < 0 && own) stencil_row_pre<SW, float>(A, A.val32, row, q);
+    SmallSums<1, WAVE> ps;
+    ps.load({d.P(P_RS)}, d.G);
+    RowPre<W, float> q;
+    if (own) q.load(A, A.val32, old, row);
     double sums[1];
     ps.reduce(sums);
     if (st != ST_RUN) return;
-    const bool dfl = deflating(d, zaz);
     const float a32 = pending ? (float)alpha : 0.0f;
     const float beta = (float)(sums[0] / rho_prev);
     if (leader()) d.sc[S_RHO0 + (k & 1)] = sums[0];
-    double acc = 0.0, sa = 0.0;
+    double red[2] = {0.0, 0.0};
     if (own) {
-        if (pending) d.xc32[row] = xo + a32 * po;
-        const float pr = si + beta * po;
-        pnew[row] = pr;
-        const DirOperand32 op{d.s32, pold, beta, d.n};
+        if (pending) d.xc32[row] = xo + a32 * me.p;
+        const float pr = me.s + beta * me.p;
+        d.sp32[k & 1][row].p = pr;
         float sum;
-        if constexpr (W < 0)
-            stencil_row_fin<SW, float, float>(A, A.val32, op, row, q, sum);
-        else
-            row_dot<W, float, float>(A, A.val32, op, row, sum);
+        q.sum(A, A.val32, DirOperand<float>{old, beta, d.n}, row, sum);
+        d.Ap32[row] = sum;
+        red[0] = (double)pr * (double)sum;
+        red[1] = (double)sum;
+    }
+    small_block_sum<2>(red);
+    if (threadIdx.x == 0) {
+        dn_part(d, k)[c] = red[0];
+        sa_part(d, k)[c] = red[1];
+    }
+}
+
+// K1 in FP32 (the symmetric form of the slot values measured slower here,
+// 121-131 against 118.5 us at 256^3, so the FP32 product keeps the full slot
+// values).  No state test: the product's stores (Ap32, its partials) are
+// read only by the fold and the update, which test it; and mixed iterations
+// are queued only while the solve runs (convergence is decided at a defect
+// correction, after which nothing is queued).
+template <int W>
+__global__ __launch_bounds__(kBlock) void k_m_spmv(EllView A, PcgDev d, const float *__restrict__ p) {
+    const int c = xcd_block(blockIdx.x, gridDim.x);
+    const int row = c * kBlock + threadIdx.x;
+    double acc = 0.0, sa = 0.0;
+    if (row < d.n) {
+        // (a SelfOperand here measured 9% slower than the separate load)
+        Operand<float> po{p};
+        const float pr = p[row];
+        float sum;
+        row_dot<W, float, float>(A, A.val32, po, row, sum);
         d.Ap32[row] = sum;
         acc = (double)pr * (double)sum;
         sa = (double)sum;
     }
-    double red[2] = {acc, sa};
-    block_reduce_n<2>(red);
-    if (threadIdx.x == 0) {
-        dn_part(d, k)[c] = red[0];
-        if (dfl) sa_part(d, k)[c] = red[1];
-    }
+    const int wv = c * kWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    acc = wave_sum_two(acc, sa);
+    if (lane == 31) d.chunk[wv] = acc;
+    if (lane == 63) d.chunk_s[wv] = acc;
 }
 
-// K1 in FP32 (SMALL as in iter_spmv; the symmetric form of the slot values
-// measured slower here, 121-131 against 118.5 us at 256^3, so the FP32
-// product keeps the full slot values)
-template <int W, bool SMALL>
-__device__ inline void m_spmv(const EllView &A, const PcgDev &d, const float *__restrict__ p) {
-    if constexpr (!SMALL) {
-        // no state test: the product's stores (Ap32, its partials) are read
-        // only by the fold and the update, which test it; and mixed
-        // iterations are queued only while the solve runs (convergence is
-        // decided at a defect correction, after which nothing is queued)
-        const int c = xcd_block(blockIdx.x, gridDim.x);
-        const int row = c * kBlock + threadIdx.x;
-        double acc = 0.0, sa = 0.0;
-        if (row < d.n) {
-            // (a SelfOperand here measured 9% slower than the separate load)
-            Operand<float> po{p};
-            const float pr = p[row];
-            float sum;
-            row_dot<W, float, float>(A, A.val32, po, row, sum);
-            d.Ap32[row] = sum;
-            acc = (double)pr * (double)sum;
-            sa = (double)sum;
-        }
-        const int wv = c * kWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-        acc = wave_sum_two(acc, sa);
-        if (lane == 31) d.chunk[wv] = acc;
-        if (lane == 63) d.chunk_s[wv] = acc;
-        return;
-    }
+// the first product of a small operator (as k_iter_spmv_small)
+template <int W>
+__global__ __launch_bounds__(kBlock) void k_m_spmv_small(EllView A, PcgDev d) {
     const int st = state_load(d.state);
     const int c = xcd_block(blockIdx.x, gridDim.x);
     const int row = c * kBlock + threadIdx.x;
     float pr = 0.0f, sum = 0.0f;
     if (row < d.n) {
-        Operand<float> po{p};
-        pr = p[row];
+        const PairOperand<float> po{d.sp32[0]};
+        pr = po.at(row);
         row_dot<W, float, float>(A, A.val32, po, row, sum);
     }
     if (st != ST_RUN) return;
@@ -1075,16 +1119,6 @@ __device__ inline void m_spmv(const EllView &A, const PcgDev &d, const float *__
     }
 }
 
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_m_spmv(EllView A, PcgDev d, const float *__restrict__ p) {
-    m_spmv<W, false>(A, d, p);
-}
-
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_m_spmv_small(EllView A, PcgDev d, const float *__restrict__ p) {
-    m_spmv<W, true>(A, d, p);
-}
-
 // (as k_iter_spmv_dict)
 template <int SW, int R>
 __global__ __launch_bounds__(kBlock) void k_m_spmv_dict(EllView A, PcgDev d, const float *__restrict__ p) {
@@ -1100,127 +1134,82 @@ __global__ __launch_bounds__(kBlock) void k_m_spmv_dict(EllView A, PcgDev d, con
     chunk_store<R, 2>(d, sh);
 }
 
-template <bool SMALL, bool LEAN = false>
+template <bool LEAN>
 __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
     float *__restrict__ r = d.r32, *__restrict__ s = d.s32;
     const float *__restrict__ Ap = d.Ap32, *__restrict__ dinv = d.dinv32;
     const bool precond = d.precond != 0;
     double rs = 0.0, rr = 0.0;
-    if constexpr (!SMALL) {
-        if (!running(d)) return;
-        // every prologue load issued before the first is used: 1.A1, the
-        // list of A 1's nonzeros, and the p.Ap and 1.Ap partials (summed
-        // together; alpha goes to its scalar slot, so later kernels need
-        // not reproduce this sum)
-        const double zaz = d.sc[S_ZAZ];
-        const int naz_all = d.azl->count;
-        int li[kAzList];
-        float lv[kAzList];
+    if (!running(d)) return;
+    // every prologue load issued before the first is used: 1.A1, the
+    // list of A 1's nonzeros, and the p.Ap and 1.Ap partials (summed
+    // together; alpha goes to its scalar slot, so later kernels need
+    // not reproduce this sum)
+    const double zaz = d.sc[S_ZAZ];
+    const int naz_all = d.azl->count;
+    int li[kAzList];
+    float lv[kAzList];
 #pragma unroll
-        for (int j = 0; j < kAzList; ++j) {
-            li[j] = d.azl->idx[j];
-            lv[j] = d.azl->val[j];
-        }
-        double sums[2];
-        if (d.Gdn <= kBlock)  // one round of the uniform loop (up to 256^3)
-            sum_partials_n<2>({d.P(P_DN), d.P(P_SA)}, d.Gdn, sums);
-        else  // all slots in one round trip
-            sum_padded<2>({d.P(P_DN), d.P(P_SA)}, {d.Gdn, d.Gdn}, sums);
-        const bool dfl = deflating(d, zaz);
-        const double sap = dfl ? sums[1] : 0.0;
-        const double dn = m_denom(sums[0], sap, zaz, dfl);
-        const double alpha = rho_slot(d, k) / dn;
-        if (dn == 0.0 || !isfinite(dn) || !isfinite(alpha)) {
-            if (leader()) state_store(d.state, ST_BREAK);
-            return;
-        }
-        store_alpha(d, k, alpha);
-        const float a32 = (float)alpha, c32 = dfl ? (float)(sap / zaz) : 0.0f;
-        const float *__restrict__ az = d.az32;
-        // A 1 from its list of nonzeros when it is short (the same values
-        // as the dense array, without streaming it), else row by row
-        const int naz = dfl ? naz_all : 0;
-        const bool listed = naz <= kAzList;
+    for (int j = 0; j < kAzList; ++j) {
+        li[j] = d.azl->idx[j];
+        lv[j] = d.azl->val[j];
+    }
+    double sums[2];
+    if (d.Gdn <= kBlock)  // one round of the uniform loop (up to 256^3)
+        sum_partials_n<2>({d.P(P_DN), d.P(P_SA)}, d.Gdn, sums);
+    else  // all slots in one round trip
+        sum_padded<2>({d.P(P_DN), d.P(P_SA)}, {d.Gdn, d.Gdn}, sums);
+    const bool dfl = deflating(d, zaz);
+    const double sap = dfl ? sums[1] : 0.0;
+    const double dn = m_denom(sums[0], sap, zaz, dfl);
+    const double alpha = rho_slot(d, k) / dn;
+    if (dn == 0.0 || !isfinite(dn) || !isfinite(alpha)) {
+        if (leader()) state_store(d.state, ST_BREAK);
+        return;
+    }
+    store_alpha(d, k, alpha);
+    const float a32 = (float)alpha, c32 = dfl ? (float)(sap / zaz) : 0.0f;
+    const float *__restrict__ az = d.az32;
+    // A 1 from its list of nonzeros when it is short (the same values
+    // as the dense array, without streaming it), else row by row
+    const int naz = dfl ? naz_all : 0;
+    const bool listed = naz <= kAzList;
 #pragma unroll
-        for (int j = 0; j < kAzList; ++j) li[j] = j < naz ? li[j] : -1;
-        struct In {
-            float r, ap, di;
-        };
-        sweep_rows<kSweepU<LEAN>>(
-            d.n,
-            [&](int row) {
-                return In{__builtin_nontemporal_load(r + row), __builtin_nontemporal_load(Ap + row),
-                          !precond ? 0.0f
-                          : LEAN   ? dict_one(d.dc_sel, d.dc_id, d.ddinv32, row)
-                                   : __builtin_nontemporal_load(dinv + row)};
-            },
-            [&](int row, const In &v) {
-                float azr = 0.0f;
-                if (dfl && !listed) {
-                    azr = az[row];
-                } else {
-                    // rows compared with the list only in a chunk that holds a
-                    // listed row (a workgroup-uniform test per chunk)
-                    const int base = __builtin_amdgcn_readfirstlane(row - (int)threadIdx.x);
-                    bool hit = false;
+    for (int j = 0; j < kAzList; ++j) li[j] = j < naz ? li[j] : -1;
+    struct In {
+        float r, ap, di;
+    };
+    sweep_rows<kSweepU<LEAN>>(
+        d.n,
+        [&](int row) {
+            return In{__builtin_nontemporal_load(r + row), __builtin_nontemporal_load(Ap + row),
+                      !precond ? 0.0f
+                      : LEAN   ? dict_one(d.dc_sel, d.dc_id, d.ddinv32, row)
+                               : __builtin_nontemporal_load(dinv + row)};
+        },
+        [&](int row, const In &v) {
+            float azr = 0.0f;
+            if (dfl && !listed) {
+                azr = az[row];
+            } else {
+                // rows compared with the list only in a chunk that holds a
+                // listed row (a workgroup-uniform test per chunk)
+                const int base = __builtin_amdgcn_readfirstlane(row - (int)threadIdx.x);
+                bool hit = false;
 #pragma unroll
-                    for (int j = 0; j < kAzList; ++j) hit = hit || (unsigned)(li[j] - base) < (unsigned)kBlock;
-                    if (hit)
+                for (int j = 0; j < kAzList; ++j) hit = hit || (unsigned)(li[j] - base) < (unsigned)kBlock;
+                if (hit)
 #pragma unroll
-                        for (int j = 0; j < kAzList; ++j) azr = row == li[j] ? lv[j] : azr;
-                }
-                const float wr = dfl ? v.ap - c32 * azr : v.ap;  // (P A p)_row
-                const float ri = v.r - a32 * wr;
-                __builtin_nontemporal_store(ri, r + row);
-                const float si = precond ? ri * v.di : ri;
-                if (!LEAN) __builtin_nontemporal_store(si, s + row);
-                rs = rs + (double)ri * (double)si;
-                rr = rr + (double)ri * (double)ri;
-            });
-    } else {
-        ThreadRows t(d.n);
-        float ro = 0.0f, apr = 0.0f, di = 0.0f, azr = 0.0f;
-        const float *__restrict__ az = d.az32;
-        const int st = state_load(d.state);
-        const bool want_az = d.deflate != 0;
-        if (t.valid()) {
-            ro = r[t.row];
-            apr = Ap[t.row];
-            if (precond) di = dinv[t.row];
-            if (want_az) azr = az[t.row];
-        }
-        const double rho = early_load(d.sc + S_RHO0 + (k & 1));
-        const double zaz = early_load(d.sc + S_ZAZ);
-        double sums[2];
-        sum_padded<2>({dn_part(d, k), sa_part(d, k)}, {d.Gdn, d.Gdn}, sums);
-        if (st != ST_RUN) return;
-        const bool dfl = deflating(d, zaz);
-        const double dn = m_denom(sums[0], sums[1], zaz, dfl);
-        const double alpha = rho / dn;
-        if (dn == 0.0 || !isfinite(dn) || !isfinite(alpha)) {
-            if (leader()) state_store(d.state, ST_BREAK);
-            return;
-        }
-        store_alpha(d, k, alpha);
-        const float a32 = (float)alpha, c32 = dfl ? (float)(sums[1] / zaz) : 0.0f;
-        while (t.valid()) {
-            const int row = t.row;
-            const float wr = dfl ? apr - c32 * azr : apr;  // (P A p)_row
-            const float ri = ro - a32 * wr;
-            r[row] = ri;
-            const float si = precond ? ri * di : ri;
-            s[row] = si;
+                    for (int j = 0; j < kAzList; ++j) azr = row == li[j] ? lv[j] : azr;
+            }
+            const float wr = dfl ? v.ap - c32 * azr : v.ap;  // (P A p)_row
+            const float ri = v.r - a32 * wr;
+            __builtin_nontemporal_store(ri, r + row);
+            const float si = precond ? ri * v.di : ri;
+            if (!LEAN) __builtin_nontemporal_store(si, s + row);
             rs = rs + (double)ri * (double)si;
             rr = rr + (double)ri * (double)ri;
-            t.next();
-            if (t.valid()) {
-                ro = r[t.row];
-                apr = Ap[t.row];
-                if (precond) di = dinv[t.row];
-                if (want_az) azr = az[t.row];
-            }
-        }
-    }
+        });
     double red[2] = {rs, rr};
     block_reduce_n<2>(red);
     if (threadIdx.x == 0) {
@@ -1228,6 +1217,78 @@ __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
         d.P(P_RR)[blockIdx.x] = red[1];
     }
     if (leader()) *d.iters = k + 1;
+}
+
+// the update of a small operator (as k_iter_update)
+template <bool WAVE>
+__global__ __launch_bounds__(kBlock) void k_m_update_small(PcgDev d, int k) {
+    const bool precond = d.precond != 0, want_az = d.deflate != 0;
+    const ThreadRows t(d.n);
+    const bool own = t.valid();
+    float ro = 0.0f, apr = 0.0f, di = 0.0f, azr = 0.0f;
+    const int st = state_load(d.state);
+    if (own) {
+        ro = d.r32[t.row];
+        apr = d.Ap32[t.row];
+        if (precond) di = d.dinv32[t.row];
+        if (want_az) azr = d.az32[t.row];
+    }
+    const double rho = early_load(d.sc + S_RHO0 + (k & 1));
+    const double zaz = early_load(d.sc + S_ZAZ);
+    SmallSums<2, WAVE> ps;
+    ps.load({dn_part(d, k), sa_part(d, k)}, d.Gdn);
+    double sums[2];
+    ps.reduce(sums);
+    if (st != ST_RUN) return;
+    const bool dfl = deflating(d, zaz);
+    const double dn = m_denom(sums[0], sums[1], zaz, dfl);
+    const double alpha = rho / dn;
+    if (dn == 0.0 || !isfinite(dn) || !isfinite(alpha)) {
+        if (leader()) state_store(d.state, ST_BREAK);
+        return;
+    }
+    store_alpha(d, k, alpha);
+    const float a32 = (float)alpha, c32 = dfl ? (float)(sums[1] / zaz) : 0.0f;
+    double red[2] = {0.0, 0.0};
+    if (own) {
+        const float wr = dfl ? apr - c32 * azr : apr;  // (P A p)_row
+        const float ri = ro - a32 * wr;
+        d.r32[t.row] = ri;
+        const float si = precond ? ri * di : ri;
+        d.sp32[k & 1][t.row].s = si;
+        red[0] = (double)ri * (double)si;
+        red[1] = (double)ri * (double)ri;
+    }
+    small_block_sum<2>(red);
+    if (threadIdx.x == 0) {
+        d.P(P_RS)[blockIdx.x] = red[0];
+        d.P(P_RR)[blockIdx.x] = red[1];
+    }
+    if (leader()) *d.iters = k + 1;
+}
+
+// the replaced s of a correction (or of the start, with the first direction
+// p = s and a zero correction) into the pairs that the next iteration reads
+__global__ __launch_bounds__(kBlock) void k_m_pairs(PcgDev d, SP<float> *__restrict__ sp, int first) {
+    FOR_ROWS(d.n, row) {
+        const float s = d.s32[row];
+        sp[row].s = s;
+        if (first) {
+            sp[row].p = s;
+            d.xc32[row] = 0.0f;
+        }
+    }
+}
+
+// k_m_fold of a small operator
+__global__ __launch_bounds__(kBlock) void k_m_fold_small(PcgDev d, int k) {
+    const float a32 = (float)alpha_slot(d, k);
+    const SP<float> *__restrict__ sp = d.sp32[k & 1];
+    FOR_ROWS(d.n, row) {
+        const float xcv = d.xc32[row] + a32 * sp[row].p;
+        d.x[row] = d.x[row] + (double)xcv;
+        d.xc32[row] = 0.0f;
+    }
 }
 
 // one workgroup: the FP32 recursive r.r for the host's correction test
@@ -1375,8 +1436,8 @@ __global__ __launch_bounds__(kBlock) void k_az32(int n, const double *__restrict
 //
 // The workspace of one FP64 solve on an operator of at most kScratchRows
 // rows lives in `scratch`, a file-scope device array (one copy per GPU, held
-// until the process ends): r, s, Ap, Dinv (kScratchRows doubles each), the
-// two direction buffers (kScratchAll each), the partial-sum arrays, the
+// until the process ends): r, Ap, Dinv (kScratchRows doubles each), the
+// two arrays of pairs (s, p) (kScratchAll pairs each), the partial-sum arrays, the
 // scalars and the state words.  Host code never passes `scratch` itself
 // (in host code the name is a stand-in, not a device address): gip_init
 // looks up its address on each device with hipGetSymbolAddress and keeps it
@@ -1387,7 +1448,7 @@ __global__ __launch_bounds__(kBlock) void k_az32(int n, const double *__restrict
 constexpr int kScratchRows = 1 << 18;
 constexpr int kScratchAll = (1 << 18) + (1 << 16);
 constexpr size_t kScratchZero = (size_t)P_COUNT * kMaxRedBlocks + S_COUNT + 1;  // partials, scalars, state words
-constexpr size_t kScratchDoubles = 4 * (size_t)kScratchRows + 2 * (size_t)kScratchAll + kScratchZero;
+constexpr size_t kScratchDoubles = 3 * (size_t)kScratchRows + 4 * (size_t)kScratchAll + kScratchZero;
 static __device__ __align__(256) double scratch[kScratchDoubles];
 constexpr int kScratchDevices = 64;
 static double *g_scratch[kScratchDevices];
@@ -1417,7 +1478,7 @@ struct gip_pcg {
     gip_ctx *ctx;
     const gip_mat *A;
     int n, n_all, grid;
-    double *r, *p, *s, *Ap, *dinv;
+    double *r, *p, *s, *Ap, *dinv;  // small operators: p and p2 are arrays of pairs (s, p), no s
     float *r32, *p32, *s32, *Ap32, *xc32, *dinv32;
     double *p2;   // second direction buffer (directions alternate by parity)
     float *p32b;  // its FP32 counterpart
@@ -1461,6 +1522,19 @@ static int pcg_grid(int n) {
             default: KERNEL<0><<<GRID, kBlock, 0, st>>>(__VA_ARGS__); break;     \
         }                                                                       \
     } while (0)
+// KERNEL<W, ARGS> over the chunks of a small operator
+#define COMMA(A, B) A, B
+#define DISPATCH_SMALL(A, KERNEL, ARGS, ...)                                              \
+    do {                                                                                  \
+        switch (kernel_width(A)) {                                                        \
+            case 5: KERNEL<5, ARGS><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__); break;    \
+            case 6: KERNEL<6, ARGS><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__); break;    \
+            case 7: KERNEL<7, ARGS><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__); break;    \
+            case -7: KERNEL<-7, ARGS><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__); break;  \
+            case -8: KERNEL<-8, ARGS><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__); break;  \
+            default: KERNEL<0, ARGS><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__); break;   \
+        }                                                                                 \
+    } while (0)
 #define DISPATCH_W(A, KERNEL, ...) DISPATCH_WG(A, S->grid, KERNEL, __VA_ARGS__)
 // the products over the symmetric form: one workgroup per chunk
 #define SYM_LAUNCH(A, KERNEL, ...)                                                    \
@@ -1497,6 +1571,10 @@ static PcgDev make_dev(gip_pcg *S, const double *b, double *x, int precond) {
     d.Ap = S->Ap;
     d.b = b;
     d.dinv = S->dinv;
+    d.sp[0] = reinterpret_cast<SP<double> *>(S->p);
+    d.sp[1] = reinterpret_cast<SP<double> *>(S->p2);
+    d.sp32[0] = reinterpret_cast<SP<float> *>(S->p32);
+    d.sp32[1] = reinterpret_cast<SP<float> *>(S->p32b);
     d.r32 = S->r32;
     d.s32 = S->s32;
     d.Ap32 = S->Ap32;
@@ -1549,9 +1627,10 @@ int gip_pcg_create(gip_ctx *c, const gip_mat *A, int32_t n_all, gip_pcg **out) {
         if (e == hipSuccess) e = hipMalloc(p, bytes);
     };
     dalloc((void **)&S->r, n * 8);
-    dalloc((void **)&S->p, na * 8);
-    dalloc((void **)&S->p2, na * 8);
-    dalloc((void **)&S->s, n * 8);
+    const size_t pb = S->fold ? 8 : sizeof(SP<double>);
+    dalloc((void **)&S->p, na * pb);
+    dalloc((void **)&S->p2, na * pb);
+    if (S->fold) dalloc((void **)&S->s, n * 8);
     dalloc((void **)&S->Ap, n * 8);
     dalloc((void **)&S->dinv, n * 8);
     dalloc((void **)&S->sc, S_COUNT * 8);
@@ -1626,10 +1705,11 @@ static int ensure_mixed(gip_pcg *S) {
     GIP_HIP_TRY(hipMemsetAsync(S->azl, 0, sizeof(AzList), S->ctx->stream));
     // the FP32 direction is an SpMV input: ghost columns included, and zero
     // there (the correction leaves the ghost values of x unchanged)
-    GIP_HIP_TRY(hipMalloc(&S->p32, na * 4));
-    GIP_HIP_TRY(hipMemsetAsync(S->p32, 0, na * 4, S->ctx->stream));
-    GIP_HIP_TRY(hipMalloc(&S->p32b, na * 4));
-    GIP_HIP_TRY(hipMemsetAsync(S->p32b, 0, na * 4, S->ctx->stream));
+    const size_t pb = S->fold ? 4 : sizeof(SP<float>);
+    GIP_HIP_TRY(hipMalloc(&S->p32, na * pb));
+    GIP_HIP_TRY(hipMemsetAsync(S->p32, 0, na * pb, S->ctx->stream));
+    GIP_HIP_TRY(hipMalloc(&S->p32b, na * pb));
+    GIP_HIP_TRY(hipMemsetAsync(S->p32b, 0, na * pb, S->ctx->stream));
     if (S->n) {
         k_to32<<<(S->n + kBlock - 1) / kBlock, kBlock, 0, S->ctx->stream>>>(S->n, S->dinv, S->dinv32);
         GIP_LAUNCH_CHECK("dinv32");
@@ -1708,6 +1788,8 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     const int pollk = o->poll > 0 ? o->poll : 16;
     const int use_coarse = o->coarse >= 0 ? 1 : 0;
     d.deflate = mixed && use_coarse;
+    // small operators: few enough partials for every wavefront to sum them all
+    const bool wave = S->grid <= kWaveParts;
     // direction of iteration k: two buffers by parity
     auto pdir = [&](int k) { return (k & 1) ? S->p2 : S->p; };
     auto pdir32 = [&](int k) { return (k & 1) ? S->p32b : S->p32; };
@@ -1750,8 +1832,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
         armed = false;
     };
     // setup, GIP_LinearSolver.h:55-80
-    DISPATCH_W(A, k_setup_resid, v, d, x0, S->n_all, S->p, S->p2);
-    k_setup_dir<<<S->grid, kBlock, 0, st>>>(d, S->p);
+    double *const dir0 = S->fold ? S->p : nullptr;  // small operators: the pairs in d
+    DISPATCH_W(A, k_setup_resid, v, d, x0, S->n_all, dir0, S->p2);
+    k_setup_dir<<<S->grid, kBlock, 0, st>>>(d, dir0);
     k_setup_fin<<<1, kBlock, 0, st>>>(d, o->tol);
     GIP_LAUNCH_CHECK("pcg setup");
     int corrections = 0, rc;
@@ -1800,14 +1883,22 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                     k_beta_fin<<<1, kBlock, 0, st>>>(d, k + 1, ufold);
                 } else {
                     const bool smp = sample_begin(k);
-                    if (k > 0 && o->tol > 0.0)
-                        DISPATCH_WG(A, S->nchunk, k_iter_dirprod, v, d, pdir(k - 1), pdir(k), k);
-                    else if (k > 0)  // fixed iteration count: no r.r test
-                        DISPATCH_WG(A, S->nchunk, k_iter_dirprod_fixed, v, d, pdir(k - 1), pdir(k), k);
+                    const bool tol = o->tol > 0.0;  // without one (fixed iteration count): no r.r test
+                    if (k == 0)
+                        DISPATCH_WG(A, S->nchunk, k_iter_spmv_small, v, d);
+                    else if (wave && tol)
+                        DISPATCH_SMALL(A, k_iter_dirprod, COMMA(true, true), v, d, k);
+                    else if (wave)
+                        DISPATCH_SMALL(A, k_iter_dirprod, COMMA(false, true), v, d, k);
+                    else if (tol)
+                        DISPATCH_SMALL(A, k_iter_dirprod, COMMA(true, false), v, d, k);
                     else
-                        DISPATCH_WG(A, S->nchunk, k_iter_spmv_small, v, d, S->p);
+                        DISPATCH_SMALL(A, k_iter_dirprod, COMMA(false, false), v, d, k);
                     sample_end(smp);
-                    k_iter_update<<<S->grid, kBlock, 0, st>>>(d, k);
+                    if (wave)
+                        k_iter_update<true><<<S->grid, kBlock, 0, st>>>(d, k);
+                    else
+                        k_iter_update<false><<<S->grid, kBlock, 0, st>>>(d, k);
                 }
             }
             GIP_LAUNCH_CHECK("pcg iteration");
@@ -1819,7 +1910,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
         if (S->fold) {
             if (k > 0) k_x_flush_pair<<<S->grid, kBlock, 0, st>>>(d, S->p, S->p2);
         } else if (k > 0) {
-            k_x_flush<<<S->grid, kBlock, 0, st>>>(d, pdir(k - 1), k - 1);
+            k_x_flush<<<S->grid, kBlock, 0, st>>>(d, k - 1);
         }
         if (S->rows)
             k_fin_rows<<<1, kBlock, 0, st>>>(d);
@@ -1831,7 +1922,10 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
         DISPATCH_W(A, k_m_resid, v, d);
         k_m_coarse<<<S->grid, kBlock, 0, st>>>(d, use_coarse);
         k_m_corr_fin<<<1, kBlock, 0, st>>>(d, 0, 1);
-        k_m_start<<<S->grid, kBlock, 0, st>>>(d, S->p32);
+        if (S->fold)
+            k_m_start<<<S->grid, kBlock, 0, st>>>(d, S->p32);
+        else
+            k_m_pairs<<<S->grid, kBlock, 0, st>>>(d, d.sp32[0], 1);
         GIP_LAUNCH_CHECK("mixed setup");
         if ((rc = poll(S, true))) return rc;
         double last_rr = S->h_sc[S_TRUE_RR];
@@ -1851,18 +1945,20 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                         DISPATCH_WG(A, S->nchunk, k_m_spmv, v, d, pdir32(k));
                     sample_end(smp);
                     k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
-                    if (lean)
-                        k_m_update<false, true><<<S->grid, kBlock, 0, st>>>(d, k);
-                    else
-                        k_m_update<false><<<S->grid, kBlock, 0, st>>>(d, k);
+                    LEAN_LAUNCH(k_m_update, S->grid, d, k);
                 } else {
                     const bool smp = sample_begin(k);
-                    if (k > 0)
-                        DISPATCH_WG(A, S->nchunk, k_m_dirprod, v, d, pdir32(k - 1), pdir32(k), k, pending);
+                    if (k == 0)
+                        DISPATCH_WG(A, S->nchunk, k_m_spmv_small, v, d);
+                    else if (wave)
+                        DISPATCH_SMALL(A, k_m_dirprod, true, v, d, k, pending);
                     else
-                        DISPATCH_WG(A, S->nchunk, k_m_spmv_small, v, d, S->p32);
+                        DISPATCH_SMALL(A, k_m_dirprod, false, v, d, k, pending);
                     sample_end(smp);
-                    k_m_update<true><<<S->grid, kBlock, 0, st>>>(d, k);
+                    if (wave)
+                        k_m_update_small<true><<<S->grid, kBlock, 0, st>>>(d, k);
+                    else
+                        k_m_update_small<false><<<S->grid, kBlock, 0, st>>>(d, k);
                     pending = 1;
                 }
             }
@@ -1874,11 +1970,15 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             const double rr32 = S->h_sc[S_RR], tol2 = S->h_sc[S_TOL2];
             const bool near_target = tol2 >= 0.0 && rr32 <= tol2;
             if (rr32 <= inner2 * last_rr || near_target || k >= o->maxit) {
-                k_m_fold<<<S->grid, kBlock, 0, st>>>(d, pdir32(k - 1), pdir32(k), k - 1, pending);
+                if (S->fold)
+                    k_m_fold<<<S->grid, kBlock, 0, st>>>(d, pdir32(k - 1), pdir32(k), k - 1, pending);
+                else
+                    k_m_fold_small<<<S->grid, kBlock, 0, st>>>(d, k - 1);
                 pending = 0;
                 DISPATCH_W(A, k_m_resid, v, d);
                 k_m_coarse<<<S->grid, kBlock, 0, st>>>(d, use_coarse);
                 k_m_corr_fin<<<1, kBlock, 0, st>>>(d, k, 0);
+                if (!S->fold) k_m_pairs<<<S->grid, kBlock, 0, st>>>(d, d.sp32[(k - 1) & 1], 0);
                 GIP_LAUNCH_CHECK("mixed correction");
                 ++corrections;
                 if ((rc = poll(S, true))) return rc;
@@ -1946,12 +2046,11 @@ int gip_pcg_solve_noalloc(gip_ctx *c, const gip_mat *A, int32_t n_all, const dou
     S.fold = false;  // at most 1024 chunks: the fused two-kernel iteration
     S.gdn = S.nchunk;
     S.r = base;
-    S.s = S.r + kScratchRows;
-    S.Ap = S.s + kScratchRows;
+    S.Ap = S.r + kScratchRows;
     S.dinv = S.Ap + kScratchRows;
     S.p = S.dinv + kScratchRows;
-    S.p2 = S.p + kScratchAll;
-    double *zero = S.p2 + kScratchAll;
+    S.p2 = S.p + 2 * (size_t)kScratchAll;
+    double *zero = S.p2 + 2 * (size_t)kScratchAll;
     S.part = zero;
     S.sc = S.part + (size_t)P_COUNT * kMaxRedBlocks;
     S.state = reinterpret_cast<int *>(S.sc + S_COUNT);

@@ -561,61 +561,144 @@ __device__ inline bool row_dot_sym(const EllView &A, const V *__restrict__ val, 
     return stencil_row_sym<-W, T, V, X>(A, val, sym, x, row, sum);
 }
 
-// The operator's part of a stencil row (slot columns and values, and for a
-// slice of kind 0, 1 or 3 its one possible tail entry), loaded apart from the
-// operand so that a kernel can request it before its prologue; the operand
-// reads follow in stencil_row_fin, in the order stencil_row uses.
-template <int SW, class V>
-struct StencilPre {
-    int c[SW];
-    V v[SW];
-    int kind, slice, tcol;  // tcol < 0: no tail entry (kinds 0, 1 and 3)
-    V tval;
+// ---- one row of a small operator, requested ahead ---------------------------
+//
+// The fused direction-product of the small operators forms its operand
+// 1.0 s + beta p at every column it reads, with a beta that its prologue has
+// yet to sum.  What the row needs from memory does not depend on beta, so
+// all of it is requested before the prologue waits: the operator's row, then
+// the (s, p) pairs at its columns, kept side by side so that a column is one
+// load, the tail's among them.  (With the operand gathered after the sums
+// and s and p apart, a kernel cost one to three round trips more: us per
+// FP64 iteration, fixed count, 32^3 9.6 -> 7.1, 46^3 11.1 -> 9.3, 80^3 27.3
+// -> 23.8; the irregular 60^3 in sliced ELL 20.9 -> 16.9.)
+
+template <class T>
+struct alignas(2 * sizeof(T)) SP {
+    T s, p;
 };
 
-template <int SW, class V>
-__device__ inline void stencil_row_pre(const EllView &A, const V *__restrict__ val, int row, StencilPre<SW, V> &q) {
+constexpr int kPreTail = 3;  // tail entries of a row requested ahead
+
+template <int SW, class T>
+struct StencilPre {
+    int c[SW], tc[kPreTail];  // columns (tail: -1 none)
+    T v[SW], tv[kPreTail];
+    SP<T> g[SW], tg[kPreTail];
+    int slice;
+    bool empty, more;  // an empty row; tails beyond kPreTail in the slice (summed from the header)
+};
+
+template <int SW, class T>
+__device__ inline void stencil_row_pre(const EllView &A, const T *__restrict__ val, const SP<T> *__restrict__ sp,
+                                       int row, StencilPre<SW, T> &q) {
     const int s = __builtin_amdgcn_readfirstlane(row >> 6);
-    const int32_t *off = A.st_off + (size_t)s * SW;
-    const V *vs = val + (size_t)s * SW * 64 + (row & 63);
+    const_as<int32_t> *off = as_const(A.st_off) + (size_t)s * SW;
+    const T *vs = val + (size_t)s * SW * 64 + (row & 63);
+    const StencilTail tl = tail_rec(as_const(A.st_tail) + s);
 #pragma unroll
     for (int k = 0; k < SW; ++k) {
         const int cc = row + off[k];
         q.c[k] = cc < 0 ? 0 : (cc > A.cmax ? A.cmax : cc);
         q.v[k] = __builtin_nontemporal_load(&vs[64 * k]);
     }
-    const StencilTail tl = A.st_tail[s];  // the 16-byte record in one load
+#pragma unroll
+    for (int k = 0; k < SW; ++k) q.g[k] = sp[q.c[k]];
     q.slice = s;
-    q.kind = tl.kind & 0xff;
-    q.tcol = -1;
-    q.tval = V(0);
-    if (q.kind == 3) {
-        if ((row & 63) == ((tl.kind >> 8) & 63)) {
-            q.tcol = (int)(uint32_t)tl.m0;
-            q.tval = val[A.tail_base + tl.tsoff];
-        }
-    } else if (q.kind == 1) {
-        const uint64_t bit = 1ull << (row & 63);
-        if (tl.m0 & bit) {
-            const int e = tl.tsoff + __popcll(tl.m0 & (bit - 1ull));
-            q.tcol = A.st_tcol[e];
-            q.tval = val[A.tail_base + e];
-        }
+    q.empty = q.more = false;
+#pragma unroll
+    for (int j = 0; j < kPreTail; ++j) {
+        q.tc[j] = -1;
+        q.tv[j] = T(0);
     }
+    const int kind = tl.kind & 0xff;
+    const uint64_t bit = 1ull << (row & 63), below = bit - 1ull;
+    if (kind == 3) {
+        if ((row & 63) == ((tl.kind >> 8) & 63)) {
+            q.tc[0] = (int)(uint32_t)tl.m0;
+            q.tv[0] = val[A.tail_base + tl.tsoff];
+        }
+    } else if (kind) {
+        const_as<StencilHdr> *h = as_const(A.st_hdr) + s;
+        int t = tl.tsoff;
+        uint64_t m = tl.m0;
+#pragma unroll
+        for (int j = 0; j < kPreTail; ++j) {
+            if (m & bit) {
+                const int e = t + __popcll(m & below);
+                q.tc[j] = A.st_tcol[e];
+                q.tv[j] = val[A.tail_base + e];
+            }
+            if (kind == 1) break;
+            t += __popcll(m);
+            m = h->m[j + 1];
+            if (!m) break;
+            if (j + 1 == kPreTail) q.more = true;
+        }
+        if (kind == 2) q.empty = (h->empty & bit) != 0;
+    }
+#pragma unroll
+    for (int j = 0; j < kPreTail; ++j)
+        if (q.tc[j] >= 0) q.tg[j] = sp[q.tc[j]];
 }
 
-template <int SW, class T, class V, class X>
-__device__ inline bool stencil_row_fin(const EllView &A, const V *__restrict__ val, const X &x, int row,
-                                       const StencilPre<SW, V> &q, T &sum) {
+// the direction at column j (past the solved rows, ghost columns, it keeps
+// its value), as the direction update computes it on the solved rows
+__device__ inline double dir_at(const SP<double> &q, int j, double beta, int n) {
+    return j < n ? 1.0 * q.s + beta * q.p : q.p;
+}
+__device__ inline float dir_at(const SP<float> &q, int j, float beta, int n) {
+    return j < n ? q.s + beta * q.p : q.p;
+}
+
+template <class T>
+struct DirOperand {
+    const SP<T> *__restrict__ sp;
+    T beta;
+    int n;
+    __device__ inline T at(int j) const { return dir_at(sp[j], j, beta, n); }
+};
+
+// the p of the pairs (the first iteration's operand)
+template <class T>
+struct PairOperand {
+    const SP<T> *__restrict__ sp;
+    __device__ inline T at(int j) const { return sp[j].p; }
+};
+
+template <int SW, class T>
+__device__ inline bool stencil_row_fin(const EllView &A, const T *__restrict__ val, const DirOperand<T> &x, int row,
+                                       const StencilPre<SW, T> &q, T &sum) {
     sum = T(0);
 #pragma unroll
-    for (int k = 0; k < SW; ++k) sum = sum + x.at(q.c[k]) * q.v[k];
-    if (q.kind == 1 || q.kind == 3) {
-        if (q.tcol >= 0) sum = sum + x.at(q.tcol) * q.tval;
-    } else if (q.kind == 2) {
-        return stencil_tail_hdr(A, val, x, q.slice, row, sum);
+    for (int k = 0; k < SW; ++k) sum = sum + dir_at(q.g[k], q.c[k], x.beta, x.n) * q.v[k];
+    if (q.more) return stencil_tail_hdr(A, val, x, q.slice, row, sum);
+#pragma unroll
+    for (int j = 0; j < kPreTail; ++j)
+        if (q.tc[j] >= 0) sum = sum + dir_at(q.tg[j], q.tc[j], x.beta, x.n) * q.tv[j];
+    return !q.empty;
+}
+
+// uniform sliced ELL of W entries per row
+template <int W, class T>
+struct EllPre {
+    int c[W];
+    T v[W];
+    SP<T> g[W];
+};
+
+template <int W, class T>
+__device__ inline void ell_row_pre(const EllView &A, const T *__restrict__ val, const SP<T> *__restrict__ sp, int row,
+                                   EllPre<W, T> &q) {
+    const int lg = A.ell_lg;
+    const int base = A.soff[row >> lg] + (row & ((1 << lg) - 1));
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+        q.c[k] = __builtin_nontemporal_load(&A.col[base + (k << lg)]);
+        q.v[k] = __builtin_nontemporal_load(&val[base + (k << lg)]);
     }
-    return true;
+#pragma unroll
+    for (int k = 0; k < W; ++k) q.g[k] = sp[q.c[k]];
 }
 
 // Row sum in stored order; returns false for an empty row.

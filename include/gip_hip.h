@@ -276,8 +276,8 @@ int gip_pcg_destroy(gip_pcg *solver);
 /* The FP64 solve of gip_pcg_solve without any allocation: no counterpart in
  * the reference; for callers that cannot allocate device or pinned memory
  * (code under stream capture, tight serving loops).  The solver workspace
- * (r, s, Ap, Dinv, two directions, partial sums, scalars, state) is a
- * device array of about 13.8 MB, one per GPU, set up by gip_init and held
+ * (r, Ap, Dinv, two arrays of (s, p) pairs, partial sums, scalars) is a
+ * device array of about 16.9 MB, one per GPU, set up by gip_init and held
  * until the process ends; its limit is 262,144 rows (nrows(A)) and 327,680
  * vector entries (n_all): larger operators, GIP_PCG_MIXED and
  * time_products are rejected with GIP_EINVAL.  Same kernels, iterates and

@@ -87,8 +87,8 @@ def test_cavity_iterates(dev, shape):
 
 
 def test_breakdown_keeps_the_updates_made(dev):
-    """A right-hand side the solve meets exactly after two iterations: the third
-    breaks down (p.Ap = 0) with x complete, whatever parity it stops at."""
+    """A solve that runs on after it has converged breaks down (p.Ap = 0) some
+    iterations later: x is complete whatever parity it stops at."""
     n = 2 ** 19 + 64
     T = sp.identity(n, format="csr") * 2.0
     T = (T + sp.csr_matrix(([1.0, 1.0], ([0, 1], [1, 0])), shape=(n, n))).tocsr()
