@@ -179,36 +179,52 @@ __global__ __launch_bounds__(kBlock) void k_b_cfl_fin(const double *part, Seg S,
 }
 
 // The PCG product and update kernels instead run one workgroup per chunk in
-// dispatch order (grid = the chunk count: the pace of a plain stream) and
-// store one partial per wavefront, with no barrier (seg_store_w); their
-// finalize kernels sum an instance's wavefront partials in chunk order
-// (seg_total_w).  A chunk of an instance that has left the PCG returns
+// dispatch order (grid = the chunk count: the pace of a plain stream), sum
+// their wavefronts by DPP and store one total per chunk (seg_store_c: one
+// barrier, which costs less than the finalize kernels' reading four times
+// as many partials, and than an 8-byte store per wavefront and sum); their
+// finalize kernels sum an instance's chunk totals in chunk order
+// (seg_total_c).  A chunk of an instance that has left the PCG returns
 // after two loads.
 template <int K>
-__device__ inline void seg_store_w(double (&v)[K], int c, double *part) {
-    const size_t w = (size_t)c * kWaves + (threadIdx.x >> 6);
+__device__ inline void seg_store_c(double (&v)[K], int c, double *part) {
+    static_assert(K <= 2, "at most two sums");
+    __shared__ double sh[kWaves][K];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double t = K == 1 ? wave_sum_63(v[0]) : wave_sum_two(v[0], v[K - 1]);
+    if (K == 1 ? lane == 63 : (lane & 31) == 31) sh[w][K == 1 ? 0 : lane >> 5] = t;
+    __syncthreads();
+    if (threadIdx.x < K) {
+        double a = sh[0][threadIdx.x];
 #pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
-    if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) part[w * K + k] = v[k];
+        for (int k = 1; k < kWaves; ++k) a = a + sh[k][threadIdx.x];
+        part[(size_t)c * K + threadIdx.x] = a;
     }
 }
 
+// (valid in thread 0)
 template <int K>
-__device__ inline void seg_total_w(const double *part, int inst, const Seg &S, double (&out)[K]) {
-    const size_t w0 = (size_t)S.inst_c0[inst] * kWaves;
-    const int nw = S.inst_nch[inst] * kWaves;
+__device__ inline void seg_total_c(const double *part, int inst, const Seg &S, double (&out)[K]) {
+    static_assert(K <= 2, "at most two sums");
+    __shared__ double sh[kWaves][K];
+    const size_t c0 = (size_t)S.inst_c0[inst];
+    const int nch = S.inst_nch[inst], lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     double acc[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = 0.0;
 #pragma unroll 8
-    for (int j = threadIdx.x; j < nw; j += kBlock)
+    for (int j = threadIdx.x; j < nch; j += kBlock)
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc[k] = acc[k] + part[(w0 + j) * K + k];
-    block_reduce_n<K>(acc);
+        for (int k = 0; k < K; ++k) acc[k] = acc[k] + part[(c0 + j) * K + k];
+    const double t = K == 1 ? wave_sum_63(acc[0]) : wave_sum_two(acc[0], acc[K - 1]);
+    if (K == 1 ? lane == 63 : (lane & 31) == 31) sh[w][K == 1 ? 0 : lane >> 5] = t;
+    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < K; ++k) out[k] = acc[k];
+    for (int k = 0; k < K; ++k) {
+        out[k] = sh[0][k];
+#pragma unroll
+        for (int q = 1; q < kWaves; ++q) out[k] = out[k] + sh[q][k];
+    }
 }
 
 // ---- batched PCG ------------------------------------------------------------
@@ -222,7 +238,7 @@ struct BPcg {
     const double *one, *az;  // MIXED coarse step: 1 on real inner rows (0 on padding), A 1
     double *sc;              // B * B_COUNT
     int *state, *iters, *active;
-    double *part;  // chunk totals or wavefront partials
+    double *part;  // chunk totals
     int maxit;
     double inner2;
 };
@@ -330,7 +346,7 @@ __global__ __launch_bounds__(kBlock) void k_bp_spmv(EllView A, BPcg d, Seg S, co
     else
         sum = d.Ap[row];
     double v[1] = {pi * sum};
-    seg_store_w<1>(v, c, d.part);
+    seg_store_c<1>(v, c, d.part);
 }
 
 // alpha = rho / p.Ap of the running instances (FP64 and MIXED)
@@ -338,7 +354,7 @@ __global__ __launch_bounds__(kBlock) void k_bp_spmv_fin(BPcg d, Seg S) {
     const int inst = blockIdx.x;
     if (d.state[inst] != BS_RUN) return;
     double out[1];
-    seg_total_w<1>(d.part, inst, S, out);
+    seg_total_c<1>(d.part, inst, S, out);
     if (threadIdx.x == 0) {
         double *q = bsc(d, inst);
         const double alpha = q[B_RHO] / out[0];
@@ -368,14 +384,14 @@ __global__ __launch_bounds__(kBlock) void k_bp_update(BPcg d, Seg S, const doubl
     }
     d.s[row] = si;
     double v[2] = {ri * si, ri * ri};
-    seg_store_w<2>(v, c, d.part);
+    seg_store_c<2>(v, c, d.part);
 }
 
 __global__ __launch_bounds__(kBlock) void k_bp_update_fin(BPcg d, Seg S) {
     const int inst = blockIdx.x;
     if (d.state[inst] != BS_RUN) return;
     double out[2];
-    seg_total_w<2>(d.part, inst, S, out);
+    seg_total_c<2>(d.part, inst, S, out);
     if (threadIdx.x == 0) {
         double *q = bsc(d, inst);
         const double r0 = q[B_RHO];
@@ -481,7 +497,7 @@ __global__ __launch_bounds__(kBlock) void k_bpm_spmv(EllView A, BPcg d, Seg S, c
     row_dot<W, float, float>(A, A.val32, po, row, sum);
     d.Ap32[row] = sum;
     double v[1] = {(double)pi * (double)sum};
-    seg_store_w<1>(v, c, d.part);
+    seg_store_c<1>(v, c, d.part);
 }
 
 __global__ __launch_bounds__(kBlock) void k_bpm_update(BPcg d, Seg S, const float *__restrict__ p, int precond) {
@@ -499,14 +515,14 @@ __global__ __launch_bounds__(kBlock) void k_bpm_update(BPcg d, Seg S, const floa
     const float si = precond ? ri * di : ri;
     __builtin_nontemporal_store(si, d.s32 + row);
     double v[2] = {(double)ri * (double)si, (double)ri * (double)ri};
-    seg_store_w<2>(v, c, d.part);
+    seg_store_c<2>(v, c, d.part);
 }
 
 __global__ __launch_bounds__(kBlock) void k_bpm_update_fin(BPcg d, Seg S) {
     const int inst = blockIdx.x;
     if (d.state[inst] != BS_RUN) return;
     double out[2];
-    seg_total_w<2>(d.part, inst, S, out);
+    seg_total_c<2>(d.part, inst, S, out);
     if (threadIdx.x == 0) {
         double *q = bsc(d, inst);
         const double r0 = q[B_RHO];
@@ -994,8 +1010,8 @@ int gip_batch_create(gip_ctx *c, int32_t ninst, const gip_cavity *const *cavs, c
         if (!rc) rc = dalloc_t(b, &b->caz, NPs);
     }
     if (!rc) rc = dalloc_t(b, &b->sc, (size_t)B * B_COUNT);
-    // chunk totals (up to 3 per chunk) or wavefront partials (up to 2 per wavefront)
-    if (!rc) rc = dalloc_t(b, &b->part, (size_t)std::max(b->NP, b->FP) / kChunk * (2 * kWaves) + 8);
+    // chunk totals (up to 3 per chunk)
+    if (!rc) rc = dalloc_t(b, &b->part, (size_t)std::max(b->NP, b->FP) / kChunk * 3 + 8);
     if (!rc) rc = dalloc_t(b, &b->state, (size_t)B);
     if (!rc) rc = dalloc_t(b, &b->iters, (size_t)B);
     if (!rc) rc = dalloc_t(b, &b->active, 1);

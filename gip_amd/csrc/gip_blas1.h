@@ -39,13 +39,49 @@ struct RedOp<RED_MIN> {
 
 constexpr int kWaves = kBlock / 64;  // wavefronts per workgroup
 
-// Sum over the wavefront (shuffle tree, no LDS or barrier); valid in lane 0.
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = v + __shfl_down(v, off, 64);
-    return v;
+// v of lane i - (CTRL - 0x110) within the lane's row of 16 (0 past the
+// row's start): a DPP row shift, moved as two 32-bit halves
+template <int CTRL>
+__device__ inline double dpp_row_shr(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
+// Wavefront sums by DPP: an inclusive scan of each row of 16 lanes, then row
+// 0's total onto row 1's and row 2's onto row 3's (row broadcast), then lane
+// 31's onto the last row: a fixed order, no LDS, no lane reads.  The total
+// is in lane 63 (18 vector instructions).
+template <int CTRL, int ROWS>
+__device__ inline double dpp_row_bcast(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+__device__ inline double half_sum_dpp(double v) {  // lanes 31 and 63: the totals of their halves
+    v = v + dpp_row_shr<0x111>(v);
+    v = v + dpp_row_shr<0x112>(v);
+    v = v + dpp_row_shr<0x114>(v);
+    v = v + dpp_row_shr<0x118>(v);
+    return v + dpp_row_bcast<0x142, 0xa>(v);
+}
+__device__ inline double wave_sum_63(double v) {
+    v = half_sum_dpp(v);
+    return v + dpp_row_bcast<0x143, 0xc>(v);
+}
+// Two sums for little more than one: the lower half of the wavefront takes
+// a, the upper half b (each lane's value and the one 32 lanes on), and the
+// halves are summed together.  a's total is in lane 31, b's in lane 63.
+__device__ inline double wave_sum_two(double a, double b) {
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    const double p = __longlong_as_double(((long long)hi[0] << 32) | (long long)lo[0]);
+    const double q = __longlong_as_double(((long long)hi[1] << 32) | (long long)lo[1]);
+    return half_sum_dpp(p + q);
+}
 // Reduce v over the workgroup; the result is valid in thread 0.
 template <int OP>
 __device__ inline double block_reduce(double v) {
