@@ -250,6 +250,13 @@ __device__ inline void leave(const BPcg &d, int inst, int st) {
     atomicSub(d.active, 1);
 }
 
+// the number of instances still running, for the host's poll
+__global__ void k_b_publish(const int *__restrict__ active, uint64_t *__restrict__ out, uint64_t seq) {
+    if (threadIdx.x != 0) return;
+    out[0] = (uint64_t)(int64_t)*active;
+    publish_seq(out + 1, seq);
+}
+
 __global__ void k_bp_init(BPcg d) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < d.B) {
@@ -655,7 +662,8 @@ struct gip_batch {
     float *r32 = nullptr, *s32 = nullptr, *Ap32 = nullptr, *xc32 = nullptr, *dinv32 = nullptr, *pq = nullptr;
     double *cone = nullptr, *caz = nullptr;  // MIXED coarse step: 1 on inner rows, A 1
     double *sc = nullptr, *part = nullptr;
-    int *state = nullptr, *iters = nullptr, *active = nullptr, *h_active = nullptr;
+    int *state = nullptr, *iters = nullptr, *active = nullptr;
+    uint64_t *h_active = nullptr, *h_active_dev = nullptr, seq = 0;  // pinned: the running count, its sequence word
     bool started = false;
     hipGraphExec_t g_pre = nullptr, g_iter = nullptr, g_post = nullptr;
     // events around the step's three phases (recorded outside any capture)
@@ -1016,7 +1024,9 @@ int gip_batch_create(gip_ctx *c, int32_t ninst, const gip_cavity *const *cavs, c
     if (!rc) rc = dalloc_t(b, &b->iters, (size_t)B);
     if (!rc) rc = dalloc_t(b, &b->active, 1);
     if (!rc) {
-        hipError_t e = hipHostMalloc((void **)&b->h_active, sizeof(int), hipHostMallocDefault);
+        hipError_t e = hipHostMalloc((void **)&b->h_active, 2 * sizeof(uint64_t), hipHostMallocCoherent);
+        if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&b->h_active_dev, b->h_active, 0);
+        if (e == hipSuccess) b->h_active[0] = b->h_active[1] = 0;
         if (e != hipSuccess) rc = hip_fail(e, "hipHostMalloc");
         for (int k = 0; k < 4 && e == hipSuccess; ++k) e = hipEventCreate(&b->ev[k]);
         if (e != hipSuccess && !rc) rc = hip_fail(e, "hipEventCreate");
@@ -1130,9 +1140,10 @@ int gip_batch_step(gip_batch *b) {
     const int max_groups = (b->o.pcg_maxit + b->o.poll - 1) / b->o.poll + 2;
     for (int g = 0; g < max_groups; ++g) {
         if ((rc = run_phase(b, enqueue_iter, &b->g_iter))) return rc;
-        GIP_HIP_TRY(hipMemcpyAsync(b->h_active, b->active, sizeof(int), hipMemcpyDeviceToHost, st));
-        GIP_HIP_TRY(hipStreamSynchronize(st));
-        if (*b->h_active <= 0) break;
+        k_b_publish<<<1, 64, 0, st>>>(b->active, b->h_active_dev, ++b->seq);
+        GIP_LAUNCH_CHECK("batch poll");
+        if ((rc = wait_published(st, b->h_active + 1, b->seq))) return rc;
+        if ((int64_t)b->h_active[0] <= 0) break;
     }
     GIP_HIP_TRY(hipEventRecord(b->ev[2], st));
     if ((rc = run_phase(b, enqueue_post, &b->g_post))) return rc;

@@ -52,12 +52,17 @@ __global__ __launch_bounds__(kBlock) void k_reduce(int n, const double *__restri
     if (threadIdx.x == 0) partials[blockIdx.x] = acc;
 }
 
-// one workgroup: combine `np` partials; CFL = 1 applies GIP_NonLinearMulticore.cpp:47-50
+// one workgroup: combine `np` partials; CFL = 1 applies GIP_NonLinearMulticore.cpp:47-50;
+// flag (may be null): the sequence word of a result the host waits for
 template <int OP, int CFL>
 __global__ __launch_bounds__(kBlock) void k_finalize(const double *__restrict__ partials, int np,
-                                                    double *__restrict__ result) {
+                                                    double *__restrict__ result, uint64_t *__restrict__ flag,
+                                                    uint64_t seq) {
     const double acc = sum_partials<OP>(partials, np);
-    if (threadIdx.x == 0) *result = CFL ? (0.8 * acc > 1e-1 ? 1e-1 : 0.8 * acc) : acc;
+    if (threadIdx.x == 0) {
+        *result = CFL ? (0.8 * acc > 1e-1 ? 1e-1 : 0.8 * acc) : acc;
+        if (flag) publish_seq(flag, seq);
+    }
 }
 
 struct CflArgs {
@@ -89,17 +94,22 @@ __global__ __launch_bounds__(kBlock) void k_cfl(int n, CflArgs a, double *__rest
 
 static inline int blocks_for(int n) { return (n + kBlock - 1) / kBlock; }
 
+static uint64_t *seq_word(gip_ctx *c) { return reinterpret_cast<uint64_t *>(c->h_result_dev + kSeqSlot); }
+
 int launch_reduce(gip_ctx *c, int op, int n, const double *x, const double *y, double *dres) {
+    // a result in the host block is waited for (fetch_result)
+    uint64_t *flag = dres == c->h_result_dev ? seq_word(c) : nullptr;
+    const uint64_t seq = flag ? ++c->seq : 0;
     int g = reduce_grid(n);
     double *part = c->d_partials;
     switch (op) {
         case RED_SUM:
             k_reduce<RED_SUM><<<g, kBlock, 0, c->stream>>>(n, x, y, part);
-            k_finalize<RED_SUM, 0><<<1, kBlock, 0, c->stream>>>(part, g, dres);
+            k_finalize<RED_SUM, 0><<<1, kBlock, 0, c->stream>>>(part, g, dres, flag, seq);
             break;
         case RED_MAXABS:
             k_reduce<RED_MAXABS><<<g, kBlock, 0, c->stream>>>(n, x, y, part);
-            k_finalize<RED_MAXABS, 0><<<1, kBlock, 0, c->stream>>>(part, g, dres);
+            k_finalize<RED_MAXABS, 0><<<1, kBlock, 0, c->stream>>>(part, g, dres, flag, seq);
             break;
         default:
             return set_error(GIP_EINVAL, "unknown reduction");
@@ -111,9 +121,10 @@ int launch_reduce(gip_ctx *c, int op, int n, const double *x, const double *y, d
 // A reduction whose result the host needs: the finalize kernel stores it
 // straight into the context's pinned host slot (no device-to-host copy
 // command; the reference's PCG sequence makes about 300 such round trips
-// per step: C100K 5.22 -> 4.87 ms per step), read after the stream drains.
+// per step: C100K 5.22 -> 4.87 ms per step), then its sequence number.
 static int fetch_result(gip_ctx *c, double *out) {
-    GIP_HIP_TRY(hipStreamSynchronize(c->stream));
+    int rc = wait_published(c->stream, reinterpret_cast<const uint64_t *>(c->h_result + kSeqSlot), c->seq);
+    if (rc) return rc;
     *out = c->h_result[0];
     return GIP_OK;
 }
@@ -194,7 +205,7 @@ int gip_cfl(gip_ctx *c, int32_t n, const double *u, const double *v, const doubl
     CflArgs a{u, v, w, dxs, gamma, rho};
     int g = reduce_grid(n);
     k_cfl<<<g, kBlock, 0, c->stream>>>(n, a, c->d_partials);
-    k_finalize<RED_MIN, 1><<<1, kBlock, 0, c->stream>>>(c->d_partials, g, c->h_result_dev);
+    k_finalize<RED_MIN, 1><<<1, kBlock, 0, c->stream>>>(c->d_partials, g, c->h_result_dev, seq_word(c), ++c->seq);
     GIP_LAUNCH_CHECK("gip_cfl");
     return fetch_result(c, dt);
 }

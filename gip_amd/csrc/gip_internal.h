@@ -66,8 +66,10 @@ struct gip_ctx {
     int device;
     hipStream_t stream;
     double *d_partials;     // kMaxRedBlocks * 4 doubles of reduction partials (one per workgroup)
-    double *h_result;       // pinned host landing slot for reduction results
+    double *h_result;       // pinned, coherent host block: reduction results at 0, the no-alloc
+                            // solve's published words at kPubSlot, sequence words at kSeqSlot
     double *h_result_dev;   // its device address: the finalize kernels store the result there
+    uint64_t seq, pub_seq;  // last sequence numbers asked for
     int num_cu;
 };
 
@@ -147,6 +149,19 @@ struct gip_mat {
 
 namespace gip {
 int reduce_grid(int n);
+
+// Words a kernel hands to the host: it stores them in pinned coherent
+// memory, then the sequence number (a system-scope release), and the host
+// waits for that number instead of copying the words and draining the
+// stream: a dot product of 97,336 entries returns in 11.0 us instead of
+// 16.5, and a solver's poll costs one short kernel instead of copies and a
+// synchronisation.  Work queued before the kernel has completed when the
+// number arrives.
+constexpr int kHostBlock = 64, kPubSlot = 8, kPubWords = 24, kSeqSlot = 40, kPubSeqSlot = 48;  // doubles
+int wait_published(hipStream_t st, const uint64_t *flag, uint64_t want);
+__device__ inline void publish_seq(uint64_t *flag, uint64_t seq) {
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // Makes (once per version of the values) and checks the symmetric form of
 // a stencil operator's slot values; *ok is true when the PCG's product may
 // read them.  Allocates on first use.

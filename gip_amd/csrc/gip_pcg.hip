@@ -49,6 +49,7 @@
 // constant mode is left to the FP64 step.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -249,8 +250,30 @@ __global__ __launch_bounds__(kBlock) void k_setup_dir(PcgDev d, double *__restri
     }
 }
 
+// What the host reads at a poll: the scalars, the state word and the
+// iteration count, by the workgroup that formed them last (flag null: not
+// asked for).
+struct Pub {
+    double *sc;
+    int *st;
+    uint64_t *flag;
+    uint64_t seq;
+};
+__device__ inline void publish(const PcgDev &d, const Pub &p) {
+    if (!p.flag) return;
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t >= 64) return;  // one wavefront: its stores come before its release
+    if (t < S_COUNT) p.sc[t] = d.sc[t];
+    if (t == S_COUNT) p.st[0] = state_load(d.state);
+    if (t == S_COUNT + 1) p.st[1] = *d.iters;
+    if (t == 0) publish_seq(p.flag, p.seq);
+}
+
+__global__ __launch_bounds__(64) void k_publish(PcgDev d, Pub pub) { publish(d, pub); }
+
 // one workgroup: rho_0, b.b, r.r, the tolerance, the state word and the iteration count
-__global__ __launch_bounds__(kBlock) void k_setup_fin(PcgDev d, double tol) {
+__global__ __launch_bounds__(kBlock) void k_setup_fin(PcgDev d, double tol, Pub pub) {
     const double rho = sum_partials<RED_SUM>(d.P(P_RS), d.G);
     const double bb = sum_partials<RED_SUM>(d.P(P_BB), d.G);
     const double rr = sum_partials<RED_SUM>(d.P(P_RR), d.G);
@@ -263,6 +286,7 @@ __global__ __launch_bounds__(kBlock) void k_setup_fin(PcgDev d, double tol) {
         state_store(d.state, (tol > 0.0 && rr <= tol2) ? ST_CONV : ST_RUN);
         *d.iters = 0;
     }
+    publish(d, pub);
 }
 
 // ---- FP64 iteration --------------------------------------------------------
@@ -927,21 +951,24 @@ __global__ __launch_bounds__(kBlock) void k_x_flush_pair(PcgDev d, const double 
 
 // one workgroup after the last iteration: the final convergence test on the
 // r.r F2 left
-__global__ __launch_bounds__(kBlock) void k_fin_rows(PcgDev d) {
-    if (threadIdx.x != 0) return;
-    const double rr = d.sc[S_RR], tol2 = d.sc[S_TOL2];
-    const int st = state_load(d.state);
-    if ((st == ST_RUN || (st & ST_MASK) == ST_CONV) && tol2 >= 0.0 && rr <= tol2) state_store(d.state, ST_CONV);
+__global__ __launch_bounds__(kBlock) void k_fin_rows(PcgDev d, Pub pub) {
+    if (threadIdx.x == 0) {
+        const double rr = d.sc[S_RR], tol2 = d.sc[S_TOL2];
+        const int st = state_load(d.state);
+        if ((st == ST_RUN || (st & ST_MASK) == ST_CONV) && tol2 >= 0.0 && rr <= tol2) state_store(d.state, ST_CONV);
+    }
+    publish(d, pub);
 }
 
 // one workgroup after the last iteration: r.r and the final convergence test
-__global__ __launch_bounds__(kBlock) void k_fin(PcgDev d) {
+__global__ __launch_bounds__(kBlock) void k_fin(PcgDev d, Pub pub) {
     const double rr = sum_partials<RED_SUM>(d.P(P_RR), d.G);
     if (threadIdx.x == 0) {
         d.sc[S_RR] = rr;
         const double tol2 = d.sc[S_TOL2];
         if (state_load(d.state) == ST_RUN && tol2 >= 0.0 && rr <= tol2) state_store(d.state, ST_CONV);
     }
+    publish(d, pub);
 }
 
 // ---- MIXED iteration (FP32 vectors and operator, FP64 dot accumulation) --------
@@ -1249,9 +1276,10 @@ __global__ __launch_bounds__(kBlock) void k_m_fold_small(PcgDev d, int k) {
 }
 
 // one workgroup: the FP32 recursive r.r for the host's correction test
-__global__ __launch_bounds__(kBlock) void k_m_status(PcgDev d) {
+__global__ __launch_bounds__(kBlock) void k_m_status(PcgDev d, Pub pub) {
     const double rr = sum_partials<RED_SUM>(d.P(P_RR), d.G);
     if (threadIdx.x == 0) d.sc[S_RR] = rr;
+    publish(d, pub);
 }
 
 // x += xc, with the last iterations' pending updates xc += alpha p first
@@ -1321,7 +1349,7 @@ __global__ __launch_bounds__(kBlock) void k_m_coarse(PcgDev d, int use) {
 // recursion's (its partials are copied over the FP32 ones); the direction is
 // kept unless the recursive r.r had drifted below a hundredth of the true
 // one, then the previous rho slot is set to +inf so the next beta is 0.
-__global__ __launch_bounds__(kBlock) void k_m_corr_fin(PcgDev d, int k, int first) {
+__global__ __launch_bounds__(kBlock) void k_m_corr_fin(PcgDev d, int k, int first, Pub pub) {
     const double rrt = sum_partials<RED_SUM>(d.P(P_RR2), d.G);
     const double rrec = first ? 0.0 : sum_partials<RED_SUM>(d.P(P_RR), d.G);
     __syncthreads();
@@ -1338,6 +1366,7 @@ __global__ __launch_bounds__(kBlock) void k_m_corr_fin(PcgDev d, int k, int firs
         const double tol2 = d.sc[S_TOL2];
         if (state_load(d.state) == ST_RUN && tol2 >= 0.0 && rrt <= tol2) state_store(d.state, ST_CONV);
     }
+    publish(d, pub);
 }
 
 // first direction p32 = s32, correction zero
@@ -1451,8 +1480,11 @@ struct gip_pcg {
                 // otherwise the fused two-kernel iteration runs
     bool rows;  // fold and more than kRowsMin rows: the row-per-thread iteration
     int *state;    // state, iters
-    int *h_state;  // pinned copy
-    double *h_sc;  // pinned scalars
+    // pinned coherent words the kernels publish to: scalars, then state and
+    // count, and the sequence word; their device address; the last number
+    double *h_pub, *h_pub_dev;
+    uint64_t *h_flag, *h_flag_dev, *seq;
+    uint64_t own_seq;
     hipEvent_t tev0, tev1;  // time_products: the sampled product launch
 };
 
@@ -1594,8 +1626,14 @@ int gip_pcg_create(gip_ctx *c, const gip_mat *A, int32_t n_all, gip_pcg **out) {
     dalloc((void **)&S->part, (size_t)P_COUNT * kMaxRedBlocks * 8);
     if (S->fold) dalloc((void **)&S->chunk, (size_t)S->nchunk * kWaves * 2 * 8);  // p.Ap, then 1.Ap
     dalloc((void **)&S->state, 2 * sizeof(int));
-    if (e == hipSuccess) e = hipHostMalloc((void **)&S->h_state, 2 * sizeof(int), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&S->h_sc, S_COUNT * 8, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&S->h_pub, kHostBlock * 8, hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&S->h_pub_dev, S->h_pub, 0);
+    if (e == hipSuccess) {
+        memset(S->h_pub, 0, kHostBlock * 8);
+        S->h_flag = reinterpret_cast<uint64_t *>(S->h_pub + kSeqSlot);
+        S->h_flag_dev = reinterpret_cast<uint64_t *>(S->h_pub_dev + kSeqSlot);
+        S->seq = &S->own_seq;
+    }
     if (e == hipSuccess) e = hipMemsetAsync(S->sc, 0, S_COUNT * 8, c->stream);
     // partial slots past each producer's grid stay zero for sum_padded
     if (e == hipSuccess) e = hipMemsetAsync(S->part, 0, (size_t)P_COUNT * kMaxRedBlocks * 8, c->stream);
@@ -1639,8 +1677,7 @@ int gip_pcg_destroy(gip_pcg *S) {
                     S->ddinv, S->ddinv32};
     for (void *p : ptrs)
         if (p) hipFree(p);
-    if (S->h_state) hipHostFree(S->h_state);
-    if (S->h_sc) hipHostFree(S->h_sc);
+    if (S->h_pub) hipHostFree(S->h_pub);
     if (S->tev0) hipEventDestroy(S->tev0);
     if (S->tev1) hipEventDestroy(S->tev1);
     delete S;
@@ -1692,13 +1729,14 @@ static int coarse_setup(gip_pcg *S) {
     return rc;
 }
 
-static int poll(gip_pcg *S, bool scalars) {
-    hipStream_t st = S->ctx->stream;
-    GIP_HIP_TRY(hipMemcpyAsync(S->h_state, S->state, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
-    if (scalars) GIP_HIP_TRY(hipMemcpyAsync(S->h_sc, S->sc, S_COUNT * 8, hipMemcpyDeviceToHost, st));
-    GIP_HIP_TRY(hipStreamSynchronize(st));
-    return GIP_OK;
+static_assert(S_COUNT + 2 <= kPubWords, "published words");
+static int *h_state(gip_pcg *S) { return reinterpret_cast<int *>(S->h_pub + S_COUNT); }
+
+// what the next kernel to publish stores, and the wait for it
+static Pub next_pub(gip_pcg *S) {
+    return Pub{S->h_pub_dev, reinterpret_cast<int *>(S->h_pub_dev + S_COUNT), S->h_flag_dev, ++*S->seq};
 }
+static int wait_pub(gip_pcg *S) { return wait_published(S->ctx->stream, S->h_flag, *S->seq); }
 
 // The solve on a solver's workspace (allocated by gip_pcg_create, or the
 // no-alloc scratch); arguments already checked.
@@ -1783,8 +1821,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             armed = true;
         }
     };
-    auto sample_read = [&]() {  // after a host synchronisation
+    auto sample_read = [&]() {  // after a wait for the host's poll
         float ms = 0.0f;
+        if (armed) hipEventSynchronize(S->tev1);
         if (armed && hipEventElapsedTime(&ms, S->tev0, S->tev1) == hipSuccess) samples.push_back(ms);
         armed = false;
     };
@@ -1792,21 +1831,21 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     double *const dir0 = S->fold ? S->p : nullptr;  // small operators: the pairs in d
     DISPATCH_W(A, k_setup_resid, v, d, x0, S->n_all, dir0, S->p2);
     k_setup_dir<<<S->grid, kBlock, 0, st>>>(d, dir0);
-    k_setup_fin<<<1, kBlock, 0, st>>>(d, o->tol);
+    const bool fixed = !mixed && !(o->tol > 0.0);
+    k_setup_fin<<<1, kBlock, 0, st>>>(d, o->tol, fixed || mixed ? Pub{} : next_pub(S));
     GIP_LAUNCH_CHECK("pcg setup");
     int corrections = 0, rc;
     // FP64 with a fixed iteration count (tol <= 0): nothing can stop the
     // solve early but a breakdown, after which every queued kernel returns
     // at once, so all iterations are queued and the host reads the state
     // once, at the end (every 4096 iterations on long runs)
-    const bool fixed = !mixed && !(o->tol > 0.0);
     if (fixed)
-        S->h_state[0] = ST_RUN;
-    else if ((rc = poll(S, true)))
+        h_state(S)[0] = ST_RUN;
+    else if (!mixed && (rc = wait_pub(S)))
         return rc;
     if (!mixed) {
         int k = 0;  // iterations queued
-        while (k < o->maxit && S->h_state[0] == ST_RUN) {
+        while (k < o->maxit && h_state(S)[0] == ST_RUN) {
             int chunk = std::min(fixed ? 4096 : pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold && !S->rows) {
@@ -1860,7 +1899,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             }
             GIP_LAUNCH_CHECK("pcg iteration");
             if (!fixed) {
-                if ((rc = poll(S, false))) return rc;
+                k_publish<<<1, 64, 0, st>>>(d, next_pub(S));
+                GIP_LAUNCH_CHECK("pcg poll");
+                if ((rc = wait_pub(S))) return rc;
                 sample_read();
             }
         }
@@ -1870,26 +1911,27 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             k_x_flush<<<S->grid, kBlock, 0, st>>>(d, k - 1);
         }
         if (S->rows)
-            k_fin_rows<<<1, kBlock, 0, st>>>(d);
+            k_fin_rows<<<1, kBlock, 0, st>>>(d, next_pub(S));
         else
-            k_fin<<<1, kBlock, 0, st>>>(d);
+            k_fin<<<1, kBlock, 0, st>>>(d, next_pub(S));
         GIP_LAUNCH_CHECK("pcg final test");
+        if ((rc = wait_pub(S))) return rc;
     } else {
         // FP64 residual of x0 (with the coarse step), FP32 copies, first direction
         DISPATCH_W(A, k_m_resid, v, d);
         k_m_coarse<<<S->grid, kBlock, 0, st>>>(d, use_coarse);
-        k_m_corr_fin<<<1, kBlock, 0, st>>>(d, 0, 1);
+        k_m_corr_fin<<<1, kBlock, 0, st>>>(d, 0, 1, next_pub(S));
         if (S->fold)
             k_m_start<<<S->grid, kBlock, 0, st>>>(d, S->p32);
         else
             k_m_pairs<<<S->grid, kBlock, 0, st>>>(d, d.sp32[0], 1);
         GIP_LAUNCH_CHECK("mixed setup");
-        if ((rc = poll(S, true))) return rc;
-        double last_rr = S->h_sc[S_TRUE_RR];
+        if ((rc = wait_pub(S))) return rc;
+        double last_rr = S->h_pub[S_TRUE_RR];
         const double it = o->inner_tol > 0.0 ? o->inner_tol : 0.1;
         const double inner2 = it * it;
         int k = 0, pending = 0;  // pending: the correction updates not yet applied (at most two)
-        while (k < o->maxit && S->h_state[0] == ST_RUN) {
+        while (k < o->maxit && h_state(S)[0] == ST_RUN) {
             int chunk = std::min(pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold) {
@@ -1919,12 +1961,12 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                     pending = 1;
                 }
             }
-            k_m_status<<<1, kBlock, 0, st>>>(d);
+            k_m_status<<<1, kBlock, 0, st>>>(d, next_pub(S));
             GIP_LAUNCH_CHECK("mixed iteration");
-            if ((rc = poll(S, true))) return rc;
+            if ((rc = wait_pub(S))) return rc;
             sample_read();
-            if (S->h_state[0] != ST_RUN) break;
-            const double rr32 = S->h_sc[S_RR], tol2 = S->h_sc[S_TOL2];
+            if (h_state(S)[0] != ST_RUN) break;
+            const double rr32 = S->h_pub[S_RR], tol2 = S->h_pub[S_TOL2];
             const bool near_target = tol2 >= 0.0 && rr32 <= tol2;
             if (rr32 <= inner2 * last_rr || near_target || k >= o->maxit) {
                 if (S->fold)
@@ -1934,27 +1976,26 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                 pending = 0;
                 DISPATCH_W(A, k_m_resid, v, d);
                 k_m_coarse<<<S->grid, kBlock, 0, st>>>(d, use_coarse);
-                k_m_corr_fin<<<1, kBlock, 0, st>>>(d, k, 0);
+                k_m_corr_fin<<<1, kBlock, 0, st>>>(d, k, 0, next_pub(S));
                 if (!S->fold) k_m_pairs<<<S->grid, kBlock, 0, st>>>(d, d.sp32[(k - 1) & 1], 0);
                 GIP_LAUNCH_CHECK("mixed correction");
                 ++corrections;
-                if ((rc = poll(S, true))) return rc;
-                last_rr = S->h_sc[S_TRUE_RR];
+                if ((rc = wait_pub(S))) return rc;
+                last_rr = S->h_pub[S_TRUE_RR];
             }
         }
     }
-    if ((rc = poll(S, true))) return rc;
     sample_read();
     int status = GIP_OK;
-    const int fin = S->h_state[0] & ST_MASK;
+    const int fin = h_state(S)[0] & ST_MASK;
     if (fin == ST_BREAK)
         status = GIP_EBREAKDOWN;
     else if (o->tol > 0.0 && fin != ST_CONV)
         status = GIP_ENOCONV;
     if (stats) {
-        stats->iters = S->h_state[1];
+        stats->iters = h_state(S)[1];
         stats->corrections = corrections;
-        const double bb = S->h_sc[S_BB], rr = S->h_sc[S_RR];
+        const double bb = S->h_pub[S_BB], rr = S->h_pub[S_RR];
         stats->relres = bb > 0.0 ? std::sqrt(rr / bb) : std::sqrt(rr);
         stats->status = status;
         stats->product_samples = (int32_t)samples.size();
@@ -1991,8 +2032,6 @@ int gip_pcg_solve_noalloc(gip_ctx *c, const gip_mat *A, int32_t n_all, const dou
     double *base = (c->device >= 0 && c->device < kScratchDevices) ? g_scratch[c->device] : nullptr;
     if (!base) return set_error(GIP_EINVAL, "gip_pcg_solve_noalloc: no scratch on this device (gip_init sets it up)");
     GIP_HIP_TRY(hipSetDevice(c->device));
-    int h_state[2] = {0, 0};
-    double h_sc[S_COUNT] = {};
     gip_pcg S{};
     S.ctx = c;
     S.A = A;
@@ -2011,8 +2050,11 @@ int gip_pcg_solve_noalloc(gip_ctx *c, const gip_mat *A, int32_t n_all, const dou
     S.part = zero;
     S.sc = S.part + (size_t)P_COUNT * kMaxRedBlocks;
     S.state = reinterpret_cast<int *>(S.sc + S_COUNT);
-    S.h_state = h_state;
-    S.h_sc = h_sc;
+    S.h_pub = c->h_result + kPubSlot;
+    S.h_pub_dev = c->h_result_dev + kPubSlot;
+    S.h_flag = reinterpret_cast<uint64_t *>(c->h_result + kPubSeqSlot);
+    S.h_flag_dev = reinterpret_cast<uint64_t *>(c->h_result_dev + kPubSeqSlot);
+    S.seq = &c->pub_seq;
     // partial slots past each producer's grid, the scalars and the state
     // words start at zero (a previous call may have left other values)
     k_zero<<<(unsigned)((kScratchZero + kBlock - 1) / kBlock), kBlock, 0, c->stream>>>(kScratchZero, zero);

@@ -18,6 +18,23 @@ int hip_fail(hipError_t e, const char *what) {
                      std::string(what) + ": " + hipGetErrorString(e));
 }
 
+int wait_published(hipStream_t st, const uint64_t *flag, uint64_t want) {
+    for (unsigned spin = 1;; ++spin) {
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == want) return GIP_OK;
+        if (spin & 0xfffff) {
+            __builtin_ia32_pause();
+            continue;
+        }
+        // the stream may have failed: then the number never comes (asked only
+        // now and then, tens of ms: the query itself queues work)
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return hip_fail(e, "waiting for a kernel's result");
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == want) return GIP_OK;
+        return set_error(GIP_EHIP, "a kernel's result did not arrive");
+    }
+}
+
 int reduce_grid(int n) {
     int g = (n + kBlock * 4 - 1) / (kBlock * 4);
     if (g < 1) g = 1;
@@ -60,8 +77,9 @@ int gip_init(int device, gip_ctx **out) {
     // default-priority, non-blocking stream
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&c->d_partials, sizeof(double) * kMaxRedBlocks * 4);
-    if (e == hipSuccess) e = hipHostMalloc(&c->h_result, sizeof(double) * 4, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc(&c->h_result, sizeof(double) * kHostBlock, hipHostMallocCoherent);
     if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->h_result_dev, c->h_result, 0);
+    if (e == hipSuccess) std::memset(c->h_result, 0, sizeof(double) * kHostBlock);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
         int rc = hip_fail(e, "context setup");
