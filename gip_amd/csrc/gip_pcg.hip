@@ -338,6 +338,37 @@ __global__ __launch_bounds__(kBlock) void k_x_flush(PcgDev d, int k) {
     FOR_ROWS(d.n, row) d.x[row] = d.x[row] + alpha * sp[row].p;  // :95
 }
 
+// Mid-size operators: up to kWideRows rows (mixed: kWideRows32) the products
+// run in workgroups of 512 threads, past 2^20 rows 1024, that store one
+// partial each, at most kMaxRedBlocks of them, which the update's prologue
+// sums like any other: no fold kernel between.  us per iteration with the
+// fold and without: FP64 clustered 81^3 29.5 / 27.7, 97^3 37.7 / 36.4, 112^3
+// 44.3 / 43.6, 128^3 56.8 / 54.5; mixed 81^3 26.8 / 24.4, 97^3 30.0 / 28.4,
+// 112^3 36.0 / 35.6, 128^3 44.9 / 45.2 (so not there); rows in scattered
+// order 81^3 37.3 / 36.5 (1024 threads: 38.8, a last round of 7 of 519
+// workgroups).  The FP64 products with the dictionary, whose wavefronts run
+// for very different times, lose more to wide workgroups than the fold
+// takes (128^3 42.0 / 46.4): they keep a fold, k_fold_wide, which forms the
+// same partials in the same order, so every layout still gives the same bits.
+constexpr int kWideRows = 1024 * kMaxRedBlocks, kWideRows32 = 3 << 19;
+static int wide_of(int n) { return n <= 512 * kMaxRedBlocks ? 512 : 1024; }
+template <int N, int M>
+__device__ inline void wide_store(const PcgDev &d, int c, const double (&sh)[N][M]) {
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < M) {
+        double v = 0.0;
+#pragma unroll
+        for (int q = 0; q < N / kWaves; ++q) {
+            double w = sh[q * kWaves][t];
+#pragma unroll
+            for (int j = 1; j < kWaves; ++j) w = w + sh[q * kWaves + j][t];
+            v = v + w;
+        }
+        d.P(t ? P_SA : P_DN)[c] = v;
+    }
+}
+
 // K1: Ap = A p (empty rows keep Ap), p.Ap partials; one row per thread.
 // Long operators: workgroups in dispatch order, one partial per wavefront
 // (with the direction and update sweeps in dispatch order too, 2% faster
@@ -348,11 +379,12 @@ __global__ __launch_bounds__(kBlock) void k_x_flush(PcgDev d, int k) {
 // reads the operator, but stores nothing.  (The same reordering in the
 // long direction and update sweeps made the solve slower: 1303 ms.)
 // SYM: the slot values from the operator's symmetric form (stencil layout).
-template <int W, bool SYM = false>
+// NB: threads of a workgroup (more than kBlock: wide_store).
+template <int W, int NB, bool SYM = false>
 __device__ inline void iter_spmv(const EllView &A, const PcgDev &d, const double *__restrict__ p) {
     const int st = state_load(d.state);  // tested after the row's loads, before any store
     const int c = blockIdx.x;
-    const int row = c * kBlock + threadIdx.x;
+    const int row = c * NB + threadIdx.x;
     double acc = 0.0, sum = 0.0, pr = 0.0;
     bool any = false;
     if (row < d.n) {
@@ -369,14 +401,20 @@ __device__ inline void iter_spmv(const EllView &A, const PcgDev &d, const double
         if (any) d.Ap[row] = sum;
         acc = pr * sum;
     }
-    // one partial per wavefront: no barrier, each wavefront retires alone
     acc = wave_sum_63(acc);
-    if ((threadIdx.x & 63) == 63) d.chunk[c * kWaves + (threadIdx.x >> 6)] = acc;
+    if constexpr (NB > kBlock) {
+        __shared__ double sh[NB / 64][1];
+        if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6][0] = acc;
+        wide_store(d, c, sh);
+    } else {
+        // one partial per wavefront: no barrier, each wavefront retires alone
+        if ((threadIdx.x & 63) == 63) d.chunk[c * kWaves + (threadIdx.x >> 6)] = acc;
+    }
 }
 
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_iter_spmv(EllView A, PcgDev d, const double *__restrict__ p) {
-    iter_spmv<W>(A, d, p);
+template <int W, int NB>
+__global__ __launch_bounds__(NB) void k_iter_spmv(EllView A, PcgDev d, const double *__restrict__ p) {
+    iter_spmv<W, NB>(A, d, p);
 }
 
 // the first product of a small operator: p_0 from the pairs, XCD-contiguous
@@ -401,9 +439,9 @@ __global__ __launch_bounds__(kBlock) void k_iter_spmv_small(EllView A, PcgDev d)
     if (threadIdx.x == 0) d.chunk[c] = acc;
 }
 
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_iter_spmv_sym(EllView A, PcgDev d, const double *__restrict__ p) {
-    iter_spmv<W, true>(A, d, p);
+template <int W, int NB>
+__global__ __launch_bounds__(NB) void k_iter_spmv_sym(EllView A, PcgDev d, const double *__restrict__ p) {
+    iter_spmv<W, NB, true>(A, d, p);
 }
 
 // K1 with the slot values from the dictionary.  The wavefront sums of a
@@ -630,6 +668,19 @@ __global__ __launch_bounds__(kBlock) void k_fold_dn(PcgDev d) {
         v = block_reduce<RED_SUM>(v);
         if (threadIdx.x == 0) d.P(P_DN)[blockIdx.x] = v;
     }
+}
+
+// wide_store's partials, of `per` chunks each, from those of the chunks (one
+// per chunk).  (Their total from one workgroup instead, so that the update
+// reads one number, was slower: FP64 128^3 42.4 / 44.0 us per iteration.)
+__global__ __launch_bounds__(kBlock) void k_fold_wide(PcgDev d, int per) {
+    if (!running(d)) return;
+    const int i = blockIdx.x * kBlock + threadIdx.x, c0 = i * per;
+    if (i >= d.Gdn) return;
+    double v = 0.0;
+    for (int q = 0; q < per; ++q)
+        if (c0 + q < d.nchunk) v = v + d.chunk[c0 + q];
+    d.P(P_DN)[i] = v;
 }
 
 // K2 (operators of at most 2^19 rows): alpha_k, r += (-alpha) Ap, s = Dinv r,
@@ -1055,10 +1106,10 @@ __global__ __launch_bounds__(kBlock) void k_m_dirprod(EllView A, PcgDev d, int k
 // read only by the fold and the update, which test it; and mixed iterations
 // are queued only while the solve runs (convergence is decided at a defect
 // correction, after which nothing is queued).
-template <int W>
-__global__ __launch_bounds__(kBlock) void k_m_spmv(EllView A, PcgDev d, const float *__restrict__ p) {
+template <int W, int NB>
+__global__ __launch_bounds__(NB) void k_m_spmv(EllView A, PcgDev d, const float *__restrict__ p) {
     const int c = xcd_block(blockIdx.x, gridDim.x);
-    const int row = c * kBlock + threadIdx.x;
+    const int row = c * NB + threadIdx.x;
     double acc = 0.0, sa = 0.0;
     if (row < d.n) {
         // (a SelfOperand here measured 9% slower than the separate load)
@@ -1070,10 +1121,17 @@ __global__ __launch_bounds__(kBlock) void k_m_spmv(EllView A, PcgDev d, const fl
         acc = (double)pr * (double)sum;
         sa = (double)sum;
     }
-    const int wv = c * kWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63;
     acc = wave_sum_two(acc, sa);
-    if (lane == 31) d.chunk[wv] = acc;
-    if (lane == 63) d.chunk_s[wv] = acc;
+    if constexpr (NB > kBlock) {
+        __shared__ double sh[NB / 64][2];
+        if ((lane & 31) == 31) sh[threadIdx.x >> 6][lane >> 5] = acc;
+        wide_store(d, c, sh);
+    } else {
+        const int wv = c * kWaves + (threadIdx.x >> 6);
+        if (lane == 31) d.chunk[wv] = acc;
+        if (lane == 63) d.chunk_s[wv] = acc;
+    }
 }
 
 // the first product of a small operator (as k_iter_spmv_small)
@@ -1525,13 +1583,41 @@ static int pcg_grid(int n) {
         }                                                                                 \
     } while (0)
 #define DISPATCH_W(A, KERNEL, ...) DISPATCH_WG(A, S->grid, KERNEL, __VA_ARGS__)
-// the products over the symmetric form: one workgroup per chunk
-#define SYM_LAUNCH(A, KERNEL, ...)                                                    \
-    do {                                                                              \
-        if (kernel_width(A) == -7)                                                    \
-            KERNEL<-7><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__);                    \
-        else                                                                          \
-            KERNEL<-8><<<S->nchunk, kBlock, 0, st>>>(__VA_ARGS__);                    \
+// the product of a long iteration, KERNEL or (FP64) its _sym form, in
+// workgroups of kWide or kBlock threads
+#define WIDTHS(KERNEL, GRID, NB, P)                                                \
+    switch (kernel_width(A)) {                                                     \
+        case 5: KERNEL<5, NB><<<GRID, NB, 0, st>>>(v, d, P); break;                \
+        case 6: KERNEL<6, NB><<<GRID, NB, 0, st>>>(v, d, P); break;                \
+        case 7: KERNEL<7, NB><<<GRID, NB, 0, st>>>(v, d, P); break;                \
+        case -7: KERNEL<-7, NB><<<GRID, NB, 0, st>>>(v, d, P); break;              \
+        case -8: KERNEL<-8, NB><<<GRID, NB, 0, st>>>(v, d, P); break;              \
+        default: KERNEL<0, NB><<<GRID, NB, 0, st>>>(v, d, P); break;               \
+    }
+#define SYM_WIDTHS(KERNEL, GRID, NB, P)                                            \
+    if (kernel_width(A) == -7)                                                     \
+        KERNEL<-7, NB><<<GRID, NB, 0, st>>>(v, d, P);                              \
+    else                                                                           \
+        KERNEL<-8, NB><<<GRID, NB, 0, st>>>(v, d, P);
+#define SYM_PRODUCT(KERNEL, P)                                                     \
+    do {                                                                           \
+        if (wide == 1024) {                                                        \
+            SYM_WIDTHS(KERNEL, nwide, 1024, P)                                     \
+        } else if (wide) {                                                         \
+            SYM_WIDTHS(KERNEL, nwide, 512, P)                                      \
+        } else {                                                                   \
+            SYM_WIDTHS(KERNEL, S->nchunk, kBlock, P)                               \
+        }                                                                          \
+    } while (0)
+#define ROW_PRODUCT(KERNEL, P)                                                     \
+    do {                                                                           \
+        if (wide == 1024) {                                                        \
+            WIDTHS(KERNEL, nwide, 1024, P)                                         \
+        } else if (wide) {                                                         \
+            WIDTHS(KERNEL, nwide, 512, P)                                          \
+        } else {                                                                   \
+            WIDTHS(KERNEL, S->nchunk, kBlock, P)                                   \
+        }                                                                          \
     } while (0)
 
 #define LEAN_LAUNCH(KERNEL, GRID, ...)                                                \
@@ -1779,6 +1865,15 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                       (!o->precond || (S->ddinv && S->dict_version == A->dict_version));
     PcgDev d = make_dev(S, b, x, o->precond ? 1 : 0);
     if (dict) d.wpc = 1;
+    const int wide = S->fold && S->n <= (mixed ? kWideRows32 : kWideRows) ? wide_of(S->n) : 0;
+    const int nwide = wide ? (S->n + wide - 1) / wide : 0;
+    if (wide) d.Gdn = nwide;
+    auto fold = [&]() {  // between a long product and its update
+        if (!wide)
+            k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
+        else if (dict)
+            k_fold_wide<<<(nwide + kBlock - 1) / kBlock, kBlock, 0, st>>>(d, wide / kBlock);
+    };
     EllView v = view(A);
     const int pollk = o->poll > 0 ? o->poll : 16;
     const int use_coarse = o->coarse >= 0 ? 1 : 0;
@@ -1854,11 +1949,11 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                     if (dict)
                         DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, pdir(k));
                     else if (sym)
-                        SYM_LAUNCH(A, k_iter_spmv_sym, v, d, pdir(k));
+                        SYM_PRODUCT(k_iter_spmv_sym, pdir(k));
                     else
-                        DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, pdir(k));
+                        ROW_PRODUCT(k_iter_spmv, pdir(k));
                     sample_end(smp);
-                    k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
+                    fold();
                     LEAN_LAUNCH(k_iter_update_grid, S->grid, d, k);
                 } else if (S->fold) {
                     // (partials: p.Ap in chunk, then r.s in chunk and r.r in chunk_s)
@@ -1867,9 +1962,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                     if (dict)
                         DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, pdir(k));
                     else if (sym)
-                        SYM_LAUNCH(A, k_iter_spmv_sym, v, d, pdir(k));
+                        SYM_PRODUCT(k_iter_spmv_sym, pdir(k));
                     else
-                        DISPATCH_WG(A, S->nchunk, k_iter_spmv, v, d, pdir(k));
+                        ROW_PRODUCT(k_iter_spmv, pdir(k));
                     sample_end(smp);
                     k_fold_two<<<S->gdn, kBlock, 0, st>>>(d, S->nchunk, d.wpc, d.chunk, nullptr, P_DN, P_DN);
                     k_alpha_fin<<<1, kBlock, 0, st>>>(d, k);
@@ -1941,9 +2036,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                     if (dict)
                         DICT_LAUNCH(k_m_spmv_dict, A->st_w, S->nchunk, st, v, d, pdir32(k));
                     else
-                        DISPATCH_WG(A, S->nchunk, k_m_spmv, v, d, pdir32(k));
+                        ROW_PRODUCT(k_m_spmv, pdir32(k));
                     sample_end(smp);
-                    k_fold_dn<<<S->gdn, kBlock, 0, st>>>(d);
+                    fold();
                     LEAN_LAUNCH(k_m_update, S->grid, d, k);
                 } else {
                     const bool smp = sample_begin(k);
