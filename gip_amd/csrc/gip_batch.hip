@@ -22,7 +22,8 @@ constexpr int kChunk = kBlock;  // rows per chunk = threads per workgroup
 enum { F_A1 = 0, F_A2, F_SIGMA, F_CORR, F_F1, F_F2, F_RHO, F_COUNT = 8 };
 enum { FAC_ONE = -1, FAC_ZERO = -2 };
 // per-instance PCG scalars
-enum { B_RHO = 0, B_ALPHA, B_BETA, B_RR, B_BB, B_TOL2, B_RHO_PREV, B_LAST_RR, B_NEED, B_ZAZ, B_C, B_COUNT = 16 };
+enum { B_RHO = 0, B_ALPHA, B_BETA, B_RR, B_BB, B_TOL2, B_RHO_PREV, B_LAST_RR, B_NEED, B_ZAZ, B_C,
+       B_RHO_K, B_RHO_K1, B_COUNT = 16 };  // rho within a group, by iteration parity
 enum { BS_RUN = 0, BS_CONV = 1, BS_BREAK = 2, BS_MAXED = 3 };
 
 struct Seg {
@@ -178,14 +179,12 @@ __global__ __launch_bounds__(kBlock) void k_b_cfl_fin(const double *part, Seg S,
     }
 }
 
-// The PCG product and update kernels instead run one workgroup per chunk in
-// dispatch order (grid = the chunk count: the pace of a plain stream), sum
-// their wavefronts by DPP and store one total per chunk (seg_store_c: one
-// barrier, which costs less than the finalize kernels' reading four times
-// as many partials, and than an 8-byte store per wavefront and sum); their
-// finalize kernels sum an instance's chunk totals in chunk order
-// (seg_total_c).  A chunk of an instance that has left the PCG returns
-// after two loads.
+// The PCG product instead runs one workgroup per chunk in dispatch order
+// (grid = the chunk count: the pace of a plain stream), sums its wavefronts
+// by DPP and stores one total per chunk (seg_store_c: one barrier, which
+// costs less than reading four times as many partials, and than an 8-byte
+// store per wavefront and sum).  A chunk of an instance that has left the
+// PCG returns after two loads.
 template <int K>
 __device__ inline void seg_store_c(double (&v)[K], int c, double *part) {
     static_assert(K <= 2, "at most two sums");
@@ -202,29 +201,70 @@ __device__ inline void seg_store_c(double (&v)[K], int c, double *part) {
     }
 }
 
-// (valid in thread 0)
-template <int K>
-__device__ inline void seg_total_c(const double *part, int inst, const Seg &S, double (&out)[K]) {
-    static_assert(K <= 2, "at most two sums");
-    __shared__ double sh[kWaves][K];
-    const size_t c0 = (size_t)S.inst_c0[inst];
-    const int nch = S.inst_nch[inst], lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    double acc[K];
+// The direction and update sweeps run one workgroup per unit of up to U
+// chunks of one instance, a row of each chunk per thread, all requested
+// before the first is used.  Their prologue sums the instance's partials of
+// the kernel before (InstSums), so every workgroup of an instance forms the
+// same alpha, or the same beta, and the kernels that did so alone, one
+// workgroup per instance, are left to instances of more than kDirectChunks
+// chunks and to the end of a group of iterations.  12 cavities of sides 32
+// to 72: 36.5 us in three kernels per iteration against 43.5 in five, and the
+// gaps between them; the step 41.0 -> 35.9 ms.
+constexpr int kDirectChunks = 2048;
+struct BUnit {
+    int32_t inst, c0, n, first;  // instance, first chunk, chunks, whether the instance's first unit
+    int32_t ic0, inc, iu0, inu;  // the instance's first chunk, chunks, first unit and units
+};
+
+// M sums of at most K x 256 partials (M per slot) from slot c0 on; every thread
+template <int M, int K>
+struct InstSums {
+    double v[K][M];
+    __device__ inline void load(const double *__restrict__ part, int c0, int n) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) acc[k] = 0.0;
-#pragma unroll 8
-    for (int j = threadIdx.x; j < nch; j += kBlock)
+        for (int k = 0; k < K; ++k) {
+            const int i = threadIdx.x + k * kBlock;
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc[k] = acc[k] + part[(c0 + j) * K + k];
-    const double t = K == 1 ? wave_sum_63(acc[0]) : wave_sum_two(acc[0], acc[K - 1]);
-    if (K == 1 ? lane == 63 : (lane & 31) == 31) sh[w][K == 1 ? 0 : lane >> 5] = t;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        out[k] = sh[0][k];
-#pragma unroll
-        for (int q = 1; q < kWaves; ++q) out[k] = out[k] + sh[q][k];
+            for (int m = 0; m < M; ++m) v[k][m] = i < n ? part[(size_t)(c0 + i) * M + m] : 0.0;
+        }
     }
+    __device__ inline void total(double (&out)[M]) const {
+        static_assert(M <= 2, "at most two sums");
+        __shared__ double sh[kWaves][M];
+        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+        double acc[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            acc[m] = 0.0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) acc[m] = acc[m] + v[k][m];
+        }
+        const double t = M == 1 ? wave_sum_63(acc[0]) : wave_sum_two(acc[0], acc[M - 1]);
+        if (M == 1 ? lane == 63 : (lane & 31) == 31) sh[w][M == 1 ? 0 : lane >> 5] = t;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            out[m] = sh[0][m];
+#pragma unroll
+            for (int q = 1; q < kWaves; ++q) out[m] = out[m] + sh[q][m];
+        }
+    }
+};
+
+// the same sums of any number of partials, for a kernel of one workgroup per instance
+template <int M>
+__device__ inline void inst_total(const double *part, int c0, int n, double (&out)[M]) {
+    constexpr int K = kDirectChunks / kBlock;
+    InstSums<M, K> ps, more;
+    ps.load(part, c0, n);
+    for (int at = K * kBlock; at < n; at += K * kBlock) {
+        more.load(part, c0 + at, n - at);
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int m = 0; m < M; ++m) ps.v[k][m] = ps.v[k][m] + more.v[k][m];
+    }
+    ps.total(out);
 }
 
 // ---- batched PCG ------------------------------------------------------------
@@ -239,15 +279,54 @@ struct BPcg {
     double *sc;              // B * B_COUNT
     int *state, *iters, *active;
     double *part;  // chunk totals
+    double *part_u;  // r.s and r.r of each unit, past the product's chunk totals
+    const BUnit *unit;
+    const int32_t *u0, *nu;  // instance -> first unit, units
+    int direct;  // no instance has more than kDirectChunks chunks
     int maxit;
     double inner2;
 };
 
 __device__ inline double *bsc(const BPcg &d, int inst) { return d.sc + (size_t)inst * B_COUNT; }
 
+// Written by the first workgroup of an instance while its others may be
+// reading it: those compute the same decision, or skip work whose result
+// nothing reads.
+__device__ inline int b_state(const BPcg &d, int inst) {
+    return __hip_atomic_load(d.state + inst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ inline void leave(const BPcg &d, int inst, int st) {
-    d.state[inst] = st;
+    __hip_atomic_store(d.state + inst, st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     atomicSub(d.active, 1);
+}
+
+// rho of iteration k of a group: where the workgroups of an instance form it
+// themselves, in two slots by parity past the group's first
+__device__ inline int rho_at(const BPcg &d, int k) { return d.direct && k > 0 ? B_RHO_K + (k & 1) : B_RHO; }
+
+// the row of chunk j of a unit (its first chunk's again past the last: a
+// load that hits, and no store)
+__device__ inline int unit_row(const BUnit &u, int j) { return (u.c0 + (j < u.n ? j : 0)) * kChunk + (int)threadIdx.x; }
+
+// the first workgroup's part at the end of iteration k - 1, formed by the
+// direction sweep of iteration k: FP64 ...
+__device__ inline void next_iter(const BPcg &d, int inst, int k, const double (&rho_rr)[2]) {
+    double *q = bsc(d, inst);
+    q[rho_at(d, k)] = rho_rr[0];
+    q[B_RR] = rho_rr[1];
+    const int it = ++d.iters[inst];
+    if (rho_rr[1] <= q[B_TOL2])
+        leave(d, inst, BS_CONV);
+    else if (it >= d.maxit)
+        leave(d, inst, BS_MAXED);
+}
+// ... and MIXED
+__device__ inline void next_iter_m(const BPcg &d, int inst, int k, const double (&rho_rr)[2]) {
+    double *q = bsc(d, inst);
+    q[rho_at(d, k)] = rho_rr[0];
+    q[B_RR] = rho_rr[1];
+    const int it = ++d.iters[inst];
+    if (rho_rr[1] <= d.inner2 * q[B_LAST_RR] || rho_rr[1] <= q[B_TOL2] || it >= d.maxit) q[B_NEED] = 1.0;
 }
 
 // the number of instances still running, for the host's poll
@@ -323,19 +402,36 @@ __global__ __launch_bounds__(kBlock) void k_bp_setup_fin(BPcg d, Seg S, double t
 }
 
 // direction of the running instances: p = 1.0 s + beta p (GIP_LinearSolver.h:113;
-// the first iteration has beta = 0 and p = 0 on the solved rows, so p = s)
-// (a grid-stride sweep: at 12-24 B per row a workgroup per chunk spends
-// more on its launch than on its rows)
-__global__ __launch_bounds__(kBlock) void k_bp_dir(BPcg d, Seg S, double *__restrict__ p) {
-    const double *__restrict__ s = d.s;
-    FOR_CHUNKS(S, c) {
-        const int inst = S.chunk_inst[c];
-        if (d.state[inst] != BS_RUN) continue;
-        const int row = c * kChunk + threadIdx.x;
-        const double beta = bsc(d, inst)[B_BETA];
-        const double si = s[row], po = p[row];
-        p[row] = 1.0 * si + beta * po;
+// the first iteration has beta = 0 and p = 0 on the solved rows, so p = s).
+// k: iteration of the group
+template <int U>
+__global__ __launch_bounds__(kBlock) void k_bp_dir(BPcg d, double *__restrict__ p, int k) {
+    const BUnit u = d.unit[blockIdx.x];
+    const int st = b_state(d, u.inst);
+    const bool form = d.direct && k > 0;
+    double si[U], po[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int row = unit_row(u, j);
+        si[j] = d.s[row];
+        po[j] = p[row];
     }
+    InstSums<2, kDirectChunks / kBlock / U> ps;
+    if (form) ps.load(d.part_u, u.iu0, u.inu);
+    const double *q = bsc(d, u.inst);
+    double beta = q[B_BETA];
+    const double r0 = q[rho_at(d, form ? k - 1 : 0)], tol2 = q[B_TOL2];
+    if (st != BS_RUN) return;
+    if (form) {
+        double rho[2];
+        ps.total(rho);
+        if (u.first && threadIdx.x == 0) next_iter(d, u.inst, k, rho);
+        if (rho[1] <= tol2) return;
+        beta = rho[0] / r0;
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+        if (j < u.n) p[unit_row(u, j)] = 1.0 * si[j] + beta * po[j];
 }
 
 // Ap = A p (one gather of p per neighbour), chunk partials of p.Ap
@@ -356,12 +452,13 @@ __global__ __launch_bounds__(kBlock) void k_bp_spmv(EllView A, BPcg d, Seg S, co
     seg_store_c<1>(v, c, d.part);
 }
 
-// alpha = rho / p.Ap of the running instances (FP64 and MIXED)
+// alpha = rho / p.Ap of the running instances (FP64 and MIXED), where an
+// instance is too large for the update to form it
 __global__ __launch_bounds__(kBlock) void k_bp_spmv_fin(BPcg d, Seg S) {
     const int inst = blockIdx.x;
     if (d.state[inst] != BS_RUN) return;
     double out[1];
-    seg_total_c<1>(d.part, inst, S, out);
+    inst_total<1>(d.part, S.inst_c0[inst], S.inst_nch[inst], out);
     if (threadIdx.x == 0) {
         double *q = bsc(d, inst);
         const double alpha = q[B_RHO] / out[0];
@@ -370,46 +467,79 @@ __global__ __launch_bounds__(kBlock) void k_bp_spmv_fin(BPcg d, Seg S) {
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_bp_update(BPcg d, Seg S, const double *__restrict__ p, int precond) {
-    const int c = blockIdx.x;
-    const int inst = S.chunk_inst[c];
-    if (d.state[inst] != BS_RUN) return;
-    const int row = c * kChunk + threadIdx.x;
-    const double alpha = bsc(d, inst)[B_ALPHA];
-    // every operand first: one memory round trip per row
-    const double xo = d.x[row], pr = p[row], ro = d.r[row], apr = d.Ap[row];
-    const double di = precond ? d.dinv[row] : 0.0;
-    d.x[row] = xo + alpha * pr;
-    const double ri = ro + (-1.0 * alpha) * apr;
-    d.r[row] = ri;
-    double si;
-    if (precond) {
-        si = 0.0;
-        si = si + ri * di;
-    } else {
-        si = ri;
+// alpha for a workgroup of an update, its loads requested at load()
+struct UnitAlpha {
+    InstSums<1, kDirectChunks / kBlock> ps;
+    double rho, alpha;
+    __device__ inline void load(const BPcg &d, const BUnit &u, int k) {
+        const double *q = bsc(d, u.inst);
+        rho = q[rho_at(d, k)];
+        alpha = q[B_ALPHA];
+        if (d.direct) ps.load(d.part, u.ic0, u.inc);
     }
-    d.s[row] = si;
-    double v[2] = {ri * si, ri * ri};
-    seg_store_c<2>(v, c, d.part);
+    // false after a breakdown
+    __device__ inline bool form(const BPcg &d, const BUnit &u) {
+        if (!d.direct) return true;
+        double dn[1];
+        ps.total(dn);
+        alpha = rho / dn[0];
+        if (dn[0] != 0.0 && isfinite(dn[0]) && isfinite(alpha)) return true;
+        if (u.first && threadIdx.x == 0) leave(d, u.inst, BS_BREAK);
+        return false;
+    }
+};
+
+template <int U>
+__global__ __launch_bounds__(kBlock) void k_bp_update(BPcg d, const double *__restrict__ p, int k, int precond) {
+    const BUnit u = d.unit[blockIdx.x];
+    const int st = b_state(d, u.inst);
+    double xo[U], pr[U], ro[U], apr[U], di[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int row = unit_row(u, j);
+        xo[j] = d.x[row];
+        pr[j] = p[row];
+        ro[j] = d.r[row];
+        apr[j] = d.Ap[row];
+        di[j] = precond ? d.dinv[row] : 0.0;
+    }
+    UnitAlpha ua;
+    ua.load(d, u, k);
+    if (st != BS_RUN || !ua.form(d, u)) return;
+    const double alpha = ua.alpha;
+    double v[2] = {0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        if (j >= u.n) break;
+        const int row = unit_row(u, j);
+        d.x[row] = xo[j] + alpha * pr[j];
+        const double ri = ro[j] + (-1.0 * alpha) * apr[j];
+        d.r[row] = ri;
+        double si;
+        if (precond) {
+            si = 0.0;
+            si = si + ri * di[j];
+        } else {
+            si = ri;
+        }
+        d.s[row] = si;
+        v[0] = v[0] + ri * si;
+        v[1] = v[1] + ri * ri;
+    }
+    seg_store_c<2>(v, blockIdx.x, d.part_u);
 }
 
-__global__ __launch_bounds__(kBlock) void k_bp_update_fin(BPcg d, Seg S) {
+// the end of iteration k of a group (every iteration's, where the next
+// direction sweep does not form its sums)
+__global__ __launch_bounds__(kBlock) void k_bp_update_fin(BPcg d, int k) {
     const int inst = blockIdx.x;
     if (d.state[inst] != BS_RUN) return;
     double out[2];
-    seg_total_c<2>(d.part, inst, S, out);
+    inst_total<2>(d.part_u, d.u0[inst], d.nu[inst], out);
     if (threadIdx.x == 0) {
         double *q = bsc(d, inst);
-        const double r0 = q[B_RHO];
-        q[B_RHO] = out[0];
-        q[B_BETA] = out[0] / r0;
-        q[B_RR] = out[1];
-        const int it = ++d.iters[inst];
-        if (out[1] <= q[B_TOL2])
-            leave(d, inst, BS_CONV);
-        else if (it >= d.maxit)
-            leave(d, inst, BS_MAXED);
+        q[B_BETA] = out[0] / q[rho_at(d, k)];
+        next_iter(d, inst, 0, out);
     }
 }
 
@@ -480,16 +610,34 @@ __global__ __launch_bounds__(kBlock) void k_bpm_setup_fin(BPcg d, Seg S, double 
 
 // (nontemporal accesses here and in the update: each array is streamed once
 // per sweep; 64-cavity batch 133 -> 126 ms of PCG per step)
-__global__ __launch_bounds__(kBlock) void k_bpm_dir(BPcg d, Seg S, float *__restrict__ p) {
-    const float *__restrict__ s = d.s32;
-    FOR_CHUNKS(S, c) {
-        const int inst = S.chunk_inst[c];
-        if (d.state[inst] != BS_RUN) continue;
-        const int row = c * kChunk + threadIdx.x;
-        const float beta = (float)bsc(d, inst)[B_BETA];
-        const float si = __builtin_nontemporal_load(s + row), po = __builtin_nontemporal_load(p + row);
-        __builtin_nontemporal_store(1.0f * si + beta * po, p + row);
+template <int U>
+__global__ __launch_bounds__(kBlock) void k_bpm_dir(BPcg d, float *__restrict__ p, int k) {
+    const BUnit u = d.unit[blockIdx.x];
+    const int st = b_state(d, u.inst);
+    const bool form = d.direct && k > 0;
+    float si[U], po[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int row = unit_row(u, j);
+        si[j] = __builtin_nontemporal_load(d.s32 + row);
+        po[j] = __builtin_nontemporal_load(p + row);
     }
+    InstSums<2, kDirectChunks / kBlock / U> ps;
+    if (form) ps.load(d.part_u, u.iu0, u.inu);
+    const double *q = bsc(d, u.inst);
+    double beta = q[B_BETA];
+    const double r0 = q[rho_at(d, form ? k - 1 : 0)];
+    if (st != BS_RUN) return;
+    if (form) {
+        double rho[2];
+        ps.total(rho);
+        if (u.first && threadIdx.x == 0) next_iter_m(d, u.inst, k, rho);
+        beta = rho[0] / r0;
+    }
+    const float b32 = (float)beta;
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+        if (j < u.n) __builtin_nontemporal_store(1.0f * si[j] + b32 * po[j], p + unit_row(u, j));
 }
 
 template <int W>
@@ -507,38 +655,51 @@ __global__ __launch_bounds__(kBlock) void k_bpm_spmv(EllView A, BPcg d, Seg S, c
     seg_store_c<1>(v, c, d.part);
 }
 
-__global__ __launch_bounds__(kBlock) void k_bpm_update(BPcg d, Seg S, const float *__restrict__ p, int precond) {
-    const int c = blockIdx.x;
-    const int inst = S.chunk_inst[c];
-    if (d.state[inst] != BS_RUN) return;
-    const int row = c * kChunk + threadIdx.x;
-    const float a32 = (float)bsc(d, inst)[B_ALPHA];
-    const float xo = __builtin_nontemporal_load(d.xc32 + row), pr = __builtin_nontemporal_load(p + row),
-                ro = __builtin_nontemporal_load(d.r32 + row), apr = __builtin_nontemporal_load(d.Ap32 + row);
-    const float di = precond ? __builtin_nontemporal_load(d.dinv32 + row) : 0.0f;
-    __builtin_nontemporal_store(xo + a32 * pr, d.xc32 + row);
-    const float ri = ro - a32 * apr;
-    __builtin_nontemporal_store(ri, d.r32 + row);
-    const float si = precond ? ri * di : ri;
-    __builtin_nontemporal_store(si, d.s32 + row);
-    double v[2] = {(double)ri * (double)si, (double)ri * (double)ri};
-    seg_store_c<2>(v, c, d.part);
+template <int U>
+__global__ __launch_bounds__(kBlock) void k_bpm_update(BPcg d, const float *__restrict__ p, int k, int precond) {
+    const BUnit u = d.unit[blockIdx.x];
+    const int st = b_state(d, u.inst);
+    float xo[U], pr[U], ro[U], apr[U], di[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int row = unit_row(u, j);
+        xo[j] = __builtin_nontemporal_load(d.xc32 + row);
+        pr[j] = __builtin_nontemporal_load(p + row);
+        ro[j] = __builtin_nontemporal_load(d.r32 + row);
+        apr[j] = __builtin_nontemporal_load(d.Ap32 + row);
+        di[j] = precond ? __builtin_nontemporal_load(d.dinv32 + row) : 0.0f;
+    }
+    UnitAlpha ua;
+    ua.load(d, u, k);
+    if (st != BS_RUN || !ua.form(d, u)) return;
+    const float a32 = (float)ua.alpha;
+    double v[2] = {0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        if (j >= u.n) break;
+        const int row = unit_row(u, j);
+        __builtin_nontemporal_store(xo[j] + a32 * pr[j], d.xc32 + row);
+        const float ri = ro[j] - a32 * apr[j];
+        __builtin_nontemporal_store(ri, d.r32 + row);
+        const float si = precond ? ri * di[j] : ri;
+        __builtin_nontemporal_store(si, d.s32 + row);
+        v[0] = v[0] + (double)ri * (double)si;
+        v[1] = v[1] + (double)ri * (double)ri;
+    }
+    seg_store_c<2>(v, blockIdx.x, d.part_u);
 }
 
-__global__ __launch_bounds__(kBlock) void k_bpm_update_fin(BPcg d, Seg S) {
+__global__ __launch_bounds__(kBlock) void k_bpm_update_fin(BPcg d, int k) {
     const int inst = blockIdx.x;
     if (d.state[inst] != BS_RUN) return;
     double out[2];
-    seg_total_c<2>(d.part, inst, S, out);
+    inst_total<2>(d.part_u, d.u0[inst], d.nu[inst], out);
     if (threadIdx.x == 0) {
         double *q = bsc(d, inst);
-        const double r0 = q[B_RHO];
+        const double r0 = q[rho_at(d, k)];
         q[B_RHO_PREV] = r0;
-        q[B_RHO] = out[0];
         q[B_BETA] = out[0] / r0;
-        q[B_RR] = out[1];
-        const int it = ++d.iters[inst];
-        if (out[1] <= d.inner2 * q[B_LAST_RR] || out[1] <= q[B_TOL2] || it >= d.maxit) q[B_NEED] = 1.0;
+        next_iter_m(d, inst, 0, out);
     }
 }
 
@@ -650,6 +811,11 @@ struct gip_batch {
     // row-space segmentations (device)
     int32_t *d_seg_in[3] = {}, *d_seg_f[3] = {};
     Seg seg_in{}, seg_f{};
+    // units of the PCG's sweeps (device)
+    BUnit *unit = nullptr;
+    int32_t *unit_u0 = nullptr, *unit_nu = nullptr;
+    int nunit = 0, unit_chunks = 1;
+    bool direct = false;
     // fields
     double *u = nullptr, *v = nullptr, *w = nullptr, *ax = nullptr, *ay = nullptr, *az = nullptr, *ax0 = nullptr,
            *ay0 = nullptr, *az0 = nullptr, *rhs = nullptr, *p = nullptr, *p0 = nullptr, *gpx = nullptr,
@@ -748,6 +914,37 @@ int make_seg(gip_batch *b, const std::vector<int64_t> &off, const std::vector<in
     return GIP_OK;
 }
 
+// The units of the direction and update sweeps: as many chunks each (1, 2 or
+// 4) as leave at least 1024 of them, four workgroups per CU.
+int make_units(gip_batch *b, const std::vector<int64_t> &off, const std::vector<int64_t> &cnt, int64_t total) {
+    const int64_t nch = total / kChunk;
+    b->unit_chunks = nch >= 4096 ? 4 : nch >= 2048 ? 2 : 1;
+    std::vector<BUnit> un;
+    std::vector<int32_t> u0, nu;
+    b->direct = true;
+    for (int i = 0; i < b->B; ++i) {
+        const int64_t c0 = off[(size_t)i] / kChunk, nc = roundup(cnt[(size_t)i], kChunk) / kChunk;
+        if (nc > kDirectChunks) b->direct = false;
+        u0.push_back((int32_t)un.size());
+        for (int64_t k = 0; k < nc; k += b->unit_chunks)
+            un.push_back(BUnit{i, (int32_t)(c0 + k), (int32_t)std::min<int64_t>(b->unit_chunks, nc - k), k == 0,
+                               (int32_t)c0, (int32_t)nc, u0.back(), 0});
+        nu.push_back((int32_t)un.size() - u0.back());
+        for (size_t k = (size_t)u0.back(); k < un.size(); ++k) un[k].inu = nu.back();
+    }
+    b->nunit = (int)un.size();
+    int rc = dalloc_t(b, &b->unit, un.size());
+    if (!rc) rc = dalloc_t(b, &b->unit_u0, u0.size());
+    if (!rc) rc = dalloc_t(b, &b->unit_nu, nu.size());
+    if (rc) return rc;
+    hipStream_t st = b->c->stream;
+    GIP_HIP_TRY(hipMemcpyAsync(b->unit, un.data(), un.size() * sizeof(BUnit), hipMemcpyHostToDevice, st));
+    GIP_HIP_TRY(hipMemcpyAsync(b->unit_u0, u0.data(), u0.size() * 4, hipMemcpyHostToDevice, st));
+    GIP_HIP_TRY(hipMemcpyAsync(b->unit_nu, nu.data(), nu.size() * 4, hipMemcpyHostToDevice, st));
+    GIP_HIP_TRY(hipStreamSynchronize(st));
+    return GIP_OK;
+}
+
 // the shared operator view and kernel width (gip_rows.h)
 EllView view_of(const gip_mat *A) { return view(A); }
 
@@ -770,6 +967,17 @@ int seg_spmv(gip_batch *b, const gip_mat *A, const double *x, double *y, bool fa
     GIP_LAUNCH_CHECK("batch segmented spmv");
     return GIP_OK;
 }
+
+// KERNEL<U> over the units
+#define UNIT_LAUNCH(KERNEL, ...)                                                                 \
+    do {                                                                                         \
+        if (b->unit_chunks == 4)                                                                 \
+            KERNEL<4><<<(unsigned)b->nunit, kBlock, 0, st>>>(__VA_ARGS__);                       \
+        else if (b->unit_chunks == 2)                                                            \
+            KERNEL<2><<<(unsigned)b->nunit, kBlock, 0, st>>>(__VA_ARGS__);                       \
+        else                                                                                     \
+            KERNEL<1><<<(unsigned)b->nunit, kBlock, 0, st>>>(__VA_ARGS__);                       \
+    } while (0)
 
 BPcg pcg_view(gip_batch *b) {
     BPcg d;
@@ -794,6 +1002,11 @@ BPcg pcg_view(gip_batch *b) {
     d.iters = b->iters;
     d.active = b->active;
     d.part = b->part;
+    d.part_u = b->part + b->seg_in.nchunk;
+    d.unit = b->unit;
+    d.u0 = b->unit_u0;
+    d.nu = b->unit_nu;
+    d.direct = b->direct;
     d.maxit = b->o.pcg_maxit;
     const double it = b->o.inner_tol > 0 ? b->o.inner_tol : 0.1;
     d.inner2 = it * it;
@@ -853,18 +1066,19 @@ int enqueue_iter(gip_batch *b) {
     const bool mixed = b->o.precision == GIP_PCG_MIXED;
     const unsigned nch = (unsigned)b->seg_in.nchunk;  // one workgroup per chunk
     for (int k = 0; k < b->o.poll; ++k) {
+        const bool fin = !b->direct || k + 1 == b->o.poll;
         if (mixed) {
-            k_bpm_dir<<<b->grid_in, kBlock, 0, st>>>(d, b->seg_in, b->pq);
+            UNIT_LAUNCH(k_bpm_dir, d, b->pq, k);
             BDISPATCH(L, nch, k_bpm_spmv, view_of(L), d, b->seg_in, b->pq);
-            k_bp_spmv_fin<<<b->B, kBlock, 0, st>>>(d, b->seg_in);
-            k_bpm_update<<<nch, kBlock, 0, st>>>(d, b->seg_in, b->pq, 1);
-            k_bpm_update_fin<<<b->B, kBlock, 0, st>>>(d, b->seg_in);
+            if (!b->direct) k_bp_spmv_fin<<<b->B, kBlock, 0, st>>>(d, b->seg_in);
+            UNIT_LAUNCH(k_bpm_update, d, b->pq, k, 1);
+            if (fin) k_bpm_update_fin<<<b->B, kBlock, 0, st>>>(d, k);
         } else {
-            k_bp_dir<<<b->grid_in, kBlock, 0, st>>>(d, b->seg_in, b->pp);
+            UNIT_LAUNCH(k_bp_dir, d, b->pp, k);
             BDISPATCH(L, nch, k_bp_spmv, view_of(L), d, b->seg_in, b->pp);
-            k_bp_spmv_fin<<<b->B, kBlock, 0, st>>>(d, b->seg_in);
-            k_bp_update<<<nch, kBlock, 0, st>>>(d, b->seg_in, b->pp, 1);
-            k_bp_update_fin<<<b->B, kBlock, 0, st>>>(d, b->seg_in);
+            if (!b->direct) k_bp_spmv_fin<<<b->B, kBlock, 0, st>>>(d, b->seg_in);
+            UNIT_LAUNCH(k_bp_update, d, b->pp, k, 1);
+            if (fin) k_bp_update_fin<<<b->B, kBlock, 0, st>>>(d, k);
         }
     }
     if (mixed) {
@@ -988,6 +1202,7 @@ int gip_batch_create(gip_ctx *c, int32_t ninst, const gip_cavity *const *cavs, c
     int rc = GIP_OK;
     if (b->ALLB > INT32_MAX / 2 || b->FP > INT32_MAX / 2) rc = set_error(GIP_EINVAL, "gip_batch_create: batch too large");
     if (!rc) rc = make_seg(b, b->off_in, npad, b->NP, b->d_seg_in, &b->seg_in);
+    if (!rc) rc = make_units(b, b->off_in, npad, b->NP);
     if (!rc) rc = make_seg(b, b->off_f, fpad, b->FP, b->d_seg_f, &b->seg_f);
     auto grid_for = [](int64_t nch) { return (int)std::min<int64_t>(std::max<int64_t>(nch, 1), 4096); };
     b->grid_in = grid_for(b->NP / kChunk);

@@ -185,3 +185,30 @@ def test_batch_argument_errors(dev):
     with pytest.raises(hip.HipError) as e:
         batch.Batch(dev, [full, lap_only], [1e-2, 1e-2], pcg_tol=1e-8)
     assert e.value.code == hip.EINVAL
+
+
+# One, two or four chunks per workgroup of the sweeps by the size of the
+# batch, partial units at an instance's end, and an instance of more than
+# 2048 chunks (81^3), with which one-workgroup kernels form the scalars: an
+# instance gives what it gives alone.  40 iterations without a tolerance, so
+# only the order of the sums differs: FP64 40 x 2 steps x 1e-16 and its
+# growth through the iteration, bounded by 1e-9; in mixed precision a flipped
+# rounding of alpha or beta to FP32 (6e-8) in each of 80 iterations, 1e-5.
+@pytest.mark.parametrize("precision,bound", [(hip.PCG_FP64, 1e-9), (hip.PCG_MIXED, 1e-5)])
+@pytest.mark.parametrize("sizes", [[20, 57, 57, 57], [20, 64, 64, 64, 64, 9], [20, 81, 9]])
+def test_instance_in_a_large_batch_is_the_instance_alone(dev, sizes, precision, bound):
+    def run(ns, poll):
+        cavs = [cavity.generate(n, gamma=1e-2) for n in ns]
+        b = batch.Batch(dev, cavs, [1e-2] * len(ns), pcg_tol=1e-30, pcg_maxit=40, precision=precision, poll=poll,
+                        use_graph=False)
+        for _ in range(2):
+            b.step()
+        out = [(b.info(k)["pcg_iters"], b.field(k, "p")) for k in range(len(ns))]
+        b.close()
+        return out
+
+    got = run(sizes, 7)
+    for k in (0, len(sizes) - 2, len(sizes) - 1):
+        (iters, p), = run([sizes[k]], 7)
+        assert got[k][0] == iters
+        assert np.abs(got[k][1] - p).max() <= bound * np.abs(p).max(), sizes[k]
