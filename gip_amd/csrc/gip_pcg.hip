@@ -183,14 +183,18 @@ constexpr int kSweepU = LEAN ? 2 : 1;
 // reads r instead of s and forms it again, with the inverse diagonal from
 // the dictionary, so the update writes r alone: two vector streams of its
 // five less.  The same expression on the same values: the same bits.
-__device__ inline double s_of(const PcgDev &d, int row, double r) {
-    if (!d.precond) return r;
+__device__ inline double s_of(double r, double di, bool precond) {
+    if (!precond) return r;
     double si = 0.0;
-    si = si + r * dict_one(d.dc_sel, d.dc_id, d.ddinv, row);  // :99-105
+    si = si + r * di;  // :99-105
     return si;
 }
-__device__ inline float s_of(const PcgDev &d, int row, float r) {
-    return d.precond ? r * dict_one(d.dc_sel, d.dc_id, d.ddinv32, row) : r;
+__device__ inline float s_of(float r, float di, bool precond) { return precond ? r * di : r; }
+__device__ inline double dict_dinv(const PcgDev &d, int row, double) {
+    return d.precond ? dict_one(d.dc_sel, d.dc_id, d.ddinv, row) : 0.0;
+}
+__device__ inline float dict_dinv(const PcgDev &d, int row, float) {
+    return d.precond ? dict_one(d.dc_sel, d.dc_id, d.ddinv32, row) : 0.0f;
 }
 
 // ---- setup ---------------------------------------------------------------
@@ -760,16 +764,24 @@ __device__ inline double x_two(double x, double a2, double p2, double a1, double
 
 // K0 (k >= 1): rho_k, the convergence test, beta, p_k = 1.0 s + beta p_{k-1}
 // into pnew (which holds p_{k-2}); PAIR: the x updates of k-2 and k-1
-template <bool LEAN, bool PAIR>
+template <bool LEAN, bool PAIR, int U>
 __global__ __launch_bounds__(kBlock) void k_iter_dir(PcgDev d, const double *__restrict__ pold,
                                                     double *__restrict__ pnew, int k) {
     double *__restrict__ x = d.x;
     const double *__restrict__ s = LEAN ? d.r : d.s;
     const int st = state_load(d.state);
-    if (st != ST_RUN && st != conv_stamp(k)) return;
+    struct In {
+        double s, di, po, x, pp;
+    };
+    const auto load = [&](int row) {
+        return In{s[row], LEAN ? dict_dinv(d, row, 0.0) : 0.0, pold[row], PAIR ? x[row] : 0.0, PAIR ? pnew[row] : 0.0};
+    };
+    AheadSweep<U, 1, decltype(load)> rows(d.n, load);
+    rows.ahead();
     const double rho = sum_partials<RED_SUM>(d.P(P_RS), d.G);  // :107
     const double a1 = PAIR ? alpha_slot(d, k - 1) : 0.0, a2 = PAIR ? alpha_slot(d, k - 2) : 0.0;
     const double tol2 = d.sc[S_TOL2];
+    if (st != ST_RUN && st != conv_stamp(k)) return;
     if (tol2 >= 0.0) {
         const double rr = sum_partials<RED_SUM>(d.P(P_RR), d.G);
         if (rr <= tol2) {  // every workgroup reaches the same decision
@@ -779,30 +791,37 @@ __global__ __launch_bounds__(kBlock) void k_iter_dir(PcgDev d, const double *__r
     }
     const double beta = rho / rho_slot(d, k - 1);  // :109
     if (leader()) d.sc[S_RHO0 + (k & 1)] = rho;
-    FOR_ROWS(d.n, row) {
-        const double sr = s[row], po = pold[row];
-        const double xo = PAIR ? x[row] : 0.0, pp = PAIR ? pnew[row] : 0.0;
-        const double si = LEAN ? s_of(d, row, sr) : sr;
-        if (PAIR) x[row] = x_two(xo, a2, pp, a1, po);
-        pnew[row] = 1.0 * si + beta * po;  // :113
-    }
+    rows.each([&](int row, const In &v) {
+        const double si = LEAN ? s_of(v.s, v.di, d.precond != 0) : v.s;
+        if (PAIR) x[row] = x_two(v.x, a2, v.pp, a1, v.po);
+        pnew[row] = 1.0 * si + beta * v.po;  // :113
+    });
 }
 
 // K2: alpha_k from the folded p.Ap partials, r += (-alpha) Ap, s = Dinv r,
 // partials of r.s and r.r (one per workgroup); each row's operands are
 // loaded together (one round trip per row)
-template <bool LEAN>
+template <bool LEAN, int U>
 __global__ __launch_bounds__(kBlock) void k_iter_update_grid(PcgDev d, int k) {
-    if (!running(d)) return;
+    const int st = state_load(d.state);
     double *__restrict__ r = d.r, *__restrict__ s = d.s;
     const double *__restrict__ Ap = d.Ap, *__restrict__ dinv = d.dinv;
     const bool precond = d.precond != 0;
+    struct In {
+        double r, ap, di;
+    };
+    const auto load = [&](int row) {
+        return In{r[row], Ap[row], LEAN ? dict_dinv(d, row, 0.0) : precond ? dinv[row] : 0.0};
+    };
+    AheadSweep<U, kSweepU<LEAN>, decltype(load)> rows(d.n, load);
+    rows.ahead();
     double dsum[1];
     if (d.Gdn <= kBlock)  // one round of the uniform loop
         sum_partials_n<1>({d.P(P_DN)}, d.Gdn, dsum);
     else
         dsum[0] = sum_partials<RED_SUM>(d.P(P_DN), d.Gdn);
     const double dn = dsum[0];
+    if (st != ST_RUN) return;
     const double alpha = rho_slot(d, k) / dn;  // :93
     if (dn == 0.0 || !isfinite(dn) || !isfinite(alpha)) {
         if (leader()) state_store(d.state, ST_BREAK);
@@ -811,28 +830,14 @@ __global__ __launch_bounds__(kBlock) void k_iter_update_grid(PcgDev d, int k) {
     store_alpha(d, k, alpha);
     const double malpha = -1.0 * alpha;
     double rs = 0.0, rr = 0.0;
-    struct In {
-        double r, ap, di;
-    };
-    sweep_rows<kSweepU<LEAN>>(
-        d.n,
-        [&](int row) {
-            return In{r[row], Ap[row], !precond ? 0.0 : LEAN ? dict_one(d.dc_sel, d.dc_id, d.ddinv, row) : dinv[row]};
-        },
-        [&](int row, const In &v) {
-            const double ri = v.r + malpha * v.ap;  // :97
-            r[row] = ri;
-            double si;
-            if (precond) {  // :99-105
-                si = 0.0;
-                si = si + ri * v.di;
-            } else {
-                si = ri;
-            }
-            if (!LEAN) s[row] = si;
-            rs = rs + ri * si;
-            rr = rr + ri * ri;
-        });
+    rows.each([&](int row, const In &v) {
+        const double ri = v.r + malpha * v.ap;  // :97
+        r[row] = ri;
+        const double si = s_of(ri, v.di, precond);
+        if (!LEAN) s[row] = si;
+        rs = rs + ri * si;
+        rr = rr + ri * ri;
+    });
     double red[2] = {rs, rr};
     block_reduce_n<2>(red);
     if (threadIdx.x == 0) {
@@ -874,7 +879,7 @@ __global__ __launch_bounds__(kBlock) void k_iter_dir_rows(PcgDev d, const double
     // stream of this mix runs 8% faster with them on this device)
     const double sr = ntload((LEAN ? d.r : d.s) + row), po = ntload(pold + row);
     const double xo = PAIR ? ntload(d.x + row) : 0.0, pp = PAIR ? ntload(pnew + row) : 0.0;
-    const double si = LEAN ? s_of(d, row, sr) : sr;
+    const double si = LEAN ? s_of(sr, dict_dinv(d, row, 0.0), d.precond != 0) : sr;
     if (PAIR) ntstore(d.x + row, x_two(xo, a2, pp, a1, po));
     ntstore(pnew + row, 1.0 * si + beta * po);  // :113
 }
@@ -1028,31 +1033,39 @@ __global__ __launch_bounds__(kBlock) void k_fin(PcgDev d, Pub pub) {
 // +inf), p32 = s32 + beta p32 into pnew; PAIR: the correction updates
 // xc += alpha p of iterations k-2 and k-1 (not yet folded by a defect
 // correction), two at a time as in k_iter_dir
-template <bool LEAN, bool PAIR>
+template <bool LEAN, bool PAIR, int U>
 __global__ __launch_bounds__(kBlock) void k_m_dir(PcgDev d, const float *__restrict__ pold, float *__restrict__ pnew,
                                                  int k) {
     float *__restrict__ xc = d.xc32;
     const float *__restrict__ s = LEAN ? d.r32 : d.s32;
-    if (!running(d)) return;
-    const double rho = sum_partials<RED_SUM>(d.P(P_RS), d.G);
-    const float a1 = PAIR ? (float)alpha_slot(d, k - 1) : 0.0f;  // as K2 formed them
-    const float a2 = PAIR ? (float)alpha_slot(d, k - 2) : 0.0f;
-    const float beta = (float)(rho / rho_slot(d, k - 1));
-    if (leader()) d.sc[S_RHO0 + (k & 1)] = rho;
+    const int st = state_load(d.state);
+    struct In {
+        float s, di, po, x, pp;
+    };
     // nontemporal accesses: each array is streamed once per sweep (mixed
     // solve at 256^3 over four runs: 392-394 ms with them, 403-405 without;
     // the sweeps' own times are unchanged within noise)
-    FOR_ROWS(d.n, row) {
-        const float sr = __builtin_nontemporal_load(s + row), po = __builtin_nontemporal_load(pold + row);
-        const float xo = PAIR ? __builtin_nontemporal_load(xc + row) : 0.0f,
-                    pp = PAIR ? __builtin_nontemporal_load(pnew + row) : 0.0f;
-        const float si = LEAN ? s_of(d, row, sr) : sr;
+    const auto load = [&](int row) {
+        return In{__builtin_nontemporal_load(s + row), LEAN ? dict_dinv(d, row, 0.0f) : 0.0f,
+                  __builtin_nontemporal_load(pold + row), PAIR ? __builtin_nontemporal_load(xc + row) : 0.0f,
+                  PAIR ? __builtin_nontemporal_load(pnew + row) : 0.0f};
+    };
+    AheadSweep<U, 1, decltype(load)> rows(d.n, load);
+    rows.ahead();
+    const double rho = sum_partials<RED_SUM>(d.P(P_RS), d.G);
+    const float a1 = PAIR ? (float)alpha_slot(d, k - 1) : 0.0f;  // as K2 formed them
+    const float a2 = PAIR ? (float)alpha_slot(d, k - 2) : 0.0f;
+    if (st != ST_RUN) return;
+    const float beta = (float)(rho / rho_slot(d, k - 1));
+    if (leader()) d.sc[S_RHO0 + (k & 1)] = rho;
+    rows.each([&](int row, const In &v) {
+        const float si = LEAN ? s_of(v.s, v.di, d.precond != 0) : v.s;
         if (PAIR) {
-            const float t = xo + a2 * pp;
-            __builtin_nontemporal_store(t + a1 * po, xc + row);
+            const float t = v.x + a2 * v.pp;
+            __builtin_nontemporal_store(t + a1 * v.po, xc + row);
         }
-        __builtin_nontemporal_store(si + beta * po, pnew + row);
-    }
+        __builtin_nontemporal_store(si + beta * v.po, pnew + row);
+    });
 }
 
 // Small operators, k >= 1: k_m_dir and the FP32 product in one kernel (as
@@ -1176,13 +1189,24 @@ __global__ __launch_bounds__(kBlock) void k_m_spmv_dict(EllView A, PcgDev d, con
     chunk_store<R, 2>(d, sh);
 }
 
-template <bool LEAN>
+template <bool LEAN, int U>
 __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
     float *__restrict__ r = d.r32, *__restrict__ s = d.s32;
     const float *__restrict__ Ap = d.Ap32, *__restrict__ dinv = d.dinv32;
     const bool precond = d.precond != 0;
     double rs = 0.0, rr = 0.0;
-    if (!running(d)) return;
+    const int st = state_load(d.state);
+    struct In {
+        float r, ap, di;
+    };
+    const auto load = [&](int row) {
+        return In{__builtin_nontemporal_load(r + row), __builtin_nontemporal_load(Ap + row),
+                  LEAN      ? dict_dinv(d, row, 0.0f)
+                  : precond ? __builtin_nontemporal_load(dinv + row)
+                            : 0.0f};
+    };
+    AheadSweep<U, kSweepU<LEAN>, decltype(load)> rows(d.n, load);
+    rows.ahead();
     // every prologue load issued before the first is used: 1.A1, the
     // list of A 1's nonzeros, and the p.Ap and 1.Ap partials (summed
     // together; alpha goes to its scalar slot, so later kernels need
@@ -1201,6 +1225,7 @@ __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
         sum_partials_n<2>({d.P(P_DN), d.P(P_SA)}, d.Gdn, sums);
     else  // all slots in one round trip
         sum_padded<2>({d.P(P_DN), d.P(P_SA)}, {d.Gdn, d.Gdn}, sums);
+    if (st != ST_RUN) return;
     const bool dfl = deflating(d, zaz);
     const double sap = dfl ? sums[1] : 0.0;
     const double dn = m_denom(sums[0], sap, zaz, dfl);
@@ -1218,17 +1243,7 @@ __global__ __launch_bounds__(kBlock) void k_m_update(PcgDev d, int k) {
     const bool listed = naz <= kAzList;
 #pragma unroll
     for (int j = 0; j < kAzList; ++j) li[j] = j < naz ? li[j] : -1;
-    struct In {
-        float r, ap, di;
-    };
-    sweep_rows<kSweepU<LEAN>>(
-        d.n,
-        [&](int row) {
-            return In{__builtin_nontemporal_load(r + row), __builtin_nontemporal_load(Ap + row),
-                      !precond ? 0.0f
-                      : LEAN   ? dict_one(d.dc_sel, d.dc_id, d.ddinv32, row)
-                               : __builtin_nontemporal_load(dinv + row)};
-        },
+    rows.each(
         [&](int row, const In &v) {
             float azr = 0.0f;
             if (dfl && !listed) {
@@ -1548,8 +1563,23 @@ struct gip_pcg {
 
 // Multiple of 8 (one share per XCD), at most kMaxRedBlocks (one partial each).
 // The product kernels run one workgroup per 256-row chunk instead.
+// Rows a thread of a mid-size sweep has, all requested before the prologue
+// (AheadSweep); 0, one (small operators) or as many as come.  512 to 1024
+// workgroups, two to four per CU, each with all its rows in flight, need a
+// quarter of the prologues that 2048 workgroups of one or two rows repeat
+// and leave no half-empty round.  us per iteration with 2048 workgroups, 4,
+// 6 and 8 rows ahead: mixed 81^3 24.5 / 19.5 / 20.3 / 20.5, 97^3 28.4 / 24.1
+// / 24.1 / 23.9, 112^3 35.5 / 34.5 / 31.4 / 30.9, 128^3 39.4 / - / - / 34.5;
+// FP64 81^3 26.8 / 24.5 / 25.5 / 27.1, 97^3 31.9 / 30.0 / 31.0 / 32.3, 112^3
+// 39.4 / 39.0 / 37.4 / 38.2, 128^3 42.6 / - / - / 40.9; clustered 81^3 27.7 /
+// 25.4 / 25.1 / 26.1, 128^3 54.9 / - / - / 52.5.  Past 2^21 rows it no longer
+// pays (160^3 mixed 68.5 / 70.4, FP64 80.8 / 83.1).
+static int ahead_rows(int n) {
+    const int nchunk = (n + kBlock - 1) / kBlock;
+    return nchunk <= kMaxRedBlocks ? 0 : nchunk <= 4096 ? 4 : nchunk <= 8192 ? 8 : 0;
+}
 static int pcg_grid(int n) {
-    int nchunk = (n + kBlock - 1) / kBlock;
+    const int u = ahead_rows(n), nchunk = ((n + kBlock - 1) / kBlock + (u ? u - 1 : 0)) / (u ? u : 1);
     int g = ((nchunk + 7) / 8) * 8;
     if (g > kMaxRedBlocks) g = kMaxRedBlocks;
     if (g < 8) g = 8;
@@ -1883,8 +1913,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     // direction of iteration k: two buffers by parity
     auto pdir = [&](int k) { return (k & 1) ? S->p2 : S->p; };
     auto pdir32 = [&](int k) { return (k & 1) ? S->p32b : S->p32; };
-    // the instance of a long direction sweep: LEAN, and whether it makes the
-    // pending x updates
+    // the instance of a long sweep: LEAN, whether a direction sweep makes the
+    // pending x updates, and (not the row-per-thread ones) the rows a thread
+    // requests ahead
 #define DIR_LAUNCH(KERNEL, GRID, PAIR, ...)                        \
     do {                                                           \
         if (lean && (PAIR))                                        \
@@ -1896,6 +1927,43 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
         else                                                       \
             KERNEL<false, false><<<GRID, kBlock, 0, st>>>(__VA_ARGS__); \
     } while (0)
+#define AHEAD_DIR(KERNEL, U, PAIR, ...)                                      \
+    do {                                                                     \
+        if (lean && (PAIR))                                                  \
+            KERNEL<true, true, U><<<S->grid, kBlock, 0, st>>>(__VA_ARGS__);  \
+        else if (lean)                                                       \
+            KERNEL<true, false, U><<<S->grid, kBlock, 0, st>>>(__VA_ARGS__); \
+        else if (PAIR)                                                       \
+            KERNEL<false, true, U><<<S->grid, kBlock, 0, st>>>(__VA_ARGS__); \
+        else                                                                 \
+            KERNEL<false, false, U><<<S->grid, kBlock, 0, st>>>(__VA_ARGS__);\
+    } while (0)
+#define SWEEP_DIR(KERNEL, PAIR, ...)                   \
+    do {                                               \
+        if (ahead == 4)                                \
+            AHEAD_DIR(KERNEL, 4, PAIR, __VA_ARGS__);   \
+        else if (ahead == 8)                           \
+            AHEAD_DIR(KERNEL, 8, PAIR, __VA_ARGS__);   \
+        else                                           \
+            AHEAD_DIR(KERNEL, 0, PAIR, __VA_ARGS__);   \
+    } while (0)
+#define AHEAD_UPDATE(KERNEL, U)                                     \
+    do {                                                            \
+        if (lean)                                                   \
+            KERNEL<true, U><<<S->grid, kBlock, 0, st>>>(d, k);      \
+        else                                                        \
+            KERNEL<false, U><<<S->grid, kBlock, 0, st>>>(d, k);     \
+    } while (0)
+#define SWEEP_UPDATE(KERNEL)            \
+    do {                                \
+        if (ahead == 4)                 \
+            AHEAD_UPDATE(KERNEL, 4);    \
+        else if (ahead == 8)            \
+            AHEAD_UPDATE(KERNEL, 8);    \
+        else                            \
+            AHEAD_UPDATE(KERNEL, 0);    \
+    } while (0)
+    const int ahead = ahead_rows(S->n);
     // time_products: events around one product launch (k >= 1) per host
     // poll, read after the poll's synchronisation
     const bool timing = o->time_products != 0;
@@ -1944,7 +2012,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             int chunk = std::min(fixed ? 4096 : pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold && !S->rows) {
-                    if (k > 0) DIR_LAUNCH(k_iter_dir, S->grid, k >= 2 && !(k & 1), d, pdir(k - 1), pdir(k), k);
+                    if (k > 0) SWEEP_DIR(k_iter_dir, k >= 2 && !(k & 1), d, pdir(k - 1), pdir(k), k);
                     const bool smp = sample_begin(k);
                     if (dict)
                         DICT_LAUNCH(k_iter_spmv_dict, A->st_w, S->nchunk, st, v, d, pdir(k));
@@ -1954,7 +2022,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                         ROW_PRODUCT(k_iter_spmv, pdir(k));
                     sample_end(smp);
                     fold();
-                    LEAN_LAUNCH(k_iter_update_grid, S->grid, d, k);
+                    SWEEP_UPDATE(k_iter_update_grid);
                 } else if (S->fold) {
                     // (partials: p.Ap in chunk, then r.s in chunk and r.r in chunk_s)
                     if (k > 0) DIR_LAUNCH(k_iter_dir_rows, S->nchunk, k >= 2 && !(k & 1), d, pdir(k - 1), pdir(k), k);
@@ -2030,7 +2098,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
             int chunk = std::min(pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold) {
-                    if (k > 0) DIR_LAUNCH(k_m_dir, S->grid, pending == 2, d, pdir32(k - 1), pdir32(k), k);
+                    if (k > 0) SWEEP_DIR(k_m_dir, pending == 2, d, pdir32(k - 1), pdir32(k), k);
                     pending = pending == 2 ? 1 : pending + 1;
                     const bool smp = sample_begin(k);
                     if (dict)
@@ -2039,7 +2107,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                         ROW_PRODUCT(k_m_spmv, pdir32(k));
                     sample_end(smp);
                     fold();
-                    LEAN_LAUNCH(k_m_update, S->grid, d, k);
+                    SWEEP_UPDATE(k_m_update);
                 } else {
                     const bool smp = sample_begin(k);
                     if (k == 0)

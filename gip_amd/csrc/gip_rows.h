@@ -783,6 +783,35 @@ __device__ inline void sweep_rows(int n, const LOAD &load, const USE &use) {
     }
 }
 
+// A sweep whose rows can be requested ahead: U > 0, at most U rows per
+// thread, all of them by ahead(), which a kernel calls before its prologue,
+// and each() takes them; U = 0, each() sweeps with V rows in flight.  load
+// and use as for sweep_rows.
+template <int U, int V, class LOAD>
+struct AheadSweep {
+    const LOAD &load;
+    int n;
+    RowSweep rs;
+    decltype(load(0)) v[U > 0 ? U : 1];
+    __device__ AheadSweep(int n_, const LOAD &l) : load(l), n(n_), rs(n_) {}
+    __device__ int row(int u) const { return (rs.c + u * rs.step) * kBlock + (int)threadIdx.x; }
+    __device__ bool own(int u) const { return rs.c + u * rs.step < rs.c1 && row(u) < n; }
+    __device__ inline void ahead() {
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = load(own(u) ? row(u) : n - 1);
+    }
+    template <class USE>
+    __device__ inline void each(const USE &use) const {
+        if constexpr (U == 0) {
+            sweep_rows<V>(n, load, use);
+            return;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (own(u)) use(row(u), v[u]);
+    }
+};
+
 // The rows FOR_ROWS gives this thread, as a cursor, so that a kernel can
 // request its first row's operands before its prologue and each next row's
 // right after storing the current one.  Only the last chunk of the matrix

@@ -102,3 +102,33 @@ def test_breakdown_keeps_the_updates_made(dev):
     print(f"[breakdown] iters {r.iters} status {r.status}", flush=True)
     assert np.all(np.isfinite(x))
     assert np.linalg.norm(b - T @ x) <= 1e-9 * np.linalg.norm(b)
+
+
+# Mid-size operators: products in workgroups of 512 (up to 2^20 rows) or 1024
+# rows, sweeps of four (up to 2^20) or eight rows per thread, and the forms on
+# both sides of 2^21 rows; partial last workgroups.  A clustered mesh (no
+# dictionary) in each layout, a uniform one with it; layouts agree bit for bit.
+@pytest.mark.parametrize("beta", [0.0, 1.5])
+@pytest.mark.parametrize("shape", [(128, 128, 64), (128, 128, 65), (128, 128, 128), (129, 128, 128)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_mid_size_forms(dev, shape, beta):
+    c = cavity.generate(*shape, gamma=1e-3, ops=cavity.OP_BITS["L"], beta=beta)
+    L, n, nall = c.op("L"), c.n_inner, c.n_all
+    b = np.zeros(nall)
+    b[:n] = cavity.rhs_normal(n, 4)
+    x0 = np.zeros(nall)
+    db, dx0, dx, orc = dev.to_device(b), dev.to_device(x0), dev.array(nall), pyoracle.Csr.of(L)
+    want = {maxit: pyoracle.pcg(orc, b, x0, n, maxit)[0] for maxit in (1, 2, 5)}
+    first = {}
+    for fmt in (hip.FMT_AUTO, hip.FMT_ELL, hip.FMT_CSR):
+        A = hip.Matrix(dev, L.rowptr, L.col, L.val, nrows=n, ncols=nall, fmt=fmt, fp32=True)
+        solver = hip.PCG(A, nall)
+        for maxit in (1, 2, 5):
+            for precision in (hip.PCG_FP64, hip.PCG_MIXED):
+                r = solver.solve(db, dx, dx0, maxit=maxit, precision=precision)
+                x = dx.download()
+                assert r.iters == maxit
+                if precision == hip.PCG_FP64:
+                    assert np.linalg.norm(x - want[maxit]) <= 1e-12 * np.linalg.norm(want[maxit]), (fmt, maxit)
+                assert np.array_equal(first.setdefault((maxit, precision), x), x), (fmt, maxit, precision)
+        del solver, A
