@@ -127,6 +127,7 @@ struct gip_mat {
     // row's slot values and diagonal, dict_n of them (0: none), current while
     // dict_version == val_version + 1
     int32_t dict_n;
+    bool dict_off;  // a captured graph may change the values unseen: not used any more
     uint64_t dict_version;
     gip::DictRec *d_dict_rec;  // per slice: which tuples its rows hold
     gip::DictSel *d_dict_sel;
@@ -170,7 +171,22 @@ int mat_sym_prepare(gip_ctx *c, gip_mat *A, bool *ok);
 // values where it pays (dict_n stays 0 otherwise), and frees it.
 int mat_dict_build(gip_ctx *c, gip_mat *A);
 void mat_dict_free(gip_mat *A);
-inline bool mat_dict_ok(const gip_mat *A) { return A->dict_n > 0 && A->dict_version == A->val_version + 1; }
+inline bool mat_dict_ok(const gip_mat *A) {
+    return A->dict_n > 0 && !A->dict_off && A->dict_version == A->val_version + 1;
+}
+inline bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+}
+// ... for a product that is launched now.  A captured one reads the stored
+// values: its replays take those of their own time, and the dictionary of
+// today is freed when the values change.
+inline bool mat_dict_now(const gip_mat *A, hipStream_t st) { return mat_dict_ok(A) && !capturing(st); }
+// values that the device writes (gip_dcsrmv_vals)
+inline void mat_values_change(gip_mat *A, hipStream_t st) {
+    ++A->val_version;
+    if (!A->dict_off && capturing(st)) A->dict_off = true;
+}
 // Looks up the no-alloc PCG scratch array's address on `device` (current);
 // called once per device by gip_init.
 int pcg_scratch_setup(int device);

@@ -358,7 +358,7 @@ int spmv_launch(gip_ctx *c, const gip_mat *A, const double *x, double *y, double
 #undef GIP_ELL_CASE
     } else if (A->format == GIP_FMT_STENCIL) {
         const EllView v = view(A);
-        const bool dict = mat_dict_ok(A), two = dict_two(A->nrows);
+        const bool dict = mat_dict_now(A, st), two = dict_two(A->nrows);
 #define GIP_ST_CASE(Wc)                                                                   \
     case Wc:                                                                              \
         if (dict && mode == 0 && two)                                                     \
@@ -428,7 +428,7 @@ int spmv32_launch(gip_ctx *c, const gip_mat *A, const float *x, float *y) {
         if (!A->d_ell_val32) return set_error(GIP_EINVAL, "operator has no FP32 values");
         const EllView v = view(A);
         const int g = nblocks(A->nrows);
-        if (mat_dict_ok(A) && A->st_w >= 7) {
+        if (A->st_w >= 7 && mat_dict_now(A, c->stream)) {
             DICT_LAUNCH(k_stencil32_dict, A->st_w, g, c->stream, v, A->nrows, x, y);
             GIP_LAUNCH_CHECK("spmv32 kernel");
             return GIP_OK;
@@ -923,7 +923,7 @@ int gip_dcsrmv_ab(gip_ctx *c, const gip_mat *A, const double *x, double *y, doub
 int gip_dcsrmv_vals(gip_ctx *c, const gip_mat *A, const double *x, gip_mat *B) {
     if (!c || !A || !B || (A->nrows && !x)) return set_error(GIP_EINVAL, "gip_dcsrmv_vals: bad argument");
     if (A->nrows != B->nnz) return set_error(GIP_EINVAL, "gip_dcsrmv_vals: rows of A must equal nnz of B");
-    ++B->val_version;
+    mat_values_change(B, c->stream);
     int rc;
     if (B->format == GIP_FMT_ELL || B->format == GIP_FMT_STENCIL)
         rc = spmv_launch(c, A, x, B->d_ell_val, 1.0, 0.0, 0, B->d_csr2ell);
@@ -945,7 +945,7 @@ int gip_dcsrmv_vals(gip_ctx *c, const gip_mat *A, const double *x, gip_mat *B) {
 int gip_dcsrmv_vals_ab(gip_ctx *c, const gip_mat *A, const double *x, gip_mat *B, double alpha, double beta) {
     if (!c || !A || !B || (A->nrows && !x)) return set_error(GIP_EINVAL, "gip_dcsrmv_vals_ab: bad argument");
     if (A->nrows != B->nnz) return set_error(GIP_EINVAL, "gip_dcsrmv_vals_ab: rows of A must equal nnz of B");
-    ++B->val_version;
+    mat_values_change(B, c->stream);
     int rc;
     if (B->format == GIP_FMT_ELL || B->format == GIP_FMT_STENCIL)
         rc = spmv_launch(c, A, x, B->d_ell_val, alpha, beta, 1, B->d_csr2ell);
@@ -1045,7 +1045,7 @@ int gip_dcsrmv_t(gip_ctx *c, const gip_mat *Ac, const double *x, double *y, int3
     if (A->nnz) {
         k_refresh<<<nblocks(A->nnz), kBlock, 0, c->stream>>>(A->nnz, value_store(A), A->d_tsrc, value_store(T), A->d_tdst);
         GIP_LAUNCH_CHECK("gip_dcsrmv_t refresh");
-        ++T->val_version;  // what was made from earlier values is stale
+        mat_values_change(T, c->stream);  // what was made from earlier values is stale
     }
     if (ncols_out) {
         k_fill0<<<nblocks(ncols_out), kBlock, 0, c->stream>>>(ncols_out, y);

@@ -106,3 +106,52 @@ def test_changed_values(dev, n):
         E.spmv_vals(mf, M)
     _products(dev, A, C, 6)
     assert np.array_equal(A.values(), C.values())
+
+
+def test_captured_products_follow_the_values(dev):
+    """A graph that holds a product or a change of values, replayed after the values changed otherwise."""
+    import torch
+
+    c = cavity.generate(64, gamma=1e-3, ops=cavity.OP_BITS["L"])  # 2^18 rows: a dictionary
+    L, n, nall = c.op("L"), c.n_inner, c.n_all
+    A = hip.Matrix.from_csr(dev, L, fp32=True)
+    C = hip.Matrix.from_csr(dev, L, fmt=hip.FMT_CSR)
+    nnz = L.val.size
+    ident = hip.Matrix(dev, np.arange(nnz + 1), np.arange(nnz), np.ones(nnz), ncols=nnz, fmt=hip.FMT_CSR)
+    rng = np.random.default_rng(0)
+    dx, sx = dev.to_device(rng.standard_normal(nall)), dev.to_device(rng.standard_normal(nall).astype(np.float32))
+    dv = dev.to_device(5.0 * L.val)
+    y, s, want, swant = dev.array(n), dev.array(n, np.float32), dev.array(n), dev.array(n, np.float32)
+    stream = torch.cuda.ExternalStream(hip.lib().gip_stream(dev.ctx))
+    product, change = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(product, stream=stream, capture_error_mode="thread_local"):
+        A.spmv(dx, y)
+        A.spmv32(sx, s)
+
+    def replayed():
+        with torch.cuda.stream(stream):
+            product.replay()
+        return y.download(), s.download()
+
+    def eager(M):
+        M.spmv(dx, want)
+        return want.download()
+
+    A.spmv32(sx, swant)
+    base, base32 = eager(C), swant.download()
+    for factor in (1.0, 2.0, 0.5, 4.0):
+        A.set_values(factor * L.val)
+        assert np.array_equal(eager(A), factor * base)
+        for _ in range(2):
+            got, got32 = replayed()
+            assert np.array_equal(got, factor * base) and np.array_equal(got32, np.float32(factor) * base32)
+    with torch.cuda.graph(change, stream=stream, capture_error_mode="thread_local"):
+        ident.spmv_vals(dv, A)
+    C.set_values(5.0 * L.val)
+    five = eager(C)
+    for _ in range(2):
+        A.set_values(L.val)
+        assert np.array_equal(eager(A), base)
+        with torch.cuda.stream(stream):
+            change.replay()
+        assert np.array_equal(eager(A), five) and np.array_equal(replayed()[0], five)
