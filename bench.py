@@ -330,11 +330,19 @@ def main():
     # input once, the output once): no column index per entry, so fewer
     # than the CSR count
     lay64, lay32 = A.product_bytes(), A.product_bytes(fp32=True)
-    # the FP64 solve multiplies a bitwise symmetric stencil operator through
-    # its symmetric form (the slots of offsets >= 0): its own bytes
-    sym_state, sym64 = A.sym_state()
-    own64 = sym64 if sym_state == 1 else lay64
-    for leg, byts, lay in ((fp64, it_fp64, own64 + 88 * N), (mixed, it_mixed, lay32 + 44 * N)):
+    # the long solves (more than 2^19 rows; mixed from 2^21) multiply this
+    # uniform mesh's operator from the dictionary of its value tuples: the
+    # input and output once, a 64-byte record per 64 rows, and a 2-byte id per
+    # row where slices straddle the mesh lines.  With it s = Dinv r is not
+    # stored (mixed: where no ids are read), and x is updated every second
+    # iteration: 7.5 vector streams beside the product instead of 11
+    dict64, dict32, ids = N > 1 << 19, N >= 1 << 21, n % 64 != 0
+    spmv64 = 16 * N + N + (2 * N if ids else 0) if N >= 1 << 18 else lay64
+    own64 = spmv64 if dict64 else lay64
+    spmv32 = 8 * N + N + (2 * N if ids else 0) if N >= 1 << 18 else lay32
+    own32 = spmv32 if dict32 else lay32
+    streams64, streams32 = (60 if dict64 else 88) * N, (30 if dict32 and not ids else 44) * N
+    for leg, byts, lay in ((fp64, it_fp64, own64 + streams64), (mixed, it_mixed, own32 + streams32)):
         ms_it = leg["ms"] / max(1, leg["iters"])
         leg["ms_per_iter"] = ms_it
         leg["iter_alg_bytes"] = byts  # CSR count of the product + the vector streams
@@ -374,19 +382,16 @@ def main():
 
     # The dominant kernel of the path: the FP64 product inside the FP64 PCG
     # (its median launch, timed by events inside the solves), achieved = the
-    # bytes the product's own layout moves per launch (over the symmetric
-    # form: the values of the slots of offsets >= 0, slot offsets and codes,
-    # tails, the input and output once).  The CSR count 12 nnz + 4 (rows+1)
+    # bytes the product's own form moves per launch (own64 above).  The CSR
+    # count 12 nnz + 4 (rows+1)
     # + 8 rows + 8 cols per launch beside it is only a CSR equivalent: the
     # layout moves fewer bytes, so that rate can exceed the peak.
     us64, us32 = fp64["product_us"], mixed["product_us"]
     # operators of at most 2^19 rows form the direction inside the product
     if info["nrows"] <= 1 << 19:
         k64, k32, form = "k_iter_dirprod", "k_m_dirprod", "stencil layout"
-    elif sym_state == 1:
-        k64, k32, form = "k_iter_spmv_sym", "k_m_spmv", "symmetric form of the stencil layout"
     else:
-        k64, k32, form = "k_iter_spmv<", "k_m_spmv", "stencil layout"
+        k64, k32, form = "k_iter_spmv_dict", "k_m_spmv_dict" if dict32 else "k_m_spmv<", "dictionary of the slot values"
     ceiling = stream_ceiling()
     ach64 = own64 / (us64 * 1e-6) / 1e9
     traffic64 = measured_traffic(n, k64)
@@ -399,14 +404,14 @@ def main():
         "kernel": f"{k64.rstrip('<')} (FP64 product of the FP64 PCG over the {form}, timed inside the solves), "
                   f"{n}^3"}
     # The dominant kernel of the timed mixed solve, its FP32 product: achieved
-    # = the layout's bytes (the FP32 CSR count includes column indices this
-    # layout never reads, and would put the rate above the peak).
-    ach32 = lay32 / (us32 * 1e-6) / 1e9
+    # = its own bytes (the FP32 CSR count includes column indices and values it
+    # never reads, and would put the rate above the peak).
+    ach32 = own32 / (us32 * 1e-6) / 1e9
     roofline_solve = {
         "bound": "hbm", "achieved": round(ach32, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": round(ach32 / HBM_PEAK_GBS, 4), "traffic": measured_traffic(n, k32),
-        "algorithmic_bytes": lay32, "us_per_launch": round(us32, 2), "csr_bytes": alg32,
-        "kernel": f"{k32} (FP32 stencil-layout product of the mixed PCG, timed inside the solves), {n}^3"}
+        "algorithmic_bytes": own32, "us_per_launch": round(us32, 2), "csr_bytes": alg32,
+        "kernel": f"{k32.rstrip('<')} (FP32 product of the mixed PCG, timed inside the solves), {n}^3"}
 
     out = {
         "metric": METRIC,
@@ -437,8 +442,8 @@ def main():
         # FP32: the layout's own bytes (its CSR count includes column indices
         # the layout never reads, so that rate is only a CSR equivalent)
         "spmv_fp64": {"ms": spmv_ms, "gbs": spmv_gbs, "algorithmic_bytes": alg,
-                      "layout_gbs": lay64 / (spmv_ms * 1e-3) / 1e9, "layout_bytes": lay64},
-        "spmv_fp32": {"ms": spmv32_ms, "gbs": lay32 / (spmv32_ms * 1e-3) / 1e9, "layout_bytes": lay32,
+                      "layout_gbs": spmv64 / (spmv_ms * 1e-3) / 1e9, "layout_bytes": spmv64},
+        "spmv_fp32": {"ms": spmv32_ms, "gbs": spmv32 / (spmv32_ms * 1e-3) / 1e9, "layout_bytes": spmv32,
                       "csr_equiv_gbs": alg32 / (spmv32_ms * 1e-3) / 1e9, "csr_bytes": alg32},
         "ns_steps": ns,
         "roofline": roofline,
@@ -489,7 +494,8 @@ def summarize_pmc(fetch_dir, write_dir, kernels):
 
 # kernel-name keys (substrings of the profiled names; "k_iter_dir(" is the
 # four-launch form's direction sweep, not k_iter_dir_rows)
-PCG_KERNELS = ("k_iter_dir_rows", "k_iter_dir(", "k_iter_spmv<", "k_iter_spmv_sym", "k_fold_two", "k_alpha_fin",
+PCG_KERNELS = ("k_iter_dir_rows", "k_iter_dir(", "k_iter_spmv<", "k_iter_spmv_dict", "k_iter_spmv_sym", "k_m_spmv_dict",
+               "k_stencil_dict", "k_fold_two", "k_alpha_fin",
                "k_iter_update_rows",
                "k_iter_update_grid", "k_beta_fin", "k_m_dir", "k_m_spmv", "k_fold_dn", "k_m_update", "k_stencil<0")
 

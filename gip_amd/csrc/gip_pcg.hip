@@ -2,9 +2,10 @@
 //
 // FP64 iteration k, the reference recurrences and roundings
 // (GIP_LinearSolver.h:85-116):
-//   direction  x += alpha_{k-1} p (the previous iteration's update, :95,
-//              moved here so that p is read once per iteration);
-//              beta = rho_k / rho_{k-1}; p = 1.0 s + beta p   (:107-113)
+//   direction  beta = rho_k / rho_{k-1}; p = 1.0 s + beta p   (:107-113);
+//              here too the x updates due (:95), since p is read anyway:
+//              the previous iteration's, or on long operators every second
+//              time the two before
 //   product    Ap = A p, partials of p.Ap                     (:87-91)
 //   update     alpha = rho_k / p.Ap; r += (-alpha) Ap; s = Dinv r;
 //              partials of r.s and r.r                        (:93-105)
@@ -13,9 +14,10 @@
 // every workgroup of a kernel re-reduces the previous kernel's partials in
 // its prologue (fence-free: plain stores, ordered by the kernel boundary;
 // every workgroup computes bit-identical scalars), so a kernel costs about
-// one memory round trip before it stores.  Up to kRowsMin rows, four
-// kernels: grid-stride sweeps whose prologues re-reduce the partials, the
-// product's partials folded first.  Longer operators sweep one row per
+// one memory round trip before it stores.  Up to kRowsMin rows, three or
+// four kernels: grid-stride sweeps whose prologues re-reduce the partials,
+// the product's folded first where they are more than 2048 or come from the
+// dictionary.  Longer operators sweep one row per
 // thread in dispatch order (the pace of a plain stream of each kernel's
 // access mix) and take their scalars from one-workgroup kernels (fold +
 // finalize) instead, since that many workgroups cannot each re-reduce the
@@ -28,7 +30,7 @@
 // and then.
 //
 // MIXED: the same iteration in FP32 (operator values, vectors and SpMV;
-// dot products accumulate in FP64; on long operators three kernels whose
+// dot products accumulate in FP64; on long operators three or four kernels whose
 // grid-stride sweeps re-reduce the partials in their prologues: the
 // row-per-thread form measured 18% slower per FP32 iteration at 256^3)
 // on the correction equation, inside an
@@ -855,13 +857,13 @@ __global__ __launch_bounds__(kBlock) void k_iter_update_grid(PcgDev d, int k) {
 // at the pace of a plain stream of their access mix.  So many workgroups
 // cannot each re-reduce the previous kernel's partials, so the scalars come
 // from one-workgroup kernels instead:
-//   K0  x += alpha_{k-1} p, p = 1.0 s + beta p        (beta, alpha from slots)
+//   K0  p = 1.0 s + beta p, x by two directions in turn (beta, alphas from slots)
 //   K1  Ap = A p, per-wavefront p.Ap partials          (iter_spmv)
 //   fold + F1: alpha = rho_k / (p.Ap)                  (breakdown test)
 //   K2  r += (-alpha) Ap, s = Dinv r, per-wavefront r.s and r.r partials
 //   fold + F2: rho_{k+1}, r.r, the convergence test, beta
-// F2 stamps a convergence with the next iteration's index; that
-// iteration's K0 (or the final flush) then applies the last x update.
+// F2 stamps a convergence with the next iteration's index; the final flush
+// then applies the x updates still due.
 
 __device__ inline double ntload(const double *p) { return __builtin_nontemporal_load(p); }
 __device__ inline void ntstore(double *p, double v) { __builtin_nontemporal_store(v, p); }

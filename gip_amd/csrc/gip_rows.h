@@ -812,19 +812,14 @@ struct AheadSweep {
     }
 };
 
-// The rows FOR_ROWS gives this thread, as a cursor, so that a kernel can
-// request its first row's operands before its prologue and each next row's
-// right after storing the current one.  Only the last chunk of the matrix
-// holds rows >= n, so the first such row ends the sweep.
+// The one row of a thread, over at least as many workgroups as there are
+// chunks, in RowSweep's order, so that a kernel can request its operands
+// before its prologue.
 struct ThreadRows {
     RowSweep rs;
     int row, n;
     __device__ explicit ThreadRows(int n_) : rs(n_), n(n_) { row = rs.c * kBlock + (int)threadIdx.x; }
     __device__ bool valid() const { return rs.c < rs.c1 && row < n; }
-    __device__ void next() {
-        rs.c += rs.step;
-        row = rs.c * kBlock + (int)threadIdx.x;
-    }
 };
 
 }  // namespace gip

@@ -251,7 +251,7 @@ typedef struct gip_pcg_opts {
                           (A p replaced by A p - A1 (1.Ap)/(1.A1)):
                           0 on (default), -1 off                                  */
     int32_t time_products; /* 1: time one product launch per host poll with events on
-                              the solver's stream (read at the poll's synchronisation);
+                              the solver's stream (read after the host's poll);
                               the median is returned in gip_pcg_stats.product_ms      */
 } gip_pcg_opts;
 typedef struct gip_pcg_stats {
