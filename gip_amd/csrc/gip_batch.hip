@@ -206,8 +206,8 @@ __device__ inline void seg_store_c(double (&v)[K], int c, double *part) {
 // before the first is used.  Their prologue sums the instance's partials of
 // the kernel before (InstSums), so every workgroup of an instance forms the
 // same alpha, or the same beta, and the kernels that did so alone, one
-// workgroup per instance, are left to instances of more than kDirectChunks
-// chunks and to the end of a group of iterations.  12 cavities of sides 32
+// workgroup per instance, are left to batches that are too large for that
+// (make_units) and to the end of a group of iterations.  12 cavities of sides 32
 // to 72: 36.5 us in three kernels per iteration against 43.5 in five, and the
 // gaps between them; the step 41.0 -> 35.9 ms.
 constexpr int kDirectChunks = 2048;
@@ -282,7 +282,7 @@ struct BPcg {
     double *part_u;  // r.s and r.r of each unit, past the product's chunk totals
     const BUnit *unit;
     const int32_t *u0, *nu;  // instance -> first unit, units
-    int direct;  // no instance has more than kDirectChunks chunks
+    int direct;  // the sweeps form the scalars themselves
     int maxit;
     double inner2;
 };
@@ -921,10 +921,15 @@ int make_units(gip_batch *b, const std::vector<int64_t> &off, const std::vector<
     b->unit_chunks = nch >= 4096 ? 4 : nch >= 2048 ? 2 : 1;
     std::vector<BUnit> un;
     std::vector<int32_t> u0, nu;
+    // every unit reads its instance's partials: up to 64 MB of them per sweep
+    // (24 mixed cavities of sides 40 to 80, 53 MB: 41.2 ms of PCG per step
+    // against 42.0 with the one-workgroup kernels; 12 of 32 to 72: 16.2 / 17.7)
     b->direct = true;
+    int64_t reads = 0;
     for (int i = 0; i < b->B; ++i) {
         const int64_t c0 = off[(size_t)i] / kChunk, nc = roundup(cnt[(size_t)i], kChunk) / kChunk;
-        if (nc > kDirectChunks) b->direct = false;
+        reads += nc * ((nc + b->unit_chunks - 1) / b->unit_chunks) * 8;
+        if (nc > kDirectChunks || reads > (int64_t)64 << 20) b->direct = false;
         u0.push_back((int32_t)un.size());
         for (int64_t k = 0; k < nc; k += b->unit_chunks)
             un.push_back(BUnit{i, (int32_t)(c0 + k), (int32_t)std::min<int64_t>(b->unit_chunks, nc - k), k == 0,
