@@ -509,7 +509,7 @@ def summary_traffic(args):
     lines = [
         f"# HBM traffic per launch of the {n}^3 PCG kernels (rocprofv3 PMC: TCC FETCH_SIZE and WRITE_SIZE in KiB per",
         "# dispatch, median over the dispatches of `bench.py --probe spmv`: 5 standalone FP64 products, 8",
-        "# iterations of the FP64 PCG, 8 of the mixed PCG, 8 of the FP64 PCG without the symmetric form, 5 copies",
+        "# iterations of the FP64 PCG, 8 of the mixed PCG, 5 copies",
         "# of 2^27 doubles)",
         "#",
         "# commands (run from the repository root on one MI355X):",
@@ -652,8 +652,7 @@ def probe_stream(args):
 
 def probe_spmv(args):
     """Five FP64 SpMVs on the n^3 Laplacian, eight iterations of the FP64 and
-    of the mixed PCG on it (their in-solve products), eight of the FP64 PCG
-    without the symmetric form, and five copies of 2^27
+    of the mixed PCG on it (their in-solve products), and five copies of 2^27
     doubles (1 GiB read + 1 GiB written each): the launches a rocprofv3 --pmc
     run counts, the copy calibrating FETCH_SIZE/WRITE_SIZE against known
     bytes."""
@@ -667,9 +666,8 @@ def probe_spmv(args):
     y = dev.array(cav.n_all)
     for _ in range(5):
         A.spmv(x, y)
-    # 8 iterations of each PCG (their products: k_iter_spmv_sym over the
-    # symmetric form, k_m_spmv), and 8 of the FP64 PCG on the operator
-    # built without the symmetric form (k_iter_spmv)
+    # 8 iterations of each PCG (their products: k_iter_spmv_dict and
+    # k_m_spmv_dict)
     A32 = hip.Matrix.from_csr(dev, L, fp32=True)
     solver = hip.PCG(A32, cav.n_all)
     b = dev.to_device(np.concatenate([cavity.rhs_normal(cav.n_inner, 1), np.zeros(cav.n_all - cav.n_inner)]))
@@ -678,11 +676,6 @@ def probe_spmv(args):
         solver.solve(b, y, z, maxit=8, tol=1e-10, precision=prec, poll=32)
     solver.destroy()
     A32.destroy()
-    F = hip.Matrix.from_csr(dev, L, sym=False)
-    solver = hip.PCG(F, cav.n_all)
-    solver.solve(b, y, z, maxit=8, tol=1e-10, poll=32)
-    solver.destroy()
-    F.destroy()
     nc = 1 << 27
     a, b = dev.array(nc), dev.array(nc)
     hip.fill(a, 1.0)

@@ -745,8 +745,9 @@ __global__ __launch_bounds__(kBlock) void k_iter_update(PcgDev d, int k) {
 //
 // A sweep of 2048 (or fewer) workgroups striding over the rows in
 // XCD-contiguous order, whose prologue re-reduces the previous kernel's
-// partials (every workgroup forms the same scalars): four launches per
-// iteration (direction, product, fold, update).  At these sizes the three
+// partials (every workgroup forms the same scalars): three or four launches
+// per iteration (direction, product, a fold where the product leaves more
+// partials than a prologue sums, update).  At these sizes the three
 // extra launches of the row-per-thread iteration cost more than its faster
 // sweeps save (FP64 solve to 1e-10, grid-stride against row-per-thread:
 // 128^3 94.9 against 107.0 ms, 160^3 205.8 / 227.7, 192^3 419.2 / 424.6;
