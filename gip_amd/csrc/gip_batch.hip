@@ -290,8 +290,10 @@ struct BPcg {
 __device__ inline double *bsc(const BPcg &d, int inst) { return d.sc + (size_t)inst * B_COUNT; }
 
 // Written by the first workgroup of an instance while its others may be
-// reading it: those compute the same decision, or skip work whose result
-// nothing reads.
+// reading it, each wavefront for itself: a sweep forms its sums, with their
+// barrier, before any wavefront acts on the word, so a wavefront that read
+// the old one still computes the same decision from whole sums (where the
+// instance leaves at its iteration limit, a direction that nothing reads).
 __device__ inline int b_state(const BPcg &d, int inst) {
     return __hip_atomic_load(d.state + inst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -421,10 +423,10 @@ __global__ __launch_bounds__(kBlock) void k_bp_dir(BPcg d, double *__restrict__ 
     const double *q = bsc(d, u.inst);
     double beta = q[B_BETA];
     const double r0 = q[rho_at(d, form ? k - 1 : 0)], tol2 = q[B_TOL2];
+    double rho[2];
+    if (form) ps.total(rho);
     if (st != BS_RUN) return;
     if (form) {
-        double rho[2];
-        ps.total(rho);
         if (u.first && threadIdx.x == 0) next_iter(d, u.inst, k, rho);
         if (rho[1] <= tol2) return;
         beta = rho[0] / r0;
@@ -467,21 +469,23 @@ __global__ __launch_bounds__(kBlock) void k_bp_spmv_fin(BPcg d, Seg S) {
     }
 }
 
-// alpha for a workgroup of an update, its loads requested at load()
+// alpha for a workgroup of an update, its loads requested at load(); sum()
+// is every wavefront's, form() that of those whose instance runs
 struct UnitAlpha {
     InstSums<1, kDirectChunks / kBlock> ps;
-    double rho, alpha;
+    double rho, alpha, dn[1];
     __device__ inline void load(const BPcg &d, const BUnit &u, int k) {
         const double *q = bsc(d, u.inst);
         rho = q[rho_at(d, k)];
         alpha = q[B_ALPHA];
         if (d.direct) ps.load(d.part, u.ic0, u.inc);
     }
+    __device__ inline void sum(const BPcg &d) {
+        if (d.direct) ps.total(dn);
+    }
     // false after a breakdown
     __device__ inline bool form(const BPcg &d, const BUnit &u) {
         if (!d.direct) return true;
-        double dn[1];
-        ps.total(dn);
         alpha = rho / dn[0];
         if (dn[0] != 0.0 && isfinite(dn[0]) && isfinite(alpha)) return true;
         if (u.first && threadIdx.x == 0) leave(d, u.inst, BS_BREAK);
@@ -505,6 +509,7 @@ __global__ __launch_bounds__(kBlock) void k_bp_update(BPcg d, const double *__re
     }
     UnitAlpha ua;
     ua.load(d, u, k);
+    ua.sum(d);
     if (st != BS_RUN || !ua.form(d, u)) return;
     const double alpha = ua.alpha;
     double v[2] = {0.0, 0.0};
@@ -627,10 +632,10 @@ __global__ __launch_bounds__(kBlock) void k_bpm_dir(BPcg d, float *__restrict__ 
     const double *q = bsc(d, u.inst);
     double beta = q[B_BETA];
     const double r0 = q[rho_at(d, form ? k - 1 : 0)];
+    double rho[2];
+    if (form) ps.total(rho);
     if (st != BS_RUN) return;
     if (form) {
-        double rho[2];
-        ps.total(rho);
         if (u.first && threadIdx.x == 0) next_iter_m(d, u.inst, k, rho);
         beta = rho[0] / r0;
     }
@@ -671,6 +676,7 @@ __global__ __launch_bounds__(kBlock) void k_bpm_update(BPcg d, const float *__re
     }
     UnitAlpha ua;
     ua.load(d, u, k);
+    ua.sum(d);
     if (st != BS_RUN || !ua.form(d, u)) return;
     const float a32 = (float)ua.alpha;
     double v[2] = {0.0, 0.0};

@@ -212,3 +212,34 @@ def test_instance_in_a_large_batch_is_the_instance_alone(dev, sizes, precision, 
         (iters, p), = run([sizes[k]], 7)
         assert got[k][0] == iters
         assert np.abs(got[k][1] - p).max() <= bound * np.abs(p).max(), sizes[k]
+
+
+# A breakdown is decided inside the update sweep, by every workgroup of the
+# instance from the same sums: the broken instance keeps the pressure it had
+# (its start, zero; in mixed precision after the coarse step, here below
+# 1e-20), in every chunk, and its neighbours advance as if it were whole.  Its
+# p.Ap overflows on a finite direction, 1e300 r (FP32: 1e20 r).
+@pytest.mark.parametrize("precision,diag,off", [(hip.PCG_FP64, 1e-300, 1e100), (hip.PCG_MIXED, 1e-20, 1e25)])
+@pytest.mark.parametrize("sizes", [[12, 20, 9], [20, 57, 9], [33, 72, 64, 64]])
+def test_a_breakdown_leaves_the_instance_and_its_neighbours_alone(dev, sizes, precision, diag, off):
+    def run(broken):
+        cavs = [cavity.generate(n, gamma=1e-2) for n in sizes]
+        if broken:
+            L = cavs[1].op("L")
+            row = np.repeat(np.arange(L.nrows), np.diff(L.rowptr))
+            L.val[:] = np.where(L.col == row, diag, off)
+        b = batch.Batch(dev, cavs, [1e-2] * len(sizes), pcg_tol=1e-8, pcg_maxit=60, precision=precision)
+        b.step()
+        out = [(b.info(k), b.field(k, "p")) for k in range(len(sizes))]
+        b.close()
+        return out
+
+    whole, got = run(False), run(True)
+    info, p = got[1]
+    n = info["n_inner"]
+    print(f"[batch breakdown {sizes}] iters {info['pcg_iters']} status {info['pcg_status']}", flush=True)
+    assert info["pcg_status"] == hip.EBREAKDOWN and info["pcg_iters"] == 0
+    assert np.abs(p[:n]).max() <= (0.0 if precision == hip.PCG_FP64 else 1e-20)
+    for k in [0] + list(range(2, len(sizes))):
+        assert got[k][0]["pcg_iters"] == whole[k][0]["pcg_iters"] > 0
+        assert np.array_equal(got[k][1], whole[k][1])
