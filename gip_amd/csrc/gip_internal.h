@@ -8,6 +8,7 @@
 
 #include "gip_hip.h"
 #include "gip_layout.h"
+#include "gip_wait.h"
 
 namespace gip {
 

@@ -19,20 +19,13 @@ int hip_fail(hipError_t e, const char *what) {
 }
 
 int wait_published(hipStream_t st, const uint64_t *flag, uint64_t want) {
-    for (unsigned spin = 1;; ++spin) {
-        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == want) return GIP_OK;
-        if (spin & 0xfffff) {
-            __builtin_ia32_pause();
-            continue;
-        }
-        // the stream may have failed: then the number never comes (asked only
-        // now and then, tens of ms: the query itself queues work)
+    const int rc = wait_seq(flag, want, [&]() {
         const hipError_t e = hipStreamQuery(st);
-        if (e == hipErrorNotReady) continue;
-        if (e != hipSuccess) return hip_fail(e, "waiting for a kernel's result");
-        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == want) return GIP_OK;
-        return set_error(GIP_EHIP, "a kernel's result did not arrive");
-    }
+        return e == hipErrorNotReady ? -1 : (int)e;
+    });
+    if (rc == WAIT_OK) return GIP_OK;
+    if (rc == WAIT_MISSING) return set_error(GIP_EHIP, "a kernel's result did not arrive");
+    return hip_fail((hipError_t)(rc - 1), "waiting for a kernel's result");
 }
 
 int reduce_grid(int n) {
