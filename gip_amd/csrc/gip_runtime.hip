@@ -19,6 +19,14 @@ int hip_fail(hipError_t e, const char *what) {
 }
 
 int wait_published(hipStream_t st, const uint64_t *flag, uint64_t want) {
+    if (seq_reached(flag, want)) return GIP_OK;
+    // a captured kernel does not run: refused as a wait for the stream is,
+    // which also ends the capture (asked while the kernel runs)
+    if (capturing(st)) {
+        const hipError_t e = hipStreamSynchronize(st);
+        return e != hipSuccess ? hip_fail(e, "a result under stream capture")
+                               : set_error(GIP_EHIP, "a result cannot be waited for under stream capture");
+    }
     const int rc = wait_seq(flag, want, [&]() {
         const hipError_t e = hipStreamQuery(st);
         return e == hipErrorNotReady ? -1 : (int)e;
