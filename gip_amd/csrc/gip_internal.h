@@ -128,7 +128,7 @@ struct gip_mat {
     // row's slot values and diagonal, dict_n of them (0: none), current while
     // dict_version == val_version + 1
     int32_t dict_n;
-    bool dict_off;  // a captured graph may change the values unseen: not used any more
+    bool vals_captured;  // a captured graph may change the values unseen: no form made from them is used any more
     uint64_t dict_version;
     gip::DictRec *d_dict_rec;  // per slice: which tuples its rows hold
     gip::DictSel *d_dict_sel;
@@ -173,7 +173,7 @@ int mat_sym_prepare(gip_ctx *c, gip_mat *A, bool *ok);
 int mat_dict_build(gip_ctx *c, gip_mat *A);
 void mat_dict_free(gip_mat *A);
 inline bool mat_dict_ok(const gip_mat *A) {
-    return A->dict_n > 0 && !A->dict_off && A->dict_version == A->val_version + 1;
+    return A->dict_n > 0 && !A->vals_captured && A->dict_version == A->val_version + 1;
 }
 inline bool capturing(hipStream_t st) {
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
@@ -186,7 +186,7 @@ inline bool mat_dict_now(const gip_mat *A, hipStream_t st) { return mat_dict_ok(
 // values that the device writes (gip_dcsrmv_vals)
 inline void mat_values_change(gip_mat *A, hipStream_t st) {
     ++A->val_version;
-    if (!A->dict_off && capturing(st)) A->dict_off = true;
+    if (!A->vals_captured && capturing(st)) A->vals_captured = true;
 }
 // Looks up the no-alloc PCG scratch array's address on `device` (current);
 // called once per device by gip_init.

@@ -450,7 +450,8 @@ int spmv32_launch(gip_ctx *c, const gip_mat *A, const float *x, float *y) {
 
 int mat_sym_prepare(gip_ctx *c, gip_mat *A, bool *ok) {
     *ok = false;
-    if (A->format != GIP_FMT_STENCIL || A->sym_nu <= 0 || !A->d_st_code || A->nrows <= 0) return GIP_OK;
+    if (A->format != GIP_FMT_STENCIL || A->sym_nu <= 0 || !A->d_st_code || A->nrows <= 0 || A->vals_captured)
+        return GIP_OK;
     if (A->sym_version == A->val_version + 1) {
         *ok = A->sym_ok > 0;
         return GIP_OK;
@@ -742,7 +743,8 @@ int gip_mat_product_bytes(const gip_mat *A, int32_t fp32, int64_t *bytes) {
 int gip_mat_sym_state(const gip_mat *A, int32_t *state, int64_t *bytes) {
     if (!A || !state) return set_error(GIP_EINVAL, "gip_mat_sym_state: bad argument");
     const bool current = A->sym_version == A->val_version + 1;
-    *state = A->format != GIP_FMT_STENCIL || A->sym_nu <= 0 ? 0 : current ? A->sym_ok : 2;
+    const bool none = A->format != GIP_FMT_STENCIL || A->sym_nu <= 0 || A->vals_captured;
+    *state = none ? 0 : current ? A->sym_ok : 2;
     // the symmetric product's own bytes: the values of the slots of offsets
     // >= 0, the slot offsets and codes, the tail records, values and
     // columns, the input once, the output once (the values of the slots of

@@ -124,7 +124,8 @@ int gip_mat_info(const gip_mat *A, int32_t *nrows, int32_t *nnz, int32_t *format
  * No counterpart in the reference: the unit of a layout's roofline. */
 int gip_mat_product_bytes(const gip_mat *A, int32_t fp32, int64_t *bytes);
 /* State of the symmetric form (GIP_MAT_NO_SYM above): 0 none (not a
- * stencil-layout operator, turned off, or offsets it cannot pair), 2 not
+ * stencil-layout operator, turned off, offsets it cannot pair, or a captured
+ * gip_dcsrmv_vals* may change the values at any replay), 2 not
  * yet made for the current values, 1 in use, -1 the values are not
  * symmetric.  bytes (optional): what one FP64 product moves with it (the
  * values of the slots of offsets >= 0, the slot metadata, the tails, the
