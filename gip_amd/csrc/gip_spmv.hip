@@ -757,6 +757,20 @@ int gip_mat_sym_state(const gip_mat *A, int32_t *state, int64_t *bytes) {
     return GIP_OK;
 }
 
+int gip_mat_dict_state(const gip_mat *A, int32_t fp32, int32_t *state, int32_t *tuples, int64_t *bytes) {
+    if (!A || !state) return set_error(GIP_EINVAL, "gip_mat_dict_state: bad argument");
+    const bool have = mat_dict_ok(A) && (!fp32 || A->d_dict_soa32);
+    *state = !have ? 0 : A->dict_ids ? 2 : 1;
+    if (tuples) *tuples = have ? A->dict_n : 0;
+    const int64_t vb = fp32 ? 4 : 8;
+    if (bytes)
+        *bytes = !have ? 0
+                       : (int64_t)A->nslices * (int64_t)sizeof(DictRec) + (A->dict_ids ? 2 * (int64_t)A->nrows : 0) +
+                             vb * A->st_w * (int64_t)A->dict_n + (int64_t)A->st_tail_nnz * vb +
+                             vb * ((int64_t)A->cols_needed + A->nrows);
+    return GIP_OK;
+}
+
 int gip_mat_autotune(gip_ctx *c, int32_t nrows, int32_t ncols, int32_t nnz, const int32_t *rowptr, const int32_t *col,
                      const double *val, int32_t flags, const double *x, double *y, int32_t reps, gip_mat **out,
                      gip_tune_report *rep) {

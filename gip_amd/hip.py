@@ -66,6 +66,7 @@ SIGNATURES = {
     "gip_mat_cols_needed": ([c_void_p, POINTER(c_int32)], c_int),
     "gip_mat_product_bytes": ([c_void_p, c_int32, POINTER(c_int64)], c_int),
     "gip_mat_sym_state": ([c_void_p, POINTER(c_int32), POINTER(c_int64)], c_int),
+    "gip_mat_dict_state": ([c_void_p, c_int32, POINTER(c_int32), POINTER(c_int32), POINTER(c_int64)], c_int),
     "gip_mat_set_lanes": ([c_void_p, c_int32], c_int),
     "gip_mat_autotune": ([c_void_p, c_int32, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p,
                           c_void_p, c_int32, POINTER(c_void_p), c_void_p], c_int),
@@ -259,6 +260,14 @@ class Matrix:
         st, b = c_int32(), c_int64()
         check(lib().gip_mat_sym_state(self.ptr, byref(st), byref(b)))
         return st.value, b.value
+
+    def dict_state(self, fp32=False):
+        """(state, tuples, bytes) of the dictionary of slot values
+        (gip_mat_dict_state): state 0 none, 1 in use, 2 in use with per-row
+        numbers; bytes one (FP32) product moves with it."""
+        st, n, b = c_int32(), c_int32(), c_int64()
+        check(lib().gip_mat_dict_state(self.ptr, 1 if fp32 else 0, byref(st), byref(n), byref(b)))
+        return st.value, n.value, b.value
 
     def values(self):
         out = np.empty(self.nnz, np.float64)

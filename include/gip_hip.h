@@ -121,6 +121,8 @@ int gip_mat_info(const gip_mat *A, int32_t *nrows, int32_t *nnz, int32_t *format
  * For CSR that is the CSR count 12 nnz + 4 (rows+1) + 8 rows + 8 cols; the
  * stencil layout stores no column per entry (one offset per slot of 64
  * rows), so it moves fewer bytes than the CSR count of the same operator.
+ * A product that reads the dictionary instead (gip_mat_dict_state) moves
+ * fewer still.
  * No counterpart in the reference: the unit of a layout's roofline. */
 int gip_mat_product_bytes(const gip_mat *A, int32_t fp32, int64_t *bytes);
 /* State of the symmetric form (GIP_MAT_NO_SYM above): 0 none (not a
@@ -131,6 +133,20 @@ int gip_mat_product_bytes(const gip_mat *A, int32_t fp32, int64_t *bytes);
  * values of the slots of offsets >= 0, the slot metadata, the tails, the
  * input and output once; 0 for state 0).  No counterpart in the reference. */
 int gip_mat_sym_state(const gip_mat *A, int32_t *state, int64_t *bytes);
+/* The dictionary of a stencil operator's slot values: an operator whose rows
+ * repeat a few value tuples (a uniform mesh) is multiplied from the distinct
+ * tuples, bit for bit the stored values, instead of 8 bytes per stored slot.
+ * Made when the values are set from the host (gip_mat_create,
+ * gip_mat_set_values); values changed on the device (gip_dcsrmv_vals*) are
+ * multiplied as stored until they are set again, and always once such a
+ * change is part of a captured graph.  state: 0 none, 1 in use, 2 in use with
+ * two bytes per row that number the tuples of slices that hold more than
+ * two.  The solver reads it from 2^19 rows on (mixed precision: 2^21).
+ * tuples (optional): the distinct ones.  bytes (optional; fp32 != 0: of the
+ * FP32 product): what one product moves with it (the records, the numbers,
+ * the tuples, the tails, the input and output once; 0 for state 0).  No
+ * counterpart in the reference. */
+int gip_mat_dict_state(const gip_mat *A, int32_t fp32, int32_t *state, int32_t *tuples, int64_t *bytes);
 /* Largest column index + 1: the length an input vector of a product must have. */
 int gip_mat_cols_needed(const gip_mat *A, int32_t *ncols);
 /* CSR operators: lanes per row (1, 2, 4, 8 = 64, 32, 16, 8 rows per

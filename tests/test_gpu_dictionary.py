@@ -155,3 +155,79 @@ def test_captured_products_follow_the_values(dev):
         with torch.cuda.stream(stream):
             change.replay()
         assert np.array_equal(eager(A), five) and np.array_equal(replayed()[0], five)
+
+
+# ---- which operators have one -------------------------------------------------
+
+OFFSETS7 = (-9, -3, -1, 0, 1, 3, 9)
+OFFSETS8 = (-9, -3, -1, 0, 1, 3, 9, 27)
+
+
+def band(n, rows, offsets=OFFSETS7):
+    """CSR arrays of a band operator whose row r holds the values rows[r] at columns r + offsets (inside the
+    operator), the number of distinct rows with zeros for the missing entries (the dictionary's tuples, since
+    every slice of 64 rows has the same slots) and whether a slice holds more than two of them."""
+    col = np.arange(n)[:, None] + np.asarray(offsets)[None, :]
+    inside = (col >= 0) & (col < n)
+    kinds, kind = np.unique(np.where(inside, rows, 0.0), axis=0, return_inverse=True)
+    k = np.sort(np.concatenate([kind.ravel(), np.full(-n % 64, kind.ravel()[-1])]).reshape(-1, 64), axis=1)
+    many = bool((np.diff(k, axis=1) != 0).sum(1).max() > 1)
+    rowptr = np.concatenate([[0], np.cumsum(inside.sum(1))]).astype(np.int32)
+    return rowptr, col[inside].astype(np.int32), np.ascontiguousarray(rows[inside]), kinds.shape[0], many
+
+
+def pick(n, k, seed, by=1):
+    """Row indices into k kinds, drawn anew every `by` rows, the first row of every kind somewhere."""
+    return np.repeat(np.random.default_rng(seed).integers(0, k, -(-n // by)), by)[:n]
+
+
+@pytest.mark.parametrize("n", [2 ** 18 + 1, 2 ** 20 - 37])
+@pytest.mark.parametrize("offsets", [(-1, 0, 1), OFFSETS7, OFFSETS8], ids=lambda o: f"{len(o)} slots")
+@pytest.mark.parametrize("kinds,by", [(1, 1), (2, 1), (3, 64), (40, 1), (3000, 64)])
+def test_tuples_of_a_band(dev, n, offsets, kinds, by):
+    """The number of tuples, whether slices need their rows' numbers, and the products."""
+    rng = np.random.default_rng(7)
+    which = pick(n, kinds, 8, by)
+    rowptr, col, val, tuples, many = band(n, rng.standard_normal((kinds, len(offsets)))[which], offsets)
+    print(f"[tuples n {n} slots {len(offsets)} kinds {kinds} by {by}] {tuples}", flush=True)
+    A = hip.Matrix(dev, rowptr, col, val, nrows=n, ncols=n, fp32=True)
+    C = hip.Matrix(dev, rowptr, col, val, nrows=n, ncols=n, fmt=hip.FMT_CSR, fp32=True)
+    state, got, nbytes = A.dict_state()
+    assert got == tuples and state == (2 if many else 1)
+    assert 16 * n < nbytes < A.product_bytes()
+    assert C.dict_state() == (0, 0, 0)
+    _products(dev, A, C, 9, fp32=True)
+
+
+def test_states(dev):
+    """64-row slices of one tuple need no numbers; values changed on the device, or without repetition, have no
+    dictionary until values are set that do."""
+    n = 2 ** 18 + 640
+    rng = np.random.default_rng(1)
+    rowptr, col, val, tuples, _ = band(n, np.tile(rng.standard_normal(3), (n, 1)), (-64, 0, 64))
+    A = hip.Matrix(dev, rowptr, col, val, nrows=n, ncols=n)
+    assert A.dict_state()[:2] == (1, tuples) and tuples == 3
+    A.set_values(rng.standard_normal(val.size))
+    assert A.dict_state() == (0, 0, 0)
+    A.set_values(val)
+    assert A.dict_state()[:2] == (1, 3)
+    nnz = val.size
+    ident = hip.Matrix(dev, np.arange(nnz + 1), np.arange(nnz), np.ones(nnz), ncols=nnz, fmt=hip.FMT_CSR)
+    ident.spmv_vals(dev.to_device(2.0 * val), A)
+    assert A.dict_state() == (0, 0, 0)
+    A.set_values(val)
+    assert A.dict_state()[:2] == (1, 3)
+
+
+@pytest.mark.parametrize("shape,state", [((128, 64, 33), 1), ((65, 64, 64), 2), ((97, 97, 97), 2)],
+                         ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else str(s))
+def test_uniform_meshes_have_one(dev, shape, state):
+    c = cavity.generate(*shape, gamma=1e-3, ops=cavity.OP_BITS["L"])
+    A = hip.Matrix.from_csr(dev, c.op("L"), fp32=True)
+    got, tuples, nbytes = A.dict_state()
+    print(f"[dictionary {shape}] state {got} tuples {tuples} bytes {nbytes} of {A.product_bytes()}", flush=True)
+    assert got == state and 0 < tuples <= c.n_inner // 8
+    assert nbytes < 0.5 * A.product_bytes() and A.dict_state(fp32=True)[2] < nbytes
+    # clustered: no two lines alike
+    c = cavity.generate(*shape, beta=1.5, gamma=1e-3, ops=cavity.OP_BITS["L"])
+    assert hip.Matrix.from_csr(dev, c.op("L")).dict_state() == (0, 0, 0)
