@@ -370,6 +370,7 @@ int mat_dict_build(gip_ctx *c, gip_mat *A) {
         A->dict_n = nd;
         A->dict_ids = cnt[2] < 0;
         A->dict_version = A->val_version + 1;
+        if (w >= kDictLineW) mat_sym_free(A);  // the solves read the dictionary in their place
     }
     return GIP_OK;
 }

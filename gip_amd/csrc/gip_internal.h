@@ -124,6 +124,7 @@ struct gip_mat {
     int32_t *d_sym_flag;
     uint64_t sym_version;  // val_version + 1 the symmetric values were made from (0: never)
     int32_t sym_ok;        // 1: in use, -1: the values are not symmetric
+    uint64_t sym_due;      // val_version + 1 of a solve that read the dictionary in its place
     // dictionary of the slot values (gip_dict.hip): the distinct tuples of a
     // row's slot values and diagonal, dict_n of them (0: none), current while
     // dict_version == val_version + 1
@@ -168,6 +169,8 @@ __device__ inline void publish_seq(uint64_t *flag, uint64_t seq) {
 // a stencil operator's slot values; *ok is true when the PCG's product may
 // read them.  Allocates on first use.
 int mat_sym_prepare(gip_ctx *c, gip_mat *A, bool *ok);
+// Frees the symmetric arrays (made again when a solve needs them).
+void mat_sym_free(gip_mat *A);
 // Makes the dictionary of a stencil operator's slot values from its current
 // values where it pays (dict_n stays 0 otherwise), and frees it.
 int mat_dict_build(gip_ctx *c, gip_mat *A);

@@ -1873,21 +1873,23 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
         int rc = coarse_setup(S);
         if (rc) return rc;
     }
-    // the symmetric form of a 7- or 8-slot stencil operator for the FP64
-    // products of the long iterations (made and checked here after a change
-    // of values; the no-alloc solve never has those iterations)
-    bool sym = false;
-    if (!mixed && S->fold && (kernel_width(A) == -7 || kernel_width(A) == -8)) {
-        int rc = mat_sym_prepare(c, const_cast<gip_mat *>(A), &sym);
-        if (rc) return rc;
-    }
-    // the dictionary of its slot values, where the operator has one, before
+    // the dictionary of a stencil operator's slot values, where it has one, before
     // either form of the stored values; in FP32 from 2^21 rows on, below
     // which the values stay in the caches (us per iteration without and with
     // it: FP64 81^3 30.9 / 27.9, 97^3 37.9 / 31.5, 128^3 58.5 / 46.6, 256^3
     // 423.7 / 324.1; mixed 97^3 31.5 / 32.3, 128^3 45.0 / 42.3, 256^3
     // 250.8 / 211.1)
     const bool dict = S->fold && A->st_w >= 7 && mat_dict_ok(A) && (!mixed || S->n >= 1 << 21);
+    // else the symmetric form of a 7- or 8-slot operator for the FP64 products
+    // of the long iterations (made and checked here after a change of values;
+    // the no-alloc solve never has those iterations)
+    bool sym = false;
+    if (!mixed && dict) {
+        const_cast<gip_mat *>(A)->sym_due = A->val_version + 1;
+    } else if (!mixed && S->fold && (kernel_width(A) == -7 || kernel_width(A) == -8)) {
+        int rc = mat_sym_prepare(c, const_cast<gip_mat *>(A), &sym);
+        if (rc) return rc;
+    }
     // ... and its inverse diagonal, while the solver's (taken when it was
     // created) is the one of the operator's present values.  us per
     // iteration with s stored and not: FP64 128^3 46.6 / 43.5, 200^3 195 /

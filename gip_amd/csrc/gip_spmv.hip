@@ -448,6 +448,13 @@ int spmv32_launch(gip_ctx *c, const gip_mat *A, const float *x, float *y) {
     return GIP_OK;
 }
 
+void mat_sym_free(gip_mat *A) {
+    if (!A->d_sym_val) return;
+    hipFree(A->d_sym_val);
+    A->d_sym_val = nullptr;
+    A->sym_version = 0;
+}
+
 int mat_sym_prepare(gip_ctx *c, gip_mat *A, bool *ok) {
     *ok = false;
     if (A->format != GIP_FMT_STENCIL || A->sym_nu <= 0 || !A->d_st_code || A->nrows <= 0 || A->vals_captured)
@@ -745,6 +752,16 @@ int gip_mat_sym_state(const gip_mat *A, int32_t *state, int64_t *bytes) {
     const bool current = A->sym_version == A->val_version + 1;
     const bool none = A->format != GIP_FMT_STENCIL || A->sym_nu <= 0 || A->vals_captured;
     *state = none ? 0 : current ? A->sym_ok : 2;
+    if (*state == 2 && A->sym_due == A->val_version + 1) {
+        // the solves read the dictionary, and nothing has asked until now: the
+        // arrays are made for the check alone
+        gip_mat *M = const_cast<gip_mat *>(A);
+        bool ok = false;
+        int rc = mat_sym_prepare(M->ctx, M, &ok);
+        if (rc) return rc;
+        *state = M->sym_ok;
+        if (mat_dict_ok(M)) mat_sym_free(M);
+    }
     // the symmetric product's own bytes: the values of the slots of offsets
     // >= 0, the slot offsets and codes, the tail records, values and
     // columns, the input once, the output once (the values of the slots of

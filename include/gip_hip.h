@@ -106,7 +106,9 @@ enum { GIP_MAT_ELL_SLICE32 = 1 << 9, GIP_MAT_ELL_SLICE128 = 1 << 10 };
  * change (gip_mat_set_values, gip_dcsrmv_vals*); an operator that fails
  * the check keeps the full product.  That first solve allocates the arrays
  * (one value per row for each stored offset: 6 for the cavity Laplacian's
- * 7 slots) and must not overlap another solve on the same operator.
+ * 7 slots) and must not overlap another solve on the same operator.  An
+ * operator with a dictionary (gip_mat_dict_state) is multiplied from that
+ * instead, and no arrays are made for its solves.
  * GIP_MAT_NO_SYM turns this off. */
 enum { GIP_MAT_NO_SYM = 1 << 11 };
 int gip_mat_create(gip_ctx *ctx, int32_t nrows, int32_t ncols, int32_t nnz, const int32_t *rowptr, const int32_t *col,
@@ -128,8 +130,10 @@ int gip_mat_product_bytes(const gip_mat *A, int32_t fp32, int64_t *bytes);
 /* State of the symmetric form (GIP_MAT_NO_SYM above): 0 none (not a
  * stencil-layout operator, turned off, offsets it cannot pair, or a captured
  * gip_dcsrmv_vals* may change the values at any replay), 2 not
- * yet made for the current values, 1 in use, -1 the values are not
- * symmetric.  bytes (optional): what one FP64 product moves with it (the
+ * yet made for the current values, 1 in use (or, where the solves read the
+ * dictionary in its place, found symmetric by this call after the first large
+ * FP64 solve: the arrays are made for the check and freed), -1 the values are
+ * not symmetric.  bytes (optional): what one FP64 product moves with it (the
  * values of the slots of offsets >= 0, the slot metadata, the tails, the
  * input and output once; 0 for state 0).  No counterpart in the reference. */
 int gip_mat_sym_state(const gip_mat *A, int32_t *state, int64_t *bytes);

@@ -10,6 +10,8 @@ slots); after a change of
 values the form is made again (scaled values) or refused (one value off
 by one unit in the last place), and the solve still equals the full one.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -134,3 +136,51 @@ def test_changed_values_remake_or_refuse_the_form(dev):
     assert np.array_equal(xa, xf)
     A.destroy()
     F.destroy()
+
+
+def test_no_arrays_beside_a_dictionary(dev):
+    """A solve that multiplies from the dictionary neither makes nor keeps the symmetric arrays (100 MB here)."""
+    torch = pytest.importorskip("torch")
+    c, L, b = _case(128)
+    A = hip.Matrix.from_csr(dev, L)
+    assert A.dict_state()[0] != 0
+    solver = hip.PCG(A, c.n_all)
+    db, dx, dz = dev.to_device(b), dev.array(c.n_all), dev.to_device(np.zeros(c.n_all))
+
+    def grown(call, want):
+        """Whether `call` changed the memory in use by want(bytes); the driver may count freed memory a little later."""
+        dev.sync()
+        free = torch.cuda.mem_get_info()[0]
+        call()
+        for _ in range(40):
+            if want(free - torch.cuda.mem_get_info()[0]):
+                return True
+            time.sleep(0.05)
+        return False
+
+    def solve():
+        solver.solve(db, dx, dz, maxit=3)
+
+    def symmetric():
+        assert A.sym_state()[0] == 1
+
+    def little(bytes_):
+        return abs(bytes_) < 16 << 20
+
+    assert grown(solve, little)
+    A.set_values(2.0 * L.val)
+    assert grown(solve, little)
+    # asked for, the symmetry is checked, and the arrays go again
+    assert grown(symmetric, little)
+    # without the dictionary (no two rows alike, still symmetric) the solve makes them; with it back they go
+    row = np.repeat(np.arange(L.nrows), np.diff(L.rowptr))
+    s = 1.0 + 0.1 * np.random.default_rng(5).random(c.n_all)
+    v = (s[row] * s[L.col]) * L.val
+    A.set_values(v)
+    assert A.dict_state()[0] == 0
+    assert grown(solve, lambda m: m > 64 << 20)
+    symmetric()
+    assert grown(lambda: A.set_values(L.val), lambda m: m < -(32 << 20))
+    assert A.sym_state()[0] == 2
+    assert grown(solve, little)
+    symmetric()
