@@ -21,7 +21,6 @@
 // in); every row's values are then compared with its tuple's, so a hash
 // collision refuses the dictionary instead of changing a value.
 #include <algorithm>
-#include <vector>
 
 #include "gip_internal.h"
 
@@ -47,14 +46,23 @@ struct DictTable {
     int32_t *row;   // lowest row holding it
     int32_t *id;    // its number
     uint32_t mask;  // slots - 1
-    int32_t *count; // [0] tuples inserted, [1] raised when the dictionary does not fit, [2] tuples listed, then -1 when
-                    // some slice needs its rows' ids
+    int32_t *count; // [0] tuples inserted, [1] raised when the dictionary does not fit, [2] raised when some slice needs
+                    // its rows' ids
     int32_t cap;
+    uint64_t *first;  // per slice: the rows that are the lowest of their tuple
+    int32_t *before;  // how many of those the slices before it in its run of kDictScan slices have
+    int32_t *run;     // and how many the runs before
 };
 
 template <class T>
 __device__ inline T dict_load(const T *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// a word of the table that may be an earlier one: an atomic update follows
+// wherever that would matter
+template <class T>
+__device__ inline T dict_hint(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 __device__ inline uint64_t dict_mix(uint64_t h, uint64_t v) {
@@ -89,8 +97,9 @@ __device__ inline int dict_find(const DictTable &T, uint64_t h) {
     return -1;
 }
 
-__global__ __launch_bounds__(kBlock) void k_dict_clear(DictTable T) {
+__global__ __launch_bounds__(kBlock) void k_dict_clear(DictTable T, int ns) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < (uint32_t)ns) T.first[i] = 0;
     if (i <= T.mask) {
         T.key[i] = 0;
         T.row[i] = INT32_MAX;
@@ -98,55 +107,115 @@ __global__ __launch_bounds__(kBlock) void k_dict_clear(DictTable T) {
     if (i < 3) T.count[i] = 0;
 }
 
-// One row per thread.  Plain atomic loads come first: once a tuple is known
-// its later rows cost two cached reads and no atomic update.
+// One row per thread, of which the lowest of each tuple in a wavefront goes to
+// the table (the wavefront's first kDictSame tuples are told apart by their
+// hashes, lanes past those go for themselves).  Run over every kDictEvery-th
+// workgroup first, then over all of them, whose tuples are nearly all known by
+// then and cost two cached reads.  With every row in one launch going for
+// itself, the rows in flight at the start (2^19, whatever the operator's
+// size) met the same few free slots, one atomic update after another, 2.5
+// ms; a counter update for each new tuple took as long on an operator
+// without repetition.  us now: uniform 97^3 87, 128^3 39, 256^3 270; no
+// two rows alike 97^3 350, 128^3 535, 256^3 610.
+constexpr int kDictSame = 4, kDictEvery = 16;
 __global__ __launch_bounds__(kBlock) void k_dict_insert(DictTable T, int n, int w, const double *__restrict__ val,
-                                                        const double *__restrict__ diag) {
-    const int r = blockIdx.x * kBlock + threadIdx.x;
-    if (r >= n || dict_load(T.count + 1)) return;
-    uint64_t t[kMaxW];
-    dict_tuple(w, val, diag, r, t);
-    const uint64_t h = dict_hash(t);
+                                                        const double *__restrict__ diag, int every) {
+    const int r = blockIdx.x * every * kBlock + threadIdx.x, lane = threadIdx.x & 63;
+    uint64_t h = 0;
+    bool todo = r < n && dict_load(T.count + 1) == 0;
+    if (todo) {
+        uint64_t t[kMaxW];
+        dict_tuple(w, val, diag, r, t);
+        h = dict_hash(t);
+    }
+    bool mine = todo;
+    for (int i = 0; i < kDictSame; ++i) {
+        const uint64_t left = __ballot(todo);
+        if (!left) break;
+        const int first = __builtin_ctzll(left);
+        const bool same = h == (uint64_t)__shfl((unsigned long long)h, first, 64);
+        mine = mine && (!todo || !same || lane == first);
+        todo = todo && !same;
+    }
+    bool added = false, lost = mine;
     uint32_t s = (uint32_t)h & T.mask;
-    for (int i = 0; i < kDictProbe; ++i, s = (s + 1) & T.mask) {
-        uint64_t k = dict_load(T.key + s);
+    for (int i = 0; mine && i < kDictProbe; ++i, s = (s + 1) & T.mask) {
+        uint64_t k = dict_hint(T.key + s);
         if (k == 0) {
             k = atomicCAS((unsigned long long *)T.key + s, 0ull, (unsigned long long)h);
-            if (k == 0) {
-                if (atomicAdd(T.count, 1) >= T.cap) atomicOr(T.count + 1, 1);
-                k = h;
-            }
+            added = k == 0;
+            if (added) k = h;
         }
         if (k == h) {
-            if (dict_load(T.row + s) > r) atomicMin(T.row + s, r);
-            return;
+            if (dict_hint(T.row + s) > r) atomicMin(T.row + s, r);
+            lost = false;
+            break;
         }
     }
-    atomicOr(T.count + 1, 1);
+    const uint64_t news = __ballot(added), bad = __ballot(lost);
+    if (lane) return;
+    const int more = __popcll(news);
+    if ((more && atomicAdd(T.count, more) + more > T.cap) || bad) atomicOr(T.count + 1, 1);
 }
 
-__global__ __launch_bounds__(kBlock) void k_dict_list(DictTable T, int32_t *__restrict__ rows) {
+// the lowest row of every tuple into its slice's mask
+__global__ __launch_bounds__(kBlock) void k_dict_mark(DictTable T) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i > T.mask || T.key[i] == 0) return;
-    const int at = atomicAdd(T.count + 2, 1);
-    if (at < T.cap) rows[at] = T.row[i];
+    const int r = T.row[i];
+    atomicOr((unsigned long long *)T.first + (r >> 6), 1ull << (r & 63));
 }
 
-// tuple i is the one of row rows[i]: its values in both table orders, its
-// number into the hash table (nothing past the slots in use: 0)
-__global__ __launch_bounds__(kBlock) void k_dict_fill(DictTable T, int nd, int w, const int32_t *__restrict__ rows,
-                                                      const double *__restrict__ val, const double *__restrict__ diag,
-                                                      double *__restrict__ tab, double *__restrict__ soa,
-                                                      double *__restrict__ ddiag) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
+// inclusive scan of one value per thread of a workgroup of kDictScan
+constexpr int kDictScan = 1024;
+__device__ inline int dict_scan(int v, int32_t (&sh)[kDictScan]) {
+    const int t = threadIdx.x;
+    sh[t] = v;
+    __syncthreads();
+    for (int off = 1; off < kDictScan; off *= 2) {
+        const int o = t >= off ? sh[t - off] : 0;
+        __syncthreads();
+        sh[t] += o;
+        __syncthreads();
+    }
+    return sh[t];
+}
+
+// The marked rows before each slice within its run of kDictScan slices, and
+// the runs' totals; then, by one workgroup, the totals before each run.
+__global__ __launch_bounds__(kDictScan) void k_dict_scan(DictTable T, int ns) {
+    __shared__ int32_t sh[kDictScan];
+    const int s = blockIdx.x * kDictScan + threadIdx.x;
+    const int own = s < ns ? __popcll(T.first[s]) : 0, sum = dict_scan(own, sh);
+    if (s < ns) T.before[s] = sum - own;
+    if (threadIdx.x == kDictScan - 1) T.run[blockIdx.x] = sum;
+}
+__global__ __launch_bounds__(kDictScan) void k_dict_runs(DictTable T, int nrun) {
+    __shared__ int32_t sh[kDictScan];
+    int base = 0;
+    for (int r0 = 0; r0 < nrun; r0 += kDictScan) {
+        const int r = r0 + threadIdx.x, own = r < nrun ? T.run[r] : 0, sum = dict_scan(own, sh);
+        if (r < nrun) T.run[r] = base + sum - own;
+        base += sh[kDictScan - 1];
+        __syncthreads();
+    }
+}
+
+// The tuples, numbered by their lowest rows: their values in both table
+// orders (nothing past the slots in use: 0).  (The numbers from a sort on the
+// host, with a copy each way, took 0.5 to 1 ms on 97^3 with 10^4 tuples.)
+__global__ __launch_bounds__(kBlock) void k_dict_fill(DictTable T, int nd, int w, const double *__restrict__ val,
+                                                      const double *__restrict__ diag, double *__restrict__ tab,
+                                                      double *__restrict__ soa, double *__restrict__ ddiag) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    if (s > T.mask || T.key[s] == 0) return;
+    const int r = T.row[s];
+    const int sl = r >> 6;
+    const int i = T.run[sl / kDictScan] + T.before[sl] + __popcll(T.first[sl] & ((1ull << (r & 63)) - 1ull));
+    T.id[s] = i;
     if (i >= nd) return;
     uint64_t t[kMaxW];
-    dict_tuple(w, val, diag, rows[i], t);
-    const int s = dict_find(T, dict_hash(t));
-    if (s < 0)
-        atomicOr(T.count + 1, 1);
-    else
-        T.id[s] = i;
+    dict_tuple(w, val, diag, r, t);
 #pragma unroll
     for (int k = 0; k < kStencilMaxW; ++k) {
         const double v = __longlong_as_double((long long)t[k]);
@@ -255,7 +324,7 @@ __global__ __launch_bounds__(kBlock) void k_dict_assign(DictTable T, int n, int 
             if (w >= kDictLineW && q.off[2] == -1 && q.off[3] == 0 && q.off[4] == 1) q.flags |= kDictLine;
         }
         if (w > 7 && q.off[7] == 0) q.flags |= kDictFree;
-        if (b < 0) T.count[2] = -1;  // some slice needs its rows' ids
+        if (b < 0) T.count[2] = 1;
         rec[sl] = q;
         sel[sl] = DictSel{a, b, mask};
     }
@@ -265,6 +334,11 @@ __global__ __launch_bounds__(kBlock) void k_dict_assign(DictTable T, int n, int 
 __global__ __launch_bounds__(kBlock) void k_dict_f32(int64_t n, const double *__restrict__ a, float *__restrict__ b) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i < n) b[i] = (float)a[i];
+}
+
+// the counters to the host
+__global__ void k_dict_report(const int32_t *__restrict__ count, int32_t *__restrict__ host) {
+    if (threadIdx.x < 3) host[threadIdx.x] = count[threadIdx.x];
 }
 
 inline int blocks(int64_t n) { return (int)((n + kBlock - 1) / kBlock); }
@@ -281,13 +355,43 @@ void mat_dict_free(gip_mat *A) {
     A->d_dict_id = nullptr;
     A->d_dict_tab = A->d_dict_soa = A->d_dict_diag = nullptr;
     A->d_dict_tab32 = A->d_dict_soa32 = nullptr;
-    A->dict_n = 0;
+    A->dict_n = A->dict_room = 0;
 }
 
-// The caller's stream has been waited for (gip_mat_create,
-// gip_mat_set_values); waits for it again before it returns.
-int mat_dict_build(gip_ctx *c, gip_mat *A) {
-    mat_dict_free(A);
+// The operator's arrays for nd tuples (kept while they are large enough: made
+// anew for every change of values, allocating and freeing them took 0.6 ms);
+// false when memory is not there.
+static bool dict_arrays(gip_mat *A, int nd) {
+    bool room = true;
+    auto get = [&](auto **p, size_t count) {
+        if (!room || *p) return;
+        if (hipMalloc(p, count * sizeof **p) != hipSuccess) {
+            (void)hipGetLastError();
+            *p = nullptr;
+            room = false;
+        }
+    };
+    if (A->dict_room && nd > A->dict_room) mat_dict_free(A);
+    if (A->dict_room) return true;
+    get(&A->d_dict_rec, (size_t)A->nslices);
+    get(&A->d_dict_sel, (size_t)A->nslices);
+    get(&A->d_dict_id, (size_t)A->nrows);
+    get(&A->d_dict_tab, (size_t)nd * 8);
+    get(&A->d_dict_soa, (size_t)nd * A->st_w);
+    get(&A->d_dict_diag, (size_t)nd);
+    if (A->d_ell_val32) {
+        get(&A->d_dict_tab32, (size_t)nd * 8);
+        get(&A->d_dict_soa32, (size_t)nd * A->st_w);
+    }
+    if (room) A->dict_room = nd;
+    return room;
+}
+
+// scratch: device memory of `bytes` bytes to work in (gip_mat_set_values has
+// the values it copied; too little: allocated).  Waits for the stream before
+// it returns.
+int mat_dict_build(gip_ctx *c, gip_mat *A, void *scratch, size_t bytes) {
+    A->dict_n = 0;
     const int n = A->nrows, w = A->st_w;
     if (A->format != GIP_FMT_STENCIL || n < kDictMinRows || n > kDictMaxRows || A->cols_needed > kDictMaxRows ||
         w < 1 || w > kStencilMaxW) return GIP_OK;
@@ -297,78 +401,68 @@ int mat_dict_build(gip_ctx *c, gip_mat *A) {
     uint32_t slots = 1024;
     while (slots < 4u * (uint32_t)T.cap) slots *= 2;
     T.mask = slots - 1;
-    char *work = nullptr;
-    int32_t *d_rows = nullptr;
     // memory that is not there is no error: the operator stays as it is
-    if (hipMalloc(&work, (size_t)slots * 16 + 64) != hipSuccess) {
+    const int ns = A->nslices, nrun = (ns + kDictScan - 1) / kDictScan;
+    const size_t need = (size_t)slots * 16 + 64 + (size_t)ns * 12 + (size_t)nrun * 4;
+    char *own = nullptr;
+    if ((!A->h_dict && hipHostMalloc((void **)&A->h_dict, 4 * sizeof(int32_t), hipHostMallocCoherent) != hipSuccess) ||
+        (bytes < need && hipMalloc(&own, need) != hipSuccess)) {
         (void)hipGetLastError();
+        mat_dict_free(A);
         return GIP_OK;
     }
+    char *const work = own ? own : static_cast<char *>(scratch);
     T.key = reinterpret_cast<uint64_t *>(work);
-    T.row = reinterpret_cast<int32_t *>(work + (size_t)slots * 8);
+    T.first = T.key + slots;
+    T.row = reinterpret_cast<int32_t *>(T.first + ns);
     T.id = T.row + slots;
-    T.count = T.id + slots;
-    k_dict_clear<<<blocks(slots), kBlock, 0, st>>>(T);
-    k_dict_insert<<<blocks(n), kBlock, 0, st>>>(T, n, w, A->d_ell_val, A->d_diag);
-    int32_t cnt[3] = {0, 1, 0};
-    hipError_t e = hipGetLastError();
+    T.before = T.id + slots;
+    T.run = T.before + ns;
+    T.count = T.run + nrun;
+    // the counters reach the host by a kernel's store: with copies from the
+    // device among them, the next copy to it ran at half its speed (0.45 GB of
+    // values 25.5 ms instead of 14.8)
+    int32_t *report = nullptr, cnt[3] = {0, 1, 0};
+    hipError_t e = hipHostGetDevicePointer((void **)&report, A->h_dict, 0);
     auto counts = [&]() {
-        if (e == hipSuccess) e = hipMemcpyAsync(cnt, T.count, sizeof cnt, hipMemcpyDeviceToHost, st);
+        if (e != hipSuccess) return;
+        k_dict_report<<<1, 64, 0, st>>>(T.count, report);
+        e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(st);
+        for (int k = 0; k < 3; ++k) cnt[k] = A->h_dict[k];
     };
-    counts();
-    const int nd = cnt[0];
-    bool ok = e == hipSuccess && !cnt[1] && nd > 0 && nd <= T.cap;
-    bool room = true;
-    auto get = [&](auto **p, size_t count) {
-        if (ok && room && hipMalloc(p, count * sizeof **p) != hipSuccess) {
-            (void)hipGetLastError();
-            *p = nullptr;
-            room = false;
-        }
-    };
-    get(&d_rows, (size_t)nd);
-    get(&A->d_dict_rec, (size_t)A->nslices);
-    get(&A->d_dict_sel, (size_t)A->nslices);
-    get(&A->d_dict_id, (size_t)n);
-    get(&A->d_dict_tab, (size_t)nd * 8);
-    get(&A->d_dict_soa, (size_t)nd * w);
-    get(&A->d_dict_diag, (size_t)nd);
-    if (A->d_ell_val32) {
-        get(&A->d_dict_tab32, (size_t)nd * 8);
-        get(&A->d_dict_soa32, (size_t)nd * w);
+    if (e == hipSuccess) {
+        const int every = kDictEvery;
+        k_dict_clear<<<blocks(std::max((int64_t)slots, (int64_t)ns)), kBlock, 0, st>>>(T, ns);
+        k_dict_insert<<<(blocks(n) + every - 1) / every, kBlock, 0, st>>>(T, n, w, A->d_ell_val, A->d_diag, every);
+        k_dict_insert<<<blocks(n), kBlock, 0, st>>>(T, n, w, A->d_ell_val, A->d_diag, 1);
+        counts();
     }
-    ok = ok && room;
+    const int nd = cnt[0];
+    bool ok = e == hipSuccess && !cnt[1] && nd > 0 && nd <= T.cap && dict_arrays(A, nd);
     if (ok) {
-        std::vector<int32_t> rows((size_t)nd);
-        k_dict_list<<<blocks(slots), kBlock, 0, st>>>(T, d_rows);
-        e = hipMemcpyAsync(rows.data(), d_rows, sizeof(int32_t) * nd, hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        std::sort(rows.begin(), rows.end());
-        if (e == hipSuccess) e = hipMemcpyAsync(d_rows, rows.data(), sizeof(int32_t) * nd, hipMemcpyHostToDevice, st);
-        if (e == hipSuccess) {
-            k_dict_fill<<<blocks(nd), kBlock, 0, st>>>(T, nd, w, d_rows, A->d_ell_val, A->d_diag, A->d_dict_tab,
-                                                       A->d_dict_soa, A->d_dict_diag);
-            k_dict_assign<<<blocks((int64_t)A->nslices * 64), kBlock, 0, st>>>(
-                T, n, A->nslices, nd, w, A->d_ell_val, A->d_diag, A->d_dict_tab, A->d_dict_diag, A->d_st_off,
-                A->d_st_tail, A->d_st_hdr, A->d_st_tcol, (int)A->st_tail_base, std::max(0, A->cols_needed - 1), A->d_dict_rec,
-                A->d_dict_sel, A->d_dict_id);
-            if (A->d_dict_tab32) {
-                k_dict_f32<<<blocks((int64_t)nd * 8), kBlock, 0, st>>>((int64_t)nd * 8, A->d_dict_tab, A->d_dict_tab32);
-                k_dict_f32<<<blocks((int64_t)nd * w), kBlock, 0, st>>>((int64_t)nd * w, A->d_dict_soa, A->d_dict_soa32);
-            }
-            e = hipGetLastError();
+        k_dict_mark<<<blocks(slots), kBlock, 0, st>>>(T);
+        k_dict_scan<<<nrun, kDictScan, 0, st>>>(T, ns);
+        k_dict_runs<<<1, kDictScan, 0, st>>>(T, nrun);
+        k_dict_fill<<<blocks(slots), kBlock, 0, st>>>(T, nd, w, A->d_ell_val, A->d_diag, A->d_dict_tab, A->d_dict_soa,
+                                                      A->d_dict_diag);
+        k_dict_assign<<<blocks((int64_t)ns * 64), kBlock, 0, st>>>(
+            T, n, ns, nd, w, A->d_ell_val, A->d_diag, A->d_dict_tab, A->d_dict_diag, A->d_st_off, A->d_st_tail,
+            A->d_st_hdr, A->d_st_tcol, (int)A->st_tail_base, std::max(0, A->cols_needed - 1), A->d_dict_rec,
+            A->d_dict_sel, A->d_dict_id);
+        if (A->d_dict_tab32) {
+            k_dict_f32<<<blocks((int64_t)nd * 8), kBlock, 0, st>>>((int64_t)nd * 8, A->d_dict_tab, A->d_dict_tab32);
+            k_dict_f32<<<blocks((int64_t)nd * w), kBlock, 0, st>>>((int64_t)nd * w, A->d_dict_soa, A->d_dict_soa32);
         }
-        counts();  // also: `rows` has been read
+        counts();
         ok = e == hipSuccess && !cnt[1];
     }
-    if (d_rows) hipFree(d_rows);
-    hipFree(work);
+    if (own) hipFree(own);
     if (!ok) mat_dict_free(A);
     if (e != hipSuccess) return hip_fail(e, "dictionary of the slot values");
     if (ok) {
         A->dict_n = nd;
-        A->dict_ids = cnt[2] < 0;
+        A->dict_ids = cnt[2] != 0;
         A->dict_version = A->val_version + 1;
         if (w >= kDictLineW) mat_sym_free(A);  // the solves read the dictionary in their place
     }

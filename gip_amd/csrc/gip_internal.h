@@ -128,7 +128,7 @@ struct gip_mat {
     // dictionary of the slot values (gip_dict.hip): the distinct tuples of a
     // row's slot values and diagonal, dict_n of them (0: none), current while
     // dict_version == val_version + 1
-    int32_t dict_n;
+    int32_t dict_n, dict_room;  // dict_room: tuples the arrays have room for
     bool vals_captured;  // a captured graph may change the values unseen: no form made from them is used any more
     uint64_t dict_version;
     gip::DictRec *d_dict_rec;  // per slice: which tuples its rows hold
@@ -137,6 +137,7 @@ struct gip_mat {
     int32_t dict_ids;          // there are such slices
     double *d_dict_tab, *d_dict_soa, *d_dict_diag;  // tuples, 8 per row of the table; slot by slot; a_ii
     float *d_dict_tab32, *d_dict_soa32;
+    int32_t *h_dict;  // pinned: the build's counters
     int32_t st_empty;  // stencil layout: some row has no entries
     // a_ii per row (the stored values of a DIAG operator), for Jacobi; for
     // the other layouts refreshed from d_diag_src (each row's last diagonal
@@ -173,7 +174,7 @@ int mat_sym_prepare(gip_ctx *c, gip_mat *A, bool *ok);
 void mat_sym_free(gip_mat *A);
 // Makes the dictionary of a stencil operator's slot values from its current
 // values where it pays (dict_n stays 0 otherwise), and frees it.
-int mat_dict_build(gip_ctx *c, gip_mat *A);
+int mat_dict_build(gip_ctx *c, gip_mat *A, void *scratch, size_t bytes);
 void mat_dict_free(gip_mat *A);
 inline bool mat_dict_ok(const gip_mat *A) {
     return A->dict_n > 0 && !A->vals_captured && A->dict_version == A->val_version + 1;

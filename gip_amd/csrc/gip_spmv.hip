@@ -320,6 +320,7 @@ static void free_mat_arrays(gip_mat *A) {
                     A->d_sym_flag, A->d_diag_src};
     for (void *p : ptrs)
         if (p) hipFree(p);
+    if (A->h_dict) hipHostFree(A->h_dict);
 }
 
 // Dispatch y (= or +=) A x in FP64.  scatter: optional output index per row.
@@ -690,7 +691,7 @@ int gip_mat_create(gip_ctx *c, int32_t nrows, int32_t ncols, int32_t nnz, const 
         hipError_t e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) rc = hip_fail(e, "gip_mat_create upload");
     }
-    if (!rc) rc = mat_dict_build(c, A);
+    if (!rc) rc = mat_dict_build(c, A, nullptr, 0);
     if (rc) {
         mat_dict_free(A);
         free_mat_arrays(A);
@@ -910,27 +911,31 @@ int gip_mat_set_values(gip_mat *A, const double *host) {
     if (!A->nnz) return GIP_OK;
     gip_ctx *c = A->ctx;
     ++A->val_version;
+    double *tmp = nullptr;
+    const size_t bytes = sizeof(double) * A->nnz;
     if (A->format == GIP_FMT_ELL || A->format == GIP_FMT_STENCIL) {
-        double *tmp = nullptr;
-        GIP_HIP_TRY(hipMalloc(&tmp, sizeof(double) * A->nnz));
-        hipError_t e = hipMemcpyAsync(tmp, host, sizeof(double) * A->nnz, hipMemcpyHostToDevice, c->stream);
+        GIP_HIP_TRY(hipMalloc(&tmp, bytes));
+        hipError_t e = hipMemcpyAsync(tmp, host, bytes, hipMemcpyHostToDevice, c->stream);
         if (e == hipSuccess) {
             k_scatter_vals<<<nblocks(A->nnz), kBlock, 0, c->stream>>>(A->nnz, tmp, A->d_csr2ell, A->d_ell_val);
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        hipFree(tmp);
-        if (e != hipSuccess) return hip_fail(e, "gip_mat_set_values");
+        if (e != hipSuccess) {
+            hipFree(tmp);
+            return hip_fail(e, "gip_mat_set_values");
+        }
         if (A->d_ell_val32) k_to_f32<<<nblocks(A->ell_stored), kBlock, 0, c->stream>>>(A->ell_stored, A->d_ell_val, A->d_ell_val32);
     } else {
         double *dst = A->format == GIP_FMT_DIAG ? A->d_diag : A->d_val;
-        GIP_HIP_TRY(hipMemcpyAsync(dst, host, sizeof(double) * A->nnz, hipMemcpyHostToDevice, c->stream));
+        GIP_HIP_TRY(hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, c->stream));
         GIP_HIP_TRY(hipStreamSynchronize(c->stream));
         if (A->d_val32) k_to_f32<<<nblocks(A->nnz), kBlock, 0, c->stream>>>(A->nnz, A->d_val, A->d_val32);
     }
-    GIP_LAUNCH_CHECK("gip_mat_set_values");
-    int rc = diag_refresh(c, A);
-    if (!rc && A->format == GIP_FMT_STENCIL) rc = mat_dict_build(c, A);
+    const hipError_t e = hipGetLastError();
+    int rc = e != hipSuccess ? hip_fail(e, "gip_mat_set_values") : diag_refresh(c, A);
+    if (!rc && A->format == GIP_FMT_STENCIL) rc = mat_dict_build(c, A, tmp, bytes);
+    if (tmp) hipFree(tmp);
     return rc;
 }
 
