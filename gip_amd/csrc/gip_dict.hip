@@ -38,6 +38,18 @@ constexpr int kDictRatio = 8;
 constexpr int kDictMax = 1 << 19;
 // Rows and columns a dictionary product addresses with 32-bit byte offsets.
 constexpr int kDictMaxRows = 1 << 28;
+// A slice of more than two tuples gathers each slot's values through its rows'
+// ids: as many cache lines of 16 FP64 tuples as its rows have tuples in.  On
+// average over the slices at most 32 of them (FP32 products: 12), past which
+// the gathers take longer than streaming the stored values.  us at 128^3 of
+// the product and the PCG iteration, rows scaled from k values at random, by
+// lines per slice; stored FP64 29.8 and 62.9, FP32 13.9 and 48.2:
+//   lines      5.9    9.9   17.5   29.4   42.0   51.1
+//   FP64      17.8   19.7   21.4   25.5   34.4   44.3
+//   FP64 PCG  51.0   52.5   54.6   59.1   70.0   81.5
+//   FP32      12.0   13.2   15.0   16.2   18.7   37.7
+//   mixed     46.6   47.2   49.2   52.6   60.3   70.2
+constexpr int kDictLines = 32, kDictLines32 = 12;
 constexpr int kDictProbe = 64;  // slots tried before the insert gives up
 constexpr int kMaxW = kStencilMaxW + 1;  // slot values and the diagonal
 
@@ -47,7 +59,7 @@ struct DictTable {
     int32_t *id;    // its number
     uint32_t mask;  // slots - 1
     int32_t *count; // [0] tuples inserted, [1] raised when the dictionary does not fit, [2] raised when some slice needs
-                    // its rows' ids
+                    // its rows' ids, [3] the lines of those slices
     int32_t cap;
     uint64_t *first;  // per slice: the rows that are the lowest of their tuple
     int32_t *before;  // how many of those the slices before it in its run of kDictScan slices have
@@ -104,7 +116,7 @@ __global__ __launch_bounds__(kBlock) void k_dict_clear(DictTable T, int ns) {
         T.key[i] = 0;
         T.row[i] = INT32_MAX;
     }
-    if (i < 3) T.count[i] = 0;
+    if (i < 4) T.count[i] = 0;
 }
 
 // One row per thread, of which the lowest of each tuple in a wavefront goes to
@@ -336,9 +348,36 @@ __global__ __launch_bounds__(kBlock) void k_dict_f32(int64_t n, const double *__
     if (i < n) b[i] = (float)a[i];
 }
 
+// The cache lines (16 FP64 tuples) that the slices with ids gather from, by
+// a few workgroups, one update each.
+constexpr int kDictLineGrid = 512;
+__global__ __launch_bounds__(kBlock) void k_dict_lines(DictTable T, int n, int ns, const DictSel *__restrict__ sel,
+                                                       const uint16_t *__restrict__ ids) {
+    __shared__ int32_t sh[kBlock / 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int lines = 0;
+    for (int s = blockIdx.x * (kBlock / 64) + wv; s < ns; s += gridDim.x * (kBlock / 64)) {
+        if (sel[s].b >= 0) continue;
+        const int r = s * 64 + lane;
+        const int line = r < n ? (sel[s].a + ids[r]) >> 4 : -1;
+        uint64_t left = __ballot(r < n);
+        while (left) {
+            const int of = __shfl(line, __builtin_ctzll(left), 64);
+            left &= ~__ballot(line == of);
+            ++lines;
+        }
+    }
+    if (lane == 0) sh[wv] = lines;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < kBlock / 64; ++k) lines += sh[k];
+        if (lines) atomicAdd(T.count + 3, lines);
+    }
+}
+
 // the counters to the host
 __global__ void k_dict_report(const int32_t *__restrict__ count, int32_t *__restrict__ host) {
-    if (threadIdx.x < 3) host[threadIdx.x] = count[threadIdx.x];
+    if (threadIdx.x < 4) host[threadIdx.x] = count[threadIdx.x];
 }
 
 inline int blocks(int64_t n) { return (int)((n + kBlock - 1) / kBlock); }
@@ -422,14 +461,14 @@ int mat_dict_build(gip_ctx *c, gip_mat *A, void *scratch, size_t bytes) {
     // the counters reach the host by a kernel's store: with copies from the
     // device among them, the next copy to it ran at half its speed (0.45 GB of
     // values 25.5 ms instead of 14.8)
-    int32_t *report = nullptr, cnt[3] = {0, 1, 0};
+    int32_t *report = nullptr, cnt[4] = {0, 1, 0, 0};
     hipError_t e = hipHostGetDevicePointer((void **)&report, A->h_dict, 0);
     auto counts = [&]() {
         if (e != hipSuccess) return;
         k_dict_report<<<1, 64, 0, st>>>(T.count, report);
         e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(st);
-        for (int k = 0; k < 3; ++k) cnt[k] = A->h_dict[k];
+        for (int k = 0; k < 4; ++k) cnt[k] = A->h_dict[k];
     };
     if (e == hipSuccess) {
         const int every = kDictEvery;
@@ -454,8 +493,9 @@ int mat_dict_build(gip_ctx *c, gip_mat *A, void *scratch, size_t bytes) {
             k_dict_f32<<<blocks((int64_t)nd * 8), kBlock, 0, st>>>((int64_t)nd * 8, A->d_dict_tab, A->d_dict_tab32);
             k_dict_f32<<<blocks((int64_t)nd * w), kBlock, 0, st>>>((int64_t)nd * w, A->d_dict_soa, A->d_dict_soa32);
         }
+        k_dict_lines<<<kDictLineGrid, kBlock, 0, st>>>(T, n, ns, A->d_dict_sel, A->d_dict_id);
         counts();
-        ok = e == hipSuccess && !cnt[1];
+        ok = e == hipSuccess && !cnt[1] && cnt[3] <= (int64_t)kDictLines * ns;
     }
     if (own) hipFree(own);
     if (!ok) mat_dict_free(A);
@@ -463,6 +503,7 @@ int mat_dict_build(gip_ctx *c, gip_mat *A, void *scratch, size_t bytes) {
     if (ok) {
         A->dict_n = nd;
         A->dict_ids = cnt[2] != 0;
+        A->dict_32 = A->d_dict_soa32 && cnt[3] <= (int64_t)kDictLines32 * ns;
         A->dict_version = A->val_version + 1;
         if (w >= kDictLineW) mat_sym_free(A);  // the solves read the dictionary in their place
     }

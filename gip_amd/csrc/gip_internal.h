@@ -135,6 +135,7 @@ struct gip_mat {
     gip::DictSel *d_dict_sel;
     uint16_t *d_dict_id;       // per row, read for slices of more than two tuples
     int32_t dict_ids;          // there are such slices
+    bool dict_32;              // FP32 products read it too
     double *d_dict_tab, *d_dict_soa, *d_dict_diag;  // tuples, 8 per row of the table; slot by slot; a_ii
     float *d_dict_tab32, *d_dict_soa32;
     int32_t *h_dict;  // pinned: the build's counters
@@ -179,6 +180,7 @@ void mat_dict_free(gip_mat *A);
 inline bool mat_dict_ok(const gip_mat *A) {
     return A->dict_n > 0 && !A->vals_captured && A->dict_version == A->val_version + 1;
 }
+inline bool mat_dict_ok32(const gip_mat *A) { return mat_dict_ok(A) && A->dict_32; }
 inline bool capturing(hipStream_t st) {
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(st, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
@@ -187,6 +189,7 @@ inline bool capturing(hipStream_t st) {
 // values: its replays take those of their own time, and the dictionary of
 // today is freed when the values change.
 inline bool mat_dict_now(const gip_mat *A, hipStream_t st) { return mat_dict_ok(A) && !capturing(st); }
+inline bool mat_dict_now32(const gip_mat *A, hipStream_t st) { return mat_dict_ok32(A) && !capturing(st); }
 // values that the device writes (gip_dcsrmv_vals)
 inline void mat_values_change(gip_mat *A, hipStream_t st) {
     ++A->val_version;

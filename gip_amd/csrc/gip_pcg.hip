@@ -1879,7 +1879,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     // it: FP64 81^3 30.9 / 27.9, 97^3 37.9 / 31.5, 128^3 58.5 / 46.6, 256^3
     // 423.7 / 324.1; mixed 97^3 31.5 / 32.3, 128^3 45.0 / 42.3, 256^3
     // 250.8 / 211.1)
-    const bool dict = S->fold && A->st_w >= 7 && mat_dict_ok(A) && (!mixed || S->n >= 1 << 21);
+    const bool dict = S->fold && A->st_w >= 7 && (mixed ? mat_dict_ok32(A) && S->n >= 1 << 21 : mat_dict_ok(A));
     // else the symmetric form of a 7- or 8-slot operator for the FP64 products
     // of the long iterations (made and checked here after a change of values;
     // the no-alloc solve never has those iterations)

@@ -429,7 +429,7 @@ int spmv32_launch(gip_ctx *c, const gip_mat *A, const float *x, float *y) {
         if (!A->d_ell_val32) return set_error(GIP_EINVAL, "operator has no FP32 values");
         const EllView v = view(A);
         const int g = nblocks(A->nrows);
-        if (A->st_w >= 7 && mat_dict_now(A, c->stream)) {
+        if (A->st_w >= 7 && mat_dict_now32(A, c->stream)) {
             DICT_LAUNCH(k_stencil32_dict, A->st_w, g, c->stream, v, A->nrows, x, y);
             GIP_LAUNCH_CHECK("spmv32 kernel");
             return GIP_OK;
@@ -777,7 +777,7 @@ int gip_mat_sym_state(const gip_mat *A, int32_t *state, int64_t *bytes) {
 
 int gip_mat_dict_state(const gip_mat *A, int32_t fp32, int32_t *state, int32_t *tuples, int64_t *bytes) {
     if (!A || !state) return set_error(GIP_EINVAL, "gip_mat_dict_state: bad argument");
-    const bool have = mat_dict_ok(A) && (!fp32 || A->d_dict_soa32);
+    const bool have = fp32 ? mat_dict_ok32(A) : mat_dict_ok(A);
     *state = !have ? 0 : A->dict_ids ? 2 : 1;
     if (tuples) *tuples = have ? A->dict_n : 0;
     const int64_t vb = fp32 ? 4 : 8;

@@ -255,3 +255,37 @@ def test_setting_values_costs_little_more_with_a_dictionary(dev, shape):
         best.append(min(times))
     print(f"[set_values {shape}] {1e3 * best[0]:.2f} ms, ELL {1e3 * best[1]:.2f}", flush=True)
     assert best[0] - best[1] < 0.7e-3
+
+
+def lines_per_slice(n, rows, offsets):
+    """Mean over the 64-row slices of the cache lines of 16 tuples that a slice of more than two tuples gathers
+    from, the tuples numbered by the first row that holds them."""
+    col = np.arange(n)[:, None] + np.asarray(offsets)[None, :]
+    _, first, kind = np.unique(np.where((col >= 0) & (col < n), rows, 0.0), axis=0, return_index=True,
+                               return_inverse=True)
+    number = np.argsort(np.argsort(first))[kind.ravel()]
+    total = 0
+    for s in range(0, n, 64):
+        own = number[s:s + 64]
+        if np.unique(own).size > 2:
+            total += np.unique(own // 16).size
+    return total / -(-n // 64)
+
+
+@pytest.mark.parametrize("kinds,by,fp64,fp32", [(100, 1, True, True), (300, 1, True, False), (5000, 1, False, False),
+                                                (20000, 1, False, False), (20000, 64, True, True),
+                                                (20000, 8, True, True)])
+def test_scattered_tuples_are_multiplied_as_stored(dev, kinds, by, fp64, fp32):
+    """Gathers from more than 32 cache lines per slice and slot (FP32: 12) would take longer than the stored values."""
+    n = 2 ** 18 + 2 ** 15
+    which = pick(n, kinds, 11, by)
+    rows = np.random.default_rng(12).standard_normal((kinds, 7))[which]
+    rowptr, col, val, _, _ = band(n, rows)
+    A = hip.Matrix(dev, rowptr, col, val, nrows=n, ncols=n, fp32=True)
+    C = hip.Matrix(dev, rowptr, col, val, nrows=n, ncols=n, fmt=hip.FMT_CSR, fp32=True)
+    lines = lines_per_slice(n, rows, OFFSETS7)
+    print(f"[scattered kinds {kinds} by {by}] {lines:.1f} lines per slice, state {A.dict_state()[0]}", flush=True)
+    assert fp64 == (lines <= 32) and fp32 == (lines <= 12)
+    assert (A.dict_state()[0] != 0) == fp64
+    assert (A.dict_state(fp32=True)[0] != 0) == fp32
+    _products(dev, A, C, 13, fp32=True)
