@@ -29,9 +29,14 @@ namespace gip {
 namespace {
 
 // Smallest operator a dictionary is made for: below it the values stay in
-// the caches between products (64^3: 4.9 us with the stored slots, 5.2 with
-// the dictionary; 97^3: 17.1 and 10.8).
+// the caches between products (us with the stored slots and with the
+// dictionary: 64^3, the smallest, 5.0 / 4.6, 72^3 7.2 / 5.4, 97^3 16.7 / 9.9).
 constexpr int kDictMinRows = 1 << 18;
+// FP32 values, half of that, stay there longer (65^3 4.4 / 4.4, 81^3 4.7 /
+// 5.1, 97^3 6.8 / 6.8, 104^3 8.5 / 8.8, 112^3 9.9 / 9.3; slices of at most
+// two tuples 128x64x64 4.3 / 4.4, 128x128x80 9.0 / 6.7): smallest operators
+// whose FP32 products read the dictionary, and where slices need ids.
+constexpr int kDictMinRows32 = 1 << 20, kDictMinIds32 = 5 << 18;
 // Tuples allowed: at most one per kDictRatio rows (a table of 64 bytes per
 // tuple then stays under the 8 bytes per row of one vector), 2^19 in all.
 constexpr int kDictRatio = 8;
@@ -503,7 +508,8 @@ int mat_dict_build(gip_ctx *c, gip_mat *A, void *scratch, size_t bytes) {
     if (ok) {
         A->dict_n = nd;
         A->dict_ids = cnt[2] != 0;
-        A->dict_32 = A->d_dict_soa32 && cnt[3] <= (int64_t)kDictLines32 * ns;
+        A->dict_32 = A->d_dict_soa32 && n >= (A->dict_ids ? kDictMinIds32 : kDictMinRows32) &&
+                     cnt[3] <= (int64_t)kDictLines32 * ns;
         A->dict_version = A->val_version + 1;
         if (w >= kDictLineW) mat_sym_free(A);  // the solves read the dictionary in their place
     }

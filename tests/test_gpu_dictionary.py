@@ -257,19 +257,13 @@ def test_setting_values_costs_little_more_with_a_dictionary(dev, shape):
     assert best[0] - best[1] < 0.7e-3
 
 
-def lines_per_slice(n, rows, offsets):
+def lines_per_slice(which):
     """Mean over the 64-row slices of the cache lines of 16 tuples that a slice of more than two tuples gathers
-    from, the tuples numbered by the first row that holds them."""
-    col = np.arange(n)[:, None] + np.asarray(offsets)[None, :]
-    _, first, kind = np.unique(np.where((col >= 0) & (col < n), rows, 0.0), axis=0, return_index=True,
-                               return_inverse=True)
-    number = np.argsort(np.argsort(first))[kind.ravel()]
-    total = 0
-    for s in range(0, n, 64):
-        own = number[s:s + 64]
-        if np.unique(own).size > 2:
-            total += np.unique(own // 16).size
-    return total / -(-n // 64)
+    from, the tuples numbered by the first row that holds them (rows without all their entries left out)."""
+    _, first, kind = np.unique(which, return_index=True, return_inverse=True)
+    number = np.argsort(np.argsort(first))[kind]
+    slices = [np.unique(number[s:s + 64]) for s in range(0, which.size, 64)]
+    return sum(np.unique(own // 16).size for own in slices if own.size > 2) / len(slices)
 
 
 @pytest.mark.parametrize("kinds,by,fp64,fp32", [(100, 1, True, True), (300, 1, True, False), (5000, 1, False, False),
@@ -277,15 +271,27 @@ def lines_per_slice(n, rows, offsets):
                                                 (20000, 8, True, True)])
 def test_scattered_tuples_are_multiplied_as_stored(dev, kinds, by, fp64, fp32):
     """Gathers from more than 32 cache lines per slice and slot (FP32: 12) would take longer than the stored values."""
-    n = 2 ** 18 + 2 ** 15
+    n = 5 * 2 ** 18  # FP32 products read ids from here on
     which = pick(n, kinds, 11, by)
-    rows = np.random.default_rng(12).standard_normal((kinds, 7))[which]
-    rowptr, col, val, _, _ = band(n, rows)
+    col = np.arange(n)[:, None] + np.asarray(OFFSETS7)[None, :]
+    inside = (col >= 0) & (col < n)
+    rowptr = np.concatenate([[0], np.cumsum(inside.sum(1))])
+    col, val = col[inside], np.random.default_rng(12).standard_normal((kinds, 7))[which][inside]
     A = hip.Matrix(dev, rowptr, col, val, nrows=n, ncols=n, fp32=True)
     C = hip.Matrix(dev, rowptr, col, val, nrows=n, ncols=n, fmt=hip.FMT_CSR, fp32=True)
-    lines = lines_per_slice(n, rows, OFFSETS7)
+    lines = lines_per_slice(which)
     print(f"[scattered kinds {kinds} by {by}] {lines:.1f} lines per slice, state {A.dict_state()[0]}", flush=True)
     assert fp64 == (lines <= 32) and fp32 == (lines <= 12)
     assert (A.dict_state()[0] != 0) == fp64
     assert (A.dict_state(fp32=True)[0] != 0) == fp32
     _products(dev, A, C, 13, fp32=True)
+
+
+@pytest.mark.parametrize("shape,fp32", [((64, 64, 65), False), ((128, 64, 64), False), ((97, 97, 97), False),
+                                        ((104, 104, 104), False), ((128, 128, 64), True), ((112, 112, 112), True)],
+                         ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else str(s))
+def test_fp32_products_that_fit_the_caches_read_the_stored_values(dev, shape, fp32):
+    c = cavity.generate(*shape, gamma=1e-3, ops=cavity.OP_BITS["L"])
+    A = hip.Matrix.from_csr(dev, c.op("L"), fp32=True)
+    assert A.dict_state()[0] != 0 and (A.dict_state(fp32=True)[0] != 0) == fp32
+    _products(dev, A, hip.Matrix.from_csr(dev, c.op("L"), fmt=hip.FMT_CSR, fp32=True), 14, fp32=True)
