@@ -308,7 +308,7 @@ int gip_adjoint_create(gip_ctx *c, const gip_cavity *cav, const gip_adjoint_opts
                                      ops[k]->val, GIP_FMT_AUTO, &a->op[k]);
     }
     if (!rc) rc = gip_mat_create(c, cav->D.nrows, cav->D.ncols, cav->D.nnz, cav->D.rowptr, cav->D.col, cav->D.val,
-                                 GIP_FMT_AUTO, &a->C);
+                                 GIP_FMT_AUTO | GIP_MAT_NO_DICT, &a->C);
     if (!rc) rc = gip_pcg_create(c, a->op[A_L], a->NA, &a->pcg);
     const size_t NA = (size_t)a->NA, F = (size_t)a->F;
     double **cells[] = {&a->u, &a->v, &a->w, &a->ax0, &a->ay0, &a->az0, &a->p0, &a->p, &a->ax, &a->ay, &a->az,

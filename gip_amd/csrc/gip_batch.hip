@@ -1292,7 +1292,9 @@ int gip_batch_create(gip_ctx *c, int32_t ninst, const gip_cavity *const *cavs, c
         int64_t nr = 0;
         assemble(b, cavs, k, rp, cl, vl, nr);
         const int32_t ncols = kCols[k] == COLS_FACES ? (int32_t)b->FP : (int32_t)b->ALLB;
-        const int32_t flags = (k == OP_L && b->o.precision == GIP_PCG_MIXED) ? GIP_MAT_FP32 : 0;
+        // the PCG's kernels and captured products read the stored values
+        const int32_t flags = ((k == OP_L && b->o.precision == GIP_PCG_MIXED) ? GIP_MAT_FP32 : 0) |
+                              (k == OP_L || b->o.use_graph ? GIP_MAT_NO_DICT : 0);
         if (b->o.autotune && k != OP_L) {
             rc = gip_mat_autotune(c, (int32_t)nr, ncols, (int32_t)vl.size(), rp.data(), cl.data(), vl.data(), flags, tx,
                                   ty, 5, &b->op[k], nullptr);
@@ -1303,7 +1305,7 @@ int gip_batch_create(gip_ctx *c, int32_t ninst, const gip_cavity *const *cavs, c
         if (!rc && k == OP_D) {
             // C takes D's pattern (GIP_DNS.h:150-151); its values are rebuilt each step
             rc = gip_mat_create(c, (int32_t)nr, ncols, (int32_t)vl.size(), rp.data(), cl.data(), vl.data(),
-                                GIP_FMT_AUTO, &b->C);
+                                GIP_FMT_AUTO | GIP_MAT_NO_DICT, &b->C);
         }
         if (!rc && k == OP_L) {
             // Jacobi inverse, zero on the padding rows (GIP_MatrixMulticore.cpp:177-210)

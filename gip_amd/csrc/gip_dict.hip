@@ -423,7 +423,7 @@ static bool dict_arrays(gip_mat *A, int nd) {
     get(&A->d_dict_tab, (size_t)nd * 8);
     get(&A->d_dict_soa, (size_t)nd * A->st_w);
     get(&A->d_dict_diag, (size_t)nd);
-    if (A->d_ell_val32) {
+    if (A->d_ell_val32 && A->st_w >= kDictLineW && A->nrows >= kDictMinRows32) {
         get(&A->d_dict_tab32, (size_t)nd * 8);
         get(&A->d_dict_soa32, (size_t)nd * A->st_w);
     }
@@ -437,8 +437,12 @@ static bool dict_arrays(gip_mat *A, int nd) {
 int mat_dict_build(gip_ctx *c, gip_mat *A, void *scratch, size_t bytes) {
     A->dict_n = 0;
     const int n = A->nrows, w = A->st_w;
+    // products of 1 and 5 slots have no dictionary kernels (spmv_launch)
     if (A->format != GIP_FMT_STENCIL || n < kDictMinRows || n > kDictMaxRows || A->cols_needed > kDictMaxRows ||
-        w < 1 || w > kStencilMaxW) return GIP_OK;
+        w < 2 || w > kStencilMaxW || w == 5 || A->no_dict || A->vals_captured) {
+        mat_dict_free(A);
+        return GIP_OK;
+    }
     hipStream_t st = c->stream;
     DictTable T{};
     T.cap = std::min(n / kDictRatio, kDictMax);

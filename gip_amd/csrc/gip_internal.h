@@ -129,6 +129,7 @@ struct gip_mat {
     // row's slot values and diagonal, dict_n of them (0: none), current while
     // dict_version == val_version + 1
     int32_t dict_n, dict_room;  // dict_room: tuples the arrays have room for
+    bool no_dict;        // GIP_MAT_NO_DICT
     bool vals_captured;  // a captured graph may change the values unseen: no form made from them is used any more
     uint64_t dict_version;
     gip::DictRec *d_dict_rec;  // per slice: which tuples its rows hold

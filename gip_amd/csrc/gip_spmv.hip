@@ -530,6 +530,7 @@ int gip_mat_create(gip_ctx *c, int32_t nrows, int32_t ncols, int32_t nnz, const 
     A->lanes = 1;
     const int32_t want = flags & 0xff;
     const bool fp32 = (flags & GIP_MAT_FP32) != 0;
+    A->no_dict = (flags & GIP_MAT_NO_DICT) != 0;
 
     // diagonal value per row (last diagonal entry wins, GIP_MatrixMulticore.cpp:191-204)
     std::vector<double> diag((size_t)nrows, 0.0);
@@ -1048,7 +1049,9 @@ static int build_transpose(gip_ctx *c, gip_mat *A) {
         }
     std::vector<double> zeros((size_t)A->nnz, 0.0);
     gip_mat *T = nullptr;
-    int rc = gip_mat_create(c, nc, A->nrows, A->nnz, trp.data(), tcl.data(), zeros.data(), GIP_FMT_AUTO, &T);
+    // its values come from A's before each product: no dictionary
+    int rc = gip_mat_create(c, nc, A->nrows, A->nnz, trp.data(), tcl.data(), zeros.data(),
+                            GIP_FMT_AUTO | GIP_MAT_NO_DICT, &T);
     if (rc) return rc;
     std::vector<int32_t> tdst((size_t)A->nnz);
     if ((T->format == GIP_FMT_ELL || T->format == GIP_FMT_STENCIL) && A->nnz) {

@@ -21,6 +21,7 @@ MAT_ELL_SLICE32 = 1 << 9
 MAT_ELL_SLICE128 = 1 << 10
 ELL_SLICE_FLAGS = {32: MAT_ELL_SLICE32, 64: 0, 128: MAT_ELL_SLICE128}
 MAT_NO_SYM = 1 << 11
+MAT_NO_DICT = 1 << 12
 SYM_STATES = {0: "none", 1: "in use", -1: "not symmetric", 2: "not made"}
 PCG_FP64, PCG_MIXED = 0, 1
 OK, EINVAL, EHIP, ENOMEM, EBREAKDOWN, ENOCONV = 0, -1, -2, -3, -4, -5
@@ -200,7 +201,7 @@ class Matrix:
     """A device operator built from host CSR arrays (int32 rowptr/col, float64 val)."""
 
     def __init__(self, dev: Device, rowptr, col, val, nrows=None, ncols=0, fmt=FMT_AUTO, fp32=False, slice=64,
-                 sym=True):
+                 sym=True, dictionary=True):
         self.dev = dev
         rowptr = np.ascontiguousarray(rowptr, dtype=np.int32)
         col = np.ascontiguousarray(col, dtype=np.int32)
@@ -211,6 +212,7 @@ class Matrix:
         if slice not in ELL_SLICE_FLAGS:
             raise ValueError("slice: rows per ELL slice, 32, 64 or 128")
         flags = fmt | (MAT_FP32 if fp32 else 0) | ELL_SLICE_FLAGS[slice] | (0 if sym else MAT_NO_SYM)
+        flags |= 0 if dictionary else MAT_NO_DICT
         check(lib().gip_mat_create(dev.ctx, self.nrows, int(ncols), self.nnz, rowptr.ctypes.data, col.ctypes.data,
                                    val.ctypes.data, flags, byref(self.ptr)))
         dev._adopt(self)

@@ -111,6 +111,10 @@ enum { GIP_MAT_ELL_SLICE32 = 1 << 9, GIP_MAT_ELL_SLICE128 = 1 << 10 };
  * instead, and no arrays are made for its solves.
  * GIP_MAT_NO_SYM turns this off. */
 enum { GIP_MAT_NO_SYM = 1 << 11 };
+/* No dictionary of the slot values (gip_mat_dict_state): for an operator
+ * whose values only products change (gip_dcsrmv_vals*), or whose products are
+ * only captured, neither of which reads one. */
+enum { GIP_MAT_NO_DICT = 1 << 12 };
 int gip_mat_create(gip_ctx *ctx, int32_t nrows, int32_t ncols, int32_t nnz, const int32_t *rowptr, const int32_t *col,
                    const double *val, int32_t flags, gip_mat **A);
 int gip_mat_destroy(gip_mat *A);

@@ -7,6 +7,8 @@ and end in a partial slice, for the operators of every shape, after changes
 of the values (made again, one value off, no repetition left, rebuilt on the
 device), and in FP32.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -237,8 +239,6 @@ def test_uniform_meshes_have_one(dev, shape, state):
 def test_setting_values_costs_little_more_with_a_dictionary(dev, shape):
     """Making the dictionary anew adds 0.1 to 0.2 ms to gip_mat_set_values here (with every row at the table for
     itself, and memory allocated for it, 1.1 and 2.8), beside the same values in a layout without one."""
-    import time
-
     c = cavity.generate(*shape, gamma=1e-3, ops=cavity.OP_BITS["L"])
     L = c.op("L")
     A, E = hip.Matrix.from_csr(dev, L), hip.Matrix.from_csr(dev, L, fmt=hip.FMT_ELL)
@@ -295,3 +295,49 @@ def test_fp32_products_that_fit_the_caches_read_the_stored_values(dev, shape, fp
     A = hip.Matrix.from_csr(dev, c.op("L"), fp32=True)
     assert A.dict_state()[0] != 0 and (A.dict_state(fp32=True)[0] != 0) == fp32
     _products(dev, A, hip.Matrix.from_csr(dev, c.op("L"), fmt=hip.FMT_CSR, fp32=True), 14, fp32=True)
+
+
+def test_no_dictionary_where_nothing_reads_one(dev):
+    """Turned off; five slots, which have no kernel for it; values that a captured graph may change, set again."""
+    c = cavity.generate(72, gamma=1e-3, ops=cavity.OP_BITS["L"])
+    L = c.op("L")
+    A, D = hip.Matrix.from_csr(dev, L, dictionary=False), hip.Matrix.from_csr(dev, L)
+    assert A.dict_state() == (0, 0, 0) and D.dict_state()[0] != 0
+    _products(dev, A, D, 15)
+    A.set_values(L.val)
+    assert A.dict_state() == (0, 0, 0)
+    n = 2 ** 18 + 64
+    rowptr, col, val, _, _ = band(n, np.tile(np.arange(1.0, 6.0), (n, 1)), (-64, -1, 0, 1, 64))
+    A = hip.Matrix(dev, rowptr, col, val, nrows=n, ncols=n, fmt=hip.FMT_STENCIL)
+    assert A.info()["format"] == hip.FMT_STENCIL and A.dict_state() == (0, 0, 0)
+    torch = pytest.importorskip("torch")
+    nnz = L.val.size
+    ident = hip.Matrix(dev, np.arange(nnz + 1), np.arange(nnz), np.ones(nnz), ncols=nnz, fmt=hip.FMT_CSR)
+    dv, change = dev.to_device(2.0 * L.val), torch.cuda.CUDAGraph()
+    stream = torch.cuda.ExternalStream(hip.lib().gip_stream(dev.ctx))
+    with torch.cuda.graph(change, stream=stream, capture_error_mode="thread_local"):
+        ident.spmv_vals(dv, D)
+    D.set_values(L.val)
+    assert D.dict_state() == (0, 0, 0)
+
+
+def test_a_batch_makes_none_for_captured_steps(dev):
+    """The operators of a batch whose steps are captured take no dictionary's memory (here about 3.5 bytes a row
+    more without the graph, over at least ten operators of 2^19 rows and more)."""
+    torch = pytest.importorskip("torch")
+    from gip_amd import batch
+
+    cavs = [cavity.generate(64, gamma=1e-2) for _ in range(4)]
+    used = []
+    for graph in (False, True, False, True):
+        dev.sync()
+        free = torch.cuda.mem_get_info()[0]
+        b = batch.Batch(dev, cavs, [1e-2] * 4, pcg_tol=1e-6, use_graph=graph)
+        used.append(free - torch.cuda.mem_get_info()[0])
+        b.close()
+        for _ in range(40):  # the driver may count freed memory a little later
+            if free - torch.cuda.mem_get_info()[0] < 4 << 20:
+                break
+            time.sleep(0.05)
+    print(f"[batch memory] without and with a graph {used}", flush=True)
+    assert min(used[0::2]) - max(used[1::2]) > 10 * 3 * 2 ** 19
