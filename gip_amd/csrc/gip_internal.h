@@ -140,7 +140,6 @@ struct gip_mat {
     double *d_dict_tab, *d_dict_soa, *d_dict_diag;  // tuples, 8 per row of the table; slot by slot; a_ii
     float *d_dict_tab32, *d_dict_soa32;
     int32_t *h_dict;  // pinned: the build's counters
-    int32_t st_empty;  // stencil layout: some row has no entries
     // a_ii per row (the stored values of a DIAG operator), for Jacobi; for
     // the other layouts refreshed from d_diag_src (each row's last diagonal
     // entry's position in the value storage, -1 for none) when values change

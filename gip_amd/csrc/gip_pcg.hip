@@ -470,15 +470,13 @@ template <int SW, int R>
 __global__ __launch_bounds__(kBlock) void k_iter_spmv_dict(EllView A, PcgDev d, const double *__restrict__ p) {
     __shared__ double sh[4 * R][1];
     const int st = state_load(d.state);
-    dict_rows<R, SW, double, double>(
-        A, A.val, d.n, p, [](int) { return 0; },
-        [&](int row, bool ok, bool any, double sum, double own, int) {
-            if (st != ST_RUN) return;
-            if (ok && any) d.Ap[row] = sum;
-            if (ok && !any) sum = d.Ap[row];  // empty row: Ap keeps its value
-            const double acc = wave_sum_63(ok ? own * sum : 0.0);
-            if ((threadIdx.x & 63) == 63) sh[(row >> 6) & (4 * R - 1)][0] = acc;
-        });
+    dict_rows<true, R, SW, double, double>(A, A.val, d.n, p, [&](int row, bool ok, bool any, double sum, double own) {
+        if (st != ST_RUN) return;
+        if (ok && any) d.Ap[row] = sum;
+        if (ok && !any) sum = d.Ap[row];  // empty row: Ap keeps its value
+        const double acc = wave_sum_63(ok ? own * sum : 0.0);
+        if ((threadIdx.x & 63) == 63) sh[(row >> 6) & (4 * R - 1)][0] = acc;
+    });
     if (st != ST_RUN) return;
     chunk_store<R, 1>(d, sh);
 }
@@ -1181,14 +1179,12 @@ __global__ __launch_bounds__(kBlock) void k_m_spmv_small(EllView A, PcgDev d) {
 template <int SW, int R>
 __global__ __launch_bounds__(kBlock) void k_m_spmv_dict(EllView A, PcgDev d, const float *__restrict__ p) {
     __shared__ double sh[4 * R][2];
-    dict_rows<R, SW, float, float>(
-        A, A.val32, d.n, p, [](int) { return 0; },
-        [&](int row, bool ok, bool, float sum, float own, int) {
-            if (ok) d.Ap32[row] = sum;
-            const int lane = threadIdx.x & 63;
-            const double acc = wave_sum_two(ok ? (double)own * (double)sum : 0.0, ok ? (double)sum : 0.0);
-            if ((lane & 31) == 31) sh[(row >> 6) & (4 * R - 1)][lane >> 5] = acc;
-        });
+    dict_rows<true, R, SW, float, float>(A, A.val32, d.n, p, [&](int row, bool ok, bool, float sum, float own) {
+        if (ok) d.Ap32[row] = sum;
+        const int lane = threadIdx.x & 63;
+        const double acc = wave_sum_two(ok ? (double)own * (double)sum : 0.0, ok ? (double)sum : 0.0);
+        if ((lane & 31) == 31) sh[(row >> 6) & (4 * R - 1)][lane >> 5] = acc;
+    });
     chunk_store<R, 2>(d, sh);
 }
 

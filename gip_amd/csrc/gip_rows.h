@@ -397,11 +397,11 @@ __device__ inline bool dict_row_slow(const EllView &A, const V *__restrict__ val
 }
 
 // Row sums with the slot values from the dictionary, R 256-row chunks per
-// workgroup: the stored values, bit for bit, in the stored order.  pre(row)
-// issues a row's other loads; use(row, ok, any, sum, own, what pre returned)
-// takes the sum, called by whole wavefronts for every slice of every chunk,
-// a thread's rows in ascending order (ok: the row exists; any: it is not
-// empty; own: the operand at the row's own column).
+// workgroup: the stored values, bit for bit, in the stored order.
+// use(row, ok, any, sum, own) takes a row's sum, called by whole wavefronts
+// for every slice of every chunk, a thread's rows in ascending order (ok: the
+// row exists; any: it is not empty; own: with OWN, the operand at the row's
+// own column, which a vector shorter than the rows may not have).
 //
 // With the slot values gone a product is bound by the bytes it keeps in
 // flight, so a wavefront takes R slices at once: their 64-byte records in
@@ -424,12 +424,11 @@ __device__ inline int dict_block(int b, int G) {
     return c < G ? c : c - G;
 }
 
-template <bool LINE, bool TUPLES, int R, int SW, class T, class V, class PRE, class USE>
+template <bool OWN, bool LINE, bool TUPLES, int R, int SW, class T, class V, class USE>
 __device__ inline void dict_rows_fast(const EllView &A, const V *__restrict__ val, const T *__restrict__ x,
-                                      const DictRec (&r)[R], const int (&ids)[R], int s0, int lane, const PRE &pre,
+                                      const DictRec (&r)[R], const int (&ids)[R], int s0, int lane,
                                       const USE &use) {
     DictX<SW, T, V> q[R];
-    decltype(pre(0)) p[R];
     V v[TUPLES ? 1 : R][SW];
 #pragma unroll
     for (int u = 0; u < R; ++u) {
@@ -442,7 +441,6 @@ __device__ inline void dict_rows_fast(const EllView &A, const V *__restrict__ va
                 v[u % (TUPLES ? 1 : R)][k] =
                     at_byte(dict_soa(A, V(0)) + (size_t)k * A.dc_n, (uint32_t)id * (uint32_t)sizeof(V));
         }
-        p[u] = pre(row);
     }
 #pragma unroll
     for (int u = 0; u < R; ++u) dict_x_loaded<LINE, !TUPLES, SW, T, V>(q[u]);
@@ -468,13 +466,13 @@ __device__ inline void dict_rows_fast(const EllView &A, const V *__restrict__ va
             for (int k = 0; k < SW; ++k) sum = sum + q[u].x[k] * v[u % (TUPLES ? 1 : R)][k];
         }
         sum = dict_tail<!TUPLES, SW, T, V>(x, r[u], q[u], lane, sum);
-        use(row, true, true, sum, LINE ? q[u].x[3 % SW] : x[row], p[u]);
+        use(row, true, true, sum, !OWN ? T(0) : LINE ? q[u].x[3 % SW] : x[row]);
     }
 }
 
-template <int R, int SW, class T, class V, class PRE, class USE>
+template <bool OWN, int R, int SW, class T, class V, class USE>
 __device__ inline void dict_rows(const EllView &A, const V *__restrict__ val, int nrows, const T *__restrict__ x,
-                                 const PRE &pre, const USE &use) {
+                                 const USE &use) {
     const int ns = (nrows + 63) >> 6, lane = threadIdx.x & 63;
     const int s0 =
         (dict_block(blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * R;
@@ -507,11 +505,11 @@ __device__ inline void dict_rows(const EllView &A, const V *__restrict__ val, in
     }
     if (SW >= kDictLineW && (all & kDictLine)) {
         if (least >= 0)
-            dict_rows_fast<true, true, R, SW, T, V>(A, val, x, r, id, s0, lane, pre, use);
+            dict_rows_fast<OWN, true, true, R, SW, T, V>(A, val, x, r, id, s0, lane, use);
         else
-            dict_rows_fast<true, false, R, SW, T, V>(A, val, x, r, id, s0, lane, pre, use);
+            dict_rows_fast<OWN, true, false, R, SW, T, V>(A, val, x, r, id, s0, lane, use);
     } else if (all & kDictFast) {
-        dict_rows_fast<false, false, R, SW, T, V>(A, val, x, r, id, s0, lane, pre, use);
+        dict_rows_fast<OWN, false, false, R, SW, T, V>(A, val, x, r, id, s0, lane, use);
     } else {
 #pragma unroll 1
         for (int u = 0; u < R; ++u) {
@@ -520,13 +518,11 @@ __device__ inline void dict_rows(const EllView &A, const V *__restrict__ val, in
             if (s >= nw) return;
             T sum = T(0), own = T(0);
             bool any = false;
-            decltype(pre(0)) p{};
             if (ok) {
-                p = pre(row);
-                own = x[row];
+                if (OWN) own = x[row];
                 any = dict_row_slow<SW, T, V>(A, val, x, dict_rec(A, s), s, row, sum);
             }
-            use(row, ok, any, sum, own, p);
+            use(row, ok, any, sum, own);
         }
     }
 }

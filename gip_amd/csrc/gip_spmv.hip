@@ -90,15 +90,11 @@ __global__ __launch_bounds__(kBlock) void k_stencil(EllView A, int nrows, const 
 }
 
 // The same products with the slot values from the dictionary.
-struct NoLoads {
-    __device__ int operator()(int) const { return 0; }
-};
-
 template <int MODE, int SW, int R>
 __global__ __launch_bounds__(kBlock) void k_stencil_dict(EllView A, int nrows, const double *__restrict__ x,
                                                         double *__restrict__ y, double a, double b,
                                                         const int32_t *__restrict__ scatter) {
-    dict_rows<R, SW, double, double>(A, A.val, nrows, x, NoLoads{}, [&](int row, bool ok, bool any, double sum, double, int) {
+    dict_rows<false, R, SW, double, double>(A, A.val, nrows, x, [&](int row, bool ok, bool any, double sum, double) {
         if (!ok || !any) return;
         const int out = scatter ? scatter[row] : row;
         if (MODE == 0)
@@ -111,10 +107,9 @@ __global__ __launch_bounds__(kBlock) void k_stencil_dict(EllView A, int nrows, c
 template <int SW, int R>
 __global__ __launch_bounds__(kBlock) void k_stencil32_dict(EllView A, int nrows, const float *__restrict__ x,
                                                           float *__restrict__ y) {
-    dict_rows<R, SW, float, float>(A, A.val32, nrows, x, NoLoads{},
-                                        [&](int row, bool ok, bool any, float sum, float, int) {
-                                            if (ok) y[row] = any ? sum : 0.0f;
-                                        });
+    dict_rows<false, R, SW, float, float>(A, A.val32, nrows, x, [&](int row, bool ok, bool any, float sum, float) {
+        if (ok) y[row] = any ? sum : 0.0f;
+    });
 }
 
 template <int W>
@@ -649,8 +644,6 @@ int gip_mat_create(gip_ctx *c, int32_t nrows, int32_t ncols, int32_t nnz, const 
         A->st_w = plan.w;
         A->st_tail_base = plan.tail_base;
         A->st_tail_nnz = (int32_t)plan.tcol.size();
-        for (const StencilHdr &h : plan.hdr)
-            if (h.empty) A->st_empty = 1;
         std::vector<double> sval((size_t)plan.stored, 0.0);
         for (int32_t j = 0; j < nnz; ++j) sval[(size_t)plan.pos[(size_t)j]] = val[j];
         rc = upload(c, &A->d_ell_val, sval.data(), sval.size());

@@ -341,3 +341,19 @@ def test_a_batch_makes_none_for_captured_steps(dev):
             time.sleep(0.05)
     print(f"[batch memory] without and with a graph {used}", flush=True)
     assert min(used[0::2]) - max(used[1::2]) > 10 * 3 * 2 ** 19
+
+
+@pytest.mark.parametrize("slots", [2, 7])
+@pytest.mark.parametrize("m", [2 ** 17 + 32, 2 ** 17 + 37])
+def test_more_rows_than_columns(dev, m, slots):
+    """Twice as many rows as columns: a row past the vector's end has no operand of its own."""
+    n, rng = 2 * m, np.random.default_rng(16)
+    r = np.arange(n)
+    col = (r % m)[:, None] + np.arange(slots)[None, :]
+    inside = col < m
+    rowptr = np.concatenate([[0], np.cumsum(inside.sum(1))])
+    val = np.broadcast_to(rng.standard_normal(slots), (n, slots))[inside]
+    A = hip.Matrix(dev, rowptr, col[inside], val, nrows=n, ncols=m, fmt=hip.FMT_STENCIL, fp32=True)
+    C = hip.Matrix(dev, rowptr, col[inside], val, nrows=n, ncols=m, fmt=hip.FMT_CSR, fp32=True)
+    assert A.cols_needed == m and A.info()["format"] == hip.FMT_STENCIL and A.dict_state()[0] != 0
+    _products(dev, A, C, 17, fp32=True)
