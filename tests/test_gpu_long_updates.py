@@ -132,3 +132,75 @@ def test_mid_size_forms(dev, shape, beta):
                     assert np.linalg.norm(x - want[maxit]) <= 1e-12 * np.linalg.norm(want[maxit]), (fmt, maxit)
                 assert np.array_equal(first.setdefault((maxit, precision), x), x), (fmt, maxit, precision)
         del solver, A
+
+
+def _band(n, kinds):
+    """A shifted 7-diagonal Laplacian, scaled symmetrically by `kinds` factors in turn: as many tuples and the few
+    of its ends; more than two tuples in a slice from three factors on."""
+    s = 1.0 + 0.05 * (np.arange(n) % kinds)
+    diags = [-(s[k:] * s[:n - k]) for k in (9, 3, 1)]
+    T = sp.diags(diags + [6.15 * s * s] + diags[::-1], [-9, -3, -1, 0, 1, 3, 9], shape=(n, n)).tocsr()
+    T.sort_indices()
+    return T
+
+
+# The long iterations with the dictionary and without: s formed again from r
+# (FP64, and FP32 where no slice needs ids) or stored, ids or scalar tuples.
+@pytest.mark.parametrize("dictionary,kinds", [(True, 1), (True, 5), (False, 5)])
+@pytest.mark.parametrize("n", [2 ** 19 + 300, 2 ** 21 + 1, 2 ** 23 + 65])
+def test_x_holds_every_update_with_the_dictionary(dev, n, dictionary, kinds):
+    rng = np.random.default_rng(n)
+    T = _band(n, kinds)
+    b, x0 = rng.standard_normal(n), 0.1 * rng.standard_normal(n)
+    orc = pyoracle.Csr(T.indptr, T.indices, T.data, n)
+    M = hip.Matrix(dev, T.indptr, T.indices, T.data, ncols=n, fp32=True, dictionary=dictionary)
+    # the two end slices hold more tuples than two whatever the factors
+    assert M.info()["format"] == hip.FMT_STENCIL and (M.dict_state()[0] != 0) == dictionary
+    assert not dictionary or M.dict_state()[1] <= 40
+    solver = hip.PCG(M, n)
+    db, dx0, dx = dev.to_device(b), dev.to_device(x0), dev.array(n)
+    for maxit in (1, 2, 3, 4):
+        for precond in (True, False):
+            r = solver.solve(db, dx, dx0, maxit=maxit, precond=precond)
+            assert r.iters == maxit and r.status == 0
+            if precond:
+                want, st, it, rel = pyoracle.pcg(orc, b, x0, n, maxit)
+                assert np.linalg.norm(dx.download() - want) <= 1e-12 * np.linalg.norm(want), maxit
+    for tol in (0.2, 0.1, 0.05):
+        r = solver.solve(db, dx, dx0, maxit=100, tol=tol, poll=3)
+        want, st, it, rel = pyoracle.pcg(orc, b, x0, n, 100, tol=tol)
+        assert r.iters == it and r.status == 0
+        assert np.linalg.norm(dx.download() - want) <= 1e-12 * np.linalg.norm(want), tol
+    for poll in (1, 2, 3):
+        r = solver.solve(db, dx, dx0, maxit=200, tol=1e-10, precision=hip.PCG_MIXED, poll=poll)
+        x = dx.download()
+        assert r.status == 0 and np.linalg.norm(b - T @ x) <= 1.01e-10 * np.linalg.norm(b)
+
+
+# Exact breakdowns: with the eigenvalue 2 (Jacobi: 1) the first iteration, with
+# 1 and 3 in equal numbers the second leaves r = 0 to the last bit, so the one
+# after stops at p.Ap = 0, an odd and an even number of iterations done (every
+# sum is one of multiples of 1/16 below 2^24: exact in any order).
+@pytest.mark.parametrize("form", ["dictionary", "stencil", "ell", "csr"])
+@pytest.mark.parametrize("n", [2 ** 19 + 64, 2 ** 21 + 64, 2 ** 23 + 64])
+@pytest.mark.parametrize("iters", [1, 2])
+def test_breakdown_after_an_odd_and_an_even_iteration(dev, n, form, iters):
+    diag = np.full(n, 2.0) if iters == 1 else np.where(np.arange(n) % 2, 3.0, 1.0)
+    col = np.arange(n)[:, None] + np.array([-9, -3, -1, 0, 1, 3, 9])[None, :]
+    inside = (col >= 0) & (col < n)
+    val = np.zeros((n, 7))
+    val[:, 3] = diag
+    rowptr = np.concatenate([[0], np.cumsum(inside.sum(1))])
+    M = hip.Matrix(dev, rowptr, col[inside], val[inside], ncols=n, dictionary=form == "dictionary",
+                   fmt={"ell": hip.FMT_ELL, "csr": hip.FMT_CSR}.get(form, hip.FMT_STENCIL))
+    assert (M.dict_state()[0] != 0) == (form == "dictionary")
+    solver = hip.PCG(M, n)
+    dx = dev.array(n)
+    for tol, poll in ((0.0, 16), (1e-300, 1), (1e-300, 16)):
+        r = solver.solve(dev.to_device(np.ones(n)), dx, dev.to_device(np.zeros(n)), maxit=50, tol=tol, poll=poll,
+                         precond=iters == 1, raise_on_breakdown=False)
+        if tol:  # r.r = 0 meets any tolerance: no breakdown, the same x
+            assert r.status == hip.OK and r.iters == iters
+        else:
+            assert r.status == hip.EBREAKDOWN and r.iters == iters
+        assert np.abs(dx.download() * diag - 1.0).max() <= 2e-16 * (iters - 1)

@@ -184,3 +184,31 @@ def test_no_arrays_beside_a_dictionary(dev):
     assert A.sym_state()[0] == 2
     assert grown(solve, little)
     symmetric()
+
+
+@pytest.mark.parametrize("beta", [0.0, 1.5])
+@pytest.mark.parametrize("shape", [(96, 96, 96), (128, 128, 64), (128, 128, 128), (113, 128, 150), (144, 128, 128),
+                                   (256, 256, 129), (208, 200, 208)], ids=lambda s: "x".join(map(str, s)))
+def test_the_form_itself_bitwise(dev, shape, beta):
+    """Operators without a dictionary, whose FP64 products do read the form: 7 and 8 slots, workgroups of 512, 1024
+    and 256 rows, and the row-per-thread iteration past 2^23 rows."""
+    c, L, b = _case(*shape, beta=beta)
+    A, F = _pair(dev, L, dictionary=False)
+    for kw in (dict(maxit=15), dict(maxit=400, tol=1e-2)):
+        ra, xa = _solve(dev, A, c, b, **kw)
+        rf, xf = _solve(dev, F, c, b, **kw)
+        assert A.dict_state()[0] == 0 and A.sym_state()[0] == 1 and F.sym_state()[0] == 0
+        print(f"[sym form {shape} beta {beta}] iters {ra.iters}", flush=True)
+        assert ra.iters == rf.iters and ra.relres == rf.relres
+        assert np.array_equal(xa, xf)
+    # one value off by one unit in the last place: the full product, not the form
+    v = L.val.copy()
+    r0 = L.nrows // 2 + 3
+    j = [j for j in range(L.rowptr[r0], L.rowptr[r0 + 1]) if r0 < L.col[j] < L.nrows][0]
+    v[j] = np.nextafter(v[j], 0.0)
+    A.set_values(v)
+    F.set_values(v)
+    ra, xa = _solve(dev, A, c, b, maxit=15)
+    rf, xf = _solve(dev, F, c, b, maxit=15)
+    assert A.sym_state()[0] == -1
+    assert np.array_equal(xa, xf)
