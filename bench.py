@@ -330,18 +330,21 @@ def main():
     # input once, the output once): no column index per entry, so fewer
     # than the CSR count
     lay64, lay32 = A.product_bytes(), A.product_bytes(fp32=True)
-    # the long solves (more than 2^19 rows; mixed from 2^21) multiply this
-    # uniform mesh's operator from the dictionary of its value tuples: the
-    # input and output once, a 64-byte record per 64 rows, and a 2-byte id per
-    # row where slices straddle the mesh lines.  With it s = Dinv r is not
-    # stored (mixed: where no ids are read), and x is updated every second
-    # iteration: 7.5 vector streams beside the product instead of 11
-    dict64, dict32, ids = N > 1 << 19, N >= 1 << 21, n % 64 != 0
-    spmv64 = 16 * N + N + (2 * N if ids else 0) if N >= 1 << 18 else lay64
-    own64 = spmv64 if dict64 else lay64
-    spmv32 = 8 * N + N + (2 * N if ids else 0) if N >= 1 << 18 else lay32
+    # the long solves (more than 2^19 rows; mixed from 2^21) multiply an
+    # operator that has a dictionary of its value tuples, as a uniform mesh's
+    # has, from that; else the FP64 ones from the symmetric form
+    state64, _, spmv64 = A.dict_state()
+    state32, _, spmv32 = A.dict_state(fp32=True)
+    spmv64, spmv32 = spmv64 if state64 else lay64, spmv32 if state32 else lay32
+    long64, dict64, dict32 = N > 1 << 19, N > 1 << 19 and state64 != 0, N >= 1 << 21 and state32 != 0
+    sym_state, sym64 = (0, 0) if dict64 or not long64 else A.sym_state()
+    own64 = spmv64 if dict64 else sym64 if sym_state == 1 else lay64
     own32 = spmv32 if dict32 else lay32
-    streams64, streams32 = (60 if dict64 else 88) * N, (30 if dict32 and not ids else 44) * N
+    # vector streams beside the product: 11; long iterations update x every
+    # second time (9.5), and with the dictionary do not store s = Dinv r
+    # (mixed: where no slice needs its rows' ids), 7.5
+    streams64 = int(8 * N * (7.5 if dict64 else 9.5 if long64 else 11))
+    streams32 = int(4 * N * (7.5 if dict32 and state32 == 1 else 9.5 if long64 else 11))
     for leg, byts, lay in ((fp64, it_fp64, own64 + streams64), (mixed, it_mixed, own32 + streams32)):
         ms_it = leg["ms"] / max(1, leg["iters"])
         leg["ms_per_iter"] = ms_it
@@ -391,7 +394,10 @@ def main():
     if info["nrows"] <= 1 << 19:
         k64, k32, form = "k_iter_dirprod", "k_m_dirprod", "stencil layout"
     else:
-        k64, k32, form = "k_iter_spmv_dict", "k_m_spmv_dict" if dict32 else "k_m_spmv<", "dictionary of the slot values"
+        k64, form = (("k_iter_spmv_dict", "dictionary of the slot values") if dict64 else
+                     ("k_iter_spmv_sym", "symmetric form of the stencil layout") if sym_state == 1 else
+                     ("k_iter_spmv<", "stencil layout"))
+        k32 = "k_m_spmv_dict" if dict32 else "k_m_spmv"
     ceiling = stream_ceiling()
     ach64 = own64 / (us64 * 1e-6) / 1e9
     traffic64 = measured_traffic(n, k64)
@@ -459,7 +465,8 @@ def summarize_pmc(fetch_dir, write_dir, kernels):
     """Per-dispatch HBM traffic of each named kernel from two rocprofv3 --pmc
     runs of `--probe spmv` (FETCH_SIZE, then WRITE_SIZE; counter CSVs under
     the two directories), scaled by what the same counters read for k_copy
-    (2^27 doubles read and written per launch).  Returns
+    (2^27 doubles read and written per launch).  A kernel counts for the
+    longest key that its name holds.  Returns
     {kernel: {"fetch_kib", "write_kib", "bytes"}} (medians over dispatches)
     and the two scale factors."""
     import csv
@@ -476,8 +483,10 @@ def summarize_pmc(fetch_dir, write_dir, kernels):
 
     fet, wri = load(fetch_dir, "FETCH_SIZE"), load(write_dir, "WRITE_SIZE")
 
+    keys = ("k_copy",) + tuple(kernels)
+
     def med(d, key):
-        hits = [v for k, vs in d.items() if key in k for v in vs]
+        hits = [v for k, vs in d.items() if max((c for c in keys if c in k), key=len, default=None) == key for v in vs]
         return float(np.median(hits)) if hits else None
 
     copy_bytes = 8 * (1 << 27)
@@ -493,11 +502,16 @@ def summarize_pmc(fetch_dir, write_dir, kernels):
 
 
 # kernel-name keys (substrings of the profiled names; "k_iter_dir(" is the
-# four-launch form's direction sweep, not k_iter_dir_rows)
-PCG_KERNELS = ("k_iter_dir_rows", "k_iter_dir(", "k_iter_spmv<", "k_iter_spmv_dict", "k_iter_spmv_sym", "k_m_spmv_dict",
-               "k_stencil_dict", "k_fold_two", "k_alpha_fin",
-               "k_iter_update_rows",
-               "k_iter_update_grid", "k_beta_fin", "k_m_dir", "k_m_spmv", "k_fold_dn", "k_m_update", "k_stencil<0")
+# four-launch form's direction sweep, not k_iter_dir_rows); the sweeps by
+# their arguments: s formed from r or stored and, of the direction sweeps,
+# whether the x updates of two iterations are made (twice the streams)
+PCG_KERNELS = tuple(f"{k}<{lean}, {pair}" for k in ("k_iter_dir_rows", "k_iter_dir", "k_m_dir")
+                    for lean in ("true", "false") for pair in ("true", "false"))
+PCG_KERNELS += tuple(f"{k}<{lean}" for k in ("k_iter_update_rows", "k_iter_update_grid", "k_m_update")
+                     for lean in ("true", "false"))
+PCG_KERNELS += ("k_iter_dir_rows", "k_iter_dir(", "k_iter_spmv<", "k_iter_spmv_dict", "k_iter_spmv_sym",
+                "k_m_spmv_dict", "k_m_spmv", "k_stencil_dict", "k_stencil<0", "k_fold_two", "k_alpha_fin",
+                "k_beta_fin", "k_fold_dn", "k_fold_wide")
 
 
 def summary_traffic(args):
@@ -509,7 +523,7 @@ def summary_traffic(args):
     lines = [
         f"# HBM traffic per launch of the {n}^3 PCG kernels (rocprofv3 PMC: TCC FETCH_SIZE and WRITE_SIZE in KiB per",
         "# dispatch, median over the dispatches of `bench.py --probe spmv`: 5 standalone FP64 products, 8",
-        "# iterations of the FP64 PCG, 8 of the mixed PCG, 5 copies",
+        "# iterations of the FP64 PCG, 8 of the mixed PCG, 8 of each on the operator without a dictionary, 5 copies",
         "# of 2^27 doubles)",
         "#",
         "# commands (run from the repository root on one MI355X):",
@@ -652,7 +666,8 @@ def probe_stream(args):
 
 def probe_spmv(args):
     """Five FP64 SpMVs on the n^3 Laplacian, eight iterations of the FP64 and
-    of the mixed PCG on it (their in-solve products), and five copies of 2^27
+    of the mixed PCG on it (their in-solve products), the same without its
+    dictionary (the symmetric form's product among them), and five copies of 2^27
     doubles (1 GiB read + 1 GiB written each): the launches a rocprofv3 --pmc
     run counts, the copy calibrating FETCH_SIZE/WRITE_SIZE against known
     bytes."""
@@ -667,15 +682,16 @@ def probe_spmv(args):
     for _ in range(5):
         A.spmv(x, y)
     # 8 iterations of each PCG (their products: k_iter_spmv_dict and
-    # k_m_spmv_dict)
-    A32 = hip.Matrix.from_csr(dev, L, fp32=True)
-    solver = hip.PCG(A32, cav.n_all)
+    # k_m_spmv_dict), and without the dictionary (k_iter_spmv_sym, k_m_spmv)
     b = dev.to_device(np.concatenate([cavity.rhs_normal(cav.n_inner, 1), np.zeros(cav.n_all - cav.n_inner)]))
     z = dev.to_device(np.zeros(cav.n_all))
-    for prec in (hip.PCG_FP64, hip.PCG_MIXED):
-        solver.solve(b, y, z, maxit=8, tol=1e-10, precision=prec, poll=32)
-    solver.destroy()
-    A32.destroy()
+    for dictionary in (True, False):
+        M = hip.Matrix.from_csr(dev, L, fp32=True, dictionary=dictionary)
+        solver = hip.PCG(M, cav.n_all)
+        for prec in (hip.PCG_FP64, hip.PCG_MIXED):
+            solver.solve(b, y, z, maxit=8, tol=1e-10, precision=prec, poll=32)
+        solver.destroy()
+        M.destroy()
     nc = 1 << 27
     a, b = dev.array(nc), dev.array(nc)
     hip.fill(a, 1.0)

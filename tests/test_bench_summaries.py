@@ -102,3 +102,24 @@ def test_kernel_summary_totals_a_results_database(tmp_path):
     assert rows[0][-1] == "k_a" and rows[0][1] == "2" and rows[0][0] == "80.00%"
     assert float(rows[0][3]) == 4.0  # average microseconds
     assert rows[1][-1] == "k_b" and rows[1][0] == "20.00%"
+
+
+def test_traffic_keeps_the_instances_of_a_kernel_apart(tmp_path):
+    """The direction sweeps that update x and those that do not, and a kernel whose name holds another's."""
+    copy_kib = COPY_BYTES / 1024
+    names = {"void gip::k_iter_dir_rows<true, true>(gip::PcgDev)": 48.0,
+             "void gip::k_iter_dir_rows<true, false>(gip::PcgDev)": 24.0,
+             "void gip::k_iter_dir<true, true, 8>(gip::PcgDev)": 47.0,
+             "void gip::k_m_dir<false, true, 0>(gip::PcgDev)": 20.0,
+             "void gip::k_m_dir<false, false, 0>(gip::PcgDev)": 12.0,
+             "void gip::k_m_spmv<-7, 512>(gip::EllView)": 38.0,
+             "void gip::k_m_spmv_dict<7, 1>(gip::EllView)": 10.0}
+    rows = [("k_copy", copy_kib)] + [(n, v) for n, v in names.items() for _ in range(3)]
+    fetch = _pmc_dir(tmp_path, "FETCH_SIZE", rows)
+    write = _pmc_dir(tmp_path, "WRITE_SIZE", [(n, v if n == "k_copy" else 0.0) for n, v in rows])
+    res, fs, ws = bench.summarize_pmc(fetch, write, bench.PCG_KERNELS)
+    assert fs == ws == 1.0
+    got = {k: r["fetch_kib"] for k, r in res.items()}
+    assert got == {"k_iter_dir_rows<true, true": 48.0, "k_iter_dir_rows<true, false": 24.0,
+                   "k_iter_dir<true, true": 47.0, "k_m_dir<false, true": 20.0, "k_m_dir<false, false": 12.0,
+                   "k_m_spmv": 38.0, "k_m_spmv_dict": 10.0}
