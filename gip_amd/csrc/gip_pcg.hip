@@ -1853,6 +1853,8 @@ static Pub next_pub(gip_pcg *S) {
 }
 static int wait_pub(gip_pcg *S) { return wait_published(S->ctx->stream, S->h_flag, *S->seq); }
 
+constexpr int kFixedPoll = 4096;
+
 // The solve on a solver's workspace (allocated by gip_pcg_create, or the
 // no-alloc scratch); arguments already checked.
 static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *x0, const gip_pcg_opts *o,
@@ -2001,8 +2003,9 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     int corrections = 0, rc;
     // FP64 with a fixed iteration count (tol <= 0): nothing can stop the
     // solve early but a breakdown, after which every queued kernel returns
-    // at once, so all iterations are queued and the host reads the state
-    // once, at the end (every 4096 iterations on long runs)
+    // at once, so the iterations are queued and the host reads the state
+    // once, at the end (on long runs every kFixedPoll iterations: 200,000 of a
+    // small operator that breaks down at once queued 1.0 s of kernels)
     if (fixed)
         h_state(S)[0] = ST_RUN;
     else if (!mixed && (rc = wait_pub(S)))
@@ -2010,7 +2013,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
     if (!mixed) {
         int k = 0;  // iterations queued
         while (k < o->maxit && h_state(S)[0] == ST_RUN) {
-            int chunk = std::min(fixed ? 4096 : pollk, o->maxit - k);
+            int chunk = std::min(fixed ? kFixedPoll : pollk, o->maxit - k);
             for (int j = 0; j < chunk; ++j, ++k) {
                 if (S->fold && !S->rows) {
                     if (k > 0) SWEEP_DIR(k_iter_dir, k >= 2 && !(k & 1), d, pdir(k - 1), pdir(k), k);
@@ -2062,7 +2065,7 @@ static int pcg_solve_impl(gip_pcg *S, const double *b, double *x, const double *
                 }
             }
             GIP_LAUNCH_CHECK("pcg iteration");
-            if (!fixed) {
+            if (!fixed || k < o->maxit) {
                 k_publish<<<1, 64, 0, st>>>(d, next_pub(S));
                 GIP_LAUNCH_CHECK("pcg poll");
                 if ((rc = wait_pub(S))) return rc;

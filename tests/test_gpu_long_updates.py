@@ -5,6 +5,8 @@ long forms (more than 2^19 and more than 2^23 rows), with and without a
 dictionary, against the oracle; the mixed solve with corrections after one,
 two and three iterations; a breakdown in the second iteration.
 """
+import time
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -204,3 +206,29 @@ def test_breakdown_after_an_odd_and_an_even_iteration(dev, n, form, iters):
         else:
             assert r.status == hip.EBREAKDOWN and r.iters == iters
         assert np.abs(dx.download() * diag - 1.0).max() <= 2e-16 * (iters - 1)
+
+
+@pytest.mark.parametrize("n", [4096, 2 ** 19 + 64])
+def test_a_long_fixed_run_ends_soon_after_a_breakdown(dev, n):
+    """200,000 iterations, of which the first breaks down: the host reads the state every 4096."""
+    rowptr = np.arange(n + 1)
+    M = hip.Matrix(dev, rowptr, np.arange(n), np.full(n, 2.0), ncols=n, fmt=hip.FMT_CSR)
+    solver, dx = hip.PCG(M, n), dev.array(n)
+    b, z = dev.to_device(np.ones(n)), dev.to_device(np.zeros(n))
+    solver.solve(b, dx, z, maxit=2, raise_on_breakdown=False)
+    t0 = time.perf_counter()
+    r = solver.solve(b, dx, z, maxit=200000, raise_on_breakdown=False)
+    took = time.perf_counter() - t0
+    print(f"[long fixed run {n}] {1e3 * took:.1f} ms", flush=True)
+    assert r.status == hip.EBREAKDOWN and r.iters == 1
+    assert np.array_equal(dx.download(), np.full(n, 0.5))
+    assert took < 0.3
+    # and one without a breakdown runs through its reads of the state
+    L = _line(n)
+    M = hip.Matrix(dev, L.indptr, L.indices, L.data, ncols=n)
+    solver = hip.PCG(M, n)
+    c = np.random.default_rng(3).standard_normal(n)
+    r = solver.solve(dev.to_device(c), dx, z, maxit=4100, raise_on_breakdown=False)
+    if r.status == 0:
+        assert r.iters == 4100
+    assert np.linalg.norm(c - L @ dx.download()) <= 1e-12 * np.linalg.norm(c)
