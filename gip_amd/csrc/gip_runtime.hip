@@ -18,6 +18,13 @@ int hip_fail(hipError_t e, const char *what) {
                      std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// gip_sync's kernel: the host waits for its number as for a result's, so a
+// call after such a result does not drain the stream from the start (dot and
+// gip_sync 21.6 -> 18.3 us, with the stream drained by both 17.8; a kernel and
+// gip_sync 12.6 -> 10.4; a step of 46^3 in two partitions, whose halo
+// exchanges call it, 10.5 -> 7.3 ms).
+__global__ void k_seq(uint64_t *flag, uint64_t seq) { publish_seq(flag, seq); }
+
 int wait_published(hipStream_t st, const uint64_t *flag, uint64_t want) {
     if (seq_reached(flag, want)) return GIP_OK;
     // a captured kernel does not run: refused as a wait for the stream is,
@@ -114,8 +121,14 @@ int gip_use_device(int device) {
 
 int gip_sync(gip_ctx *c) {
     if (!c) return set_error(GIP_EINVAL, "null context");
-    GIP_HIP_TRY(hipStreamSynchronize(c->stream));
-    return GIP_OK;
+    uint64_t want;
+    {
+        std::lock_guard<std::mutex> lock(c->sync_mu);
+        want = ++c->sync_seq;
+        k_seq<<<1, 1, 0, c->stream>>>(reinterpret_cast<uint64_t *>(c->h_result_dev + kSyncSlot), want);
+        GIP_LAUNCH_CHECK("gip_sync");
+    }
+    return wait_published(c->stream, reinterpret_cast<const uint64_t *>(c->h_result + kSyncSlot), want);
 }
 
 void *gip_stream(gip_ctx *c) { return c ? (void *)c->stream : nullptr; }
