@@ -1370,13 +1370,13 @@ int gip_batch_step(gip_batch *b) {
         if ((rc = run_phase(b, enqueue_iter, &b->g_iter))) return rc;
         k_b_publish<<<1, 64, 0, st>>>(b->active, b->h_active_dev, ++b->seq);
         GIP_LAUNCH_CHECK("batch poll");
-        if ((rc = wait_published(st, b->h_active + 1, b->seq))) return rc;
+        if ((rc = wait_published(b->c, b->h_active + 1, b->seq))) return rc;
         if ((int64_t)b->h_active[0] <= 0) break;
     }
     GIP_HIP_TRY(hipEventRecord(b->ev[2], st));
     if ((rc = run_phase(b, enqueue_post, &b->g_post))) return rc;
     GIP_HIP_TRY(hipEventRecord(b->ev[3], st));
-    GIP_HIP_TRY(hipStreamSynchronize(st));
+    GIP_HIP_TRY(drain(b->c));
     for (int k = 0; k < 3; ++k) GIP_HIP_TRY(hipEventElapsedTime(&b->phase_ms[k], b->ev[k], b->ev[k + 1]));
     return GIP_OK;
 }

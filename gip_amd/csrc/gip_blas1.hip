@@ -123,7 +123,7 @@ int launch_reduce(gip_ctx *c, int op, int n, const double *x, const double *y, d
 // command; the reference's PCG sequence makes about 300 such round trips
 // per step: C100K 5.22 -> 4.87 ms per step), then its sequence number.
 static int fetch_result(gip_ctx *c, double *out) {
-    int rc = wait_published(c->stream, reinterpret_cast<const uint64_t *>(c->h_result + kSeqSlot), c->seq);
+    int rc = wait_published(c, reinterpret_cast<const uint64_t *>(c->h_result + kSeqSlot), c->seq);
     if (rc) return rc;
     *out = c->h_result[0];
     return GIP_OK;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include <string>
@@ -74,6 +75,7 @@ struct gip_ctx {
     uint64_t seq, pub_seq;  // last sequence numbers asked for
     std::mutex sync_mu;     // gip_sync: numbers are given out in the order of the launches
     uint64_t sync_seq;
+    std::atomic<bool> published;  // a result was waited for since the stream was last drained (wait_published, drain)
     int num_cu;
 };
 
@@ -166,7 +168,8 @@ int reduce_grid(int n);
 // synchronisation.  Work queued before the kernel has completed when the
 // number arrives.
 constexpr int kHostBlock = 64, kPubSlot = 8, kPubWords = 24, kSeqSlot = 40, kPubSeqSlot = 48, kSyncSlot = 56;  // doubles
-int wait_published(hipStream_t st, const uint64_t *flag, uint64_t want);
+int wait_published(gip_ctx *c, const uint64_t *flag, uint64_t want);
+hipError_t drain(gip_ctx *c);  // hipStreamSynchronize
 __device__ inline void publish_seq(uint64_t *flag, uint64_t seq) {
     __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }

@@ -1851,7 +1851,7 @@ static int *h_state(gip_pcg *S) { return reinterpret_cast<int *>(S->h_pub + S_CO
 static Pub next_pub(gip_pcg *S) {
     return Pub{S->h_pub_dev, reinterpret_cast<int *>(S->h_pub_dev + S_COUNT), S->h_flag_dev, ++*S->seq};
 }
-static int wait_pub(gip_pcg *S) { return wait_published(S->ctx->stream, S->h_flag, *S->seq); }
+static int wait_pub(gip_pcg *S) { return wait_published(S->ctx, S->h_flag, *S->seq); }
 
 constexpr int kFixedPoll = 4096;
 

@@ -18,14 +18,23 @@ int hip_fail(hipError_t e, const char *what) {
                      std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// gip_sync's kernel: the host waits for its number as for a result's, so a
-// call after such a result does not drain the stream from the start (dot and
-// gip_sync 21.6 -> 18.3 us, with the stream drained by both 17.8; a kernel and
-// gip_sync 12.6 -> 10.4; a step of 46^3 in two partitions, whose halo
-// exchanges call it, 10.5 -> 7.3 ms).
+// gip_sync's kernel after a published result: the host waits for its number
+// as for the result's, so it does not pay for draining what the result's wait
+// left (dot and gip_sync 21.6 -> 18.3 us, with the stream drained by both
+// 17.8; a step of 46^3 in two partitions, whose halo exchanges call it, 10.5
+// -> 7.3 ms).  With the stream drained since, the runtime's own wait is the
+// cheaper one (an idle stream 0.4 us against 6.1).
 __global__ void k_seq(uint64_t *flag, uint64_t seq) { publish_seq(flag, seq); }
 
-int wait_published(hipStream_t st, const uint64_t *flag, uint64_t want) {
+hipError_t drain(gip_ctx *c) {
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) c->published = false;
+    return e;
+}
+
+int wait_published(gip_ctx *c, const uint64_t *flag, uint64_t want) {
+    const hipStream_t st = c->stream;
+    c->published = true;
     if (seq_reached(flag, want)) return GIP_OK;
     // a captured kernel does not run: refused as a wait for the stream is,
     // which also ends the capture (asked while the kernel runs)
@@ -121,6 +130,10 @@ int gip_use_device(int device) {
 
 int gip_sync(gip_ctx *c) {
     if (!c) return set_error(GIP_EINVAL, "null context");
+    if (!c->published || capturing(c->stream)) {
+        GIP_HIP_TRY(drain(c));
+        return GIP_OK;
+    }
     uint64_t want;
     {
         std::lock_guard<std::mutex> lock(c->sync_mu);
@@ -128,7 +141,7 @@ int gip_sync(gip_ctx *c) {
         k_seq<<<1, 1, 0, c->stream>>>(reinterpret_cast<uint64_t *>(c->h_result_dev + kSyncSlot), want);
         GIP_LAUNCH_CHECK("gip_sync");
     }
-    return wait_published(c->stream, reinterpret_cast<const uint64_t *>(c->h_result + kSyncSlot), want);
+    return wait_published(c, reinterpret_cast<const uint64_t *>(c->h_result + kSyncSlot), want);
 }
 
 void *gip_stream(gip_ctx *c) { return c ? (void *)c->stream : nullptr; }
@@ -144,7 +157,7 @@ int gip_malloc(gip_ctx *c, size_t bytes, void **dptr) {
 int gip_free(gip_ctx *c, void *dptr) {
     if (!c) return set_error(GIP_EINVAL, "null context");
     if (!dptr) return GIP_OK;
-    GIP_HIP_TRY(hipStreamSynchronize(c->stream));
+    GIP_HIP_TRY(drain(c));
     GIP_HIP_TRY(hipFree(dptr));
     return GIP_OK;
 }
@@ -153,7 +166,7 @@ int gip_memcpy_h2d(gip_ctx *c, void *dst, const void *src, size_t bytes) {
     if (!c || (bytes && (!dst || !src))) return set_error(GIP_EINVAL, "null argument");
     if (!bytes) return GIP_OK;
     GIP_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
-    GIP_HIP_TRY(hipStreamSynchronize(c->stream));  // the host buffer may be reused at return
+    GIP_HIP_TRY(drain(c));  // the host buffer may be reused at return
     return GIP_OK;
 }
 
@@ -161,7 +174,7 @@ int gip_memcpy_d2h(gip_ctx *c, void *dst, const void *src, size_t bytes) {
     if (!c || (bytes && (!dst || !src))) return set_error(GIP_EINVAL, "null argument");
     if (!bytes) return GIP_OK;
     GIP_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-    GIP_HIP_TRY(hipStreamSynchronize(c->stream));
+    GIP_HIP_TRY(drain(c));
     return GIP_OK;
 }
 

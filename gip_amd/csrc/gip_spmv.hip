@@ -893,7 +893,7 @@ int gip_mat_get_values(const gip_mat *A, double *host) {
     int rc = values_csr_order(A, tmp);
     if (!rc) {
         hipError_t e = hipMemcpyAsync(host, tmp, sizeof(double) * A->nnz, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        if (e == hipSuccess) e = drain(c);
         if (e != hipSuccess) rc = hip_fail(e, "gip_mat_get_values");
     }
     hipFree(tmp);
@@ -914,7 +914,7 @@ int gip_mat_set_values(gip_mat *A, const double *host) {
             k_scatter_vals<<<nblocks(A->nnz), kBlock, 0, c->stream>>>(A->nnz, tmp, A->d_csr2ell, A->d_ell_val);
             e = hipGetLastError();
         }
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        if (e == hipSuccess) e = drain(c);
         if (e != hipSuccess) {
             hipFree(tmp);
             return hip_fail(e, "gip_mat_set_values");
@@ -923,7 +923,7 @@ int gip_mat_set_values(gip_mat *A, const double *host) {
     } else {
         double *dst = A->format == GIP_FMT_DIAG ? A->d_diag : A->d_val;
         GIP_HIP_TRY(hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, c->stream));
-        GIP_HIP_TRY(hipStreamSynchronize(c->stream));
+        GIP_HIP_TRY(drain(c));
         if (A->d_val32) k_to_f32<<<nblocks(A->nnz), kBlock, 0, c->stream>>>(A->nnz, A->d_val, A->d_val32);
     }
     const hipError_t e = hipGetLastError();

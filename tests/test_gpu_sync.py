@@ -61,3 +61,26 @@ def test_several_threads_wait_on_one_context(dev):
     dev.sync()
     for v in y:
         assert np.array_equal(v.download(), np.full(n, float(calls)))
+
+
+def test_an_idle_stream_costs_no_kernel(dev):
+    """After a copy to the host, which drains the stream, the call returns at once (0.4 us; a kernel and its wait
+    6.1); after a host result it waits for a kernel of its own (6.4 more than the result, the runtime's wait 9.6)."""
+    import time
+
+    x = dev.to_device(np.ones(1000))
+
+    def best(call, reps=300):
+        times = []
+        for _ in range(5):
+            t0 = time.perf_counter()
+            for _ in range(reps):
+                call()
+            times.append((time.perf_counter() - t0) / reps)
+        return 1e6 * min(times)
+
+    x.download()
+    idle = best(dev.sync)
+    one, both = best(lambda: hip.dot(x, x)), best(lambda: (hip.dot(x, x), dev.sync()))
+    print(f"[gip_sync] idle {idle:.2f} us, dot {one:.2f}, dot and gip_sync {both:.2f}", flush=True)
+    assert idle < 3.0 and both - one < 8.5
